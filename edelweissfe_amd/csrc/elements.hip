@@ -1,6 +1,7 @@
 // Element, material and assembly kernels for gfx950.
 //
-// element_kernel: one 64-lane wavefront owns EPW elements.
+// hex8_kernel (hexa8) is described at its definition; element_kernel (hexa20) follows the same
+// three phases, one 64-lane wavefront owning EPW elements.
 //   phase 1, one lane per (element, QP): Jacobian from the gathered node
 //            coordinates and the shape-function derivatives at the reference's
 //            evaluation point, dN/dx, strain increment from the gathered dU,
@@ -24,6 +25,7 @@
 //   (nonlinearimplicitstatic.py:843-844) in element order.  No atomics: the
 //   result is bitwise reproducible.
 #include <cstdlib>
+#include <type_traits>
 
 #include "efe_internal.h"
 #include "materials.h"
@@ -34,6 +36,31 @@ template <int MAT>
 struct MatState {
     static constexpr int n = (MAT == EFE_LINEAR_ELASTIC) ? 0 : 1;
 };
+
+// The compact tangent of QP q of element e for the matrix-free product, from cc = [A, B, cnn, cn1,
+// c1n, n]: ncw = 8 [A, B, cnn, n] or 10 [A, B, cnn, cn1, c1n, n] (cn1 = c1n = 0 but DP) values, the
+// coefficients times f = w detJ; n is deviatoric (n_33 = -n_11 - n_22): its five other components
+// are stored.
+template <typename CT>
+__device__ __forceinline__ void store_compact(CT* __restrict__ mfC, int E, int e, int q, int ncw, double f, const double (&cc)[11]) {
+    const int64_t stride = E;
+    CT* dc = mfC + (int64_t)q * ncw * E + e;
+    *dc = (CT)(f * cc[0]);
+    dc += stride;
+    dc[0] = (CT)(f * cc[1]);
+    dc[stride] = (CT)(f * cc[2]);
+    dc += 2 * stride;
+    if (ncw == 10) {
+        dc[0] = (CT)(f * cc[3]);
+        dc[stride] = (CT)(f * cc[4]);
+        dc += 2 * stride;
+    }
+    dc[0] = (CT)cc[5];
+    dc[stride] = (CT)cc[6];
+    dc[2 * stride] = (CT)cc[8];
+    dc[3 * stride] = (CT)cc[9];
+    dc[4 * stride] = (CT)cc[10];
+}
 
 // MF (matrix-free form, KT = float): phase 1 also stores the compact tangent
 // w detJ [A, B, cnn, (cn1, c1n,)] and the deviatoric n (five components) per QP for the
@@ -50,7 +77,8 @@ __global__ __launch_bounds__(64) void element_kernel(int E, int N, const double*
                                                      const double* __restrict__ dU,
                                                      const double* __restrict__ sRef, double* __restrict__ sTmp,
                                                      KT* __restrict__ Kscr, double* __restrict__ Pscr,
-                                                     int* __restrict__ status, float* __restrict__ mfC,
+                                                     int* __restrict__ status,
+                                                     float* __restrict__ mfC,
                                                      int* __restrict__ specStatus,
                                                      const int32_t* __restrict__ specOfElem,
                                                      const int32_t* __restrict__ cpos,
@@ -58,7 +86,7 @@ __global__ __launch_bounds__(64) void element_kernel(int E, int N, const double*
                                                      const int32_t* __restrict__ elist, int ecount, int ncw) {
     constexpr int NS = 12 + MatState<MAT>::n;
     constexpr int NP = (MAT == EFE_LINEAR_ELASTIC) ? 2 : 6;
-    // the tangent of every QP in compact form, w detJ [A, B, c_nn, (c_n1, c_1n)] then n:
+    // the tangent of every QP in compact form, w detJ [A - B/3, B/2, c_nn, (c_n1, c_1n)] then n:
     // C = A 1(x)1 + B Idev + c_nn n(x)n (+ c_n1 n(x)1 + c_1n 1(x)n for Drucker-Prager)
     constexpr int NCC = (MAT == EFE_DRUCKER_PRAGER) ? 11 : 9;
     __shared__ double g_s[EPW][Q * NN * 3];
@@ -153,15 +181,7 @@ __global__ __launch_bounds__(64) void element_kernel(int E, int N, const double*
             *status = 1;
             if (specStatus) specStatus[specOfElem[e]] = 1;  // which specimen asked (batched contexts)
         }
-        if (MF && formK) {  // ncw = 8 [A, B, cnn, n] or 10 [A, B, cnn, cn1, c1n, n] (cn1 = c1n = 0 but DP);
-            // n is deviatoric (n_33 = -n_11 - n_22): its five other components are stored
-            const double fq = det * qpw[q];
-            float* dc = mfC + (int64_t)q * ncw * E + e;
-            for (int k = 0; k < ncw - 5; ++k) dc[(int64_t)k * E] = (float)(fq * cc[k]);
-            const int nk[5] = {0, 1, 3, 4, 5};
-#pragma unroll
-            for (int k = 0; k < 5; ++k) dc[(int64_t)(ncw - 5 + k) * E] = (float)cc[5 + nk[k]];
-        }
+        if (mfC && formK) store_compact(mfC, E, e, q, ncw, det * qpw[q], cc);
 #pragma unroll
         for (int c = 0; c < 6; ++c) {
             sTmp[c * EQ + sidx] = s[c];
@@ -171,8 +191,10 @@ __global__ __launch_bounds__(64) void element_kernel(int E, int N, const double*
         (void)NS;
         const double f = det * qpw[q];
         if (formK) {
+            fC_s[el][q * NCC + 0] = (KT)(f * (cc[0] - cc[1] * (1.0 / 3.0)));
+            fC_s[el][q * NCC + 1] = (KT)(f * (0.5 * cc[1]));
 #pragma unroll
-            for (int k = 0; k < NCC - 6; ++k) fC_s[el][q * NCC + k] = (KT)(f * cc[k]);
+            for (int k = 2; k < NCC - 6; ++k) fC_s[el][q * NCC + k] = (KT)(f * cc[k]);
 #pragma unroll
             for (int k = 0; k < 6; ++k) fC_s[el][q * NCC + NCC - 6 + k] = (KT)cc[5 + k];
         }
@@ -186,15 +208,10 @@ __global__ __launch_bounds__(64) void element_kernel(int E, int N, const double*
     constexpr bool SYM = !MF && MAT != EFE_DRUCKER_PRAGER;
     constexpr int NB = MF ? NN : (SYM ? NN * (NN + 1) / 2 : NN * NN);  // blocks per element formed here
     // a residual-only pass (formK = 0) leaves the tangent blocks alone
-    // Lanes take an element's blocks one after the other.  (Taking the EPW elements of one
-    // block position side by side, so that the stores form runs of adjacent blocks, was
-    // measured 8 % slower at 64^3 with per-lane stores, as the tangent reads lose their
-    // broadcast, and no faster with the staged stores below.)  The assembled
+    // Lanes take an element's blocks one after the other.  The assembled
     // passes write their blocks through LDS, kStage blocks (and their transposes) at a time:
     // the wavefront then stores consecutive words, about seven 72-byte blocks per store
-    // instruction instead of one scattered block per lane.  Measured on the 64^3 hexa8 J2
-    // tangent pass: 1.00 ms with per-lane stores, 0.95 / 0.91 / 0.88 / 0.95 ms staging 8 / 16 /
-    // 32 / 64 blocks (0.53 ms with no block stores at all); 48^3 hexa20R DP: 2.34 -> 2.27 ms.
+    // instruction instead of one scattered block per lane (48^3 hexa20R DP: 2.34 -> 2.27 ms).
     const int ntask = formK ? EPW * NB : 0;
     for (int t0 = 0; t0 < ntask; t0 += 64) {
         const int t = t0 + lane;
@@ -214,45 +231,41 @@ __global__ __launch_bounds__(64) void element_kernel(int E, int N, const double*
             b = r0 - a * NN;
         }
         const int e = t < ntask ? elem(el) : -1;
-        KT acc[9];
+        KT acc[9], tr = (KT)0;
 #pragma unroll
         for (int k = 0; k < 9; ++k) acc[k] = (KT)0;
         if (e >= 0) {
             for (int q = 0; q < Q; ++q) {
                 const KT ax = (KT)g_s[el][(q * NN + a) * 3 + 0], ay = (KT)g_s[el][(q * NN + a) * 3 + 1], az = (KT)g_s[el][(q * NN + a) * 3 + 2];
                 const KT bx = (KT)g_s[el][(q * NN + b) * 3 + 0], by = (KT)g_s[el][(q * NN + b) * 3 + 1], bz = (KT)g_s[el][(q * NN + b) * 3 + 2];
-                // CB[:, j] = C B_b e_j from the compact tangent: the strain of column j has the
-                // normal component b_j and two engineering shears (12/13, 12/23, 13/23)
+                // the block as in hex8_kernel: lambda = A - B/3, mu = B/2 and h = n g
                 const KT* cq = fC_s[el] + q * NCC;
-                const KT cA = cq[0], cB = cq[1], cnn = cq[2];
-                const KT cn1 = NCC == 11 ? cq[3] : (KT)0, c1n = NCC == 11 ? cq[4] : (KT)0;
+                const KT lam = cq[0], mu = cq[1], cnn = cq[2];
                 const KT* n = cq + NCC - 6;
-                const KT bv[3] = {bx, by, bz};
-                KT CB[6][3];
+                const KT av[3] = {ax, ay, az}, bv[3] = {bx, by, bz};
+                const KT ha[3] = {n[0] * ax + n[3] * ay + n[4] * az, n[3] * ax + n[1] * ay + n[5] * az,
+                                  n[4] * ax + n[5] * ay + n[2] * az};
+                const KT hb[3] = {n[0] * bx + n[3] * by + n[4] * bz, n[3] * bx + n[1] * by + n[5] * bz,
+                                  n[4] * bx + n[5] * by + n[2] * bz};
+                KT u[3], v[3], w[3];
 #pragma unroll
-                for (int j = 0; j < 3; ++j) {
-                    KT v[6] = {0, 0, 0, 0, 0, 0};
-                    v[j] = bv[j];
-                    if (j == 0) { v[3] = by; v[4] = bz; }
-                    if (j == 1) { v[3] = bx; v[5] = bz; }
-                    if (j == 2) { v[4] = bx; v[5] = by; }
-                    const KT tr = bv[j];
-                    KT ne = n[j] * bv[j];
-#pragma unroll
-                    for (int k = 3; k < 6; ++k) ne += n[k] * v[k];
-                    const KT sn = cnn * ne + cn1 * tr, s1 = cA * tr + c1n * ne, t3 = tr * (KT)(1.0 / 3.0);
-#pragma unroll
-                    for (int i = 0; i < 3; ++i) CB[i][j] = s1 + cB * (v[i] - t3) + sn * n[i];
-#pragma unroll
-                    for (int k = 3; k < 6; ++k) CB[k][j] = (KT)0.5 * cB * v[k] + sn * n[k];
+                for (int i = 0; i < 3; ++i) {
+                    u[i] = lam * av[i];
+                    v[i] = cnn * ha[i];
+                    w[i] = mu * av[i];
+                    if (NCC == 11) {
+                        u[i] += cq[3] * ha[i];
+                        v[i] += cq[4] * av[i];
+                    }
                 }
+                tr += w[0] * bx + w[1] * by + w[2] * bz;
 #pragma unroll
-                for (int j = 0; j < 3; ++j) {
-                    acc[0 + j] += ax * CB[0][j] + ay * CB[3][j] + az * CB[4][j];
-                    acc[3 + j] += ay * CB[1][j] + ax * CB[3][j] + az * CB[5][j];
-                    acc[6 + j] += az * CB[2][j] + ax * CB[4][j] + ay * CB[5][j];
-                }
+                for (int i = 0; i < 3; ++i)
+#pragma unroll
+                    for (int j = 0; j < 3; ++j) acc[i * 3 + j] += u[i] * bv[j] + v[i] * hb[j] + w[j] * bv[i];
             }
+#pragma unroll
+            for (int i = 0; i < 3; ++i) acc[i * 4] += tr;
         }
         if (MF) {  // K_aa element-major at the start of the scratch: [e][a][9]
             if (e >= 0) store_block(Kscr + ((int64_t)e * NN + a) * kBlockPitch, acc);
@@ -309,6 +322,378 @@ __global__ __launch_bounds__(64) void element_kernel(int E, int N, const double*
         dst[2] = -p2;
     }
     __syncthreads();  // the LDS tiles are refilled by the next round
+    }
+}
+
+// ---- hexa8 passes --------------------------------------------------------------------------------
+//
+// One wavefront takes 8 elements, lane 8 el + j standing for node j, QP j and block row j of element
+// el in turn:
+//   fields   each lane loads one node (its coordinates and increment: every node of an element once,
+//            not once per QP); three butterfly steps over the lanes of an element turn the nodal
+//            values into the coefficients of 1, x, y, xy, ... (the trilinear field in monomials), and
+//            a natural gradient at a QP then takes 9 FMA instead of 24;
+//   QP       J^-1, strain increment, material update; loads of the state start before the fields;
+//   forces   M = w detJ sigma J^-T of every QP to LDS; lane a sums M_q grad N_a(q) over the QPs;
+//   blocks   g_a = grad N_a and h_a = n g_a of every QP to LDS; lane a accumulates the blocks
+//            (a, a + o), o = 0..4 for a symmetric tangent (36 blocks of the 64, o = 4 for a < 4),
+//            four passes of two o otherwise.  With C = A 1(x)1 + B Idev + cnn n(x)n + cn1 n(x)1 +
+//            c1n 1(x)n, lambda = A - B/3, mu = B/2:
+//              K_ab = sum_q (lambda g_a + cn1 h_a) g_b^T + (c1n g_a + cnn h_a) h_b^T
+//                     + mu (g_b g_a^T + (g_a . g_b) I),
+//            30 FMA per block and QP (the 6x6 form took about 100), the factors of g_a and h_a
+//            formed once per lane and QP for all its blocks.
+// What bounds it: the blocks' scattered 72-byte stores (1.2 GB at 64^3 in FP64) and, with 210 VGPRs
+// and 26 KB of LDS a wavefront, 6 wavefronts per CU to hide the gathers behind; the residual pass moves
+// 0.49 GB at 4.2 TB/s.  64^3 J2, one lane per (element, QP) with table gradients before -> now:
+// residual pass 221 -> 117 us (3 wavefronts per SIMD; held to 128 VGPRs it spills and takes 133), FP64
+// tangent pass 865 -> 630, FP32 731 -> 411, matrix-free 225 -> 184; linear elastic FP64 828 -> 540;
+// Drucker-Prager FP64 985 -> 878.
+//
+// The QP evaluated at (eta_q, xi_q, zeta_q) of the table lies in the octant of node q, so a
+// lane's sign pattern serves it as node and as QP.
+
+// value of the lane whose number differs in bit H (1, 2 or 4) of the lane number
+template <int H>
+__device__ __forceinline__ double lane_xor8(double v) {
+    int lo = __double2loint(v), hi = __double2hiint(v);
+    if constexpr (H == 1) {  // quad_perm [1, 0, 3, 2]
+        lo = __builtin_amdgcn_update_dpp(0, lo, 0xB1, 0xF, 0xF, true);
+        hi = __builtin_amdgcn_update_dpp(0, hi, 0xB1, 0xF, 0xF, true);
+    } else if constexpr (H == 2) {  // quad_perm [2, 3, 0, 1]
+        lo = __builtin_amdgcn_update_dpp(0, lo, 0x4E, 0xF, 0xF, true);
+        hi = __builtin_amdgcn_update_dpp(0, hi, 0x4E, 0xF, 0xF, true);
+    } else {  // row_half_mirror (xor 7), then quad_perm [3, 2, 1, 0] (xor 3)
+        lo = __builtin_amdgcn_update_dpp(0, lo, 0x141, 0xF, 0xF, true);
+        hi = __builtin_amdgcn_update_dpp(0, hi, 0x141, 0xF, 0xF, true);
+        lo = __builtin_amdgcn_update_dpp(0, lo, 0x1B, 0xF, 0xF, true);
+        hi = __builtin_amdgcn_update_dpp(0, hi, 0x1B, 0xF, 0xF, true);
+    }
+    return __hiloint2double(hi, lo);
+}
+
+// value of lane 0 of the 8 lanes of an element
+__device__ __forceinline__ double lane_first8(double v, bool upper) {
+    int lo = __double2loint(v), hi = __double2hiint(v);
+    lo = __builtin_amdgcn_update_dpp(0, lo, 0x00, 0xF, 0xF, true);  // lane 0 of each quad
+    hi = __builtin_amdgcn_update_dpp(0, hi, 0x00, 0xF, 0xF, true);
+    const int lm = __builtin_amdgcn_update_dpp(0, lo, 0x141, 0xF, 0xF, true);  // row_half_mirror
+    const int hm = __builtin_amdgcn_update_dpp(0, hi, 0x141, 0xF, 0xF, true);
+    return __hiloint2double(upper ? hm : hi, upper ? lm : lo);
+}
+
+// octant of node (and QP) j: node numbers run (-,-,-) (-,-,+) (+,-,+) (+,-,-), then the same with +y
+__host__ __device__ constexpr bool oct_x(int j) { return (j & 2) != 0; }
+__host__ __device__ constexpr bool oct_y(int j) { return j >= 4; }
+__host__ __device__ constexpr bool oct_z(int j) { return (j & 3) == 1 || (j & 3) == 2; }
+
+template <int MAT, typename KT, bool MF, bool TAN>
+struct Hex8Lds {
+    static constexpr bool SYM = MAT != EFE_DRUCKER_PRAGER;
+    static constexpr int NSC = SYM ? 3 : 5;                 // factors per QP: lambda, mu, cnn (, cn1, c1n)
+    static constexpr int QS = 6 * 64 + 1;                   // pitch of a QP's g and h: the lanes of a store, 8
+                                                            // QPs of 8 elements, spread over the banks
+    static constexpr int kBlocks = SYM ? 288 : 128;         // blocks staged for the stores at a time
+    static constexpr size_t fields = 6 * 64 * sizeof(double), forces = 9 * 64 * sizeof(double);
+    static constexpr size_t grads = TAN ? (8 * QS + 8 * 8 * NSC) * sizeof(KT) : 0;
+    static constexpr size_t stage = TAN && !MF ? kBlocks * (9 * sizeof(KT) + (SYM ? 2 : 1) * sizeof(int)) : 0;
+    static constexpr size_t ab = fields > forces ? fields : forces;
+    // one pass: the blocks take the place of g and h; two: g and h stay for the second
+    static constexpr size_t stageAt = SYM ? 0 : (grads + 7) / 8 * 8;
+    static constexpr size_t cd = grads > stageAt + stage ? grads : stageAt + stage;
+    static constexpr size_t bytes = ab > cd ? ab : cd;
+};
+
+template <int MAT, typename KT, bool MF, bool TAN>
+__global__ __launch_bounds__(64) void hex8_kernel(
+    int E, int N, const double* __restrict__ coords, const int32_t* __restrict__ conn,
+    const double* __restrict__ props, int propStride, const double* __restrict__ dU,
+    const double* __restrict__ sRef, double* __restrict__ sTmp, KT* __restrict__ Kscr, double* __restrict__ Pscr,
+    int* __restrict__ status, KT* __restrict__ mfC, int* __restrict__ specStatus,
+    const int32_t* __restrict__ specOfElem, const int32_t* __restrict__ cpos, const int* __restrict__ specActive,
+    const int32_t* __restrict__ elist, int ecount, int ncw) {
+    using L = Hex8Lds<MAT, KT, MF, TAN>;
+    constexpr int NP = (MAT == EFE_LINEAR_ELASTIC) ? 2 : 6;
+    constexpr bool HAS_K = MatState<MAT>::n != 0;
+    __shared__ __align__(16) char lds[L::bytes];
+    const int lane = threadIdx.x, el = lane >> 3, j = lane & 7;
+    const int64_t EQ = (int64_t)E * 8;
+    int e = -1;  // -1 past the end and, in batched contexts, for specimens the pass skips
+    {
+        const int i = blockIdx.x * 8 + el;
+        if (i < ecount) {
+            e = elist ? elist[i] : i;
+            if (specActive && !specActive[specOfElem[e]]) e = -1;
+        }
+    }
+    const bool live = e >= 0;
+    const int64_t sidx = (int64_t)(live ? e : 0) * 8 + j;
+    double s[6], eps[6], ms = 0.0;
+#pragma unroll
+    for (int c = 0; c < 6; ++c) s[c] = eps[c] = 0.0;
+    double w[6] = {0, 0, 0, 0, 0, 0};
+    if (live) {
+        const int nd = conn[(int64_t)((0x65217430u >> (4 * j)) & 7) * E + e];  // the node of octant bits j
+#pragma unroll
+        for (int c = 0; c < 6; ++c) s[c] = sRef[c * EQ + sidx];
+#pragma unroll
+        for (int c = 0; c < 6; ++c) eps[c] = sRef[(6 + c) * EQ + sidx];
+        if (HAS_K) ms = sRef[12 * EQ + sidx];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            w[c] = coords[(int64_t)c * N + nd];
+            w[3 + c] = dU[3 * (int64_t)nd + c];
+        }
+    }
+    {
+        const double s1 = (j & 1) ? -1.0 : 1.0, s2 = (j & 2) ? -1.0 : 1.0, s4 = (j & 4) ? -1.0 : 1.0;
+        double* cf = (double*)lds;
+#pragma unroll
+        for (int c = 0; c < 6; ++c) {
+            // lanes with the bit set take own - other, the others own + other
+            // (values relative to the first node, so that round-off goes with the element's own scale)
+            double v = w[c] - lane_first8(w[c], (j & 4) != 0);
+            v = fma(s1, lane_xor8<1>(v), v);
+            v = fma(s2, lane_xor8<2>(v), v);
+            v = fma(s4, lane_xor8<4>(v), v);
+            cf[c * 64 + lane] = 0.125 * v;
+        }
+    }
+    __syncthreads();
+    const double g0 = 0.57735026918962576451;
+    const double x = oct_x(j) ? g0 : -g0, y = oct_y(j) ? g0 : -g0, z = oct_z(j) ? g0 : -g0;
+    double J[9], H[9];
+    {
+        const double* cf = (const double*)lds + el * 8;
+        const double xy = x * y, yz = y * z, xz = x * z;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const double* cx = cf + i * 64;
+            const double* cu = cf + (3 + i) * 64;
+            // d/dx = c1 + c3 y + c5 z + c7 yz, d/dy = c2 + c3 x + c6 z + c7 xz, d/dz = c4 + c5 x + c6 y + c7 xy
+            J[0 * 3 + i] = cx[1] + cx[3] * y + cx[5] * z + cx[7] * yz;
+            J[1 * 3 + i] = cx[2] + cx[3] * x + cx[6] * z + cx[7] * xz;
+            J[2 * 3 + i] = cx[4] + cx[5] * x + cx[6] * y + cx[7] * xy;
+            H[i * 3 + 0] = cu[1] + cu[3] * y + cu[5] * z + cu[7] * yz;
+            H[i * 3 + 1] = cu[2] + cu[3] * x + cu[6] * z + cu[7] * xz;
+            H[i * 3 + 2] = cu[4] + cu[5] * x + cu[6] * y + cu[7] * xy;
+        }
+    }
+    const double det = J[0] * (J[4] * J[8] - J[5] * J[7]) - J[1] * (J[3] * J[8] - J[5] * J[6]) +
+                       J[2] * (J[3] * J[7] - J[4] * J[6]);  // the Gauss weights are 1
+    const double id = live ? 1.0 / det : 0.0;
+    const double iJ[9] = {(J[4] * J[8] - J[5] * J[7]) * id, (J[2] * J[7] - J[1] * J[8]) * id,
+                          (J[1] * J[5] - J[2] * J[4]) * id, (J[5] * J[6] - J[3] * J[8]) * id,
+                          (J[0] * J[8] - J[2] * J[6]) * id, (J[2] * J[3] - J[0] * J[5]) * id,
+                          (J[3] * J[7] - J[4] * J[6]) * id, (J[1] * J[6] - J[0] * J[7]) * id,
+                          (J[0] * J[4] - J[1] * J[3]) * id};
+    double cc[11];
+#pragma unroll
+    for (int k = 0; k < 11; ++k) cc[k] = 0.0;
+    if (live) {
+        double gr[9];  // d u_i / d x_k
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+                gr[i * 3 + k] = H[i * 3] * iJ[k * 3] + H[i * 3 + 1] * iJ[k * 3 + 1] + H[i * 3 + 2] * iJ[k * 3 + 2];
+        const double de[6] = {gr[0], gr[4], gr[8], gr[1] + gr[3], gr[2] + gr[6], gr[5] + gr[7]};
+        double p[NP];
+#pragma unroll
+        for (int k = 0; k < NP; ++k) p[k] = propStride ? props[(int64_t)k * propStride + e] : props[k];
+        double C[36];
+        int st = 0;
+        if (MAT == EFE_LINEAR_ELASTIC) st = efe::le_update(p, s, de, C, cc);
+        else if (MAT == EFE_VONMISES) st = efe::vm_update(p, s, ms, de, C, cc);
+        else st = efe::dp_update(p, s, ms, de, C, cc);
+        if (st) {
+            *status = 1;
+            if (specStatus) specStatus[specOfElem[e]] = 1;  // which specimen asked (batched contexts)
+        }
+#pragma unroll
+        for (int c = 0; c < 6; ++c) {
+            sTmp[c * EQ + sidx] = s[c];
+            sTmp[(6 + c) * EQ + sidx] = eps[c] + de[c];
+        }
+        if (HAS_K) sTmp[12 * EQ + sidx] = ms;
+        if (TAN && mfC) store_compact(mfC, E, e, j, ncw, det, cc);
+    }
+    // reference gradients of an octant pair: t*(b)[c] = (1 +- g s)(1 +- g s) / 8 of the two other axes
+    double tx[2][2], ty[2][2], tz[2][2];
+    {
+        const double px[2] = {1.0 - x, 1.0 + x}, py[2] = {1.0 - y, 1.0 + y}, pz[2] = {1.0 - z, 1.0 + z};
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                tx[a][b] = 0.125 * py[a] * pz[b];
+                ty[a][b] = 0.125 * px[a] * pz[b];
+                tz[a][b] = 0.125 * px[a] * py[b];
+            }
+    }
+    // forces
+    double* Ms = (double*)lds;
+    __syncthreads();  // the coefficients have been read
+    {
+        const double S[9] = {s[0], s[3], s[4], s[3], s[1], s[5], s[4], s[5], s[2]};
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+                Ms[el * 72 + (i * 3 + k) * 8 + j] =
+                    det * (S[i * 3] * iJ[k] + S[i * 3 + 1] * iJ[3 + k] + S[i * 3 + 2] * iJ[6 + k]);
+    }
+    __syncthreads();
+    {
+        const double sx = oct_x(j) ? 1.0 : -1.0, sy = oct_y(j) ? 1.0 : -1.0, sz = oct_z(j) ? 1.0 : -1.0;
+        double f[3] = {0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const double* M = Ms + el * 72 + i * 24;
+            double fx = 0, fy = 0, fz = 0;
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                fx += M[q] * tx[oct_y(q)][oct_z(q)];
+                fy += M[8 + q] * ty[oct_x(q)][oct_z(q)];
+                fz += M[16 + q] * tz[oct_x(q)][oct_y(q)];
+            }
+            f[i] = sx * fx + sy * fy + sz * fz;
+        }
+        if (live) {
+            double* dst = Pscr + ((int64_t)e * 8 + j) * 3;
+            dst[0] = -f[0];
+            dst[1] = -f[1];
+            dst[2] = -f[2];
+        }
+    }
+    if constexpr (TAN) {
+        __syncthreads();
+        KT* gh = (KT*)lds;
+        KT* sc = gh + 8 * L::QS;
+        {
+            const double nn[9] = {cc[5], cc[8], cc[9], cc[8], cc[6], cc[10], cc[9], cc[10], cc[7]};
+#pragma unroll
+            for (int a = 0; a < 8; ++a) {
+                const double d0 = oct_x(a) ? tx[oct_y(a)][oct_z(a)] : -tx[oct_y(a)][oct_z(a)];
+                const double d1 = oct_y(a) ? ty[oct_x(a)][oct_z(a)] : -ty[oct_x(a)][oct_z(a)];
+                const double d2 = oct_z(a) ? tz[oct_x(a)][oct_y(a)] : -tz[oct_x(a)][oct_y(a)];
+                double g[3];
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    g[c] = iJ[c * 3] * d0 + iJ[c * 3 + 1] * d1 + iJ[c * 3 + 2] * d2;
+                    gh[j * L::QS + c * 64 + el * 8 + a] = (KT)g[c];
+                }
+                if (MAT != EFE_LINEAR_ELASTIC)
+#pragma unroll
+                    for (int c = 0; c < 3; ++c)
+                        gh[j * L::QS + (3 + c) * 64 + el * 8 + a] =
+                            (KT)(nn[c * 3] * g[0] + nn[c * 3 + 1] * g[1] + nn[c * 3 + 2] * g[2]);
+            }
+            KT* d = sc + (j * 8 + el) * L::NSC;
+            d[0] = (KT)(det * (cc[0] - cc[1] * (1.0 / 3.0)));
+            d[1] = (KT)(det * (0.5 * cc[1]));
+            d[2] = (KT)(det * cc[2]);
+            if (!L::SYM) {
+                d[L::NSC - 2] = (KT)(det * cc[3]);
+                d[L::NSC - 1] = (KT)(det * cc[4]);
+            }
+        }
+        __syncthreads();
+        constexpr int NO = MF ? 1 : (L::SYM ? 5 : 2);  // blocks per lane and pass
+        constexpr int NPASS = MF || L::SYM ? 1 : 4;
+#pragma unroll 1
+        for (int pass = 0; pass < NPASS; ++pass) {
+            KT acc[NO][9], tr[NO];
+#pragma unroll
+            for (int o = 0; o < NO; ++o) {
+                tr[o] = (KT)0;
+#pragma unroll
+                for (int k = 0; k < 9; ++k) acc[o][k] = (KT)0;
+            }
+#pragma unroll 1
+            for (int q = 0; q < 8; ++q) {
+                const KT* gq = gh + q * L::QS + el * 8;
+                const KT* d = sc + (q * 8 + el) * L::NSC;
+                KT u[3], v[3], wv[3];
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    const KT ga = gq[c * 64 + j];
+                    u[c] = d[0] * ga;
+                    wv[c] = d[1] * ga;
+                    if (MAT != EFE_LINEAR_ELASTIC) {
+                        const KT ha = gq[(3 + c) * 64 + j];
+                        v[c] = d[2] * ha;
+                        if (!L::SYM) {
+                            u[c] += d[L::NSC - 2] * ha;
+                            v[c] += d[L::NSC - 1] * ga;
+                        }
+                    }
+                }
+#pragma unroll
+                for (int o = 0; o < NO; ++o) {
+                    const int b = (j + o + pass * NO) & 7;
+                    KT gb[3], hb[3];
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) {
+                        gb[c] = gq[c * 64 + b];
+                        if (MAT != EFE_LINEAR_ELASTIC) hb[c] = gq[(3 + c) * 64 + b];
+                    }
+                    tr[o] += wv[0] * gb[0] + wv[1] * gb[1] + wv[2] * gb[2];
+#pragma unroll
+                    for (int i = 0; i < 3; ++i)
+#pragma unroll
+                        for (int k = 0; k < 3; ++k) {
+                            KT t = acc[o][i * 3 + k] + u[i] * gb[k] + wv[k] * gb[i];
+                            if (MAT != EFE_LINEAR_ELASTIC) t += v[i] * hb[k];
+                            acc[o][i * 3 + k] = t;
+                        }
+                }
+            }
+#pragma unroll
+            for (int o = 0; o < NO; ++o)
+#pragma unroll
+                for (int i = 0; i < 3; ++i) acc[o][i * 4] += tr[o];
+            if constexpr (MF) {  // K_aa element-major at the start of the scratch: [e][a][9]
+                if (live) store_block(Kscr + ((int64_t)e * 8 + j) * kBlockPitch, acc[0]);
+            } else {
+                // the blocks, then their positions (and those of the transposes, -1: none), in LDS; the
+                // wavefront stores them word by word, about seven 72-byte blocks per instruction
+                KT* stg = (KT*)(lds + L::stageAt);
+                int* pos = (int*)(stg + L::kBlocks * 9);
+                const int32_t* cp = cpos + (int64_t)(live ? e : 0) * 64;
+                int p0[NO], p1[NO];
+#pragma unroll
+                for (int o = 0; o < NO; ++o) {
+                    const int b = (j + o + pass * NO) & 7;
+                    const bool mine = live && (!L::SYM || o < 4 || j < 4);
+                    p0[o] = mine ? cp[j * 8 + b] : -1;
+                    p1[o] = L::SYM && mine && o ? cp[b * 8 + j] : -1;
+                }
+                __syncthreads();  // g and h have been read
+#pragma unroll
+                for (int o = 0; o < NO; ++o) {
+                    if (L::SYM && o == 4 && j >= 4) continue;
+                    // slots 0..255: the offsets 0..3; 256..287: offset 4 of the lanes j < 4
+                    const int slot = o < 4 ? o * 64 + lane : 256 + el * 4 + j;
+#pragma unroll
+                    for (int k = 0; k < 9; ++k) stg[slot * 9 + k] = acc[o][k];
+                    pos[slot] = p0[o];
+                    if (L::SYM) pos[L::kBlocks + slot] = p1[o];
+                }
+                __syncthreads();
+                for (int t = lane; t < L::kBlocks * 9; t += 64) {
+                    const int bi = t / 9, v = t - bi * 9;
+                    const int pb = pos[bi];
+                    if (pb >= 0) Kscr[(int64_t)pb * kBlockPitch + v] = stg[t];
+                    if constexpr (L::SYM) {  // K_ba = K_ab^T
+                        const int pt = pos[L::kBlocks + bi];
+                        const int vt = (v % 3) * 3 + v / 3;
+                        if (pt >= 0) Kscr[(int64_t)pt * kBlockPitch + v] = stg[bi * 9 + vt];
+                    }
+                }
+                if (pass + 1 < NPASS) __syncthreads();  // the staged blocks have been read
+            }
+        }
     }
 }
 
@@ -424,15 +809,15 @@ __global__ __launch_bounds__(256) void assemble_kernel(
     }
 }
 
-// assemble_kernel with the element scratch read run by run: the wavefront of a slice loads
-// contribution run j (the j-th contribution of its 64 rows, 64 contiguous blocks) with nine
-// coalesced 512-byte loads (FP64), stages it in LDS and each lane takes its own block from
-// there, loading run j + 1 meanwhile.  Every line of the scratch is fetched once (the per-lane
-// nine-load form re-fetched lines its wavefronts had in flight when they were evicted).  The
-// lanes walk their rows' contributions in the same order, so K, Minv, P, F and the correction are
-// bitwise those of assemble_kernel.
-template <typename KT>
-__global__ __launch_bounds__(256) void assemble_runs_kernel(
+// assemble_kernel with the element scratch read run by run and the row's blocks shared out over W
+// wavefronts: a workgroup takes one slice, wavefront w the w-th part of every row's blocks.  It loads
+// each contribution run of its part (the j-th contributions of the 64 rows, 64 contiguous blocks)
+// with nine coalesced 512-byte loads (FP64), stages it in LDS and each lane takes its own block
+// from there, loading the next run meanwhile.  A block is summed by one lane in the order of
+// assemble_kernel, so K and Minv are bitwise the same for every W; P and F are summed by the last
+// wavefront, the correction from the W parts in order.
+template <typename KT, int W>
+__global__ __launch_bounds__(64 * W) void assemble_runs_kernel(
     int N, const int32_t* __restrict__ bptr, const int32_t* __restrict__ bcol, const int32_t* __restrict__ coff,
     const int32_t* __restrict__ nptr, const int32_t* __restrict__ nlist,
     const int32_t* __restrict__ slice_off, const KT* __restrict__ Kscr, const double* __restrict__ Pscr,
@@ -441,17 +826,16 @@ __global__ __launch_bounds__(256) void assemble_runs_kernel(
     const int32_t* __restrict__ slotNode, const int32_t* __restrict__ cslice, const int* __restrict__ specActive,
     const int32_t* __restrict__ specOfNode) {
     constexpr int RUN = 9 * kSlice;  // values of one contribution run
-    __shared__ KT runbuf[256 / kSlice][RUN];
+    __shared__ KT runbuf[W][RUN];
     const int per = gridDim.x >> 3;
-    const int blk = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-    const int ps = blk * blockDim.x + threadIdx.x;
-    const int s = ps / kSlice, l = ps - (ps / kSlice) * kSlice;  // one slice per wavefront: l is the lane
-    if (s * kSlice >= N) return;                                  // the whole wavefront
-    KT* buf = runbuf[threadIdx.x / kSlice];
+    const int s = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (s * kSlice >= N) return;  // the whole workgroup
+    const int l = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int ps = s * kSlice + l;
+    KT* buf = runbuf[wv];
     const bool valid = ps < N;
     const int n = valid ? slotNode[ps] : 0;
     const bool work = valid && !(specActive && !specActive[specOfNode[n]]);
-    if (valid && !work && dirv) dircorr[3 * n] = dircorr[3 * n + 1] = dircorr[3 * n + 2] = 0.0;
     bool fr[3] = {false, false, false};
     if (work && ndir) {
         fr[0] = dirflag[3 * n];
@@ -460,36 +844,48 @@ __global__ __launch_bounds__(256) void assemble_runs_kernel(
     }
     double t0 = 0, t1 = 0, t2 = 0;
     double dg[9] = {1, 0, 0, 0, 1, 0, 0, 0, 1};
+    bool haveDiag = false;
     const int64_t vbase = (int64_t)slice_off[s] * 9 + l;
-    int b0 = 0, b = 0, b1 = 0, c0 = 0, cnt = 0, cend = 0;
+    int b0 = 0, b = 0, b1 = 0, c0 = 0, c1 = 0, cend = 0;  // this part's blocks [b, b1), contributions [c0, c1)
     if (work) {
-        b0 = b = bptr[n];
-        b1 = bptr[n + 1];
-        c0 = coff[b0];
-        cnt = coff[b1] - c0;
-        cend = coff[b + 1] - c0;
+        b0 = bptr[n];
+        const int deg = bptr[n + 1] - b0;
+        b = b0 + deg * wv / W;
+        b1 = b0 + deg * (wv + 1) / W;
+        const int first = coff[b0];
+        c0 = coff[b] - first;
+        c1 = coff[b1] - first;
+        if (b < b1) cend = coff[b + 1] - first;
     }
     KT acc[9];
 #pragma unroll
     for (int v = 0; v < 9; ++v) acc[v] = (KT)0;
-    const int J = cslice[s + 1] - cslice[s];
-    if (__any(work)) {
+    // the runs of this part over the 64 rows (rows of one kind, the same for all)
+    int jlo = c0 < c1 ? c0 : 0x7fffffff, jhi = c1;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        jlo = min(jlo, __shfl_xor(jlo, o, 64));
+        jhi = max(jhi, __shfl_xor(jhi, o, 64));
+    }
+    jlo = __builtin_amdgcn_readfirstlane(jlo);
+    jhi = __builtin_amdgcn_readfirstlane(jhi);
+    if (jlo < jhi) {
         const KT* runs = Kscr + (int64_t)cslice[s] * RUN;
         KT nxt[9];
 #pragma unroll
-        for (int t = 0; t < 9; ++t) nxt[t] = J > 0 ? runs[t * kSlice + l] : (KT)0;
-        for (int j = 0; j < J; ++j) {
+        for (int t = 0; t < 9; ++t) nxt[t] = __builtin_nontemporal_load(runs + (int64_t)jlo * RUN + t * kSlice + l);
+        for (int j = jlo; j < jhi; ++j) {
 #pragma unroll
             for (int t = 0; t < 9; ++t) buf[t * kSlice + l] = nxt[t];
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            if (j + 1 < J) {
+            if (j + 1 < jhi) {
                 const KT* nr = runs + (int64_t)(j + 1) * RUN;
 #pragma unroll
                 for (int t = 0; t < 9; ++t) nxt[t] = __builtin_nontemporal_load(nr + t * kSlice + l);
             }
-            if (work && j < cnt) {
+            if (j >= c0 && j < c1) {
 #pragma unroll
                 for (int v = 0; v < 9; ++v) acc[v] += buf[l * 9 + v];
                 if (j + 1 == cend) {  // the last contribution of block b: finish it
@@ -512,13 +908,14 @@ __global__ __launch_bounds__(256) void assemble_runs_kernel(
 #pragma unroll
                     for (int v = 0; v < 9; ++v) Kval[vbase + (int64_t)(k * 9 + v) * kSlice] = acc[v];
                     if (m == n) {
+                        haveDiag = true;
 #pragma unroll
                         for (int v = 0; v < 9; ++v) dg[v] = (double)acc[v];
                     }
 #pragma unroll
                     for (int v = 0; v < 9; ++v) acc[v] = (KT)0;
                     ++b;
-                    if (b < b1) cend = coff[b + 1] - c0;
+                    if (b < b1) cend = coff[b + 1] - coff[b0];
                 }
             }
             // every lane has read its block before the next run overwrites the buffer
@@ -527,12 +924,13 @@ __global__ __launch_bounds__(256) void assemble_runs_kernel(
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         }
     }
-    if (!work) return;
-    double iv[9];
-    inv3(dg, iv);
+    if (work && haveDiag) {
+        double iv[9];
+        inv3(dg, iv);
 #pragma unroll
-    for (int v = 0; v < 9; ++v) Minv[(int64_t)n * 9 + v] = (KT)iv[v];
-    if (P) {
+        for (int v = 0; v < 9; ++v) Minv[(int64_t)n * 9 + v] = (KT)iv[v];
+    }
+    if (work && P && wv == W - 1) {
         double p0 = 0, p1 = 0, p2 = 0, f0 = 0, f1 = 0, f2 = 0;
 #pragma unroll 4
         for (int c = nptr[n]; c < nptr[n + 1]; ++c) {
@@ -552,9 +950,22 @@ __global__ __launch_bounds__(256) void assemble_runs_kernel(
         F[3 * n + 2] = f2;
     }
     if (dirv) {
-        dircorr[3 * n] = fr[0] ? 0.0 : t0;
-        dircorr[3 * n + 1] = fr[1] ? 0.0 : t1;
-        dircorr[3 * n + 2] = fr[2] ? 0.0 : t2;
+        double(*sum)[3][64] = (double(*)[3][64])runbuf;  // [W][3][64], within the run buffers
+        static_assert(sizeof(runbuf) >= (size_t)W * 3 * 64 * sizeof(double), "the parts' sums fit");
+        __syncthreads();
+        sum[wv][0][l] = t0;
+        sum[wv][1][l] = t1;
+        sum[wv][2][l] = t2;
+        __syncthreads();
+        if (wv == 0 && valid) {
+            // a skipped specimen's increment is not solved: its correction is zero
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                double t = 0;
+                for (int k = 0; k < W; ++k) t += sum[k][i][l];
+                dircorr[3 * n + i] = !work || fr[i] ? 0.0 : t;
+            }
+        }
     }
 }
 
@@ -792,24 +1203,42 @@ void launch_elem_t(efe_ctx* c, const double* dU) {
 
 template <int NN, int Q, int MAT, typename KT>
 int launch_elem_epw(efe_ctx* c, const double* dU) {
-    // default: hexa8 4 (assembled passes) or 8 (matrix-free and residual-only passes: phase 1,
-    // one lane per element and QP, then fills the wavefront; 64^3: matrix-free 0.34 against
-    // 0.51 ms, residual-only 0.27 against 0.34 ms), hexa20R 2, hexa20 1
+    // default: hexa20R 2, hexa20 1
     int epw = c->epw;
-    if (epw <= 0) epw = (NN == 8) ? ((c->mfPass || !c->formK) ? 8 : 4) : (Q == 8 ? 2 : 1);
+    if (epw <= 0) epw = Q == 8 ? 2 : 1;
     switch (epw) {
         case 1: launch_elem_t<NN, Q, MAT, KT, 1>(c, dU); break;
         case 2: launch_elem_t<NN, Q, MAT, KT, 2>(c, dU); break;
-        case 4:
-            if (NN == 8) { launch_elem_t<NN, Q, MAT, KT, (NN == 8 ? 4 : 1)>(c, dU); break; }
-            [[fallthrough]];
-        case 8:
-            if (NN == 8 && Q == 8) { launch_elem_t<NN, Q, MAT, KT, (NN == 8 && Q == 8 ? 8 : 1)>(c, dU); break; }
-            [[fallthrough]];
         default:
             efe_set_error("elements per workgroup must be 1, 2, 4 or 8 (hexa20: 1 or 2)");
             return EFE_ERR_ARG;
     }
+    return EFE_OK;
+}
+
+// hexa8: 8 elements per wavefront whatever is set (of the choices there are)
+template <int MAT, typename KT>
+int launch_hex8(efe_ctx* c, const double* dU) {
+    if (c->epw > 0 && c->epw != 1 && c->epw != 2 && c->epw != 4 && c->epw != 8) {
+        efe_set_error("elements per workgroup must be 1, 2, 4 or 8 (hexa20: 1 or 2)");
+        return EFE_ERR_ARG;
+    }
+    const int grid = (c->curCount + 7) / 8;
+    if (grid == 0) return EFE_OK;
+    const int propStride = c->props_per_element ? c->E : 0;
+    const int* act = c->useActive ? c->specActive : nullptr;
+#define HEX8_ARGS(T, C)                                                                                            \
+    c->E, c->N, c->coords, c->conn, c->props, propStride, dU, c->stateRef, c->stateTmp, (T*)c->Kscr, c->Pscr,         \
+        c->status, C, c->specStatus, c->specOfElem, c->cpos, act, c->curList, c->curCount, c->mfNC
+    if (!c->formK)
+        hex8_kernel<MAT, double, false, false><<<grid, 64, 0, c->stream>>>(HEX8_ARGS(double, (double*)nullptr));
+    else if (c->mfPass)
+        hex8_kernel<MAT, float, true, true><<<grid, 64, 0, c->stream>>>(HEX8_ARGS(float, c->mfC));
+    else if constexpr (sizeof(KT) == 8)
+        hex8_kernel<MAT, double, false, true><<<grid, 64, 0, c->stream>>>(HEX8_ARGS(double, (double*)nullptr));
+    else
+        hex8_kernel<MAT, float, false, true><<<grid, 64, 0, c->stream>>>(HEX8_ARGS(float, (float*)nullptr));
+#undef HEX8_ARGS
     return EFE_OK;
 }
 
@@ -827,7 +1256,14 @@ int launch_elem_mat(efe_ctx* c, const double* dU) {
 template <typename KT>
 int launch_elem_type(efe_ctx* c, const double* dU) {
     switch (c->eltype) {
-        case EFE_C3D8: return launch_elem_mat<8, 8, KT>(c, dU);
+        case EFE_C3D8:
+            switch (c->curMat) {
+                case EFE_LINEAR_ELASTIC: return launch_hex8<EFE_LINEAR_ELASTIC, KT>(c, dU);
+                case EFE_VONMISES: return launch_hex8<EFE_VONMISES, KT>(c, dU);
+                case EFE_DRUCKER_PRAGER: return launch_hex8<EFE_DRUCKER_PRAGER, KT>(c, dU);
+            }
+            efe_set_error("unknown material");
+            return EFE_ERR_ARG;
         case EFE_C3D20: return launch_elem_mat<20, 27, KT>(c, dU);
         case EFE_C3D20R: return launch_elem_mat<20, 8, KT>(c, dU);
     }
@@ -871,10 +1307,22 @@ int efe_launch_assembly(efe_ctx* c, double* P, double* F, const double* dir_valu
     c->N, c->bptr, c->bcol, c->coff, c->nptr, c->nlist, c->slice_off, (const KT*)c->Kscr, c->Pscr, c->dirflag,       \
         c->ndir, dir_values, dir_correction, K, M, P, F, c->slotNode, c->cslice, c->useActive ? c->specActive : nullptr, \
         c->specOfNode
-        if (precision == EFE_FP32)
-            assemble_runs_kernel<float><<<grid, bs, 0, c->stream>>>(ASM_ARGS(float, c->K32, c->Minv32));
-        else
-            assemble_runs_kernel<double><<<grid, bs, 0, c->stream>>>(ASM_ARGS(double, c->K64, c->Minv64));
+#define ASM_LAUNCH(W)                                                                                                  \
+    do {                                                                                                               \
+        if (precision == EFE_FP32)                                                                                     \
+            assemble_runs_kernel<float, W><<<gs, 64 * W, 0, c->stream>>>(ASM_ARGS(float, c->K32, c->Minv32));          \
+        else                                                                                                           \
+            assemble_runs_kernel<double, W><<<gs, 64 * W, 0, c->stream>>>(ASM_ARGS(double, c->K64, c->Minv64));        \
+    } while (0)
+        const int gs = (c->nslices + 7) & ~7;
+        // a row's contributions are one dependent walk (80 to 160 runs in hexa20): 8 wavefronts per
+        // slice take it in parts, 4 where the slices alone fill the chip and the values are FP64.
+        // At 1 / 4 / 8 / 16 wavefronts: 525 nodes 55 / 36 / 31 / 37 us, hexa20 17 x 15 x 13 148 / 103 /
+        // 100 / 121 us, 64^3 hexa8 477 / 468 / 473 / 494 us, FP32 373 / 287 / 275 / 301 us (one wavefront
+        // per slice and four slices per workgroup before: 67, 186, 520 and 390 us).
+        if (precision == EFE_FP64 && c->nslices >= 1536) ASM_LAUNCH(4);
+        else ASM_LAUNCH(8);
+#undef ASM_LAUNCH
 #undef ASM_ARGS
         EFE_HIP(hipGetLastError());
         c->Kprec = precision;

@@ -361,8 +361,8 @@ int efe_collect_results(efe_ctx* ctx, int32_t which, const int32_t* elements, in
  * zero (the initial state of a fresh model, element.py:207-240). */
 int efe_set_qp_state(efe_ctx* ctx, const double* in);
 
-/* Elements per workgroup of the element kernel and threads per workgroup of the
- * Krylov kernels; 0 keeps the current choice. */
+/* Elements per workgroup of the element kernel (hexa20; hexa8 passes take 8 whatever of 1, 2, 4
+ * and 8 is set) and threads per workgroup of the Krylov kernels; 0 keeps the current choice. */
 int efe_set_launch(efe_ctx* ctx, int32_t elements_per_workgroup, int32_t krylov_block);
 
 /* Device times (ms) measured with HIP events on the context's streams (host out[16]):
