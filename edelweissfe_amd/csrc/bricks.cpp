@@ -1,0 +1,235 @@
+// Bricks of the hexa8 matrix-free operator (matfree.hip): the elements grouped into compact
+// workgroup-sized sets, with every index table the product needs.
+//
+// A product stages each brick's distinct nodes once and writes one partial force per (brick,
+// node), so its traffic beyond the tangents goes with the nodes per element of a brick: 2.5 for
+// 256 consecutive elements of a box in lattice order (two thin slabs of nodes), 1.6 for the
+// 8 x 8 x 4 sets found here.  The elements are split recursively across the longest side
+// (measured in mean element sizes), at a gap between layers of elements where there is one, at
+// the position that needs the fewest bricks, else nearest the middle; a set is a brick once it
+// has at most kBrick elements and kBrickNodes staged nodes, whatever the mesh.
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+#include <future>
+#include <system_error>
+
+#include "efe_internal.h"
+
+namespace {
+
+struct Splitter {
+    const std::vector<float>& cen;  // [3][E] element centroids in mean element sizes
+    std::vector<int32_t>& order;    // element indices, rearranged in place
+    int E;
+
+    // Splits [lo, hi) of the order and returns the position of the cut.
+    int cut(int lo, int hi, std::vector<int32_t>& bins, std::vector<int32_t>& tmp) const {
+        const int n = hi - lo;
+        float mn[3] = {3e38f, 3e38f, 3e38f}, mx[3] = {-3e38f, -3e38f, -3e38f};
+        for (int i = lo; i < hi; ++i)
+            for (int k = 0; k < 3; ++k) {
+                const float v = cen[(size_t)k * E + order[i]];
+                mn[k] = std::min(mn[k], v);
+                mx[k] = std::max(mx[k], v);
+            }
+        int ax = 0;
+        for (int k = 1; k < 3; ++k)
+            if (mx[k] - mn[k] > 1.001f * (mx[ax] - mn[ax])) ax = k;
+        const float ext = mx[ax] - mn[ax];
+        if (!(ext > 0.0f)) return lo + n / 2;  // coincident centroids: the order as it is
+        const float* c = cen.data() + (size_t)ax * E;
+        const int nb = std::min(4096, std::max(64, 4 * n));
+        const float scale = (float)nb / ext;
+        auto bin = [&](int e) {
+            const float f = (c[e] - mn[ax]) * scale;
+            return f >= (float)(nb - 1) ? nb - 1 : (f > 0.0f ? (int)f : 0);
+        };
+        bins.assign(nb + 1, 0);
+        for (int i = lo; i < hi; ++i) ++bins[bin(order[i]) + 1];
+        for (int b = 0; b < nb; ++b) bins[b + 1] += bins[b];  // bins[b]: elements before bin b
+        int best = -1;
+        int64_t bestCost = INT64_MAX;
+        for (int b = 1; b < nb; ++b) {
+            const int l = bins[b];
+            if (4 * (int64_t)l < n || 4 * (int64_t)l > 3 * (int64_t)n) continue;
+            const bool gap = bins[b + 1] == l;  // an empty bin: between two layers
+            const int64_t bricks = (l + kBrick - 1) / kBrick + (n - l + kBrick - 1) / kBrick;
+            const int64_t cost = ((gap ? 0 : 1) * (int64_t)(E + 1) + bricks) * (int64_t)(n + 1) + std::abs(2 * l - n);
+            if (cost < bestCost) {
+                bestCost = cost;
+                best = b;
+            }
+        }
+        if (best < 0) {  // most centroids in one bin: halve by position
+            std::nth_element(order.begin() + lo, order.begin() + lo + n / 2, order.begin() + hi,
+                             [&](int32_t a, int32_t b) { return c[a] != c[b] ? c[a] < c[b] : a < b; });
+            return lo + n / 2;
+        }
+        tmp.clear();
+        int w = lo;
+        for (int i = lo; i < hi; ++i) {
+            const int32_t e = order[i];
+            if (bin(e) < best) order[w++] = e;
+            else tmp.push_back(e);
+        }
+        std::copy(tmp.begin(), tmp.end(), order.begin() + w);
+        return w;
+    }
+};
+
+// the tables of one brick; entries are moved into the global tables afterwards
+struct Brick {
+    int lo = 0, hi = 0;
+    std::vector<int32_t> nodes;   // staged nodes (a node with more than 8 incidences repeats)
+    std::vector<uint16_t> linc;   // [nodes][8] incidences a * kBrick + t, 0xffff: none
+    std::vector<uint16_t> lidx;   // [elements][8]
+};
+
+// Fills the tables of the elements order[lo, hi); false when more than kBrickNodes are staged.
+bool fill(Brick& b, const std::vector<int32_t>& order, const int32_t* conn, std::vector<int32_t>& scratch) {
+    const int ne = b.hi - b.lo;
+    scratch.clear();
+    for (int t = 0; t < ne; ++t)
+        for (int a = 0; a < 8; ++a) scratch.push_back(conn[(size_t)order[b.lo + t] * 8 + a]);
+    std::vector<int32_t> sorted(scratch);
+    std::sort(sorted.begin(), sorted.end());
+    b.nodes.clear();
+    for (size_t i = 0; i < sorted.size();) {  // one entry per 8 incidences of a node
+        size_t j = i;
+        while (j < sorted.size() && sorted[j] == sorted[i]) ++j;
+        for (size_t k = i; k < j; k += 8) b.nodes.push_back(sorted[i]);
+        i = j;
+    }
+    if ((int)b.nodes.size() > kBrickNodes) return false;
+    b.linc.assign(b.nodes.size() * 8, 0xffff);
+    b.lidx.resize((size_t)ne * 8);
+    std::vector<uint8_t> fillc(b.nodes.size(), 0);
+    for (int t = 0; t < ne; ++t)  // element order inside every node's list
+        for (int a = 0; a < 8; ++a) {
+            const int32_t nd = scratch[(size_t)t * 8 + a];
+            int l = (int)(std::lower_bound(b.nodes.begin(), b.nodes.end(), nd) - b.nodes.begin());
+            while (fillc[l] == 8) ++l;
+            b.lidx[(size_t)t * 8 + a] = (uint16_t)l;
+            b.linc[(size_t)l * 8 + fillc[l]++] = (uint16_t)(a * kBrick + t);
+        }
+    return true;
+}
+
+// a task of its own thread, or run at get() when there is no thread to be had
+template <typename Fn>
+std::future<void> aside(Fn fn) {
+    try {
+        return std::async(std::launch::async, fn);
+    } catch (const std::system_error&) {
+        return std::async(std::launch::deferred, fn);
+    }
+}
+
+void grow(const Splitter& sp, int lo, int hi, const int32_t* conn, std::vector<Brick>& out, int depth) {
+    std::vector<int32_t> bins, tmp, scratch;
+    if (hi - lo <= kBrick) {
+        Brick b;
+        b.lo = lo;
+        b.hi = hi;
+        std::sort(sp.order.begin() + lo, sp.order.begin() + hi);
+        if (fill(b, sp.order, conn, scratch)) {
+            out.push_back(std::move(b));
+            return;
+        }
+    }
+    const int mid = sp.cut(lo, hi, bins, tmp);
+    if (depth > 0 && hi - lo > 8192) {  // the two halves side by side
+        std::vector<Brick> right;
+        std::future<void> f = aside([&] { grow(sp, mid, hi, conn, right, depth - 1); });
+        grow(sp, lo, mid, conn, out, depth - 1);
+        f.get();
+        out.insert(out.end(), std::make_move_iterator(right.begin()), std::make_move_iterator(right.end()));
+        return;
+    }
+    grow(sp, lo, mid, conn, out, 0);
+    grow(sp, mid, hi, conn, out, 0);
+}
+
+}  // namespace
+
+void efe_build_bricks(BrickPattern& bp, int N, int E, const int32_t* conn, const double* coords,
+                      const int32_t* specOfNode) {
+    // centroids in mean element sizes
+    std::vector<float> cen((size_t)3 * E);
+    double lo3[3], size[3] = {0, 0, 0};
+    for (int k = 0; k < 3; ++k) lo3[k] = coords[k];
+    for (int n = 1; n < N; ++n)
+        for (int k = 0; k < 3; ++k) lo3[k] = std::min(lo3[k], coords[(size_t)3 * n + k]);
+    for (int e = 0; e < E; ++e)
+        for (int k = 0; k < 3; ++k) {
+            double mn = coords[(size_t)3 * conn[(size_t)8 * e] + k], mx = mn, s = 0.0;
+            for (int a = 0; a < 8; ++a) {
+                const double v = coords[(size_t)3 * conn[(size_t)8 * e + a] + k];
+                mn = std::min(mn, v);
+                mx = std::max(mx, v);
+                s += v;
+            }
+            size[k] += mx - mn;
+            cen[(size_t)k * E + e] = (float)(s * 0.125 - lo3[k]);
+        }
+    for (int k = 0; k < 3; ++k) {
+        const double h = size[k] / E;
+        if (h > 0.0 && std::isfinite(h))
+            for (int e = 0; e < E; ++e) cen[(size_t)k * E + e] = (float)(cen[(size_t)k * E + e] / h);
+    }
+    bp.order.resize(E);
+    for (int e = 0; e < E; ++e) bp.order[e] = e;
+    std::vector<int> seg;  // a brick holds elements of one specimen
+    if (specOfNode) {
+        auto spec = [&](int e) { return specOfNode[conn[(size_t)8 * e]]; };
+        std::stable_sort(bp.order.begin(), bp.order.end(), [&](int32_t a, int32_t b) { return spec(a) < spec(b); });
+        for (int i = 0; i < E; ++i)
+            if (i == 0 || spec(bp.order[i]) != spec(bp.order[i - 1])) seg.push_back(i);
+    } else {
+        seg.push_back(0);
+    }
+    seg.push_back(E);
+    Splitter sp{cen, bp.order, E};
+    std::vector<Brick> bricks;
+    if (seg.size() == 2) {
+        grow(sp, 0, E, conn, bricks, 3);
+    } else {  // specimens shared out over threads, collected in specimen order
+        const int ns = (int)seg.size() - 1, nt = std::min(8, ns);
+        std::vector<std::vector<Brick>> per(ns);
+        std::vector<std::future<void>> th;
+        for (int t = 0; t < nt; ++t)
+            th.push_back(aside([&, t] {
+                for (int s = t; s < ns; s += nt) grow(sp, seg[s], seg[s + 1], conn, per[s], 0);
+            }));
+        for (auto& x : th) x.get();
+        for (auto& v : per)
+            bricks.insert(bricks.end(), std::make_move_iterator(v.begin()), std::make_move_iterator(v.end()));
+    }
+    const int G = (int)bricks.size();
+    bp.e0.assign(1, 0);
+    bp.lptr.assign(1, 0);
+    for (const Brick& b : bricks) {
+        bp.e0.push_back(b.hi);
+        bp.lptr.push_back(bp.lptr.back() + (int32_t)b.nodes.size());
+    }
+    const size_t L = bp.lptr.back();
+    bp.pos.resize(E);
+    bp.lnode.resize(L);
+    bp.lpos.resize(L);
+    bp.linc.resize(L * 8);
+    bp.lidx.resize((size_t)E * 8);
+    bp.pptr.assign(N + 1, 0);
+    for (int g = 0; g < G; ++g) {
+        const Brick& b = bricks[g];
+        std::copy(b.nodes.begin(), b.nodes.end(), bp.lnode.begin() + bp.lptr[g]);
+        std::copy(b.linc.begin(), b.linc.end(), bp.linc.begin() + (size_t)bp.lptr[g] * 8);
+        std::copy(b.lidx.begin(), b.lidx.end(), bp.lidx.begin() + (size_t)b.lo * 8);
+        for (int i = b.lo; i < b.hi; ++i) bp.pos[bp.order[i]] = g * kBrick + (i - b.lo);
+        for (int32_t nd : b.nodes) ++bp.pptr[nd + 1];
+    }
+    // partial slots in node order, the bricks of a node in ascending order
+    for (int n = 0; n < N; ++n) bp.pptr[n + 1] += bp.pptr[n];
+    std::vector<int32_t> next(bp.pptr.begin(), bp.pptr.end() - 1);
+    for (size_t i = 0; i < L; ++i) bp.lpos[i] = next[bp.lnode[i]]++;
+}

@@ -2,7 +2,9 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <future>
 #include <string>
+#include <system_error>
 #include <utility>
 #include <vector>
 
@@ -160,6 +162,9 @@ int efe_prepare_elements(efe_ctx* c, int precision) {
     }
     if (precision == EFE_FP32_MATFREE)
         if (int rc = efe_mf_alloc(c)) return rc;
+    // the FP64 CG on hexa8 with a symmetric tangent runs on the bricks (krylov.hip)
+    if (precision == EFE_FP64 && c->eltype == EFE_C3D8 && c->mfNC != 10)
+        if (int rc = efe_mf_alloc_bricks(c, true)) return rc;
     return EFE_OK;
 }
 
@@ -229,10 +234,31 @@ int efe_ctx_create(const efe_mesh_desc* d, efe_ctx** out) {
         c->groupMat[0] = c->material;
         c->groupCount[0] = c->E;
     }
-    c->mfNC = (mat_of ? mat_count[EFE_DRUCKER_PRAGER] > 0 : d->material == EFE_DRUCKER_PRAGER) ? 10 : 8;
+    const bool anyDP = mat_of ? mat_count[EFE_DRUCKER_PRAGER] > 0 : d->material == EFE_DRUCKER_PRAGER;
+    const bool allLE = mat_of ? mat_count[EFE_LINEAR_ELASTIC] == d->n_elements : d->material == EFE_LINEAR_ELASTIC;
+    c->mfNC = anyDP ? 10 : (NN == 20 ? 8 : (allLE ? 0 : 7));
     c->stream = (hipStream_t)d->stream;
     c->nspec = d->specimen_of_node ? d->n_specimens : 1;
     std::string err;
+    for (int64_t i = 0; i < (int64_t)c->E * NN; ++i)
+        if (d->conn[i] < 0 || d->conn[i] >= c->N) {
+            efe_set_error("connectivity references a node outside [0, n_nodes)");
+            delete c;
+            return EFE_ERR_ARG;
+        }
+    // the bricks of the matrix-free product, beside the pattern
+    BrickPattern bp;
+    std::future<void> bricks;
+    if (c->eltype == EFE_C3D8) {
+        auto build = [&bp, N = c->N, E = c->E, conn = d->conn, xyz = d->coords, spec = d->specimen_of_node] {
+            efe_build_bricks(bp, N, E, conn, xyz, spec);
+        };
+        try {
+            bricks = std::async(c->E > 4096 ? std::launch::async : std::launch::deferred, build);
+        } catch (const std::system_error&) {  // no thread to be had: at get(), as for small meshes
+            bricks = std::async(std::launch::deferred, build);
+        }
+    }
     if (!efe_build_pattern(c->hp, c->N, c->E, NN, d->conn, err)) {
         efe_set_error(err);
         delete c;
@@ -364,6 +390,10 @@ int efe_ctx_create(const efe_mesh_desc* d, efe_ctx** out) {
     if ((rc = dalloc((void**)&c->red, (size_t)c->redn * sizeof(double)))) return fail(rc);
     for (auto& ev : c->ev) EFE_HIP(hipEventCreate(&ev));
     EFE_HIP(hipStreamSynchronize(st));
+    if (c->eltype == EFE_C3D8) {
+        bricks.get();
+        if ((rc = efe_mf_upload_bricks(c, bp, d->coords))) return fail(rc);
+    }
     *out = c;
     return EFE_OK;
 }
@@ -428,6 +458,7 @@ int efe_set_dirichlet(efe_ctx* c, const int32_t* dofs, int32_t n) {
     EFE_HIP(hipMemcpyAsync(c->dirflag, f.data(), f.size(), hipMemcpyHostToDevice, c->stream));
     EFE_HIP(hipStreamSynchronize(c->stream));
     c->ndir = n;
+    ++c->dirVersion;
     return EFE_OK;
 }
 
@@ -457,6 +488,7 @@ int efe_compute_elements(efe_ctx* c, const double* U, const double* dU, const do
     EFE_HIP(hipEventRecord(c->ev[2], c->stream));
     c->kscrValid = precision != EFE_FP32_MATFREE;
     c->pscrValid = true;
+    if (precision == EFE_FP64 && !c->useActive) c->mf64Dir = c->dirVersion;  // a pass over some specimens keeps it
     int hs = 0;
     EFE_HIP(hipMemcpyAsync(&hs, c->status, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     EFE_HIP(hipStreamSynchronize(c->stream));

@@ -62,6 +62,27 @@ struct HostPattern {
     int64_t padded_blocks = 0;
 };
 
+// Bricks of the hexa8 matrix-free operator: at most kBrick elements and kBrickNodes staged nodes.
+constexpr int kBrick = 256;
+constexpr int kBrickNodes = 512;
+
+struct BrickPattern {
+    std::vector<int32_t> e0;      // [G+1] first element (of `order`) of each brick
+    std::vector<int32_t> order;   // [E] elements brick by brick, ascending inside a brick
+    std::vector<int32_t> pos;     // [E] element -> brick * kBrick + its place in the brick
+    std::vector<int32_t> lptr;    // [G+1] first staged node of each brick
+    std::vector<int32_t> lnode;   // [L] node of each staged entry (a node with more than 8 incidences
+                                  // in a brick has several entries)
+    std::vector<int32_t> lpos;    // [L] its slot among the node's partials
+    std::vector<int32_t> pptr;    // [N+1] partials of each node, in brick order
+    std::vector<uint16_t> linc;   // [L][8] incidences a * kBrick + t in element order, 0xffff: none
+    std::vector<uint16_t> lidx;   // [E][8] staged entries of the elements of `order`
+};
+
+// conn [E][8], coords [N][3], specOfNode [N] or null (a brick then holds one specimen's elements)
+void efe_build_bricks(BrickPattern& bp, int N, int E, const int32_t* conn, const double* coords,
+                      const int32_t* specOfNode);
+
 // Multicolor block ILU(0) structure (rows in elimination order = (color, node)).
 struct IluPattern {
     int ncolors = 0;
@@ -117,26 +138,33 @@ struct efe_ctx {
     double* dJdxi = nullptr;     // [Q][NN][3] the table J is formed with (hexa20: the reference's third row)
     double* shapeN = nullptr;    // [Q][NN] at the table points (body force)
     double* shapeNe = nullptr;   // [Q][NN] at the evaluation points (QP coordinates)
-    // matrix-free FP32 operator: [Q][NC][E] compact tangent, [E*NN][3] node-sorted force slots,
-    // dnxi32 = FP32 dNdxi then dJdxi ([2][Q][NN][3])
+    // matrix-free FP32 operator of hexa20: [Q][NC][E] compact tangent, [E*NN][3] node-sorted force
+    // slots, dnxi32 = FP32 dNdxi then dJdxi ([2][Q][NN][3]).  hexa8 (bricks): mfC / mfC64
+    // [brick][Q][NC][kBrick] compact tangents of the last FP32 matrix-free / FP64 tangent pass
     float *mfC = nullptr, *mfF = nullptr, *dnxi32 = nullptr;
-    // hexa8 matrix-free operator by workgroup bricks (256 consecutive elements): per workgroup its
-    // local nodes (lptr [G+1] into lnode / lpos / lincp), per local node its partial-force slot in
-    // node order (lpos) and its element-node incidences t*8+a (linc, element order, from lincp);
-    // per element its 8 local node indices (lidx); per node its partial range (pptr [N+1]) in
-    // the partial forces mfbF [L][3]
+    double* mfC64 = nullptr;
+    // hexa8 bricks (bricks.cpp): BrickPattern's tables on the device, the staged nodes'
+    // coordinates, and the partial forces [L][3] in the precision of the product
     bool mfb = false;
-    int mfbG = 0;                // workgroups (bricks); in batched contexts a brick holds one specimen's elements
-    int32_t* mfbE0 = nullptr;    // [G+1] first element of each brick
-    int32_t *mfbLptr = nullptr, *mfbLnode = nullptr, *mfbLpos = nullptr, *mfbLincp = nullptr, *mfbPptr = nullptr;
+    int mfbG = 0;                // bricks
+    int64_t mfbL = 0;            // staged nodes over all bricks
+    void* mfbTables = nullptr;   // one allocation: the tables below
+    int32_t *mfbE0 = nullptr, *mfbOrder = nullptr, *mfbPos = nullptr;
+    int32_t *mfbLptr = nullptr, *mfbLnode = nullptr, *mfbLpos = nullptr, *mfbPptr = nullptr;
     uint16_t *mfbLinc = nullptr, *mfbLidx = nullptr;
-    float* mfbF = nullptr;
+    double* mfbX = nullptr;      // [3][L]
+    float *mfbEl = nullptr, *mfbF = nullptr;       // [2][G * kBrick] bulk modulus and 2 G; [L][3]
+    double *mfbEl64 = nullptr, *mfbF64 = nullptr;
+    int dirVersion = 0;          // incremented by every efe_set_dirichlet
+    int mf64Dir = -1;            // dirVersion of the pass whose tangents mfC64 holds (-1: none)
     int32_t* elemPos = nullptr;  // [NN][E] index of (e, a) in the node-sorted incidence list nlist
                                  // (force slot of the matrix-free operator; block-row (e, a) of the
                                  // element scratch starts at block elemPos * NN)
     bool mfPass = false;             // the current element launch is a matrix-free pass
-    int mfNC = 8;                    // compact tangent values per QP of the matrix-free operator
-                                     // (10 when a Drucker-Prager section is present)
+    int mfNC = 8;                    // compact tangent values per QP of the matrix-free operator:
+                                     // 10 with a Drucker-Prager section, else 8 (hexa20), 7 (hexa8:
+                                     // A = K det w is formed from the bulk modulus) or 0 (hexa8,
+                                     // linear elastic only)
     // material groups (sections): the element kernel runs once per group over its element list
     int ngroups = 1;
     int groupMat[3] = {0, 0, 0};
@@ -218,8 +246,17 @@ int efe_launch_geostatic(efe_ctx* c, const double* def, const int32_t* elements,
 // matrix-free FP32 operator (matfree.hip)
 int efe_mf_alloc(efe_ctx* c);
 int efe_launch_mf_assembly(efe_ctx* c, double* P, double* F, const double* dir_values, double* dir_correction);
-// hexa8 bricks: the product's node partials (mfbF over mfbPptr) and per-brick partials of p.Kp
-void efe_mf_launch_apply_partials(efe_ctx* c, hipStream_t st, const float* p, double* part, const int* flags);
+// hexa8 bricks: the tables on the device (at creation), and the buffers of FP32 or FP64 products
+int efe_mf_upload_bricks(efe_ctx* c, const BrickPattern& bp, const double* coords);
+int efe_mf_alloc_bricks(efe_ctx* c, bool fp64);
+// whether the FP64 CG may run on the bricks: tangents of the last FP64 pass, Dirichlet set unchanged
+bool efe_mf_bricks64(const efe_ctx* c);
+// hexa8 bricks: the product's node partials (mfbF / mfbF64 over mfbPptr) and per-brick partials of
+// p.Kp; active: per-specimen flags (batched contexts) or null
+void efe_mf_launch_apply_partials(efe_ctx* c, hipStream_t st, const float* p, double* part, const int* flags,
+                                  const int* active = nullptr);
+void efe_mf_launch_apply_partials(efe_ctx* c, hipStream_t st, const double* p, double* part, const int* flags,
+                                  const int* active = nullptr);
 void efe_mf_launch_operator(efe_ctx* c, hipStream_t st, const float* p, float* q, double* part, const int* flags,
                             int nwg, int bs, int kr);
 void efe_mf_free(efe_ctx* c);

@@ -38,15 +38,27 @@ struct MatState {
 };
 
 // The compact tangent of QP q of element e for the matrix-free product, from cc = [A, B, cnn, cn1,
-// c1n, n]: ncw = 8 [A, B, cnn, n] or 10 [A, B, cnn, cn1, c1n, n] (cn1 = c1n = 0 but DP) values, the
-// coefficients times f = w detJ; n is deviatoric (n_33 = -n_11 - n_22): its five other components
-// are stored.
+// c1n, n]: ncw = 8 [A, B, cnn, n], 7 (A left out), 10 [A, B, cnn, cn1, c1n, n] (cn1 = c1n = 0 but
+// DP) or 0 values, the coefficients times f = w detJ; n is deviatoric (n_33 = -n_11 - n_22): its
+// five other components are stored.  Element e lies at its place mfPos in the bricks (hexa8), or in
+// element order.  (Constant indices into cc only: a variable one would put it into scratch memory.)
 template <typename CT>
-__device__ __forceinline__ void store_compact(CT* __restrict__ mfC, int E, int e, int q, int ncw, double f, const double (&cc)[11]) {
-    const int64_t stride = E;
-    CT* dc = mfC + (int64_t)q * ncw * E + e;
-    *dc = (CT)(f * cc[0]);
-    dc += stride;
+__device__ __forceinline__ void store_compact(CT* __restrict__ mfC, const int32_t* __restrict__ mfPos, int E, int Q,
+                                              int e, int q, int ncw, double f, const double (&cc)[11]) {
+    if (!ncw) return;
+    CT* dc;
+    int64_t stride = E;
+    if (mfPos) {
+        const int pos = mfPos[e];
+        stride = kBrick;
+        dc = mfC + ((int64_t)(pos / kBrick) * Q + q) * ncw * kBrick + pos % kBrick;
+    } else {
+        dc = mfC + (int64_t)q * ncw * E + e;
+    }
+    if (ncw != 7) {
+        *dc = (CT)(f * cc[0]);
+        dc += stride;
+    }
     dc[0] = (CT)(f * cc[1]);
     dc[stride] = (CT)(f * cc[2]);
     dc += 2 * stride;
@@ -181,7 +193,7 @@ __global__ __launch_bounds__(64) void element_kernel(int E, int N, const double*
             *status = 1;
             if (specStatus) specStatus[specOfElem[e]] = 1;  // which specimen asked (batched contexts)
         }
-        if (mfC && formK) store_compact(mfC, E, e, q, ncw, det * qpw[q], cc);
+        if (mfC && formK) store_compact(mfC, (const int32_t*)nullptr, E, Q, e, q, ncw, det * qpw[q], cc);
 #pragma unroll
         for (int c = 0; c < 6; ++c) {
             sTmp[c * EQ + sidx] = s[c];
@@ -409,7 +421,7 @@ __global__ __launch_bounds__(64) void hex8_kernel(
     int E, int N, const double* __restrict__ coords, const int32_t* __restrict__ conn,
     const double* __restrict__ props, int propStride, const double* __restrict__ dU,
     const double* __restrict__ sRef, double* __restrict__ sTmp, KT* __restrict__ Kscr, double* __restrict__ Pscr,
-    int* __restrict__ status, KT* __restrict__ mfC, int* __restrict__ specStatus,
+    int* __restrict__ status, KT* __restrict__ mfC, const int32_t* __restrict__ mfPos, int* __restrict__ specStatus,
     const int32_t* __restrict__ specOfElem, const int32_t* __restrict__ cpos, const int* __restrict__ specActive,
     const int32_t* __restrict__ elist, int ecount, int ncw) {
     using L = Hex8Lds<MAT, KT, MF, TAN>;
@@ -516,7 +528,7 @@ __global__ __launch_bounds__(64) void hex8_kernel(
             sTmp[(6 + c) * EQ + sidx] = eps[c] + de[c];
         }
         if (HAS_K) sTmp[12 * EQ + sidx] = ms;
-        if (TAN && mfC) store_compact(mfC, E, e, j, ncw, det, cc);
+        if (TAN && mfC) store_compact(mfC, mfPos, E, 8, e, j, ncw, det, cc);
     }
     // reference gradients of an octant pair: t*(b)[c] = (1 +- g s)(1 +- g s) / 8 of the two other axes
     double tx[2][2], ty[2][2], tz[2][2];
@@ -1229,13 +1241,13 @@ int launch_hex8(efe_ctx* c, const double* dU) {
     const int* act = c->useActive ? c->specActive : nullptr;
 #define HEX8_ARGS(T, C)                                                                                            \
     c->E, c->N, c->coords, c->conn, c->props, propStride, dU, c->stateRef, c->stateTmp, (T*)c->Kscr, c->Pscr,         \
-        c->status, C, c->specStatus, c->specOfElem, c->cpos, act, c->curList, c->curCount, c->mfNC
+        c->status, C, c->mfbPos, c->specStatus, c->specOfElem, c->cpos, act, c->curList, c->curCount, c->mfNC
     if (!c->formK)
         hex8_kernel<MAT, double, false, false><<<grid, 64, 0, c->stream>>>(HEX8_ARGS(double, (double*)nullptr));
     else if (c->mfPass)
         hex8_kernel<MAT, float, true, true><<<grid, 64, 0, c->stream>>>(HEX8_ARGS(float, c->mfC));
     else if constexpr (sizeof(KT) == 8)
-        hex8_kernel<MAT, double, false, true><<<grid, 64, 0, c->stream>>>(HEX8_ARGS(double, (double*)nullptr));
+        hex8_kernel<MAT, double, false, true><<<grid, 64, 0, c->stream>>>(HEX8_ARGS(double, c->mfC64));
     else
         hex8_kernel<MAT, float, false, true><<<grid, 64, 0, c->stream>>>(HEX8_ARGS(float, (float*)nullptr));
 #undef HEX8_ARGS

@@ -22,7 +22,7 @@
 // r.z partial buffers alternate with the iteration parity, so a batch of an even number
 // of iterations is a fixed sequence of launches that is captured once into a hipGraph
 // and replayed.
-// With the hexa8 brick operator (matrix-free FP32), A is the brick product alone, its
+// With the hexa8 brick operator (matrix-free FP32, and FP64), A is the brick product alone, its
 // partials the bricks' shares of p.Kp (Dirichlet DOFs masked), and B gathers each node's
 // brick partials itself (q is never stored): p.q = the bricks' sum + the sum of p^2 over the
 // Dirichlet DOFs, whose partials C (and the init) form with p.
@@ -52,11 +52,11 @@ struct KrylovWork {
     double* hpart = nullptr; // pinned host scalars
     hipStream_t ks = nullptr;
     hipEvent_t evA = nullptr, evB = nullptr, t0 = nullptr, t1 = nullptr;
-    hipGraphExec_t graph[3] = {nullptr, nullptr, nullptr};  // FP64, FP32 assembled, FP32 matrix-free
-    int graph_batch[3] = {0, 0, 0};
-    int graph_block[3] = {0, 0, 0};
+    hipGraphExec_t graph[4] = {};  // FP64 assembled, FP32 assembled, FP32 matrix-free, FP64 bricks
+    int graph_batch[4] = {};
+    int graph_block[4] = {};
     // the operator buffers a batch graph was captured with (a graph keeps their addresses)
-    const void* graph_ops[3][4] = {};
+    const void* graph_ops[4][4] = {};
 };
 
 namespace {
@@ -333,15 +333,15 @@ __global__ __launch_bounds__(BS) void pcg_direction_kernel(int N, const T* __res
     }
 }
 
-// B for the hexa8 brick operator (FP32): p.q = the bricks' partials (nop of them) + the
+// B for the hexa8 brick operator: p.q = the bricks' partials (nop of them) + the
 // Dirichlet p.p partials; q of node n = the sum of its brick partials (in brick order), p on
 // its Dirichlet DOFs, formed here and not stored.
-template <int BS>
-__global__ __launch_bounds__(BS) void pcg_update_mfb_kernel(int N, const float* __restrict__ Minv,
-                                                            float* __restrict__ x, float* __restrict__ r,
-                                                            float* __restrict__ z, const float* __restrict__ p,
+template <typename T, int BS>
+__global__ __launch_bounds__(BS) void pcg_update_mfb_kernel(int N, const T* __restrict__ Minv,
+                                                            T* __restrict__ x, T* __restrict__ r,
+                                                            T* __restrict__ z, const T* __restrict__ p,
                                                             const int32_t* __restrict__ gptr,
-                                                            const float* __restrict__ gF,
+                                                            const T* __restrict__ gF,
                                                             const uint8_t* __restrict__ dirflag,
                                                             double* __restrict__ part, int ps, int nop, int nvec,
                                                             int par, const int* __restrict__ flags, int kr) {
@@ -352,33 +352,33 @@ __global__ __launch_bounds__(BS) void pcg_update_mfb_kernel(int N, const float* 
     double sc[3];
     reduce_partials_nv<BS, 3>(part, offs, ns, sc, sh);
     const double pq = sc[0] + sc[1], rz = sc[2];
-    const float alpha = (float)(rz / pq);
+    const T alpha = (T)(rz / pq);
     const int blk = xcd_block();
     double rzn = 0, rr = 0;
     for (int it = 0; it < kr; ++it) {
         const int n = (blk * kr + it) * BS + threadIdx.x;
         if (n >= N) break;
-        float qv[3] = {0.0f, 0.0f, 0.0f};
+        T qv[3] = {(T)0, (T)0, (T)0};
         const int g0 = gptr[n], g1 = gptr[n + 1];
         for (int c = g0; c < g1; ++c) {
             qv[0] += gF[3 * (int64_t)c];
             qv[1] += gF[3 * (int64_t)c + 1];
             qv[2] += gF[3 * (int64_t)c + 2];
         }
-        float rv[3];
+        T rv[3];
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
-            const float pv = p[3 * n + i];
-            const float q = dirflag[3 * n + i] ? pv : qv[i];
+            const T pv = p[3 * n + i];
+            const T q = dirflag[3 * n + i] ? pv : qv[i];
             x[3 * n + i] += alpha * pv;
             rv[i] = r[3 * n + i] - alpha * q;
             r[3 * n + i] = rv[i];
             rr += (double)rv[i] * rv[i];
         }
-        const float* M = Minv + (int64_t)n * 9;
+        const T* M = Minv + (int64_t)n * 9;
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
-            const float zi = M[3 * i] * rv[0] + M[3 * i + 1] * rv[1] + M[3 * i + 2] * rv[2];
+            const T zi = M[3 * i] * rv[0] + M[3 * i + 1] * rv[1] + M[3 * i + 2] * rv[2];
             z[3 * n + i] = zi;
             rzn += (double)rv[i] * zi;
         }
@@ -565,19 +565,20 @@ __global__ __launch_bounds__(BS) void norms_batched_kernel(const int64_t* __rest
 
 template <typename T, int BS>
 void launch_iter(efe_ctx* c, KrylovWork* w, hipStream_t st, T* x, T* r, T* z, T* p, T* q, const T* K,
-                 const T* Minv, int par, int j) {
+                 const T* Minv, bool bricks, int par, int j) {
     const int grid = w->nwg;
     const int kr = w->kr;
     const int gv = w->nwgv, krv = w->krv;
-    if constexpr (sizeof(T) == 4) {
-        if (!K && c->mfb) {  // hexa8 bricks: the product's partials gathered by the update
-            efe_mf_launch_apply_partials(c, st, p, w->part, w->flags);
-            pcg_update_mfb_kernel<BS><<<gv, BS, 0, st>>>(c->N, Minv, x, r, z, p, c->mfbPptr, c->mfbF, c->dirflag,
-                                                         w->part, w->ps, round8(c->mfbG), gv, par, w->flags, krv);
-            pcg_direction_kernel<T, BS, true><<<gv, BS, 0, st>>>(c->N, z, p, w->part, w->ps, gv, par, j, w->dscal,
-                                                                 w->flags, krv, c->dirflag);
-            return;
-        }
+    if (bricks) {  // hexa8 bricks: the product's partials gathered by the update
+        const T* gF;
+        if constexpr (sizeof(T) == 8) gF = c->mfbF64;
+        else gF = c->mfbF;
+        efe_mf_launch_apply_partials(c, st, p, w->part, w->flags);
+        pcg_update_mfb_kernel<T, BS><<<gv, BS, 0, st>>>(c->N, Minv, x, r, z, p, c->mfbPptr, gF, c->dirflag, w->part,
+                                                        w->ps, round8(c->mfbG), gv, par, w->flags, krv);
+        pcg_direction_kernel<T, BS, true><<<gv, BS, 0, st>>>(c->N, z, p, w->part, w->ps, gv, par, j, w->dscal,
+                                                             w->flags, krv, c->dirflag);
+        return;
     }
     if (K)
         spmv_kernel<T, BS><<<grid, BS, 0, st>>>(c->N, c->slice_off, c->scol, c->slotNode, K, p, q, w->part, w->flags,
@@ -591,12 +592,12 @@ void launch_iter(efe_ctx* c, KrylovWork* w, hipStream_t st, T* x, T* r, T* z, T*
 
 template <typename T>
 void launch_iter_bs(efe_ctx* c, KrylovWork* w, hipStream_t st, T* x, T* r, T* z, T* p, T* q, const T* K,
-                    const T* Minv, int par, int j) {
+                    const T* Minv, bool bricks, int par, int j) {
     switch (w->block) {
-        case 64: launch_iter<T, 64>(c, w, st, x, r, z, p, q, K, Minv, par, j); break;
-        case 128: launch_iter<T, 128>(c, w, st, x, r, z, p, q, K, Minv, par, j); break;
-        case 512: launch_iter<T, 512>(c, w, st, x, r, z, p, q, K, Minv, par, j); break;
-        default: launch_iter<T, 256>(c, w, st, x, r, z, p, q, K, Minv, par, j); break;
+        case 64: launch_iter<T, 64>(c, w, st, x, r, z, p, q, K, Minv, bricks, par, j); break;
+        case 128: launch_iter<T, 128>(c, w, st, x, r, z, p, q, K, Minv, bricks, par, j); break;
+        case 512: launch_iter<T, 512>(c, w, st, x, r, z, p, q, K, Minv, bricks, par, j); break;
+        default: launch_iter<T, 256>(c, w, st, x, r, z, p, q, K, Minv, bricks, par, j); break;
     }
 }
 
@@ -653,7 +654,7 @@ int ensure_work(efe_ctx* c) {
         EFE_HIP(hipEventCreate(&w->t0));
         EFE_HIP(hipEventCreate(&w->t1));
     }
-    for (int i = 0; i < 3; ++i) {
+    for (int i = 0; i < 4; ++i) {
         if (w->graph[i]) hipGraphExecDestroy(w->graph[i]);
         w->graph[i] = nullptr;
     }
@@ -690,7 +691,7 @@ int ensure_work(efe_ctx* c) {
 
 template <typename T>
 int pcg_solve(efe_ctx* c, const double* b, double* xout, const efe_solve_opts* o, efe_solve_info* info, T* x, T* r,
-              T* z, T* p, T* q, const T* K, const T* Minv, int gi) {
+              T* z, T* p, T* q, const T* K, const T* Minv, bool bricks, int gi) {
     KrylovWork* w = c->kw;
     hipStream_t st = w->ks;
     w->kr = w->krp[sizeof(T) == 4 ? 1 : 0];
@@ -700,7 +701,7 @@ int pcg_solve(efe_ctx* c, const double* b, double* xout, const efe_solve_opts* o
     // order after the caller's stream
     EFE_HIP(hipEventRecord(w->evA, c->stream));
     EFE_HIP(hipStreamWaitEvent(st, w->evA, 0));
-    launch_init_bs<T>(c, w, st, b, Minv, x, r, z, p, !K && c->mfb);
+    launch_init_bs<T>(c, w, st, b, Minv, x, r, z, p, bricks);
     EFE_HIP(hipGetLastError());
     // b.b (host) to fix the absolute tolerance
     sum_partials_kernel<<<1, 256, 0, st>>>(w->part + 4 * w->ps, w->nwgv, w->dscal + 1);
@@ -727,7 +728,8 @@ int pcg_solve(efe_ctx* c, const double* b, double* xout, const efe_solve_opts* o
     w->hpart[1] = tol2;
     EFE_HIP(hipMemcpyAsync(w->dscal, w->hpart + 1, sizeof(double), hipMemcpyHostToDevice, st));
     // (re)build the captured batch when its shape or an operator buffer changed
-    const void* ops[4] = {K, Minv, c->mfC, c->mfbF};
+    const void* ops[4] = {K, Minv, sizeof(T) == 8 ? (void*)c->mfC64 : (void*)c->mfC,
+                          sizeof(T) == 8 ? (void*)c->mfbF64 : (void*)c->mfbF};
     bool same = true;
     for (int i = 0; i < 4; ++i) same = same && w->graph_ops[gi][i] == ops[i];
     if (!w->graph[gi] || w->graph_batch[gi] != batch || w->graph_block[gi] != w->block || !same) {
@@ -735,7 +737,7 @@ int pcg_solve(efe_ctx* c, const double* b, double* xout, const efe_solve_opts* o
         w->graph[gi] = nullptr;
         hipGraph_t g;
         EFE_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeRelaxed));
-        for (int j = 0; j < batch; ++j) launch_iter_bs<T>(c, w, st, x, r, z, p, q, K, Minv, j & 1, j);
+        for (int j = 0; j < batch; ++j) launch_iter_bs<T>(c, w, st, x, r, z, p, q, K, Minv, bricks, j & 1, j);
         EFE_HIP(hipStreamEndCapture(st, &g));
         EFE_HIP(hipGraphInstantiate(&w->graph[gi], g, nullptr, nullptr, 0));
         EFE_HIP(hipGraphDestroy(g));
@@ -804,10 +806,16 @@ int efe_krylov_solve(efe_ctx* c, const double* b, double* x, const efe_solve_opt
     if (rc != EFE_OK) return rc;
     KrylovWork* w = c->kw;
     if (o->precision == EFE_FP32_MATFREE)
-        return pcg_solve<float>(c, b, x, o, info, w->x32, w->r32, w->z32, w->p32, w->q32, nullptr, c->Minv32, 2);
+        return pcg_solve<float>(c, b, x, o, info, w->x32, w->r32, w->z32, w->p32, w->q32, nullptr, c->Minv32, c->mfb, 2);
     if (o->precision == EFE_FP32)
-        return pcg_solve<float>(c, b, x, o, info, w->x32, w->r32, w->z32, w->p32, w->q32, c->K32, c->Minv32, 1);
-    return pcg_solve<double>(c, b, x, o, info, w->x64, w->r64, w->z64, w->p64, w->q64, c->K64, c->Minv64, 0);
+        return pcg_solve<float>(c, b, x, o, info, w->x32, w->r32, w->z32, w->p32, w->q32, c->K32, c->Minv32, false, 1);
+    // hexa8 with a symmetric tangent: the FP64 brick product moves 614 bytes per element where the
+    // assembled one moves 2135.  PCG iteration at 8^3 / 20^3 / 40^3 / 64^3: 19.8 / 22.9 / 46.9 /
+    // 123.7 us assembled, 18.9 / 20.7 / 31.2 / 62.7 us on the bricks.  The assembled operator serves
+    // the other elements and materials, and a Dirichlet set changed since the pass.
+    if (efe_mf_bricks64(c))
+        return pcg_solve<double>(c, b, x, o, info, w->x64, w->r64, w->z64, w->p64, w->q64, nullptr, c->Minv64, true, 3);
+    return pcg_solve<double>(c, b, x, o, info, w->x64, w->r64, w->z64, w->p64, w->q64, c->K64, c->Minv64, false, 0);
 }
 
 int efe_launch_spmv64(efe_ctx* c, const double* x, double* y) {
@@ -837,7 +845,7 @@ int efe_launch_norms(efe_ctx* c, const double* R, const double* ddU, const doubl
 void efe_krylov_free(efe_ctx* c) {
     KrylovWork* w = c->kw;
     if (!w) return;
-    for (int i = 0; i < 3; ++i)
+    for (int i = 0; i < 4; ++i)
         if (w->graph[i]) hipGraphExecDestroy(w->graph[i]);
     hipFree(w->x64); hipFree(w->r64); hipFree(w->z64); hipFree(w->p64); hipFree(w->q64);
     hipFree(w->x32); hipFree(w->r32); hipFree(w->z32); hipFree(w->p32); hipFree(w->q32);

@@ -1,28 +1,34 @@
-// Matrix-free FP32 operator for the mixed-precision form (EFE_FP32_MATFREE).
+// Matrix-free products K p from the tangents at the QPs.
 //
 // The element pass stores, per element and QP, the compact tangent
 // w detJ [A, B, cnn, (cn1, c1n,)] and the deviatoric direction n as n_11, n_22, n_12, n_13,
-// n_23 (n_33 = -n_11 - n_22): 8 floats, 10 for Drucker-Prager, of
-// C = A 1(x)1 + B Idev + cnn n(x)n + cn1 n(x)1 + c1n 1(x)n, in [QP][field][element] order
-// so that consecutive lanes read consecutive elements.  y = K p is then, per element (one
+// n_23 (n_33 = -n_11 - n_22) of
+// C = A 1(x)1 + B Idev + cnn n(x)n + cn1 n(x)1 + c1n 1(x)n.  y = K p is then, per element (one
 // thread):
 //   J   = sum_a dN_a/dxi (x) (x_a - x_0)              (rebuilt: cheaper than storing J^-1)
 //   H   = sum_a p_a (x) dN_a/dxi                      (3x3)
 //   eps = sym(H J^-1)                                 (engineering Voigt)
 //   sig = C eps                                       (compact form, ~30 flops)
 //   M_ik = sum_j sig_ij J^-1_jk
-//   f_a = M dN_a/dxi                                  -> node-sorted force slots
-// followed by a per-node sum of its slots in element order (the order of the assembled
-// path's row sums), so the product is deterministic.  Dirichlet DOFs are
-// eliminated symmetrically, as in the assembled operator: p is read as 0 on them and their
-// rows return p (unit diagonal).  The same two kernels with the prescribed values as p and
-// no elimination give the right-hand-side correction K[:, dir] dir_values.
+//   f_a = M dN_a/dxi
+// followed by a sum of the element forces per node in a fixed order, so the product is
+// deterministic.  Dirichlet DOFs are eliminated symmetrically, as in the assembled operator: p is
+// read as 0 on them and their rows return p (unit diagonal).  The same kernels with the
+// prescribed values as p and no elimination give the right-hand-side correction
+// K[:, dir] dir_values.
 //
-// Algorithmic bytes per application: 32..40 per element-QP pair (tangent), 4 per
-// element-node (connectivity) and 2 x 4 per element-node (slot index, force slot written and
-// read), plus the node vectors; against 9 x 4 + 4 bytes per 3x3 block of the assembled FP32
-// operator.  It also removes the FP32 assembly from every Newton iteration.
+// hexa20 (EFE_FP32_MATFREE): 8 or 10 floats per QP in [QP][field][element] order, the forces to
+// node-sorted slots, one per (element, node), summed per node by a second kernel.
+//
+// hexa8: bricks of up to 256 elements (bricks.cpp), in FP32 (EFE_FP32_MATFREE) and in FP64: the
+// FP64 tangent pass of elastic and J2 models stores its compact tangents too, and the FP64 CG
+// runs on them instead of the assembled operator.  Bytes per element and product: 64 NC / 8 (FP32
+// half of it) for the tangents (NC = 7), ~1.6 staged nodes of 48 + 2 x 24 (12) bytes, 16 of local
+// indices: 614 in FP64, against 2135 of the assembled blocks at 64^3 (27 x 72 + 27 x 4 per node).
+// Measured at 64^3 in FP64: 100 us per assembled product (5.6 TB/s), 43 us per brick product with
+// the tangents from HBM, ~36 us with them in the Infinity Cache; PCG iteration 123.7 -> 62.7 us.
 #include <algorithm>
+#include <cstring>
 #include <type_traits>
 #include <vector>
 
@@ -230,8 +236,8 @@ __global__ __launch_bounds__(256) void mf_apply_kernel(int E, int N, const int32
     }
 }
 
-// Hexa8 with 2x2x2 Gauss points: the same product with the trilinear interpolation written
-// in monomials.  A nodal field v gives v(x, y, z) = c0 + c_x x + c_y y + c_z z + c_xy xy +
+// Hexa8 with 2x2x2 Gauss points: the product with the trilinear interpolation written in
+// monomials.  A nodal field v gives v(x, y, z) = c0 + c_x x + c_y y + c_z z + c_xy xy +
 // c_yz yz + c_xz xz + c_xyz xyz with c = (1/8) H v (H: the +-1 Walsh matrix of the node
 // signs, applied as a 3-stage butterfly), so its natural gradient at a point costs 3 FMA per
 // direction instead of a sum over the 8 nodes; the element forces f_a = sum_q M_q grad N_a(q)
@@ -246,94 +252,58 @@ __global__ __launch_bounds__(256) void mf_apply_kernel(int E, int N, const int32
 __constant__ int8_t kHex8Canon[8] = {0, 3, 4, 7, 1, 2, 5, 6};  // node of canonical index k
 
 // in place: w[k] (canonical order) -> r[k] = sum_j prod_{i in bits(k)} s_i(j) w[j]
-__device__ __forceinline__ void walsh3(float (&w)[8]) {
+template <typename T>
+__device__ __forceinline__ void walsh3(T (&w)[8]) {
 #pragma unroll
     for (int h = 1; h < 8; h <<= 1)
 #pragma unroll
         for (int k = 0; k < 8; ++k)
             if (!(k & h)) {
-                const float lo = w[k], hi = w[k | h];
+                const T lo = w[k], hi = w[k | h];
                 w[k] = lo + hi;
                 w[k | h] = hi - lo;
             }
 }
 
 // in place: A[k] (monomial coefficients, A[0] = 0) -> f[k] = sum_S A_S prod_{i in S} s_i(k)
-__device__ __forceinline__ void walsh3_t(float (&w)[8]) {
+template <typename T>
+__device__ __forceinline__ void walsh3_t(T (&w)[8]) {
 #pragma unroll
     for (int h = 1; h < 8; h <<= 1)
 #pragma unroll
         for (int k = 0; k < 8; ++k)
             if (!(k & h)) {
-                const float lo = w[k], hi = w[k | h];
+                const T lo = w[k], hi = w[k | h];
                 w[k] = lo - hi;
                 w[k | h] = lo + hi;
             }
 }
 
-template <int NC, typename TP>
-__global__ __launch_bounds__(256) void mf_apply_hex8_kernel(int E, int N, const int32_t* __restrict__ conn,
-                                                            const double* __restrict__ coords,
-                                                            const float* __restrict__ dnxi,
-                                                            const float* __restrict__ mfC, const TP* __restrict__ p,
-                                                            const uint8_t* __restrict__ dirflag, int mask,
-                                                            const int* __restrict__ flags,
-                                                            const int32_t* __restrict__ pos, float* __restrict__ Fs,
-                                                            const int* __restrict__ active,
-                                                            const int32_t* __restrict__ specOfElem) {
-    (void)dnxi;
-    if (flags && flags[0]) return;
-    const int e = xcd_block_mf() * 256 + threadIdx.x;
-    if (e >= E) return;
-    if (active && !active[specOfElem[e]]) return;  // frozen specimen of a batched solve
-    // monomial coefficients (1/8 included) of p and of the coordinates relative to node 0
-    // (formed in FP64, so that FP32 keeps the element's own scale)
-    float cp[3][8], cx[3][8];
-    double x0[3];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        const int a = kHex8Canon[k];
-        const int nd = conn[(int64_t)a * E + e];
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            float v = (float)p[3 * nd + i];
-            if (mask && dirflag[3 * nd + i]) v = 0.0f;
-            cp[i][k] = v;
-            const double xc = coords[(int64_t)i * N + nd];
-            if (k == 0) x0[i] = xc;
-            cx[i][k] = (float)(xc - x0[i]);
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        walsh3(cp[i]);
-        walsh3(cx[i]);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            cp[i][k] *= 0.125f;
-            cx[i][k] *= 0.125f;
-        }
-    }
-    // force coefficients in the same basis, x 8
-    float fa[3][8];
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int k = 0; k < 8; ++k) fa[i][k] = 0.0f;
-    const float g = 0.57735026918962576451f;
-    // not unrolled: the unrolled loop hoists the tangent loads of all QPs and needs 154
-    // VGPRs (3 waves per SIMD instead of 4), measured slower; so is loading the next QP's
-    // tangent ahead
+// The element's forces in the monomial basis (fa, x 8) from those of p (cp) and of the coordinates
+// (cx), summed over its QPs, whose tangents start at Cg.  HOT: plain loads, which leave the tangents
+// in the Infinity Cache for the next product; else non-temporal ones.  The loop is not unrolled:
+// unrolled, it hoists the tangent loads of all QPs and needs half as many registers again.
+template <int NC, typename T, bool HOT>
+__device__ __forceinline__ void brick_qps(const T* __restrict__ Cg, T bulk, T shear2, const T (&cp)[3][8],
+                                          const T (&cx)[3][8], T (&fa)[3][8]) {
+    const T gq = (T)0.57735026918962576451;
 #pragma unroll 1
     for (int q = 0; q < 8; ++q) {
         // evaluation point (eta_q, xi_q, zeta_q) of the QP table xi = (-,-,-,-,+,+,+,+),
         // eta = (-,-,+,+,-,-,+,+), zeta = (-,+,+,-,-,+,+,-) (times 1/sqrt 3)
         const int r = q & 3;
-        const float x = (r < 2 ? -g : g), y = (q < 4 ? -g : g), z = ((r == 1 || r == 2) ? g : -g);
-        const float xy = x * y, yz = y * z, xz = x * z;
+        const T x = (r < 2 ? -gq : gq), y = (q < 4 ? -gq : gq), z = ((r == 1 || r == 2) ? gq : -gq);
+        const T xy = x * y, yz = y * z, xz = x * z;
+        T cf[NC ? NC : 1];
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+            const T* src = Cg + (q * NC + k) * kBrick;
+            if constexpr (HOT) cf[k] = *src;
+            else cf[k] = __builtin_nontemporal_load(src);
+        }
         // natural gradients: d/dx = c1 + c3 y + c5 z + c7 yz, d/dy = c2 + c3 x + c6 z + c7 xz,
         // d/dz = c4 + c5 x + c6 y + c7 xy   (index = canonical monomial bits)
-        float H[9], J[9];
+        T H[9], J[9];
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
             H[i * 3 + 0] = cp[i][1] + cp[i][3] * y + cp[i][5] * z + cp[i][7] * yz;
@@ -343,47 +313,54 @@ __global__ __launch_bounds__(256) void mf_apply_hex8_kernel(int E, int N, const 
             J[1 * 3 + i] = cx[i][2] + cx[i][3] * x + cx[i][6] * z + cx[i][7] * xz;
             J[2 * 3 + i] = cx[i][4] + cx[i][5] * x + cx[i][6] * y + cx[i][7] * xy;
         }
-        const float det = J[0] * (J[4] * J[8] - J[5] * J[7]) - J[1] * (J[3] * J[8] - J[5] * J[6]) +
-                          J[2] * (J[3] * J[7] - J[4] * J[6]);
-        const float id = 1.0f / det;
-        const float iJ[9] = {(J[4] * J[8] - J[5] * J[7]) * id, (J[2] * J[7] - J[1] * J[8]) * id,
-                             (J[1] * J[5] - J[2] * J[4]) * id, (J[5] * J[6] - J[3] * J[8]) * id,
-                             (J[0] * J[8] - J[2] * J[6]) * id, (J[2] * J[3] - J[0] * J[5]) * id,
-                             (J[3] * J[7] - J[4] * J[6]) * id, (J[1] * J[6] - J[0] * J[7]) * id,
-                             (J[0] * J[4] - J[1] * J[3]) * id};
-        float gr[9];
+        const T det = J[0] * (J[4] * J[8] - J[5] * J[7]) - J[1] * (J[3] * J[8] - J[5] * J[6]) +
+                      J[2] * (J[3] * J[7] - J[4] * J[6]);
+        const T id = (T)1 / det;
+        const T iJ[9] = {(J[4] * J[8] - J[5] * J[7]) * id, (J[2] * J[7] - J[1] * J[8]) * id,
+                         (J[1] * J[5] - J[2] * J[4]) * id, (J[5] * J[6] - J[3] * J[8]) * id,
+                         (J[0] * J[8] - J[2] * J[6]) * id, (J[2] * J[3] - J[0] * J[5]) * id,
+                         (J[3] * J[7] - J[4] * J[6]) * id, (J[1] * J[6] - J[0] * J[7]) * id,
+                         (J[0] * J[4] - J[1] * J[3]) * id};
+        T gr[9];
 #pragma unroll
         for (int i = 0; i < 3; ++i)
 #pragma unroll
             for (int j = 0; j < 3; ++j)
                 gr[i * 3 + j] = H[i * 3] * iJ[j * 3] + H[i * 3 + 1] * iJ[j * 3 + 1] + H[i * 3 + 2] * iJ[j * 3 + 2];
-        const float ep[6] = {gr[0], gr[4], gr[8], gr[1] + gr[3], gr[2] + gr[6], gr[5] + gr[7]};
-        float cf[NC];
+        const T ep[6] = {gr[0], gr[4], gr[8], gr[1] + gr[3], gr[2] + gr[6], gr[5] + gr[7]};
+        // the Gauss weights of hexa8 are 1: w detJ = det
+        const T A = NC == 10 ? cf[0] : bulk * det;
+        const T B = NC == 10 ? cf[1] : (NC == 7 ? cf[0] : shear2 * det);
+        const T tr = ep[0] + ep[1] + ep[2], t3 = tr * (T)(1.0 / 3.0);
+        T s1 = A * tr, sg[6];
+        if constexpr (NC != 0) {
+            const T* nc = cf + (NC == 10 ? 5 : 2);
+            const T n[6] = {nc[0], nc[1], -(nc[0] + nc[1]), nc[2], nc[3], nc[4]};  // n deviatoric
+            const T ne_ = n[0] * ep[0] + n[1] * ep[1] + n[2] * ep[2] + n[3] * ep[3] + n[4] * ep[4] + n[5] * ep[5];
+            T sn = (NC == 10 ? cf[2] : cf[1]) * ne_;
+            if constexpr (NC == 10) {
+                sn += cf[3] * tr;
+                s1 += cf[4] * ne_;
+            }
 #pragma unroll
-        for (int k = 0; k < NC; ++k) cf[k] = __builtin_nontemporal_load(mfC + (int64_t)(q * NC + k) * E + e);
-        const float A = cf[0], B = cf[1], cnn = cf[2];
-        const float cn1 = NC == 10 ? cf[3] : 0.0f, c1n = NC == 10 ? cf[4] : 0.0f;
-        const float* nc = cf + (NC == 10 ? 5 : 3);
-        const float n[6] = {nc[0], nc[1], -(nc[0] + nc[1]), nc[2], nc[3], nc[4]};  // n deviatoric
-        const float tr = ep[0] + ep[1] + ep[2];
-        const float ne = n[0] * ep[0] + n[1] * ep[1] + n[2] * ep[2] + n[3] * ep[3] + n[4] * ep[4] + n[5] * ep[5];
-        const float t3 = tr * (1.0f / 3.0f);
-        const float sn = cnn * ne + cn1 * tr;
-        const float s1 = A * tr + c1n * ne;
-        float sg[6];
+            for (int i = 0; i < 3; ++i) sg[i] = s1 + B * (ep[i] - t3) + sn * n[i];
 #pragma unroll
-        for (int i = 0; i < 3; ++i) sg[i] = s1 + B * (ep[i] - t3) + sn * n[i];
+            for (int i = 3; i < 6; ++i) sg[i] = (T)0.5 * B * ep[i] + sn * n[i];
+        } else {
 #pragma unroll
-        for (int i = 3; i < 6; ++i) sg[i] = 0.5f * B * ep[i] + sn * n[i];
-        const float S[9] = {sg[0], sg[3], sg[4], sg[3], sg[1], sg[5], sg[4], sg[5], sg[2]};
+            for (int i = 0; i < 3; ++i) sg[i] = s1 + B * (ep[i] - t3);
+#pragma unroll
+            for (int i = 3; i < 6; ++i) sg[i] = (T)0.5 * B * ep[i];
+        }
+        const T S[9] = {sg[0], sg[3], sg[4], sg[3], sg[1], sg[5], sg[4], sg[5], sg[2]};
         // f_a,i += sum_k M_ik dN_a/dxi_k with M_ik = sum_j sig_ij iJ_jk, in monomials:
         // fa[1] += M0, fa[2] += M1, fa[4] += M2, fa[3] += M0 y + M1 x, fa[5] += M0 z + M2 x,
         // fa[6] += M1 z + M2 y, fa[7] += M0 yz + M1 xz + M2 xy   (M_k = column k, x 1/8)
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
-            const float m0 = S[i * 3] * iJ[0] + S[i * 3 + 1] * iJ[3] + S[i * 3 + 2] * iJ[6];
-            const float m1 = S[i * 3] * iJ[1] + S[i * 3 + 1] * iJ[4] + S[i * 3 + 2] * iJ[7];
-            const float m2 = S[i * 3] * iJ[2] + S[i * 3 + 1] * iJ[5] + S[i * 3 + 2] * iJ[8];
+            const T m0 = S[i * 3] * iJ[0] + S[i * 3 + 1] * iJ[3] + S[i * 3 + 2] * iJ[6];
+            const T m1 = S[i * 3] * iJ[1] + S[i * 3 + 1] * iJ[4] + S[i * 3 + 2] * iJ[7];
+            const T m2 = S[i * 3] * iJ[2] + S[i * 3 + 1] * iJ[5] + S[i * 3 + 2] * iJ[8];
             fa[i][1] += m0;
             fa[i][2] += m1;
             fa[i][4] += m2;
@@ -393,79 +370,78 @@ __global__ __launch_bounds__(256) void mf_apply_hex8_kernel(int E, int N, const 
             fa[i][7] += m0 * yz + m1 * xz + m2 * xy;
         }
     }
-#pragma unroll
-    for (int i = 0; i < 3; ++i) walsh3_t(fa[i]);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        const int a = kHex8Canon[k];
-        float* dst = Fs + (int64_t)pos[(int64_t)a * E + e] * 3;
-#pragma unroll
-        for (int i = 0; i < 3; ++i) dst[i] = 0.125f * fa[i][k];
-    }
 }
 
-// Hexa8 product by workgroup bricks: workgroup g takes the run of up to 256 consecutive elements
-// e0s[g] .. e0s[g + 1] - 1 (every 256 elements; in batched contexts a run never crosses a
-// specimen boundary).  Its local nodes (the distinct nodes of those elements, ascending) are
-// staged once into LDS with coalesced loads: p (Dirichlet DOFs masked) and the FP64
-// coordinates.  Each thread takes its element's 8 nodes from LDS (local indices lidx), forms the
-// element forces exactly as mf_apply_hex8_kernel, and writes them to LDS; then each local node's
-// forces are summed in element order (incidence list linc) into one partial per (workgroup,
-// node), stored at its slot lpos of the node-ordered partial list.  The gather then sums a
-// node's partials (1 to 8, ~2.4 on a box) in workgroup order: the element-order sum of the
-// per-slot path, grouped by workgroup.  Versus one slot per (element, node): 8 p and 8 coordinate
-// gathers per element become ~2.5 staged loads, and 8 scattered 12-byte stores become ~2.5.
-constexpr int kBrick = 256;       // elements per workgroup
-constexpr int kBrickNodes = 768;  // local nodes a workgroup can stage (an interior hexa8 pencil: 650)
+// What a workgroup of the brick product reads besides the tangents (bricks.cpp).
+struct BrickTables {
+    const int32_t *lptr, *lnode, *lpos, *e0;
+    const uint16_t *linc, *lidx;
+    const double* X;   // [3][L] coordinates of the staged nodes
+    int64_t L;
+    int G, hot;
+};
 
-template <int NC, typename TP>
-__global__ __launch_bounds__(kBrick) void mfb_apply_hex8_kernel(
-    int E, int N, const int32_t* __restrict__ lptr, const int32_t* __restrict__ lnode,
-    const int32_t* __restrict__ lpos, const int32_t* __restrict__ lincp, const uint16_t* __restrict__ linc,
-    const uint16_t* __restrict__ lidx, const double* __restrict__ coords, const float* __restrict__ mfC,
-    const TP* __restrict__ p, const uint8_t* __restrict__ dirflag, int mask, const int* __restrict__ flags,
-    float* __restrict__ Fpart, int G, const int32_t* __restrict__ e0s, const int* __restrict__ active,
-    const int32_t* __restrict__ specOfElem, double* __restrict__ part) {
-    // LDS, reused: first the staged node data (p 3 x 768 floats, x 3 x 768 doubles), then the
-    // element forces (256 x 8 x 3 floats)
-    __shared__ double lds[3 * kBrickNodes + (3 * kBrickNodes + 1) / 2];
+// Hexa8 product by bricks: workgroup g takes the up to kBrick elements of brick g, one lane each.
+// The brick's distinct nodes (p with Dirichlet DOFs masked, and the coordinates, which lie in
+// staging order) go to LDS once; each lane forms its element's forces in the monomial basis and
+// leaves them in LDS; each staged node's forces are summed in element order into one partial
+// per (brick, node), stored at its slot of the node-ordered partial list.
+//
+// NC values per QP are read: 7 (w detJ [B, c_nn], n_11, n_22, n_12, n_13, n_23), with the
+// volumetric coefficient A = K w detJ formed from the element's bulk modulus and the determinant
+// at hand; 10 with Drucker-Prager (A, B, c_nn, c_n1, c_1n and n as stored); 0 when every
+// element is linear elastic (B = 2 G w detJ likewise).  T is the precision of the arithmetic,
+// the tangents and the partials.
+template <int NC, typename T, typename TP>
+__global__ __launch_bounds__(kBrick) void brick_apply_kernel(
+    BrickTables bt, const T* __restrict__ el, const T* __restrict__ C, const TP* __restrict__ p,
+    const uint8_t* __restrict__ dirflag, int mask, const int* __restrict__ flags, T* __restrict__ Fpart,
+    const int* __restrict__ active, const int32_t* __restrict__ order, const int32_t* __restrict__ specOfElem,
+    double* __restrict__ part) {
+    // LDS, reused: first the staged nodes (x 3 doubles, p 3 T), then the element forces (24 T a lane)
+    constexpr int kStage = 3 * kBrickNodes * (int)(sizeof(double) + sizeof(T));
+    constexpr int kForce = 24 * kBrick * (int)sizeof(T);
+    __shared__ __align__(16) char lds[kStage > kForce ? kStage : kForce];
     __shared__ double red[kBrick / 64];
-    double* sx = lds;
-    float* sp = (float*)(lds + 3 * kBrickNodes);
-    float* sf = (float*)lds;
+    double* sx = (double*)lds;
+    T* sp = (T*)(lds + 3 * kBrickNodes * sizeof(double));
+    T* sf = (T*)lds;
     if (flags && flags[0]) return;
     const int g = xcd_block_mf();
-    if (g >= G) {  // the grid is rounded up to a multiple of 8
+    if (g >= bt.G) {  // the grid is rounded up to a multiple of 8
         if (part && threadIdx.x == 0) part[g] = 0.0;
         return;
     }
-    const int eb = e0s[g], ee = e0s[g + 1];
-    // batched solves: a brick of a frozen specimen leaves its partials alone (the gather skips
-    // that specimen's nodes)
-    if (active && !active[specOfElem[eb]]) return;
+    const int eb = bt.e0[g], ne = bt.e0[g + 1] - eb;
+    // batched solves: a brick of a frozen specimen leaves its partials alone (nobody reads them)
+    if (active && !active[specOfElem[order[eb]]]) return;
     const int t = threadIdx.x;
-    const int l0 = lptr[g], nl = lptr[g + 1] - l0;
+    const int l0 = bt.lptr[g], nl = bt.lptr[g + 1] - l0;
     for (int i = t; i < nl; i += kBrick) {
-        const int nd = lnode[l0 + i];
+        const int nd = bt.lnode[l0 + i];
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-            float v = (float)p[3 * nd + c];
-            if (mask && dirflag[3 * nd + c]) v = 0.0f;
+            T v = (T)p[3 * nd + c];
+            if (mask && dirflag[3 * nd + c]) v = (T)0;
             sp[c * kBrickNodes + i] = v;
-            sx[c * kBrickNodes + i] = coords[(int64_t)c * N + nd];
+            sx[c * kBrickNodes + i] = bt.X[c * bt.L + l0 + i];
         }
     }
+    const bool live = t < ne;
+    const T* Cg = C + (int64_t)g * (8 * NC * kBrick) + t;
+    const T bulk = NC != 10 && live ? el[g * kBrick + t] : (T)0;
+    const T shear2 = NC == 0 && live ? el[(int64_t)bt.G * kBrick + g * kBrick + t] : (T)0;
+    // 8 local indices in one 16-byte load
+    const uint4 li4 = live ? *reinterpret_cast<const uint4*>(bt.lidx + (int64_t)(eb + t) * 8) : uint4{0, 0, 0, 0};
     __syncthreads();
-    const int e = eb + t;
-    const bool live = e < ee;
-    float cp[3][8], cx[3][8];
+    T cp[3][8], cx[3][8];
     if (live) {
-        // 8 local indices in one 16-byte load
-        const uint4 li4 = *reinterpret_cast<const uint4*>(lidx + (int64_t)e * 8);
         const uint32_t lw[4] = {li4.x, li4.y, li4.z, li4.w};
         int loc[8];
 #pragma unroll
         for (int a = 0; a < 8; ++a) loc[a] = (int)((lw[a >> 1] >> (16 * (a & 1))) & 0xffffu);
+        // coordinates relative to node 0, the difference formed in FP64, so that FP32 keeps the
+        // element's own scale
         double x0[3];
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
@@ -475,7 +451,7 @@ __global__ __launch_bounds__(kBrick) void mfb_apply_hex8_kernel(
                 cp[i][k] = sp[i * kBrickNodes + l];
                 const double xc = sx[i * kBrickNodes + l];
                 if (k == 0) x0[i] = xc;
-                cx[i][k] = (float)(xc - x0[i]);
+                cx[i][k] = (T)(xc - x0[i]);
             }
         }
     }
@@ -490,78 +466,17 @@ __global__ __launch_bounds__(kBrick) void mfb_apply_hex8_kernel(
             walsh3(cx[i]);
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
-                cp[i][k] *= 0.125f;
-                cx[i][k] *= 0.125f;
+                cp[i][k] *= (T)0.125;
+                cx[i][k] *= (T)0.125;
             }
         }
-        float fa[3][8];
+        T fa[3][8];
 #pragma unroll
         for (int i = 0; i < 3; ++i)
 #pragma unroll
-            for (int k = 0; k < 8; ++k) fa[i][k] = 0.0f;
-        const float gq = 0.57735026918962576451f;
-#pragma unroll 1
-        for (int q = 0; q < 8; ++q) {
-            const int r = q & 3;
-            const float x = (r < 2 ? -gq : gq), y = (q < 4 ? -gq : gq), z = ((r == 1 || r == 2) ? gq : -gq);
-            const float xy = x * y, yz = y * z, xz = x * z;
-            float H[9], J[9];
-#pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                H[i * 3 + 0] = cp[i][1] + cp[i][3] * y + cp[i][5] * z + cp[i][7] * yz;
-                H[i * 3 + 1] = cp[i][2] + cp[i][3] * x + cp[i][6] * z + cp[i][7] * xz;
-                H[i * 3 + 2] = cp[i][4] + cp[i][5] * x + cp[i][6] * y + cp[i][7] * xy;
-                J[0 * 3 + i] = cx[i][1] + cx[i][3] * y + cx[i][5] * z + cx[i][7] * yz;
-                J[1 * 3 + i] = cx[i][2] + cx[i][3] * x + cx[i][6] * z + cx[i][7] * xz;
-                J[2 * 3 + i] = cx[i][4] + cx[i][5] * x + cx[i][6] * y + cx[i][7] * xy;
-            }
-            const float det = J[0] * (J[4] * J[8] - J[5] * J[7]) - J[1] * (J[3] * J[8] - J[5] * J[6]) +
-                              J[2] * (J[3] * J[7] - J[4] * J[6]);
-            const float id = 1.0f / det;
-            const float iJ[9] = {(J[4] * J[8] - J[5] * J[7]) * id, (J[2] * J[7] - J[1] * J[8]) * id,
-                                 (J[1] * J[5] - J[2] * J[4]) * id, (J[5] * J[6] - J[3] * J[8]) * id,
-                                 (J[0] * J[8] - J[2] * J[6]) * id, (J[2] * J[3] - J[0] * J[5]) * id,
-                                 (J[3] * J[7] - J[4] * J[6]) * id, (J[1] * J[6] - J[0] * J[7]) * id,
-                                 (J[0] * J[4] - J[1] * J[3]) * id};
-            float gr[9];
-#pragma unroll
-            for (int i = 0; i < 3; ++i)
-#pragma unroll
-                for (int j = 0; j < 3; ++j)
-                    gr[i * 3 + j] = H[i * 3] * iJ[j * 3] + H[i * 3 + 1] * iJ[j * 3 + 1] + H[i * 3 + 2] * iJ[j * 3 + 2];
-            const float ep[6] = {gr[0], gr[4], gr[8], gr[1] + gr[3], gr[2] + gr[6], gr[5] + gr[7]};
-            float cf[NC];
-#pragma unroll
-            for (int k = 0; k < NC; ++k) cf[k] = __builtin_nontemporal_load(mfC + (int64_t)(q * NC + k) * E + e);
-            const float A = cf[0], B = cf[1], cnn = cf[2];
-            const float cn1 = NC == 10 ? cf[3] : 0.0f, c1n = NC == 10 ? cf[4] : 0.0f;
-            const float* nc = cf + (NC == 10 ? 5 : 3);
-            const float n[6] = {nc[0], nc[1], -(nc[0] + nc[1]), nc[2], nc[3], nc[4]};  // n deviatoric
-            const float tr = ep[0] + ep[1] + ep[2];
-            const float ne = n[0] * ep[0] + n[1] * ep[1] + n[2] * ep[2] + n[3] * ep[3] + n[4] * ep[4] + n[5] * ep[5];
-            const float t3 = tr * (1.0f / 3.0f);
-            const float sn = cnn * ne + cn1 * tr;
-            const float s1 = A * tr + c1n * ne;
-            float sg[6];
-#pragma unroll
-            for (int i = 0; i < 3; ++i) sg[i] = s1 + B * (ep[i] - t3) + sn * n[i];
-#pragma unroll
-            for (int i = 3; i < 6; ++i) sg[i] = 0.5f * B * ep[i] + sn * n[i];
-            const float S[9] = {sg[0], sg[3], sg[4], sg[3], sg[1], sg[5], sg[4], sg[5], sg[2]};
-#pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                const float m0 = S[i * 3] * iJ[0] + S[i * 3 + 1] * iJ[3] + S[i * 3 + 2] * iJ[6];
-                const float m1 = S[i * 3] * iJ[1] + S[i * 3 + 1] * iJ[4] + S[i * 3 + 2] * iJ[7];
-                const float m2 = S[i * 3] * iJ[2] + S[i * 3 + 1] * iJ[5] + S[i * 3 + 2] * iJ[8];
-                fa[i][1] += m0;
-                fa[i][2] += m1;
-                fa[i][4] += m2;
-                fa[i][3] += m0 * y + m1 * x;
-                fa[i][5] += m0 * z + m2 * x;
-                fa[i][6] += m1 * z + m2 * y;
-                fa[i][7] += m0 * yz + m1 * xz + m2 * xy;
-            }
-        }
+            for (int k = 0; k < 8; ++k) fa[i][k] = (T)0;
+        if (g < bt.hot) brick_qps<NC, T, true>(Cg, bulk, shear2, cp, cx, fa);
+        else brick_qps<NC, T, false>(Cg, bulk, shear2, cp, cx, fa);
         if (part)
 #pragma unroll
             for (int i = 0; i < 3; ++i)
@@ -569,26 +484,30 @@ __global__ __launch_bounds__(kBrick) void mfb_apply_hex8_kernel(
                 for (int k = 0; k < 8; ++k) en += (double)cp[i][k] * (double)fa[i][k];
 #pragma unroll
         for (int i = 0; i < 3; ++i) walsh3_t(fa[i]);
-        // forces [i][t * 8 + a] (component-major: lanes t write 8 apart, then the node sums read
-        // runs of one component)
+        // forces [i][a][t]: consecutive lanes in consecutive banks
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
             const int a = kHex8Canon[k];
 #pragma unroll
-            for (int i = 0; i < 3; ++i) sf[i * (kBrick * 8) + t * 8 + a] = 0.125f * fa[i][k];
+            for (int i = 0; i < 3; ++i) sf[(i * 8 + a) * kBrick + t] = (T)0.125 * fa[i][k];
         }
     }
     __syncthreads();
-    // one partial per local node: its incidences in element order
+    // one partial per staged node: its up to 8 incidences in element order
     for (int i = t; i < nl; i += kBrick) {
-        float f0 = 0.0f, f1 = 0.0f, f2 = 0.0f;
-        for (int c = lincp[l0 + i]; c < lincp[l0 + i + 1]; ++c) {
-            const int s = linc[c];
-            f0 += sf[s];
-            f1 += sf[kBrick * 8 + s];
-            f2 += sf[2 * kBrick * 8 + s];
+        const uint4 w4 = *reinterpret_cast<const uint4*>(bt.linc + (int64_t)(l0 + i) * 8);
+        const uint32_t w[4] = {w4.x, w4.y, w4.z, w4.w};
+        T f0 = (T)0, f1 = (T)0, f2 = (T)0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint32_t s = (w[j >> 1] >> (16 * (j & 1))) & 0xffffu;
+            if (s != 0xffffu) {
+                f0 += sf[s];
+                f1 += sf[8 * kBrick + s];
+                f2 += sf[16 * kBrick + s];
+            }
         }
-        float* dst = Fpart + (int64_t)lpos[l0 + i] * 3;
+        T* dst = Fpart + (int64_t)bt.lpos[l0 + i] * 3;
         dst[0] = f0;
         dst[1] = f1;
         dst[2] = f2;
@@ -738,34 +657,60 @@ inline int round8_mf(int n) { return (n + 7) & ~7; }
     c->E, c->N, c->conn, c->coords, c->dnxi32, c->mfC, p, c->dirflag, mask, flags, c->elemPos, c->mfF, active, \
         c->specOfElem
 
+// T: precision of the product (float: the matrix-free operator; double: bricks of the FP64 pass)
+template <typename T, typename TP>
+void launch_bricks(efe_ctx* c, hipStream_t st, const TP* p, int mask, const int* flags, const int* active,
+                   double* part) {
+    // The Infinity Cache (256 MB) serves the tangents from one product to the next when they and
+    // what a PCG iteration touches beside them fit: plain loads then, else non-temporal ones, which
+    // keep the tangents from displacing the rest.  PCG iteration at 64^3 FP64 (117 + 90 MB) 69.6 ->
+    // 62.7 us, 80^3 FP32 (115 + 90 MB) 82 -> 72 us; beyond it plain loads cost more: 80^3 FP64
+    // (229 + 160 MB) 129 -> 152 us, 96^3 FP32 119 -> 139 us.  Below ~24 MB the L2s hold them either
+    // way (36^3 FP64 25.3 us non-temporal, 26.4 plain).
+    const int64_t tangents = (int64_t)c->E * 8 * c->mfNC * (int64_t)sizeof(T);
+    const int64_t rest = c->mfbL * (int64_t)(48 + 3 * sizeof(T)) + (int64_t)c->E * (16 + sizeof(T)) +
+                         (int64_t)c->N * 21 * (int64_t)sizeof(T);
+    const bool hot = tangents > (int64_t)24e6 && tangents + rest <= (int64_t)216e6;
+    const BrickTables bt{c->mfbLptr, c->mfbLnode, c->mfbLpos, c->mfbE0, c->mfbLinc, c->mfbLidx, c->mfbX, c->mfbL,
+                         c->mfbG, hot ? c->mfbG : 0};
+    const int grid = round8_mf(c->mfbG);
+    const T *el, *C;
+    T* F;
+    if constexpr (sizeof(T) == 8) {
+        el = c->mfbEl64;
+        C = c->mfC64;
+        F = c->mfbF64;
+    } else {
+        el = c->mfbEl;
+        C = c->mfC;
+        F = c->mfbF;
+    }
+#define BRICK_ARGS bt, el, C, p, c->dirflag, mask, flags, F, active, c->mfbOrder, c->specOfElem, part
+    if (c->mfNC == 10) {
+        if constexpr (sizeof(T) == 4) brick_apply_kernel<10, T, TP><<<grid, kBrick, 0, st>>>(BRICK_ARGS);
+    } else if (c->mfNC == 7) {
+        brick_apply_kernel<7, T, TP><<<grid, kBrick, 0, st>>>(BRICK_ARGS);
+    } else {
+        brick_apply_kernel<0, T, TP><<<grid, kBrick, 0, st>>>(BRICK_ARGS);
+    }
+#undef BRICK_ARGS
+}
+
 template <typename TP>
 void launch_apply(efe_ctx* c, hipStream_t st, const TP* p, int mask, const int* flags,
                   const int* active = nullptr, double* part = nullptr) {
-    const int grid = round8_mf((c->E + 255) / 256);
-    const bool dp = c->mfNC == 10;
-    if (c->mfb) {  // bricks (hexa8); grid: the bricks, rounded up to a multiple of 8
-        const int gb = round8_mf(c->mfbG);
-#define MFB_ARGS                                                                                                 \
-    c->E, c->N, c->mfbLptr, c->mfbLnode, c->mfbLpos, c->mfbLincp, c->mfbLinc, c->mfbLidx, c->coords, c->mfC, p, \
-        c->dirflag, mask, flags, c->mfbF, c->mfbG, c->mfbE0, active, c->specOfElem, part
-        if (dp) mfb_apply_hex8_kernel<10, TP><<<gb, kBrick, 0, st>>>(MFB_ARGS);
-        else mfb_apply_hex8_kernel<8, TP><<<gb, kBrick, 0, st>>>(MFB_ARGS);
-#undef MFB_ARGS
+    if (c->mfb) {
+        launch_bricks<float, TP>(c, st, p, mask, flags, active, part);
         return;
     }
-    switch (c->eltype) {
-        case EFE_C3D8:
-            if (dp) mf_apply_hex8_kernel<10, TP><<<grid, 256, 0, st>>>(MF_ARGS);
-            else mf_apply_hex8_kernel<8, TP><<<grid, 256, 0, st>>>(MF_ARGS);
-            break;
-        case EFE_C3D20:
-            if (dp) mf_apply_kernel<20, 27, 10, TP><<<grid, 256, 0, st>>>(MF_ARGS);
-            else mf_apply_kernel<20, 27, 8, TP><<<grid, 256, 0, st>>>(MF_ARGS);
-            break;
-        default:
-            if (dp) mf_apply_kernel<20, 8, 10, TP><<<grid, 256, 0, st>>>(MF_ARGS);
-            else mf_apply_kernel<20, 8, 8, TP><<<grid, 256, 0, st>>>(MF_ARGS);
-            break;
+    const int grid = round8_mf((c->E + 255) / 256);
+    const bool dp = c->mfNC == 10;
+    if (c->eltype == EFE_C3D20) {
+        if (dp) mf_apply_kernel<20, 27, 10, TP><<<grid, 256, 0, st>>>(MF_ARGS);
+        else mf_apply_kernel<20, 27, 8, TP><<<grid, 256, 0, st>>>(MF_ARGS);
+    } else {
+        if (dp) mf_apply_kernel<20, 8, 10, TP><<<grid, 256, 0, st>>>(MF_ARGS);
+        else mf_apply_kernel<20, 8, 8, TP><<<grid, 256, 0, st>>>(MF_ARGS);
     }
 }
 
@@ -789,103 +734,95 @@ void launch_gather_op(efe_ctx* c, hipStream_t st, const float* p, float* q, doub
 }  // namespace
 
 namespace {
-// Brick tables of the hexa8 operator; left off when a workgroup's elements touch more than
-// kBrickNodes nodes (a mesh in an order without locality).  Bricks are runs of up to kBrick
-// consecutive elements; in batched contexts every specimen's elements start a new brick, so
-// that a specimen's partial sums are grouped the same alone and in any batch (its elements
-// must then be one contiguous run per specimen, else the per-slot operator stays).
-int mfb_build(efe_ctx* c) {
-    if (c->eltype != EFE_C3D8 || c->mfb) return EFE_OK;
-    const int E = c->E, N = c->N;
-    std::vector<int32_t> e0s(1, 0);
-    if (c->specOfNode) {
-        std::vector<int32_t> se(E);
-        EFE_HIP(hipMemcpy(se.data(), c->specOfElem, (size_t)E * sizeof(int32_t), hipMemcpyDeviceToHost));
-        for (int e = 1; e < E; ++e) {
-            if (se[e] < se[e - 1]) return EFE_OK;  // specimens' elements not in runs
-            if (se[e] != se[e - 1] || e - e0s.back() == kBrick) e0s.push_back(e);
-        }
-    } else {
-        for (int e = kBrick; e < E; e += kBrick) e0s.push_back(e);
+template <typename T>
+int up(T** dst, const std::vector<T>& v) {
+    EFE_HIP(hipMalloc((void**)dst, (v.size() ? v.size() : 1) * sizeof(T)));
+    if (!v.empty()) EFE_HIP(hipMemcpy((void*)*dst, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
+    return EFE_OK;
+}
+
+// bulk modulus and 2 G of the elements, brick by brick
+template <typename T>
+int build_moduli(efe_ctx* c, T** dst) {
+    const int E = c->E;
+    std::vector<double> pr(c->props_per_element ? (size_t)2 * E : 2);
+    std::vector<int32_t> pos(E);
+    EFE_HIP(hipMemcpy(pr.data(), c->props, pr.size() * sizeof(double), hipMemcpyDeviceToHost));
+    EFE_HIP(hipMemcpy(pos.data(), c->mfbPos, (size_t)E * sizeof(int32_t), hipMemcpyDeviceToHost));
+    const size_t n = (size_t)c->mfbG * kBrick;
+    std::vector<T> v(2 * n, (T)0);
+    for (int e = 0; e < E; ++e) {
+        const double y = c->props_per_element ? pr[e] : pr[0], nu = c->props_per_element ? pr[(size_t)E + e] : pr[1];
+        v[pos[e]] = (T)(y / (3.0 * (1.0 - 2.0 * nu)));
+        v[n + pos[e]] = (T)(y / (1.0 + nu));
     }
-    e0s.push_back(E);
-    const int G = (int)e0s.size() - 1;
-    std::vector<int32_t> conn((size_t)8 * E);  // [a][e]
-    EFE_HIP(hipMemcpy(conn.data(), c->conn, conn.size() * sizeof(int32_t), hipMemcpyDeviceToHost));
-    std::vector<int32_t> lptr(G + 1, 0), lnode, lincp, pcount(N, 0);
-    std::vector<uint16_t> linc((size_t)8 * E), lidx((size_t)8 * E);
-    lnode.reserve((size_t)3 * E);
-    lincp.reserve((size_t)3 * E + 1);
-    std::vector<int32_t> mark(N, -1);
-    std::vector<int32_t> nodes, cnt, fill;
-    for (int g = 0; g < G; ++g) {
-        const int e0 = e0s[g], e1 = e0s[g + 1];
-        nodes.clear();
-        for (int e = e0; e < e1; ++e)
-            for (int a = 0; a < 8; ++a) nodes.push_back(conn[(size_t)a * E + e]);
-        std::sort(nodes.begin(), nodes.end());
-        nodes.erase(std::unique(nodes.begin(), nodes.end()), nodes.end());
-        const int nl = (int)nodes.size();
-        if (nl > kBrickNodes) return EFE_OK;  // no locality: keep the per-slot operator
-        for (int i = 0; i < nl; ++i) mark[nodes[i]] = i;
-        cnt.assign(nl + 1, 0);
-        for (int e = e0; e < e1; ++e)
-            for (int a = 0; a < 8; ++a) {
-                const int l = mark[conn[(size_t)a * E + e]];
-                lidx[(size_t)e * 8 + a] = (uint16_t)l;
-                ++cnt[l + 1];
-            }
-        for (int i = 0; i < nl; ++i) cnt[i + 1] += cnt[i];
-        const int base = e0 * 8;  // linc entries of workgroup g start at its first element's
-        fill.assign(cnt.begin(), cnt.end() - 1);
-        for (int e = e0; e < e1; ++e)  // element order inside every local node's list
-            for (int a = 0; a < 8; ++a) {
-                const int l = mark[conn[(size_t)a * E + e]];
-                linc[(size_t)base + fill[l]++] = (uint16_t)((e - e0) * 8 + a);
-            }
-        for (int i = 0; i < nl; ++i) {
-            lnode.push_back(nodes[i]);
-            lincp.push_back(base + cnt[i]);
-            ++pcount[nodes[i]];
-            mark[nodes[i]] = -1;
-        }
-        lptr[g + 1] = (int32_t)lnode.size();
-    }
-    lincp.push_back(8 * E);
-    // partial slots in node order, the workgroups of a node in ascending order
-    const int64_t L = (int64_t)lnode.size();
-    std::vector<int32_t> pptr(N + 1, 0), lpos(L);
-    for (int n = 0; n < N; ++n) pptr[n + 1] = pptr[n] + pcount[n];
-    std::vector<int32_t> next(pptr.begin(), pptr.end() - 1);
-    for (int64_t i = 0; i < L; ++i) lpos[i] = next[lnode[i]]++;
-    // the end of each local node's incidence list is the start of the next one's; the last
-    // local node of a workgroup ends where the next workgroup's first begins (lincp[L] = 8 E)
-    auto up = [&](auto** dst, const auto& v) -> int {
-        using T = typename std::remove_reference<decltype(v[0])>::type;
-        EFE_HIP(hipMalloc((void**)dst, (v.size() ? v.size() : 1) * sizeof(T)));
-        if (!v.empty()) EFE_HIP(hipMemcpy((void*)*dst, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
-        return EFE_OK;
+    return up(dst, v);
+}
+}  // namespace
+
+// The brick tables, once per context.  (The element passes keep the element order: walking the
+// bricks, whose state lies in runs of ~8 elements, took the 64^3 tangent pass from 0.87 to 1.06 ms.)
+// One allocation and one copy hold them all.
+int efe_mf_upload_bricks(efe_ctx* c, const BrickPattern& bp, const double* coords) {
+    const int64_t L = (int64_t)bp.lnode.size();
+    std::vector<double> X((size_t)3 * L);
+    for (int64_t i = 0; i < L; ++i)
+        for (int k = 0; k < 3; ++k) X[(size_t)k * L + i] = coords[(size_t)3 * bp.lnode[i] + k];
+    struct Part {
+        const void* src;
+        size_t bytes;
+        void** dst;
     };
-    int rc;
-    if ((rc = up(&c->mfbLptr, lptr)) || (rc = up(&c->mfbLnode, lnode)) || (rc = up(&c->mfbLpos, lpos)) ||
-        (rc = up(&c->mfbLincp, lincp)) || (rc = up(&c->mfbPptr, pptr)) || (rc = up(&c->mfbLinc, linc)) ||
-        (rc = up(&c->mfbLidx, lidx)) || (rc = up(&c->mfbE0, e0s)))
-        return rc;
-    EFE_HIP(hipMalloc(&c->mfbF, (size_t)L * 3 * sizeof(float)));
-    c->mfbG = G;
+    auto part = [](const auto& v, auto** dst) { return Part{v.data(), v.size() * sizeof(v[0]), (void**)dst}; };
+    const Part parts[] = {part(bp.e0, &c->mfbE0),       part(bp.order, &c->mfbOrder), part(bp.pos, &c->mfbPos),
+                          part(bp.lptr, &c->mfbLptr),   part(bp.lnode, &c->mfbLnode), part(bp.lpos, &c->mfbLpos),
+                          part(bp.pptr, &c->mfbPptr),   part(bp.linc, &c->mfbLinc),   part(bp.lidx, &c->mfbLidx),
+                          part(X, &c->mfbX)};
+    size_t total = 0;
+    for (const Part& q : parts) total += (q.bytes + 255) & ~(size_t)255;
+    std::vector<char> host(total);
+    EFE_HIP(hipMalloc(&c->mfbTables, total));
+    size_t off = 0;
+    for (const Part& q : parts) {
+        if (q.bytes) memcpy(host.data() + off, q.src, q.bytes);
+        *q.dst = (char*)c->mfbTables + off;
+        off += (q.bytes + 255) & ~(size_t)255;
+    }
+    EFE_HIP(hipMemcpy(c->mfbTables, host.data(), total, hipMemcpyHostToDevice));
+    c->mfbL = L;
+    c->mfbG = (int)bp.e0.size() - 1;
     c->mfb = true;
     return EFE_OK;
 }
-}  // namespace
+
+int efe_mf_alloc_bricks(efe_ctx* c, bool fp64) {
+    EFE_HIP(hipStreamSynchronize(c->stream));  // the uploads below use the default stream
+    const size_t nc = (size_t)c->mfbG * kBrick * 8 * (c->mfNC ? c->mfNC : 1);
+    if (fp64) {
+        if (c->mfC64) return EFE_OK;
+        if (int rc = build_moduli(c, &c->mfbEl64)) return rc;
+        EFE_HIP(hipMalloc(&c->mfbF64, (size_t)c->mfbL * 3 * sizeof(double)));
+        EFE_HIP(hipMalloc(&c->mfC64, nc * sizeof(double)));
+    } else {
+        if (c->mfC) return EFE_OK;
+        if (int rc = build_moduli(c, &c->mfbEl)) return rc;
+        EFE_HIP(hipMalloc(&c->mfbF, (size_t)c->mfbL * 3 * sizeof(float)));
+        EFE_HIP(hipMalloc(&c->mfC, nc * sizeof(float)));
+    }
+    return EFE_OK;
+}
+
+bool efe_mf_bricks64(const efe_ctx* c) { return c->mfC64 && c->mf64Dir == c->dirVersion; }
 
 int efe_mf_alloc(efe_ctx* c) {
     const int NC = c->mfNC;
     if (c->mfC) return EFE_OK;
+    if (!c->Minv32) EFE_HIP(hipMalloc(&c->Minv32, (size_t)c->N * 9 * sizeof(float)));
+    if (c->eltype == EFE_C3D8) return efe_mf_alloc_bricks(c, false);
     const size_t EQ = (size_t)c->E * c->Q;
     const int64_t L = (int64_t)c->E * c->NN;
     EFE_HIP(hipMalloc(&c->mfC, EQ * NC * sizeof(float)));
     EFE_HIP(hipMalloc(&c->mfF, (size_t)L * 3 * sizeof(float)));
-    if (!c->Minv32) EFE_HIP(hipMalloc(&c->Minv32, (size_t)c->N * 9 * sizeof(float)));
     // FP32 copies of the natural shape-function derivatives at the evaluation points and of
     // the table J is formed with, one after the other
     const size_t nd = (size_t)c->Q * c->NN * 3;
@@ -896,7 +833,7 @@ int efe_mf_alloc(efe_ctx* c) {
     for (size_t i = 0; i < 2 * nd; ++i) hf[i] = (float)h[i];
     EFE_HIP(hipMalloc(&c->dnxi32, 2 * nd * sizeof(float)));
     EFE_HIP(hipMemcpy(c->dnxi32, hf.data(), 2 * nd * sizeof(float), hipMemcpyHostToDevice));
-    return mfb_build(c);
+    return EFE_OK;
 }
 
 // Diagonal blocks, Minv, P, F and (optionally) the right-hand-side correction K[:, dir] dir_values.
@@ -939,8 +876,14 @@ void efe_mf_launch_operator(efe_ctx* c, hipStream_t st, const float* p, float* q
 // The brick product alone (hexa8 bricks only): the node partials of K p for the caller's own
 // gather, and per brick the partial of p . K p (Dirichlet DOFs masked) at part[g], g below
 // round8(mfbG).
-void efe_mf_launch_apply_partials(efe_ctx* c, hipStream_t st, const float* p, double* part, const int* flags) {
-    launch_apply<float>(c, st, p, 1, flags, nullptr, part);
+void efe_mf_launch_apply_partials(efe_ctx* c, hipStream_t st, const float* p, double* part, const int* flags,
+                                  const int* active) {
+    launch_bricks<float, float>(c, st, p, 1, flags, active, part);
+}
+
+void efe_mf_launch_apply_partials(efe_ctx* c, hipStream_t st, const double* p, double* part, const int* flags,
+                                  const int* active) {
+    launch_bricks<double, double>(c, st, p, 1, flags, active, part);
 }
 
 // y = K x for FP64 vectors with the matrix-free FP32 operator (Dirichlet eliminated).
@@ -969,16 +912,10 @@ void efe_mf_launch_operator_batched(efe_ctx* c, hipStream_t st, const float* p, 
 }
 
 void efe_mf_free(efe_ctx* c) {
-    hipFree(c->mfC);
-    hipFree(c->mfF);
-    hipFree(c->dnxi32);
-    c->mfC = c->mfF = c->dnxi32 = nullptr;
-    void* b[] = {c->mfbLptr, c->mfbLnode, c->mfbLpos, c->mfbLincp, c->mfbPptr, c->mfbLinc, c->mfbLidx, c->mfbF,
-                 c->mfbE0};
+    void* b[] = {c->mfC, c->mfF, c->dnxi32, c->mfC64, c->mfbTables, c->mfbEl, c->mfbF, c->mfbEl64, c->mfbF64};
     for (void* q : b)
         if (q) hipFree(q);
-    c->mfbLptr = c->mfbLnode = c->mfbLpos = c->mfbLincp = c->mfbPptr = c->mfbE0 = nullptr;
-    c->mfbLinc = c->mfbLidx = nullptr;
-    c->mfbF = nullptr;
+    c->mfC = c->mfF = c->dnxi32 = nullptr;
+    c->mfC64 = nullptr;
     c->mfb = false;
 }
