@@ -19,7 +19,7 @@ struct BatchWork {
     int N = 0, S = 0, prec = -1;
     void *x = nullptr, *r = nullptr, *z = nullptr, *p = nullptr, *q = nullptr;
     double *nv0 = nullptr, *nv1 = nullptr;     // per-node values
-    double* sc = nullptr;                      // per specimen: [0] rz, [1] rtol2, [2] rr, [3] tol2, [4] beta
+    double* sc = nullptr;                      // per specimen: [0] rz, [1] rtol2, [2] rr, [3] tol2, [4] beta, [5] rz of odd iterations
     int *active = nullptr, *iters = nullptr;   // per specimen
     int* nactive = nullptr;                    // device count
     int* acc = nullptr;                        // per specimen accept flags
@@ -28,6 +28,11 @@ struct BatchWork {
     int32_t *chunkNode0 = nullptr, *chunkSpec = nullptr;  // [C] first node, specimen
     int32_t* specChunk = nullptr;              // [S+1] first chunk of each specimen
     double *pqp = nullptr, *rzp = nullptr, *rrp = nullptr;  // [C] chunk partials of p.q, r.z, r.r
+    // hexa8 bricks: first brick of each specimen [S+1], per brick the partial of p.Kp [round8(G)], and
+    // the second set of active flags [S] (the flags alternate with the iteration)
+    int32_t* specBrick = nullptr;
+    double* brickPq = nullptr;
+    int* active2 = nullptr;
     int* hbuf = nullptr;                       // pinned
     hipStream_t ks = nullptr;
     hipEvent_t evA = nullptr, evB = nullptr;
@@ -50,7 +55,8 @@ struct BatchWork {
 namespace {
 
 constexpr int BS = 256;
-enum { RZ = 0, RTOL2 = 1, RR = 2, TOL2 = 3, BETA = 4, NSC = 5 };
+constexpr int kOpBricks64 = 16;  // operator code of the FP64 bricks (else the precision code)
+enum { RZ = 0, RTOL2 = 1, RR = 2, TOL2 = 3, BETA = 4, RZ2 = 5, NSC = 6 };
 
 // Fixed-order workgroup sums: an xor butterfly inside each wavefront (all lanes end with
 // bitwise identical sums), then the per-wave sums in wave order.
@@ -295,11 +301,144 @@ __global__ __launch_bounds__(BS) void b_direction_kernel(int N, const int32_t* _
     for (int i = 0; i < 3; ++i) p[3 * n + i] = z[3 * n + i] + beta * p[3 * n + i];
 }
 
-__global__ void b_count_kernel(int S, const int* __restrict__ active, int* __restrict__ nactive) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// Hexa8 bricks, iteration of parity par (three kernels: the brick product, this, the direction).
+// p.q = the specimen's brick partials (Dirichlet DOFs masked) + the Dirichlet p.p chunk partials
+// pdp; q of a node = the sum of its brick partials, p on its Dirichlet DOFs, formed here and not
+// stored; then as b_update_kernel.
+template <typename T>
+__global__ __launch_bounds__(BS) void b_update_mfb_kernel(
+    const int32_t* __restrict__ chunkNode0, const int32_t* __restrict__ chunkSpec,
+    const int32_t* __restrict__ specChunk, const int32_t* __restrict__ specBrick, const int64_t* __restrict__ noff,
+    const int* __restrict__ active, const double* __restrict__ sc, int par, const double* __restrict__ brickPq,
+    const double* __restrict__ pdp, const T* __restrict__ Minv, T* __restrict__ x, T* __restrict__ r,
+    T* __restrict__ z, const T* __restrict__ p, const int32_t* __restrict__ gptr, const T* __restrict__ gF,
+    const uint8_t* __restrict__ dirflag, double* __restrict__ rzp, double* __restrict__ rrp) {
+    __shared__ double sh[2 * (BS / 64)];
+    const int c = blockIdx.x;
+    const int s = chunkSpec[c];
+    if (!active[s]) return;
+    const double pq = chunk_sum(brickPq, specBrick[s], specBrick[s + 1]) +
+                      chunk_sum(pdp, specChunk[s], specChunk[s + 1]);
+    const T alpha = (T)(sc[s * NSC + (par ? RZ2 : RZ)] / pq);
+    const int n = chunkNode0[c] + threadIdx.x;
+    double part[2] = {0.0, 0.0};  // r.z, r.r
+    if (n < noff[s + 1]) {
+        T qv[3] = {(T)0, (T)0, (T)0};
+        const int g1 = gptr[n + 1];
+        for (int k = gptr[n]; k < g1; ++k) {
+            qv[0] += gF[3 * (int64_t)k];
+            qv[1] += gF[3 * (int64_t)k + 1];
+            qv[2] += gF[3 * (int64_t)k + 2];
+        }
+        T rv[3];
+        double rr = 0, rz = 0;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const T pv = p[3 * n + i];
+            x[3 * n + i] += alpha * pv;
+            rv[i] = r[3 * n + i] - alpha * (dirflag[3 * n + i] ? pv : qv[i]);
+            r[3 * n + i] = rv[i];
+            rr += (double)rv[i] * rv[i];
+        }
+        const T* M = Minv + (int64_t)n * 9;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const T zi = M[3 * i] * rv[0] + M[3 * i + 1] * rv[1] + M[3 * i + 2] * rv[2];
+            z[3 * n + i] = zi;
+            rz += (double)rv[i] * zi;
+        }
+        part[0] = rz;
+        part[1] = rr;
+    }
+    wsums<2>(part, sh);
+    if (threadIdx.x == 0) {
+        rzp[c] = part[0];
+        rrp[c] = part[1];
+    }
+}
+
+// b_beta_kernel and b_direction_kernel in one (workgroup per chunk): every workgroup of a specimen
+// forms beta and the stop test from the chunk partials; its first one stores the specimen's scalars.
+// What this kernel stores for the next iteration (r.z, the active flag) it never reads: both
+// alternate with the parity.  Also the Dirichlet p.p partial of the chunk.
+template <typename T>
+__global__ __launch_bounds__(BS) void b_direction_mfb_kernel(
+    const int32_t* __restrict__ chunkNode0, const int32_t* __restrict__ chunkSpec,
+    const int32_t* __restrict__ specChunk, const int64_t* __restrict__ noff, const int* __restrict__ active,
+    int* __restrict__ activeNext, double* __restrict__ sc, int par, const double* __restrict__ rzp,
+    const double* __restrict__ rrp, int* __restrict__ iters, const T* __restrict__ z, T* __restrict__ p,
+    const uint8_t* __restrict__ dirflag, double* __restrict__ pdp) {
+    __shared__ double sh[BS / 64];
+    const int c = blockIdx.x;
+    const int s = chunkSpec[c];
+    const bool first = c == specChunk[s] && threadIdx.x == 0;
+    if (!active[s]) {
+        if (first) activeNext[s] = 0;
+        return;
+    }
+    const double rz = chunk_sum(rzp, specChunk[s], specChunk[s + 1]);
+    const double rr = chunk_sum(rrp, specChunk[s], specChunk[s + 1]);
+    const double rzo = sc[s * NSC + (par ? RZ2 : RZ)];
+    const bool done = rr <= sc[s * NSC + TOL2] || !(rr == rr) || !(rz == rz);
+    if (first) {
+        sc[s * NSC + (par ? RZ : RZ2)] = rz;
+        sc[s * NSC + RR] = rr;
+        iters[s] += 1;
+        activeNext[s] = done ? 0 : 1;
+    }
+    if (done) return;
+    const T beta = (T)(rz / rzo);
+    const int n = chunkNode0[c] + threadIdx.x;
+    double pd[1] = {0.0};
+    if (n < noff[s + 1]) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const T pv = z[3 * n + i] + beta * p[3 * n + i];
+            p[3 * n + i] = pv;
+            if (dirflag[3 * n + i]) pd[0] += (double)pv * pv;
+        }
+    }
+    wsums<1>(pd, sh);
+    if (threadIdx.x == 0) pdp[c] = pd[0];
+}
+
+// Dirichlet p.p chunk partials of the first iteration
+template <typename T>
+__global__ __launch_bounds__(BS) void b_pd_chunk_kernel(const int32_t* __restrict__ chunkNode0,
+                                                        const int32_t* __restrict__ chunkSpec,
+                                                        const int64_t* __restrict__ noff,
+                                                        const int* __restrict__ active, const T* __restrict__ p,
+                                                        const uint8_t* __restrict__ dirflag,
+                                                        double* __restrict__ pdp) {
+    __shared__ double sh[BS / 64];
+    const int c = blockIdx.x;
+    const int s = chunkSpec[c];
+    if (!active[s]) return;
+    const int n = chunkNode0[c] + threadIdx.x;
+    double pd[1] = {0.0};
+    if (n < noff[s + 1])
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            if (dirflag[3 * n + i]) pd[0] += (double)p[3 * n + i] * p[3 * n + i];
+    wsums<1>(pd, sh);
+    if (threadIdx.x == 0) pdp[c] = pd[0];
+}
+
+// one workgroup
+__global__ __launch_bounds__(BS) void b_count_kernel(int S, const int* __restrict__ active,
+                                                     int* __restrict__ nactive) {
+    __shared__ int sh[BS / 64];
     int c = 0;
-    for (int s = 0; s < S; ++s) c += active[s] ? 1 : 0;
-    *nactive = c;
+    for (int s = threadIdx.x; s < S; s += BS) c += active[s] ? 1 : 0;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = c;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int t = 0;
+        for (int i = 0; i < BS / 64; ++i) t += sh[i];
+        *nactive = t;
+    }
 }
 
 template <typename T>
@@ -316,6 +455,24 @@ template <typename T>
 void launch_b_batch(efe_ctx* c, BatchWork* w, hipStream_t st, const T* K, const T* Minv, int batch) {
     const int N = c->N, S = c->nspec;
     T *x = (T*)w->x, *r = (T*)w->r, *z = (T*)w->z, *p = (T*)w->p, *q = (T*)w->q;
+    if (!K && c->mfb) {  // hexa8 bricks
+        const T* gF;
+        if constexpr (sizeof(T) == 8) gF = c->mfbF64;
+        else gF = c->mfbF;
+        for (int j = 0; j < batch; ++j) {
+            const int par = j & 1;
+            int *act = par ? w->active2 : w->active, *next = par ? w->active : w->active2;
+            efe_mf_launch_apply_partials(c, st, p, w->brickPq, nullptr, act);
+            b_update_mfb_kernel<T><<<w->C, BS, 0, st>>>(w->chunkNode0, w->chunkSpec, w->specChunk, w->specBrick,
+                                                        c->specNodeOff, act, w->sc, par, w->brickPq, w->pqp, Minv, x,
+                                                        r, z, p, c->mfbPptr, gF, c->dirflag, w->rzp, w->rrp);
+            b_direction_mfb_kernel<T><<<w->C, BS, 0, st>>>(w->chunkNode0, w->chunkSpec, w->specChunk, c->specNodeOff,
+                                                           act, next, w->sc, par, w->rzp, w->rrp, w->iters, z, p,
+                                                           c->dirflag, w->pqp);
+        }
+        b_count_kernel<<<1, BS, 0, st>>>(S, w->active, w->nactive);
+        return;
+    }
     for (int j = 0; j < batch; ++j) {
         if (K)
             b_spmv_kernel<T><<<gridn(N), BS, 0, st>>>(N, c->specOfNode, w->active, c->slice_off, c->scol,
@@ -329,7 +486,18 @@ void launch_b_batch(efe_ctx* c, BatchWork* w, hipStream_t st, const T* K, const 
         b_beta_kernel<<<S, 64, 0, st>>>(w->specChunk, w->rzp, w->rrp, w->sc, w->active, w->iters);
         b_direction_kernel<T><<<gridn(N), BS, 0, st>>>(N, c->specOfNode, w->active, w->sc, z, p);
     }
-    b_count_kernel<<<1, 1, 0, st>>>(S, w->active, w->nactive);
+    b_count_kernel<<<1, BS, 0, st>>>(S, w->active, w->nactive);
+}
+
+// start of a solve: x = 0, r, z, p, the per-specimen r.z and r.r and the specimens that iterate
+template <typename T>
+void launch_b_init(efe_ctx* c, BatchWork* w, hipStream_t st, const double* b, const T* K, const T* Minv) {
+    b_init_kernel<T><<<gridn(c->N), BS, 0, st>>>(c->N, c->specOfNode, w->active, b, Minv, (T*)w->x, (T*)w->r, (T*)w->z,
+                                                 (T*)w->p, w->nv0, w->nv1);
+    b_init_reduce_kernel<<<c->nspec, BS, 0, st>>>(c->specNodeOff, w->nv0, w->nv1, w->sc, w->active, w->iters);
+    if (!K && c->mfb)
+        b_pd_chunk_kernel<T><<<w->C, BS, 0, st>>>(w->chunkNode0, w->chunkSpec, c->specNodeOff, w->active, (T*)w->p,
+                                                  c->dirflag, w->pqp);
 }
 
 int ensure_batch(efe_ctx* c, int prec) {
@@ -379,6 +547,18 @@ int ensure_batch(efe_ctx* c, int prec) {
         EFE_HIP(hipMemcpyAsync(w->specChunk, sco.data(), sco.size() * sizeof(int32_t), hipMemcpyHostToDevice,
                                c->stream));
         EFE_HIP(hipStreamSynchronize(c->stream));
+        if (c->mfb) {  // bricks hold one specimen's elements, in specimen order
+            std::vector<int32_t> e0((size_t)c->mfbG + 1), order(c->E), se(c->E), sb((size_t)c->nspec + 1, 0);
+            EFE_HIP(hipMemcpy(e0.data(), c->mfbE0, e0.size() * sizeof(int32_t), hipMemcpyDeviceToHost));
+            EFE_HIP(hipMemcpy(order.data(), c->mfbOrder, order.size() * sizeof(int32_t), hipMemcpyDeviceToHost));
+            EFE_HIP(hipMemcpy(se.data(), c->specOfElem, se.size() * sizeof(int32_t), hipMemcpyDeviceToHost));
+            for (int g = 0; g < c->mfbG; ++g) ++sb[se[order[e0[g]]] + 1];
+            for (int sp = 0; sp < c->nspec; ++sp) sb[sp + 1] += sb[sp];
+            EFE_HIP(hipMalloc(&w->specBrick, sb.size() * sizeof(int32_t)));
+            EFE_HIP(hipMemcpy(w->specBrick, sb.data(), sb.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+            EFE_HIP(hipMalloc(&w->brickPq, (size_t)((c->mfbG + 7) & ~7) * sizeof(double)));
+            EFE_HIP(hipMalloc(&w->active2, (size_t)c->nspec * sizeof(int)));
+        }
         EFE_HIP(hipEventCreateWithFlags(&w->evA, hipEventDisableTiming));
         EFE_HIP(hipEventCreateWithFlags(&w->evB, hipEventDisableTiming));
     }
@@ -411,13 +591,13 @@ int batched_pcg_run(efe_ctx* c, const double* b, double* xout, const efe_solve_o
     hipStream_t st = w->ks;
     const int N = c->N, S = c->nspec, D = c->D;
     std::vector<double> sc((size_t)S * NSC, 0.0);
-    b_init_kernel<T><<<gridn(N), BS, 0, st>>>(N, c->specOfNode, w->active, b, Minv, (T*)w->x, (T*)w->r, (T*)w->z,
-                                              (T*)w->p, w->nv0, w->nv1);
-    b_init_reduce_kernel<<<S, BS, 0, st>>>(c->specNodeOff, w->nv0, w->nv1, w->sc, w->active, w->iters);
+    launch_b_init<T>(c, w, st, b, K, Minv);
     EFE_HIP(hipGetLastError());
     int batch = o->check_every > 0 ? o->check_every : 16;
+    if (batch & 1) ++batch;  // the scalars alternate with the iteration's parity
     const int maxit = o->max_iter > 0 ? o->max_iter : 10000;
-    if (!w->graph || w->graph_batch != batch || w->graph_op != o->precision) {
+    const int op = o->precision == EFE_FP64 && !K ? kOpBricks64 : o->precision;
+    if (!w->graph || w->graph_batch != batch || w->graph_op != op) {
         if (w->graph) hipGraphExecDestroy(w->graph);
         w->graph = nullptr;
         hipGraph_t g;
@@ -427,7 +607,7 @@ int batched_pcg_run(efe_ctx* c, const double* b, double* xout, const efe_solve_o
         EFE_HIP(hipGraphInstantiate(&w->graph, g, nullptr, nullptr, 0));
         EFE_HIP(hipGraphDestroy(g));
         w->graph_batch = batch;
-        w->graph_op = o->precision;
+        w->graph_op = op;
     }
     int it = 0;
     info->status = EFE_OK;
@@ -515,7 +695,9 @@ int efe_batched_linsolve(efe_ctx* c, const double* b, double* x, const efe_solve
     if (o->precision == EFE_FP32)
         return batched_pcg<float>(c, b, x, o, spec_tol, spec_rtol, spec_active, spec_iters, info, c->K32,
                                   c->Minv32);
-    return batched_pcg<double>(c, b, x, o, spec_tol, spec_rtol, spec_active, spec_iters, info, c->K64, c->Minv64);
+    // the hexa8 bricks of the FP64 pass (else the assembled operator); see efe_krylov_solve
+    const double* K = efe_mf_bricks64(c, spec_active) ? nullptr : c->K64;
+    return batched_pcg<double>(c, b, x, o, spec_tol, spec_rtol, spec_active, spec_iters, info, K, c->Minv64);
 }
 
 // per-specimen convergence quantities: [max|R|, ||ddU||_inf, ||F||_1, NaN]
@@ -813,9 +995,7 @@ int newton_pass_launch(efe_ctx* c, hipStream_t st, int variant, int prec, bool h
     nr_decide_kernel<<<1, BS, 0, st>>>(S, variant == 2, w->ni, w->nd, w->nout, c->specStatus, w->nopt, w->active,
                                        w->sc, w->ncount);
     if (variant == 1) nr_sub_kernel<<<gd, BS, 0, st>>>(D, w->rhs, w->corr);
-    b_init_kernel<T><<<gridn(N), BS, 0, st>>>(N, c->specOfNode, w->active, w->rhs, Minv, (T*)w->x, (T*)w->r,
-                                              (T*)w->z, (T*)w->p, w->nv0, w->nv1);
-    b_init_reduce_kernel<<<S, BS, 0, st>>>(c->specNodeOff, w->nv0, w->nv1, w->sc, w->active, w->iters);
+    launch_b_init<T>(c, w, st, w->rhs, K, Minv);
     launch_b_batch<T>(c, w, st, K, Minv, batch);
     EFE_HIP(hipGetLastError());
     return EFE_OK;
@@ -844,10 +1024,11 @@ int newton_round(efe_ctx* c, const efe_newton_opts* o, bool hasPExt, bool anyFir
                  const T* K, const T* Minv) {
     BatchWork* w = c->bw;
     hipStream_t st = c->stream;
-    const int batch = o->check_every > 0 ? o->check_every : 16;
+    const int batch = ((o->check_every > 0 ? o->check_every : 16) + 1) & ~1;
+    const int op = o->precision == EFE_FP64 && !K ? kOpBricks64 : o->precision;
     const int maxit = o->krylov_max_iter > 0 ? o->krylov_max_iter : 10000;
     // the PCG batch graph of later batches (also the one efe_linsolve_batched replays)
-    if (!w->graph || w->graph_batch != batch || w->graph_op != o->precision) {
+    if (!w->graph || w->graph_batch != batch || w->graph_op != op) {
         if (w->graph) hipGraphExecDestroy(w->graph);
         w->graph = nullptr;
         hipGraph_t g;
@@ -857,7 +1038,7 @@ int newton_round(efe_ctx* c, const efe_newton_opts* o, bool hasPExt, bool anyFir
         EFE_HIP(hipGraphInstantiate(&w->graph, g, nullptr, nullptr, 0));
         EFE_HIP(hipGraphDestroy(g));
         w->graph_batch = batch;
-        w->graph_op = o->precision;
+        w->graph_op = op;
     }
     for (int pass = 0;; ++pass) {
         if (pass > maxPasses) {
@@ -955,15 +1136,19 @@ int efe_newton_round_batched_impl(efe_ctx* c, double* dU, double* P, double* F, 
     else if (o->precision == EFE_FP32)
         rc = newton_round<float>(c, o, PExt != nullptr, anyFirst, maxPasses, &passes, c->K32, c->Minv32);
     else
-        rc = newton_round<double>(c, o, PExt != nullptr, anyFirst, maxPasses, &passes, c->K64, c->Minv64);
+        // every specimen that solves in the round was computed in it: its tangents are in the bricks
+        rc = newton_round<double>(c, o, PExt != nullptr, anyFirst, maxPasses, &passes, c->mfC64 ? nullptr : c->K64,
+                                  c->Minv64);
     c->stream = home;
     c->useActive = wasActive;
+    c->hostActive.assign(S, 0);  // specActive holds the round's flags now: no pass is known to cover anyone
     if (rc) {
         hipStreamSynchronize(st);
         return rc;
     }
     c->kscrValid = o->precision != EFE_FP32_MATFREE;
     c->pscrValid = true;
+    if (o->precision == EFE_FP64) efe_mf_mark64(c, live);
     c->Kprec = o->precision;
     c->Kversion++;
     c->tot[EFE_T_ELEMENT_PASSES] += passes;
@@ -994,7 +1179,8 @@ void efe_batched_free(efe_ctx* c) {
                     w->nout,   w->pqp,    w->rzp,    w->rrp,        w->chunkNode0, w->chunkSpec,
                     w->specChunk, w->ni,  w->nd,     w->nopt,       w->nout2,      w->ncount,
                     w->du,     w->nP,     w->nF,     w->pext,       w->dtv,        w->dirv,
-                    w->corr,   w->rhs,    w->ddu};
+                    w->corr,   w->rhs,    w->ddu,         w->specBrick,  w->brickPq,
+                    w->active2};
     for (void* p : bufs)
         if (p) hipFree(p);
     for (hipGraphExec_t g : w->ngraph)

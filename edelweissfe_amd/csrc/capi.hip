@@ -488,7 +488,7 @@ int efe_compute_elements(efe_ctx* c, const double* U, const double* dU, const do
     EFE_HIP(hipEventRecord(c->ev[2], c->stream));
     c->kscrValid = precision != EFE_FP32_MATFREE;
     c->pscrValid = true;
-    if (precision == EFE_FP64 && !c->useActive) c->mf64Dir = c->dirVersion;  // a pass over some specimens keeps it
+    if (precision == EFE_FP64) efe_mf_mark64(c, c->useActive ? c->hostActive.data() : nullptr);
     int hs = 0;
     EFE_HIP(hipMemcpyAsync(&hs, c->status, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     EFE_HIP(hipStreamSynchronize(c->stream));
@@ -780,6 +780,7 @@ int efe_set_active_specimens(efe_ctx* c, const uint8_t* active) {
     EFE_HIP(hipMemcpyAsync(c->specActive, a.data(), a.size() * sizeof(int), hipMemcpyHostToDevice, c->stream));
     EFE_HIP(hipStreamSynchronize(c->stream));  // a must outlive the copy
     c->useActive = true;
+    c->hostActive.assign(active, active + c->nspec);
     return EFE_OK;
 }
 

@@ -156,7 +156,10 @@ struct efe_ctx {
     float *mfbEl = nullptr, *mfbF = nullptr;       // [2][G * kBrick] bulk modulus and 2 G; [L][3]
     double *mfbEl64 = nullptr, *mfbF64 = nullptr;
     int dirVersion = 0;          // incremented by every efe_set_dirichlet
-    int mf64Dir = -1;            // dirVersion of the pass whose tangents mfC64 holds (-1: none)
+    // per specimen, the dirVersion of the last FP64 pass over it, whose tangents mfC64 holds (-1: none),
+    // and whether the element passes cover it (efe_set_active_specimens)
+    std::vector<int> mf64Dir;
+    std::vector<uint8_t> hostActive;
     int32_t* elemPos = nullptr;  // [NN][E] index of (e, a) in the node-sorted incidence list nlist
                                  // (force slot of the matrix-free operator; block-row (e, a) of the
                                  // element scratch starts at block elemPos * NN)
@@ -249,8 +252,10 @@ int efe_launch_mf_assembly(efe_ctx* c, double* P, double* F, const double* dir_v
 // hexa8 bricks: the tables on the device (at creation), and the buffers of FP32 or FP64 products
 int efe_mf_upload_bricks(efe_ctx* c, const BrickPattern& bp, const double* coords);
 int efe_mf_alloc_bricks(efe_ctx* c, bool fp64);
-// whether the FP64 CG may run on the bricks: tangents of the last FP64 pass, Dirichlet set unchanged
-bool efe_mf_bricks64(const efe_ctx* c);
+// whether the FP64 CG of the specimens in `which` (null: all) may run on the bricks: tangents of the
+// last FP64 pass, Dirichlet set unchanged since; and: an FP64 pass has covered `which`
+bool efe_mf_bricks64(const efe_ctx* c, const uint8_t* which = nullptr);
+void efe_mf_mark64(efe_ctx* c, const uint8_t* which);
 // hexa8 bricks: the product's node partials (mfbF / mfbF64 over mfbPptr) and per-brick partials of
 // p.Kp; active: per-specimen flags (batched contexts) or null
 void efe_mf_launch_apply_partials(efe_ctx* c, hipStream_t st, const float* p, double* part, const int* flags,

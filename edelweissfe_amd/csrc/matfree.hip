@@ -812,7 +812,18 @@ int efe_mf_alloc_bricks(efe_ctx* c, bool fp64) {
     return EFE_OK;
 }
 
-bool efe_mf_bricks64(const efe_ctx* c) { return c->mfC64 && c->mf64Dir == c->dirVersion; }
+bool efe_mf_bricks64(const efe_ctx* c, const uint8_t* which) {
+    if (!c->mfC64 || c->mf64Dir.empty()) return false;
+    for (int s = 0; s < c->nspec; ++s)
+        if ((!which || which[s]) && c->mf64Dir[s] != c->dirVersion) return false;
+    return true;
+}
+
+void efe_mf_mark64(efe_ctx* c, const uint8_t* which) {
+    c->mf64Dir.resize(c->nspec, -1);
+    for (int s = 0; s < c->nspec; ++s)
+        if (!which || which[s]) c->mf64Dir[s] = c->dirVersion;
+}
 
 int efe_mf_alloc(efe_ctx* c) {
     const int NC = c->mfNC;

@@ -91,3 +91,64 @@ def test_fp64_bricks_follow_a_changed_dirichlet_set():
     sysm.spmv(x, y)
     sysm.close()
     assert rel_err(y.cpu().numpy()[free], b.cpu().numpy()[free]) < 1e-9
+
+
+@pytest.mark.parametrize("precision", ["fp64", "matfree"])
+@pytest.mark.parametrize("sizes", [(1,), (3, 1, 7), (9, 4, 6, 8)])
+def test_batched_bricks_solve_every_specimen_as_alone(sizes, precision):
+    """The batched PCG on the bricks against each specimen's own context, which runs the same
+    bricks: the same solutions to round-off (FP64: both to 1e-13 of b, 1e-9 as above; FP32: 1e-7
+    of b, within 2e-4 = condition number times that), excluded specimens zero; in FP64 also against
+    the assembled operator, which a set of Dirichlet DOFs set after the pass leaves."""
+    from edelweissfe_amd import _lib
+    from edelweissfe_amd.device import DeviceSystem
+
+    prec, rtol, tol = ((_lib.EFE_FP64, 1e-13, 1e-9) if precision == "fp64" else (_lib.EFE_FP32_MATFREE, 1e-7, 2e-4))
+    models = [device_model((m, m, m), (1.0, 1.0, 1.0), "C3D8", "vonmises", J2, jitter=0.1, seed=i)
+              for i, m in enumerate(sizes)]
+    S = len(models)
+    off = np.concatenate([[0], np.cumsum([m.nNodes for m in models])])
+    coords = np.concatenate([m.coordinates for m in models])
+    conn = np.concatenate([m.connectivity + o for m, o in zip(models, off)])
+    batch = DeviceSystem(coords, conn, "C3D8", "vonmises", J2, n_specimens=S,
+                         specimen_of_node=np.repeat(np.arange(S), np.diff(off)).astype(np.int32))
+    rng = np.random.default_rng(7)
+    dirs = [np.r_[m.dofsOfNodeSet("gen_bottom"), m.dofsOfNodeSet("gen_top", [1])] for m in models]
+    alld = np.concatenate([d + 3 * o for d, o in zip(dirs, off)])
+    dU = rng.uniform(-1, 1, batch.n_dof) * 1e-3
+    b = rng.standard_normal(batch.n_dof)
+    act = np.ones(S, np.uint8)
+    if S > 2:
+        act[1] = 0
+
+    def solve():
+        x = batch.zeros()
+        info, its = batch.linsolve_batched(torch.as_tensor(b, device="cuda"), x, np.zeros(S), act, precision=prec,
+                                           rtol=rtol, check_every=7)
+        assert info.status == 0 and (its[act != 0] > 0).all()
+        return x.cpu().numpy()
+
+    P, F = batch.zeros(), batch.zeros()
+    batch.set_dirichlet(alld)
+    batch.compute_elements(torch.as_tensor(dU, device="cuda"), P, F, precision=prec)
+    x = solve()
+    if precision == "fp64":
+        batch.set_dirichlet(alld)
+        xa = solve()
+    for s, m in enumerate(models):
+        sl = slice(3 * off[s], 3 * off[s + 1])
+        free = np.ones(3 * m.nNodes, bool)
+        free[np.unique(dirs[s])] = False
+        if not act[s]:
+            assert (x[sl][free] == 0.0).all()
+            continue
+        one = DeviceSystem(m.coordinates, m.connectivity, "C3D8", "vonmises", J2)
+        one.set_dirichlet(dirs[s])
+        P1, F1, x1 = one.zeros(), one.zeros(), one.zeros()
+        one.compute_elements(torch.as_tensor(dU[sl], device="cuda"), P1, F1, precision=prec)
+        assert one.linsolve(torch.as_tensor(b[sl], device="cuda"), x1, precision=prec, rtol=rtol).status == 0
+        one.close()
+        assert rel_err(x[sl], x1.cpu().numpy()) < tol
+        if precision == "fp64":
+            assert rel_err(xa[sl], x1.cpu().numpy()) < tol
+    batch.close()
