@@ -548,11 +548,9 @@ int ensure_batch(efe_ctx* c, int prec) {
                                c->stream));
         EFE_HIP(hipStreamSynchronize(c->stream));
         if (c->mfb) {  // bricks hold one specimen's elements, in specimen order
-            std::vector<int32_t> e0((size_t)c->mfbG + 1), order(c->E), se(c->E), sb((size_t)c->nspec + 1, 0);
-            EFE_HIP(hipMemcpy(e0.data(), c->mfbE0, e0.size() * sizeof(int32_t), hipMemcpyDeviceToHost));
-            EFE_HIP(hipMemcpy(order.data(), c->mfbOrder, order.size() * sizeof(int32_t), hipMemcpyDeviceToHost));
-            EFE_HIP(hipMemcpy(se.data(), c->specOfElem, se.size() * sizeof(int32_t), hipMemcpyDeviceToHost));
-            for (int g = 0; g < c->mfbG; ++g) ++sb[se[order[e0[g]]] + 1];
+            std::vector<int32_t> spec(c->mfbG), sb((size_t)c->nspec + 1, 0);
+            EFE_HIP(hipMemcpy(spec.data(), c->mfbSpec, spec.size() * sizeof(int32_t), hipMemcpyDeviceToHost));
+            for (int32_t sp : spec) ++sb[sp + 1];
             for (int sp = 0; sp < c->nspec; ++sp) sb[sp + 1] += sb[sp];
             EFE_HIP(hipMalloc(&w->specBrick, sb.size() * sizeof(int32_t)));
             EFE_HIP(hipMemcpy(w->specBrick, sb.data(), sb.size() * sizeof(int32_t), hipMemcpyHostToDevice));

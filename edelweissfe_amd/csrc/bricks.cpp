@@ -178,19 +178,19 @@ void efe_build_bricks(BrickPattern& bp, int N, int E, const int32_t* conn, const
         if (h > 0.0 && std::isfinite(h))
             for (int e = 0; e < E; ++e) cen[(size_t)k * E + e] = (float)(cen[(size_t)k * E + e] / h);
     }
-    bp.order.resize(E);
-    for (int e = 0; e < E; ++e) bp.order[e] = e;
+    std::vector<int32_t> order(E);
+    for (int e = 0; e < E; ++e) order[e] = e;
     std::vector<int> seg;  // a brick holds elements of one specimen
     if (specOfNode) {
         auto spec = [&](int e) { return specOfNode[conn[(size_t)8 * e]]; };
-        std::stable_sort(bp.order.begin(), bp.order.end(), [&](int32_t a, int32_t b) { return spec(a) < spec(b); });
+        std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) { return spec(a) < spec(b); });
         for (int i = 0; i < E; ++i)
-            if (i == 0 || spec(bp.order[i]) != spec(bp.order[i - 1])) seg.push_back(i);
+            if (i == 0 || spec(order[i]) != spec(order[i - 1])) seg.push_back(i);
     } else {
         seg.push_back(0);
     }
     seg.push_back(E);
-    Splitter sp{cen, bp.order, E};
+    Splitter sp{cen, order, E};
     std::vector<Brick> bricks;
     if (seg.size() == 2) {
         grow(sp, 0, E, conn, bricks, 3);
@@ -206,30 +206,27 @@ void efe_build_bricks(BrickPattern& bp, int N, int E, const int32_t* conn, const
         for (auto& v : per)
             bricks.insert(bricks.end(), std::make_move_iterator(v.begin()), std::make_move_iterator(v.end()));
     }
-    const int G = (int)bricks.size();
-    bp.e0.assign(1, 0);
-    bp.lptr.assign(1, 0);
-    for (const Brick& b : bricks) {
-        bp.e0.push_back(b.hi);
-        bp.lptr.push_back(bp.lptr.back() + (int32_t)b.nodes.size());
-    }
-    const size_t L = bp.lptr.back();
+    const int G = bp.G = (int)bricks.size();
+    // tables at a fixed pitch per brick, so that a workgroup finds its own without reading offsets
     bp.pos.resize(E);
-    bp.lnode.resize(L);
-    bp.lpos.resize(L);
-    bp.linc.resize(L * 8);
-    bp.lidx.resize((size_t)E * 8);
+    bp.lidx.assign((size_t)G * kBrick * 8, 0xffff);
+    bp.lnode.assign((size_t)G * kBrickNodes, -1);
+    bp.lpos.assign((size_t)G * kBrickNodes, 0);
+    bp.linc.assign((size_t)G * kBrickNodes * 8, 0xffff);
     bp.pptr.assign(N + 1, 0);
     for (int g = 0; g < G; ++g) {
         const Brick& b = bricks[g];
-        std::copy(b.nodes.begin(), b.nodes.end(), bp.lnode.begin() + bp.lptr[g]);
-        std::copy(b.linc.begin(), b.linc.end(), bp.linc.begin() + (size_t)bp.lptr[g] * 8);
-        std::copy(b.lidx.begin(), b.lidx.end(), bp.lidx.begin() + (size_t)b.lo * 8);
-        for (int i = b.lo; i < b.hi; ++i) bp.pos[bp.order[i]] = g * kBrick + (i - b.lo);
+        std::copy(b.nodes.begin(), b.nodes.end(), bp.lnode.begin() + (size_t)g * kBrickNodes);
+        std::copy(b.linc.begin(), b.linc.end(), bp.linc.begin() + (size_t)g * kBrickNodes * 8);
+        std::copy(b.lidx.begin(), b.lidx.end(), bp.lidx.begin() + (size_t)g * kBrick * 8);
+        for (int i = b.lo; i < b.hi; ++i) bp.pos[order[i]] = g * kBrick + (i - b.lo);
         for (int32_t nd : b.nodes) ++bp.pptr[nd + 1];
+        if (specOfNode) bp.spec.push_back(specOfNode[b.nodes[0]]);
     }
     // partial slots in node order, the bricks of a node in ascending order
     for (int n = 0; n < N; ++n) bp.pptr[n + 1] += bp.pptr[n];
+    bp.L = bp.pptr[N];
     std::vector<int32_t> next(bp.pptr.begin(), bp.pptr.end() - 1);
-    for (size_t i = 0; i < L; ++i) bp.lpos[i] = next[bp.lnode[i]]++;
+    for (size_t i = 0; i < bp.lnode.size(); ++i)
+        if (bp.lnode[i] >= 0) bp.lpos[i] = next[bp.lnode[i]]++;
 }

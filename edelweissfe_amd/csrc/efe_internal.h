@@ -67,16 +67,16 @@ constexpr int kBrick = 256;
 constexpr int kBrickNodes = 512;
 
 struct BrickPattern {
-    std::vector<int32_t> e0;      // [G+1] first element (of `order`) of each brick
-    std::vector<int32_t> order;   // [E] elements brick by brick, ascending inside a brick
-    std::vector<int32_t> pos;     // [E] element -> brick * kBrick + its place in the brick
-    std::vector<int32_t> lptr;    // [G+1] first staged node of each brick
-    std::vector<int32_t> lnode;   // [L] node of each staged entry (a node with more than 8 incidences
-                                  // in a brick has several entries)
-    std::vector<int32_t> lpos;    // [L] its slot among the node's partials
+    int G = 0;
+    int64_t L = 0;                // partials: (brick, node) pairs
+    std::vector<int32_t> pos;     // [E] element -> brick * kBrick + its place (ascending in a brick)
+    std::vector<uint16_t> lidx;   // [G * kBrick][8] staged entries of the element there, 0xffff: none
+    std::vector<int32_t> lnode;   // [G * kBrickNodes] node of each staged entry, -1: none (a node with
+                                  // more than 8 incidences in a brick has several entries)
+    std::vector<int32_t> lpos;    // [G * kBrickNodes] its slot among the node's partials
+    std::vector<uint16_t> linc;   // [G * kBrickNodes][8] incidences a * kBrick + t, element order, 0xffff: none
     std::vector<int32_t> pptr;    // [N+1] partials of each node, in brick order
-    std::vector<uint16_t> linc;   // [L][8] incidences a * kBrick + t in element order, 0xffff: none
-    std::vector<uint16_t> lidx;   // [E][8] staged entries of the elements of `order`
+    std::vector<int32_t> spec;    // [G] specimen of each brick (specimens given)
 };
 
 // conn [E][8], coords [N][3], specOfNode [N] or null (a brick then holds one specimen's elements)
@@ -147,12 +147,11 @@ struct efe_ctx {
     // coordinates, and the partial forces [L][3] in the precision of the product
     bool mfb = false;
     int mfbG = 0;                // bricks
-    int64_t mfbL = 0;            // staged nodes over all bricks
+    int64_t mfbL = 0;            // partials
     void* mfbTables = nullptr;   // one allocation: the tables below
-    int32_t *mfbE0 = nullptr, *mfbOrder = nullptr, *mfbPos = nullptr;
-    int32_t *mfbLptr = nullptr, *mfbLnode = nullptr, *mfbLpos = nullptr, *mfbPptr = nullptr;
+    int32_t *mfbPos = nullptr, *mfbLnode = nullptr, *mfbLpos = nullptr, *mfbPptr = nullptr, *mfbSpec = nullptr;
     uint16_t *mfbLinc = nullptr, *mfbLidx = nullptr;
-    double* mfbX = nullptr;      // [3][L]
+    double* mfbX = nullptr;      // [3][G * kBrickNodes]
     float *mfbEl = nullptr, *mfbF = nullptr;       // [2][G * kBrick] bulk modulus and 2 G; [L][3]
     double *mfbEl64 = nullptr, *mfbF64 = nullptr;
     int dirVersion = 0;          // incremented by every efe_set_dirichlet

@@ -374,16 +374,16 @@ __device__ __forceinline__ void brick_qps(const T* __restrict__ Cg, T bulk, T sh
 
 // What a workgroup of the brick product reads besides the tangents (bricks.cpp).
 struct BrickTables {
-    const int32_t *lptr, *lnode, *lpos, *e0;
+    const int32_t *lnode, *lpos, *spec;
     const uint16_t *linc, *lidx;
-    const double* X;   // [3][L] coordinates of the staged nodes
-    int64_t L;
+    const double* X;  // [3][G * kBrickNodes] coordinates of the staged nodes
     int G, hot;
 };
 
 // Hexa8 product by bricks: workgroup g takes the up to kBrick elements of brick g, one lane each.
 // The brick's distinct nodes (p with Dirichlet DOFs masked, and the coordinates, which lie in
-// staging order) go to LDS once; each lane forms its element's forces in the monomial basis and
+// staging order) go to LDS once, after two dependent loads (the node, then its values: the tables
+// have a fixed pitch, and the flags are waited for beside them); each lane forms its element's forces in the monomial basis and
 // leaves them in LDS; each staged node's forces are summed in element order into one partial
 // per (brick, node), stored at its slot of the node-ordered partial list.
 //
@@ -396,8 +396,7 @@ template <int NC, typename T, typename TP>
 __global__ __launch_bounds__(kBrick) void brick_apply_kernel(
     BrickTables bt, const T* __restrict__ el, const T* __restrict__ C, const TP* __restrict__ p,
     const uint8_t* __restrict__ dirflag, int mask, const int* __restrict__ flags, T* __restrict__ Fpart,
-    const int* __restrict__ active, const int32_t* __restrict__ order, const int32_t* __restrict__ specOfElem,
-    double* __restrict__ part) {
+    const int* __restrict__ active, double* __restrict__ part) {
     // LDS, reused: first the staged nodes (x 3 doubles, p 3 T), then the element forces (24 T a lane)
     constexpr int kStage = 3 * kBrickNodes * (int)(sizeof(double) + sizeof(T));
     constexpr int kForce = 24 * kBrick * (int)sizeof(T);
@@ -406,33 +405,38 @@ __global__ __launch_bounds__(kBrick) void brick_apply_kernel(
     double* sx = (double*)lds;
     T* sp = (T*)(lds + 3 * kBrickNodes * sizeof(double));
     T* sf = (T*)lds;
-    if (flags && flags[0]) return;
     const int g = xcd_block_mf();
     if (g >= bt.G) {  // the grid is rounded up to a multiple of 8
         if (part && threadIdx.x == 0) part[g] = 0.0;
         return;
     }
-    const int eb = bt.e0[g], ne = bt.e0[g + 1] - eb;
-    // batched solves: a brick of a frozen specimen leaves its partials alone (nobody reads them)
-    if (active && !active[specOfElem[order[eb]]]) return;
+    constexpr int NS = kBrickNodes / kBrick;  // staged nodes per lane
     const int t = threadIdx.x;
-    const int l0 = bt.lptr[g], nl = bt.lptr[g + 1] - l0;
-    for (int i = t; i < nl; i += kBrick) {
-        const int nd = bt.lnode[l0 + i];
+    const int64_t l0 = (int64_t)g * kBrickNodes + t;
+    int nd[NS];
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            T v = (T)p[3 * nd + c];
-            if (mask && dirflag[3 * nd + c]) v = (T)0;
-            sp[c * kBrickNodes + i] = v;
-            sx[c * kBrickNodes + i] = bt.X[c * bt.L + l0 + i];
+    for (int k = 0; k < NS; ++k) nd[k] = bt.lnode[l0 + k * kBrick];
+    // the element's 8 staged entries in one 16-byte load; 0xffff: no element for this lane
+    const uint4 li4 = *reinterpret_cast<const uint4*>(bt.lidx + ((int64_t)g * kBrick + t) * 8);
+    const T bulk = NC != 10 ? el[g * kBrick + t] : (T)0;
+    const T shear2 = NC == 0 ? el[(int64_t)bt.G * kBrick + g * kBrick + t] : (T)0;
+    if (flags && flags[0]) return;
+    // batched solves: a brick of a frozen specimen leaves its partials alone (nobody reads them)
+    if (active && !active[bt.spec[g]]) return;
+#pragma unroll
+    for (int k = 0; k < NS; ++k)
+        if (nd[k] >= 0) {
+            const int i = t + k * kBrick;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                T v = (T)p[3 * (int64_t)nd[k] + c];
+                if (mask && dirflag[3 * (int64_t)nd[k] + c]) v = (T)0;
+                sp[c * kBrickNodes + i] = v;
+                sx[c * kBrickNodes + i] = bt.X[(int64_t)c * bt.G * kBrickNodes + l0 + k * kBrick];
+            }
         }
-    }
-    const bool live = t < ne;
+    const bool live = (li4.x & 0xffffu) != 0xffffu;
     const T* Cg = C + (int64_t)g * (8 * NC * kBrick) + t;
-    const T bulk = NC != 10 && live ? el[g * kBrick + t] : (T)0;
-    const T shear2 = NC == 0 && live ? el[(int64_t)bt.G * kBrick + g * kBrick + t] : (T)0;
-    // 8 local indices in one 16-byte load
-    const uint4 li4 = live ? *reinterpret_cast<const uint4*>(bt.lidx + (int64_t)(eb + t) * 8) : uint4{0, 0, 0, 0};
     __syncthreads();
     T cp[3][8], cx[3][8];
     if (live) {
@@ -459,6 +463,15 @@ __global__ __launch_bounds__(kBrick) void brick_apply_kernel(
     // with part given: the brick's sum of p_e . f_e (its share of p . K p), formed in the
     // monomial basis: f = H^T fa / 8 and cp = H p / 8 with H H = 8 I give p . f = cp . fa
     double en = 0.0;
+    uint4 inc[NS];
+    int lp[NS];
+    auto load_lists = [&] {  // of the staged nodes, for the sums at the end
+#pragma unroll
+        for (int k = 0; k < NS; ++k) {
+            inc[k] = *reinterpret_cast<const uint4*>(bt.linc + (l0 + k * kBrick) * 8);
+            lp[k] = bt.lpos[l0 + k * kBrick];
+        }
+    };
     if (live) {
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
@@ -482,6 +495,7 @@ __global__ __launch_bounds__(kBrick) void brick_apply_kernel(
             for (int i = 0; i < 3; ++i)
 #pragma unroll
                 for (int k = 0; k < 8; ++k) en += (double)cp[i][k] * (double)fa[i][k];
+        load_lists();
 #pragma unroll
         for (int i = 0; i < 3; ++i) walsh3_t(fa[i]);
         // forces [i][a][t]: consecutive lanes in consecutive banks
@@ -491,12 +505,15 @@ __global__ __launch_bounds__(kBrick) void brick_apply_kernel(
 #pragma unroll
             for (int i = 0; i < 3; ++i) sf[(i * 8 + a) * kBrick + t] = (T)0.125 * fa[i][k];
         }
+    } else {
+        load_lists();
     }
     __syncthreads();
     // one partial per staged node: its up to 8 incidences in element order
-    for (int i = t; i < nl; i += kBrick) {
-        const uint4 w4 = *reinterpret_cast<const uint4*>(bt.linc + (int64_t)(l0 + i) * 8);
-        const uint32_t w[4] = {w4.x, w4.y, w4.z, w4.w};
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+        if (nd[k] < 0) continue;
+        const uint32_t w[4] = {inc[k].x, inc[k].y, inc[k].z, inc[k].w};
         T f0 = (T)0, f1 = (T)0, f2 = (T)0;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
@@ -507,7 +524,7 @@ __global__ __launch_bounds__(kBrick) void brick_apply_kernel(
                 f2 += sf[16 * kBrick + s];
             }
         }
-        T* dst = Fpart + (int64_t)bt.lpos[l0 + i] * 3;
+        T* dst = Fpart + (int64_t)lp[k] * 3;
         dst[0] = f0;
         dst[1] = f1;
         dst[2] = f2;
@@ -671,8 +688,8 @@ void launch_bricks(efe_ctx* c, hipStream_t st, const TP* p, int mask, const int*
     const int64_t rest = c->mfbL * (int64_t)(48 + 3 * sizeof(T)) + (int64_t)c->E * (16 + sizeof(T)) +
                          (int64_t)c->N * 21 * (int64_t)sizeof(T);
     const bool hot = tangents > (int64_t)24e6 && tangents + rest <= (int64_t)216e6;
-    const BrickTables bt{c->mfbLptr, c->mfbLnode, c->mfbLpos, c->mfbE0, c->mfbLinc, c->mfbLidx, c->mfbX, c->mfbL,
-                         c->mfbG, hot ? c->mfbG : 0};
+    const BrickTables bt{c->mfbLnode, c->mfbLpos, c->mfbSpec, c->mfbLinc, c->mfbLidx, c->mfbX,
+                         c->mfbG,     hot ? c->mfbG : 0};
     const int grid = round8_mf(c->mfbG);
     const T *el, *C;
     T* F;
@@ -685,7 +702,7 @@ void launch_bricks(efe_ctx* c, hipStream_t st, const TP* p, int mask, const int*
         C = c->mfC;
         F = c->mfbF;
     }
-#define BRICK_ARGS bt, el, C, p, c->dirflag, mask, flags, F, active, c->mfbOrder, c->specOfElem, part
+#define BRICK_ARGS bt, el, C, p, c->dirflag, mask, flags, F, active, part
     if (c->mfNC == 10) {
         if constexpr (sizeof(T) == 4) brick_apply_kernel<10, T, TP><<<grid, kBrick, 0, st>>>(BRICK_ARGS);
     } else if (c->mfNC == 7) {
@@ -764,20 +781,20 @@ int build_moduli(efe_ctx* c, T** dst) {
 // bricks, whose state lies in runs of ~8 elements, took the 64^3 tangent pass from 0.87 to 1.06 ms.)
 // One allocation and one copy hold them all.
 int efe_mf_upload_bricks(efe_ctx* c, const BrickPattern& bp, const double* coords) {
-    const int64_t L = (int64_t)bp.lnode.size();
-    std::vector<double> X((size_t)3 * L);
-    for (int64_t i = 0; i < L; ++i)
-        for (int k = 0; k < 3; ++k) X[(size_t)k * L + i] = coords[(size_t)3 * bp.lnode[i] + k];
+    const size_t L = bp.lnode.size();
+    std::vector<double> X(3 * L, 0.0);
+    for (size_t i = 0; i < L; ++i)
+        if (bp.lnode[i] >= 0)
+            for (int k = 0; k < 3; ++k) X[k * L + i] = coords[(size_t)3 * bp.lnode[i] + k];
     struct Part {
         const void* src;
         size_t bytes;
         void** dst;
     };
     auto part = [](const auto& v, auto** dst) { return Part{v.data(), v.size() * sizeof(v[0]), (void**)dst}; };
-    const Part parts[] = {part(bp.e0, &c->mfbE0),       part(bp.order, &c->mfbOrder), part(bp.pos, &c->mfbPos),
-                          part(bp.lptr, &c->mfbLptr),   part(bp.lnode, &c->mfbLnode), part(bp.lpos, &c->mfbLpos),
-                          part(bp.pptr, &c->mfbPptr),   part(bp.linc, &c->mfbLinc),   part(bp.lidx, &c->mfbLidx),
-                          part(X, &c->mfbX)};
+    const Part parts[] = {part(bp.pos, &c->mfbPos),   part(bp.lnode, &c->mfbLnode), part(bp.lpos, &c->mfbLpos),
+                          part(bp.pptr, &c->mfbPptr), part(bp.linc, &c->mfbLinc),   part(bp.lidx, &c->mfbLidx),
+                          part(bp.spec, &c->mfbSpec), part(X, &c->mfbX)};
     size_t total = 0;
     for (const Part& q : parts) total += (q.bytes + 255) & ~(size_t)255;
     std::vector<char> host(total);
@@ -789,8 +806,8 @@ int efe_mf_upload_bricks(efe_ctx* c, const BrickPattern& bp, const double* coord
         off += (q.bytes + 255) & ~(size_t)255;
     }
     EFE_HIP(hipMemcpy(c->mfbTables, host.data(), total, hipMemcpyHostToDevice));
-    c->mfbL = L;
-    c->mfbG = (int)bp.e0.size() - 1;
+    c->mfbL = bp.L;
+    c->mfbG = bp.G;
     c->mfb = true;
     return EFE_OK;
 }
