@@ -4,9 +4,10 @@
 //
 // Block ILU(0): the zero-fill incomplete factorisation on the 3x3-block pattern of K, in
 // the elimination order (color, node) of a greedy coloring of the node graph.  The
-// factor is kept in block CSR with rows in that order, so every color is one contiguous
+// factor is formed in block CSR with rows in that order, so every color is one contiguous
 // range of mutually independent rows: the factorisation and both triangular sweeps take
-// one launch per color (8 on a hexa8 grid) instead of one per dependency level.
+// one launch per color (8 on a hexa8 grid) instead of one per dependency level.  The sweeps
+// read a copy of it in slices.
 //
 // GMRES: right preconditioning (the Arnoldi residual is the true residual of K x = b),
 // classical Gram-Schmidt with one re-orthogonalisation (all projections of a step in one
@@ -20,13 +21,21 @@
 
 #include "efe_internal.h"
 
+// One color of a sweep: slices of 64 / G rows by decreasing length, so step k belongs to the first
+// count[k] slices, at base[k] + slice; kernel arguments, so that no load waits for an offset.
+constexpr int kSweepLevels = 8;
+struct SweepColor {
+    int slices = 0, levels = 0, row0 = 0, more = 0, G = 0;  // more: first of levels kSweepLevels.. in Sweep::more
+    int base[kSweepLevels] = {}, count[kSweepLevels] = {};
+};
+
 struct GmresWork {
     int D = 0, N = 0, m = 0, nwg = 0;
     // ILU structure
     bool ilu_ready = false;
     int ncolors = 0;
     std::vector<int> cstart;
-    std::vector<int> clow, cup;  // per color: most blocks before / after the diagonal in a row
+    std::vector<int> cup;  // per color: most blocks after the diagonal in a row
     int32_t *fptr = nullptr, *fcol = nullptr, *fidx = nullptr, *dslot = nullptr, *perm = nullptr;
     int64_t nbF = 0;
     int maxUpper = 0;  // most blocks in a row's upper part
@@ -34,14 +43,23 @@ struct GmresWork {
     double *F64 = nullptr, *Dinv64 = nullptr;
     float *F32 = nullptr, *Dinv32 = nullptr;
     int factored_version[2] = {-1, -1};
+    // the sweeps' copy of the factor: [0] the blocks before the diagonal, [1] those after it
+    struct Sweep {
+        std::vector<SweepColor> color;
+        int64_t steps = 0;
+        int2* rows = nullptr;          // [slices][64/G] (node, factor row), node -1: none
+        int2* more = nullptr;          // levels past SweepColor's own: (first step, slices)
+        int32_t *col = nullptr, *src = nullptr;  // [steps][64] node of the entry (kNoBlock: none), its block
+        double* v64 = nullptr;         // [steps][9][64]
+        float* v32 = nullptr;
+    } sweep[2];
     // Krylov basis and work vectors (one precision at a time)
     void* V = nullptr;   // [(m+1)][D]
     void* w = nullptr;
     void* z = nullptr;
     void* x = nullptr;
-    void* t = nullptr;   // permuted vector for the ILU sweeps
     int vprec = -1;
-    double* part = nullptr;  // [(m+1)][nwg]
+    double *part = nullptr, *pnorm = nullptr;  // [(m+1)][nwg]; behind it the partial norms
     double* hdev = nullptr;  // [3][m+2]: h1, h2, norm
     double* hhost = nullptr; // pinned
     hipStream_t ks = nullptr;
@@ -358,29 +376,6 @@ __global__ __launch_bounds__(BS) void ilu_factor_reg_kernel(int r0, int r1, cons
     }
 }
 
-// t = perm(v): t[factor row i] = v[node perm[i]]
-template <typename T>
-__global__ void permute_in_kernel(int N, const int32_t* __restrict__ perm, const T* __restrict__ v,
-                                  T* __restrict__ t) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    const int n = perm[i];
-    t[3 * i] = v[3 * n];
-    t[3 * i + 1] = v[3 * n + 1];
-    t[3 * i + 2] = v[3 * n + 2];
-}
-
-template <typename T>
-__global__ void permute_out_kernel(int N, const int32_t* __restrict__ perm, const T* __restrict__ t,
-                                   T* __restrict__ v) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    const int n = perm[i];
-    v[3 * n] = t[3 * i];
-    v[3 * n + 1] = t[3 * i + 1];
-    v[3 * n + 2] = t[3 * i + 2];
-}
-
 // Sum of the 3-vectors of a group of G lanes (fixed butterfly order).
 template <typename T, int G>
 __device__ __forceinline__ void group_sum3(T& a, T& b, T& c) {
@@ -392,98 +387,144 @@ __device__ __forceinline__ void group_sum3(T& a, T& b, T& c) {
     }
 }
 
-// forward sweep of one color: t_i -= sum_{k before i} L_ik t_k (unit block-lower);
-// G lanes per row, each over every G-th block of the row's lower part.  A lane takes U of its
-// blocks at a time: their column indices, then the t entries they name, then the blocks are
-// loaded together, so one pass costs two dependent memory round trips, not two per block.
-// Each lane adds its blocks in the same order as one at a time.
-// With Dinv given (the last color, whose rows have no blocks after them), the backward sweep's
-// t_i = Dinv_i (t_i - 0) follows in the same launch.
-template <typename T, int G, int U>
-__global__ __launch_bounds__(BS) void ilu_lower_kernel(int r0, int r1, const int32_t* __restrict__ fptr,
-                                                       const int32_t* __restrict__ fcol,
-                                                       const int32_t* __restrict__ dslot, const T* __restrict__ F,
-                                                       T* __restrict__ t, const T* __restrict__ Dinv) {
-    const int tid = blockIdx.x * BS + threadIdx.x;
-    const int i = r0 + tid / G, lane = tid % G;
-    if (i >= r1) return;
-    const int b0 = fptr[i], d = b0 + dslot[i];
-    T y0 = 0, y1 = 0, y2 = 0;
-    for (int kb0 = b0 + lane; kb0 < d; kb0 += G * U) {
-        int kk[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) kk[u] = kb0 + u * G < d ? fcol[kb0 + u * G] : -1;
-        T x[U][3];
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-            for (int c = 0; c < 3; ++c) x[u][c] = kk[u] >= 0 ? t[3 * kk[u] + c] : (T)0;
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (kk[u] < 0) break;
-            const T* a = F + (int64_t)(kb0 + u * G) * 9;
-            y0 += a[0] * x[u][0] + a[1] * x[u][1] + a[2] * x[u][2];
-            y1 += a[3] * x[u][0] + a[4] * x[u][1] + a[5] * x[u][2];
-            y2 += a[6] * x[u][0] + a[7] * x[u][1] + a[8] * x[u][2];
-        }
+// ---- triangular sweeps ---------------------------------------------------------------------------
+//
+// A color is 1/20 of a hexa20 mesh's rows (1/8 of hexa8's) and must be complete before the next one
+// starts, so at ordinary sizes a sweep is bound by the latency of its launches: each of the 38 per
+// application waits for its dependent loads and little else.  The sweeps therefore read a copy of
+// the factor in the order they take it: a wavefront has a slice of 64 / G rows, sorted by length
+// within the color, G lanes per row; its blocks lie in steps of 64 (one per lane), a block's 9 values
+// 64 apart, and where a step lies follows from the kernel's arguments.  Nodes, columns and values
+// then take one round of loads, each contiguous over the wavefront, and the entries of z, the row's
+// own values and its Dinv a second.  z is in node order and takes the forward values in place (color
+// 0 has none: its rows read v), so that no vector is permuted.  A CU fills its L1 at 64 bytes a cycle,
+// so few workgroups per color leave most of that idle: a wavefront is a workgroup of its own, and G
+// is the smallest of 8, 16 and 32 with which a row's blocks take one batch of kSweepUnroll steps (a
+// second batch is a third round of loads).  hexa20R FP64, GMRES iteration 24 x 22 x 20 / 8 x 8 x 8:
+// row pointers, columns, z and strided 72-byte blocks in turn 309 / 257 us; this layout in
+// workgroups of 4 wavefronts, G = 16 314 / 247; of one 297 / 219 (G = 32 throughout 310 / 217; next
+// color's lines fetched into the L2 by further workgroups 297 / 216 but 697 for 613 at 40 x 36 x 32).
+
+constexpr int32_t kNoBlock = INT32_MIN;
+constexpr int kSweepUnroll = 4;  // steps loaded together
+
+__device__ __forceinline__ int2 sweep_level(const SweepColor& sc, const int2* more, int k) {
+    return k < kSweepLevels ? make_int2(sc.base[k], sc.count[k]) : more[sc.more + k - kSweepLevels];
+}
+
+// col and src of every entry of a color's slices: entry (step k, lane) is block G k + lane of the row
+// (before the diagonal: from the row's first; after it: from the one after the diagonal).  Columns of
+// color 0 (factor rows below c1) are marked -1 - node in the forward sweep.
+template <int G>
+__global__ __launch_bounds__(BS) void sweep_fill_kernel(SweepColor sc, int upper, int c1, const int2* __restrict__ more,
+                                                        const int2* __restrict__ rows,
+                                                        const int32_t* __restrict__ fptr,
+                                                        const int32_t* __restrict__ fcol,
+                                                        const int32_t* __restrict__ dslot,
+                                                        const int32_t* __restrict__ perm, int32_t* __restrict__ col,
+                                                        int32_t* __restrict__ src) {
+    const int w = (blockIdx.x * BS + threadIdx.x) / 64, lane = threadIdx.x & 63;
+    if (w >= sc.slices) return;
+    const int2 rw = rows[sc.row0 + w * (64 / G) + lane / G];
+    int b = 0, e = 0;
+    if (rw.x >= 0) {
+        const int d = fptr[rw.y] + dslot[rw.y];
+        b = upper ? d + 1 : fptr[rw.y];
+        e = upper ? fptr[rw.y + 1] : d;
     }
-    group_sum3<T, G>(y0, y1, y2);
-    if (lane == 0) {
-        y0 = t[3 * i] - y0;
-        y1 = t[3 * i + 1] - y1;
-        y2 = t[3 * i + 2] - y2;
-        if (Dinv) {
-            const T* m = Dinv + (int64_t)i * 9;
-            const T z0 = y0 - (T)0, z1 = y1 - (T)0, z2 = y2 - (T)0;  // as the backward sweep forms them
-            y0 = m[0] * z0 + m[1] * z1 + m[2] * z2;
-            y1 = m[3] * z0 + m[4] * z1 + m[5] * z2;
-            y2 = m[6] * z0 + m[7] * z1 + m[8] * z2;
+    for (int s = 0, k = b + lane % G; s < sc.levels; ++s, k += G) {
+        const int2 lv = sweep_level(sc, more, s);
+        if (w >= lv.y) break;
+        const int64_t i = (int64_t)(lv.x + w) * 64 + lane;
+        if (k < e) {
+            const int f = fcol[k], m = perm[f];
+            col[i] = !upper && f < c1 ? -1 - m : m;
+            src[i] = k;
+        } else {
+            col[i] = kNoBlock;
+            src[i] = -1;
         }
-        t[3 * i] = y0;
-        t[3 * i + 1] = y1;
-        t[3 * i + 2] = y2;
     }
 }
 
-// backward sweep of one color: t_i = Dinv_i (t_i - sum_{j after i} U_ij t_j); blocks taken U
-// at a time per lane as in the forward sweep
-template <typename T, int G, int U>
-__global__ __launch_bounds__(BS) void ilu_upper_kernel(int r0, int r1, const int32_t* __restrict__ fptr,
-                                                       const int32_t* __restrict__ fcol,
-                                                       const int32_t* __restrict__ dslot, const T* __restrict__ F,
-                                                       const T* __restrict__ Dinv, T* __restrict__ t) {
-    const int tid = blockIdx.x * BS + threadIdx.x;
-    const int i = r0 + tid / G, lane = tid % G;
-    if (i >= r1) return;
-    const int e = fptr[i + 1];
-    T y0 = 0, y1 = 0, y2 = 0;
-    for (int jb0 = fptr[i] + dslot[i] + 1 + lane; jb0 < e; jb0 += G * U) {
-        int jj[U];
+// the values of a sweep's entries from the factor
+template <typename T>
+__global__ __launch_bounds__(BS) void sweep_pack_kernel(int64_t steps, const int32_t* __restrict__ src,
+                                                        const T* __restrict__ F, T* __restrict__ val) {
+    const int64_t s = ((int64_t)blockIdx.x * BS + threadIdx.x) / 64;
+    const int lane = threadIdx.x & 63;
+    if (s >= steps) return;
+    const int k = src[s * 64 + lane];
 #pragma unroll
-        for (int u = 0; u < U; ++u) jj[u] = jb0 + u * G < e ? fcol[jb0 + u * G] : -1;
-        T x[U][3];
+    for (int v = 0; v < 9; ++v) val[(s * 9 + v) * 64 + lane] = k >= 0 ? F[(int64_t)k * 9 + v] : (T)0;
+}
+
+// One color of a sweep: z_n = own_n - sum of the row's blocks times their entries (columns marked
+// -1 - m read v, the others z), times Dinv when given.
+template <typename T, int G>
+__global__ __launch_bounds__(64) void sweep_kernel(SweepColor sc, const int2* __restrict__ more,
+                                                   const int2* __restrict__ rows, const int32_t* __restrict__ col,
+                                                   const T* __restrict__ val, const T* __restrict__ Dinv,
+                                                   const T* __restrict__ v, const T* own, T* z) {
+    constexpr int U = kSweepUnroll;
+    const int w = xcd_block_g();  // slice
+    const int lane = threadIdx.x, r = lane % G;
+    if (w >= sc.slices) return;
+    const int2 rw = rows[sc.row0 + w * (64 / G) + lane / G];
+    T y0 = 0, y1 = 0, y2 = 0, o[3] = {0, 0, 0}, m[3] = {0, 0, 0};
+    auto steps = [&](int b0, int c0, int b1, int c1, int b2, int c2, int b3, int c3, bool first) {
+        const int bs[U] = {b0, b1, b2, b3}, ct[U] = {c0, c1, c2, c3};
+        int c[U];
+        T a[U][9], x[U][3];
 #pragma unroll
         for (int u = 0; u < U; ++u)
+            if (w < ct[u]) {  // uniform over the wavefront
+                const int64_t i = bs[u] + w;
+                c[u] = col[i * 64 + lane];
 #pragma unroll
-            for (int c = 0; c < 3; ++c) x[u][c] = jj[u] >= 0 ? t[3 * jj[u] + c] : (T)0;
+                for (int k = 0; k < 9; ++k) a[u][k] = val[(i * 9 + k) * 64 + lane];
+            }
+        if (first && r < 3 && rw.x >= 0) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (jj[u] < 0) break;
-            const T* a = F + (int64_t)(jb0 + u * G) * 9;
-            y0 += a[0] * x[u][0] + a[1] * x[u][1] + a[2] * x[u][2];
-            y1 += a[3] * x[u][0] + a[4] * x[u][1] + a[5] * x[u][2];
-            y2 += a[6] * x[u][0] + a[7] * x[u][1] + a[8] * x[u][2];
+            for (int k = 0; k < 3; ++k) o[k] = own[3 * (int64_t)rw.x + k];
+            if (Dinv)
+#pragma unroll
+                for (int k = 0; k < 3; ++k) m[k] = Dinv[(int64_t)rw.y * 9 + 3 * r + k];
         }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (w < ct[u]) {
+                x[u][0] = x[u][1] = x[u][2] = (T)0;
+                if (c[u] != kNoBlock) {
+                    const T* xs = c[u] < 0 ? v + 3 * (int64_t)(-1 - c[u]) : z + 3 * (int64_t)c[u];
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) x[u][k] = xs[k];
+                }
+            }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (w < ct[u]) {
+                y0 += a[u][0] * x[u][0] + a[u][1] * x[u][1] + a[u][2] * x[u][2];
+                y1 += a[u][3] * x[u][0] + a[u][4] * x[u][1] + a[u][5] * x[u][2];
+                y2 += a[u][6] * x[u][0] + a[u][7] * x[u][1] + a[u][8] * x[u][2];
+            }
+    };
+    steps(sc.base[0], sc.count[0], sc.base[1], sc.count[1], sc.base[2], sc.count[2], sc.base[3], sc.count[3], true);
+    if (w < sc.count[U])
+        steps(sc.base[4], sc.count[4], sc.base[5], sc.count[5], sc.base[6], sc.count[6], sc.base[7], sc.count[7], false);
+    for (int k = kSweepLevels; k < sc.levels; ++k) {
+        const int2 lv = more[sc.more + k - kSweepLevels];
+        if (w >= lv.y) break;
+        steps(lv.x, lv.y, 0, 0, 0, 0, 0, 0, false);
     }
     group_sum3<T, G>(y0, y1, y2);
-    if (lane == 0) {
-        y0 = t[3 * i] - y0;
-        y1 = t[3 * i + 1] - y1;
-        y2 = t[3 * i + 2] - y2;
-        const T* m = Dinv + (int64_t)i * 9;
-        t[3 * i] = m[0] * y0 + m[1] * y1 + m[2] * y2;
-        t[3 * i + 1] = m[3] * y0 + m[4] * y1 + m[5] * y2;
-        t[3 * i + 2] = m[6] * y0 + m[7] * y1 + m[8] * y2;
+    if (r < 3 && rw.x >= 0) {
+        y0 = o[0] - y0;
+        y1 = o[1] - y1;
+        y2 = o[2] - y2;
+        T out = r == 0 ? y0 : r == 1 ? y1 : y2;
+        if (Dinv) out = m[0] * y0 + m[1] * y1 + m[2] * y2;
+        z[3 * (int64_t)rw.x + r] = out;
     }
 }
 
@@ -540,38 +581,171 @@ __global__ __launch_bounds__(BS) void gm_spmv_kernel(int N, const int32_t* __res
     }
 }
 
-// partial dots of w with basis vectors V_0..V_j (blockIdx.y = vector)
+// partial sums of w . w, and their sum
 template <typename T>
-__global__ __launch_bounds__(BS) void mdot_kernel(int D, const T* __restrict__ V, const T* __restrict__ w,
-                                                  double* __restrict__ part, int nwg) {
+__global__ __launch_bounds__(BS) void norm_kernel(int D, const T* __restrict__ w, double* __restrict__ part, int nwg) {
     __shared__ double sh[BS];
-    const int blk = blockIdx.x;
-    const T* vi = V + (int64_t)blockIdx.y * D;
     double s = 0.0;
 #pragma unroll 4
-    for (int i = blk * BS + threadIdx.x; i < D; i += nwg * BS) s += (double)vi[i] * (double)w[i];
+    for (int i = blockIdx.x * BS + threadIdx.x; i < D; i += nwg * BS) s += (double)w[i] * (double)w[i];
     s = bsum(s, sh);
-    if (threadIdx.x == 0) part[(int64_t)blockIdx.y * nwg + blk] = s;
+    if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
-__global__ __launch_bounds__(BS) void mdot_reduce_kernel(const double* __restrict__ part, int nwg,
-                                                         double* __restrict__ out, int accumulate) {
+__global__ __launch_bounds__(BS) void norm_reduce_kernel(const double* __restrict__ part, int nwg,
+                                                         double* __restrict__ out) {
     __shared__ double sh[BS];
     double s = 0.0;
-    for (int i = threadIdx.x; i < nwg; i += BS) s += part[(int64_t)blockIdx.x * nwg + i];
+    for (int i = threadIdx.x; i < nwg; i += BS) s += part[i];
     s = bsum(s, sh);
-    if (threadIdx.x == 0) out[blockIdx.x] = accumulate ? out[blockIdx.x] + s : s;
+    if (threadIdx.x == 0) *out = s;
 }
 
-// w -= sum_i h_i V_i  (sign = -1) or w = sum_i h_i V_i (sign = 0)
+// sum over the wavefront of the NV values of each lane: lane l gets that of value l / (64 / NV)
+template <int NV>
+__device__ __forceinline__ double wave_sums(double (&s)[NV]) {
+    const int lane = threadIdx.x & 63;
+    int m = 32;
+#pragma unroll
+    for (int n = NV / 2; n >= 1; n >>= 1, m >>= 1) {
+        const bool hi = lane & m;
+#pragma unroll
+        for (int q = 0; q < n; ++q) {
+            const double send = hi ? s[q] : s[q + n], keep = hi ? s[q + n] : s[q];
+            s[q] = keep + __shfl_xor(send, m);
+        }
+    }
+    for (; m >= 1; m >>= 1) s[0] += __shfl_xor(s[0], m);
+    return s[0];
+}
+
+// Classical Gram-Schmidt of w against V_0..V_{nv-1}.  A dot product has to be complete before the next
+// step, and at ordinary sizes a launch costs more than its data: the dot kernel leaves the partial
+// sums of its workgroups, and each workgroup of the kernel that needs them adds them up for itself.
+// So that this stays short, the workgroups per group of kDotVecs vectors get fewer as the groups get
+// more.  hexa20R 24 x 22 x 20 FP64, GMRES(50) iteration: with a reduction launch per dot and the norm
+// apart (9 launches) 297 us, now (5) 279.  Several vectors held in registers across the correction and
+// the second dot spill from 24 on (FP64), and the restart length is the caller's: not done.
+constexpr int kDotVecs = 8, kCombineWG = 512, kMaxVecs = 257;
+
+inline int dot_wgs(int nv) { return nv <= kDotVecs ? 256 : nv <= 3 * kDotVecs ? 128 : 64; }
+
+// part[k][workgroup] = partial sums of V_k . w, kDotVecs vectors per workgroup
+template <typename T>
+__global__ __launch_bounds__(BS) void orth_dot_kernel(int D, int nv, const T* __restrict__ V, const T* __restrict__ w,
+                                                      double* __restrict__ part) {
+    constexpr int NV = kDotVecs, W = BS / 64;
+    __shared__ double red[W][NV];
+    const int nwg = gridDim.x, k0 = blockIdx.y * NV;
+    const T* v[NV];
+    double s[NV];
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+        v[q] = V + (int64_t)(k0 + q < nv ? k0 + q : nv - 1) * D;
+        s[q] = 0.0;
+    }
+#pragma unroll 2
+    for (int i = blockIdx.x * BS + threadIdx.x; i < D; i += nwg * BS) {
+        const double x = (double)w[i];
+#pragma unroll
+        for (int q = 0; q < NV; ++q) s[q] += (double)v[q][i] * x;
+    }
+    const double t = wave_sums<NV>(s);
+    const int lane = threadIdx.x & 63;
+    if (lane % (64 / NV) == 0) red[threadIdx.x / 64][lane / (64 / NV)] = t;
+    __syncthreads();
+    if ((int)threadIdx.x < NV && k0 + (int)threadIdx.x < nv) {
+        double y = 0.0;
+#pragma unroll
+        for (int q = 0; q < W; ++q) y += red[q][threadIdx.x];
+        part[(int64_t)(k0 + threadIdx.x) * nwg + blockIdx.x] = y;
+    }
+}
+
+// h_k = sum of part[k] (to hout from the first workgroup), w -= sum h_k V_k; with NORM, pnorm = the
+// workgroups' partial sums of w . w
+template <typename T, bool NORM>
+__global__ __launch_bounds__(BS) void orth_combine_kernel(int D, int nv, int nwg, const T* __restrict__ V,
+                                                          T* __restrict__ w, const double* __restrict__ part,
+                                                          double* __restrict__ hout, double* __restrict__ pnorm) {
+    constexpr int PRE = 8;
+    __shared__ double hs[kMaxVecs], red[BS / 64];
+    int i = blockIdx.x * BS + threadIdx.x;
+    T a[PRE], x = 0;
+    if (i < D) {  // in flight while the sums are formed
+        x = w[i];
+#pragma unroll
+        for (int q = 0; q < PRE; ++q) a[q] = V[(int64_t)(q < nv ? q : nv - 1) * D + i];
+    }
+    for (int k = threadIdx.x / 8; k < nv; k += BS / 8) {
+        double h = 0.0;
+#pragma unroll 8
+        for (int q = threadIdx.x & 7; q < nwg; q += 8) h += part[(int64_t)k * nwg + q];
+        h += __shfl_xor(h, 1);
+        h += __shfl_xor(h, 2);
+        h += __shfl_xor(h, 4);
+        if ((threadIdx.x & 7) == 0) {
+            hs[k] = h;
+            if (blockIdx.x == 0) hout[k] = h;
+        }
+    }
+    __syncthreads();
+    double nrm = 0.0;
+    for (bool first = true; i < D; i += gridDim.x * BS, first = false) {
+        double acc;
+        int k = 0;
+        if (first) {
+            acc = (double)x;
+            const int n = nv < PRE ? nv : PRE;
+#pragma unroll
+            for (int q = 0; q < PRE; ++q)
+                if (q < n) acc -= hs[q] * (double)a[q];
+            k = n;
+        } else {
+            acc = (double)w[i];
+        }
+#pragma unroll 8
+        for (; k < nv; ++k) acc -= hs[k] * (double)V[(int64_t)k * D + i];
+        const T y = (T)acc;
+        w[i] = y;
+        nrm += (double)y * (double)y;
+    }
+    if (NORM) {
+#pragma unroll
+        for (int m = 32; m >= 1; m >>= 1) nrm += __shfl_xor(nrm, m);
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x / 64] = nrm;
+        __syncthreads();
+        if (threadIdx.x == 0) pnorm[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+    }
+}
+
+// v = w / ||w|| with ||w||^2 the sum of the np <= kCombineWG values pin
+template <typename T>
+__global__ __launch_bounds__(BS) void orth_scale_kernel(int D, int np, const T* __restrict__ w, const double* __restrict__ pin,
+                                                        double* __restrict__ nrm2, T* __restrict__ v) {
+    __shared__ double red[BS / 64];
+    const int i = blockIdx.x * BS + threadIdx.x;
+    const T x = i < D ? w[i] : (T)0;
+    static_assert(kCombineWG == 2 * BS, "two values per thread");
+    double s = ((int)threadIdx.x < np ? pin[threadIdx.x] : 0.0) + ((int)threadIdx.x + BS < np ? pin[threadIdx.x + BS] : 0.0);
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) s += __shfl_xor(s, m);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x / 64] = s;
+    __syncthreads();
+    s = (red[0] + red[1]) + (red[2] + red[3]);
+    if (i == 0) *nrm2 = s;
+    if (i < D) v[i] = (T)((double)x / sqrt(s));
+}
+
+// w = sum_i h_i V_i
 template <typename T>
 __global__ void combine_kernel(int D, int nv, const T* __restrict__ V, const double* __restrict__ h,
-                               T* __restrict__ w, int overwrite) {
+                               T* __restrict__ w) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= D) return;
-    double acc = overwrite ? 0.0 : (double)w[i];
+    double acc = 0.0;
 #pragma unroll 4
-    for (int k = 0; k < nv; ++k) acc += (overwrite ? 1.0 : -1.0) * h[k] * (double)V[(int64_t)k * D + i];
+    for (int k = 0; k < nv; ++k) acc += h[k] * (double)V[(int64_t)k * D + i];
     w[i] = (T)acc;
 }
 
@@ -603,6 +777,58 @@ __global__ void finish_kernel(int D, const T* __restrict__ x, const double* __re
 }
 
 int grid_of(int n) { return (n + BS - 1) / BS; }
+
+// The slices and levels of one sweep.
+int build_sweep(GmresWork* g, int upper, const std::vector<int32_t>& fptr, const std::vector<int32_t>& dslot,
+                const std::vector<int32_t>& perm) {
+    GmresWork::Sweep& sw = g->sweep[upper];
+    std::vector<int32_t> order;
+    std::vector<int2> rows, more;
+    sw.color.assign(g->ncolors, SweepColor());
+    sw.steps = 0;
+    auto len = [&](int i) { return upper ? fptr[i + 1] - fptr[i] - dslot[i] - 1 : dslot[i]; };
+    for (int col = 0; col < g->ncolors; ++col) {
+        const int r0 = g->cstart[col], r1 = g->cstart[col + 1];
+        SweepColor& sc = sw.color[col];
+        order.resize(r1 - r0);
+        for (int i = r0; i < r1; ++i) order[i - r0] = i;
+        std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) { return len(a) > len(b); });
+        const int most = order.empty() ? 0 : len(order[0]);
+        const int G = sc.G = most <= kSweepUnroll * 8 ? 8 : most <= kSweepUnroll * 16 ? 16 : 32, R = 64 / G;
+        sc.row0 = (int)rows.size();
+        sc.slices = (int)((order.size() + R - 1) / R);
+        sc.more = (int)more.size();
+        for (int k = 0; k < sc.slices * R; ++k)
+            rows.push_back(k < (int)order.size() ? make_int2(perm[order[k]], order[k]) : make_int2(-1, -1));
+        for (int k = 0, n = sc.slices;; ++k) {
+            while (n > 0 && len(order[(n - 1) * R]) <= k * G) --n;  // slices with a step k
+            if (n == 0) break;
+            if (k < kSweepLevels) {
+                sc.base[k] = (int)sw.steps;
+                sc.count[k] = n;
+            } else {
+                more.push_back(make_int2((int)sw.steps, n));
+            }
+            sc.levels = k + 1;
+            sw.steps += n;
+        }
+    }
+    const size_t ne = std::max<size_t>(1, (size_t)sw.steps * 64);
+    EFE_HIP(hipMalloc(&sw.rows, std::max<size_t>(1, rows.size()) * sizeof(int2)));
+    EFE_HIP(hipMalloc(&sw.more, std::max<size_t>(1, more.size()) * sizeof(int2)));
+    EFE_HIP(hipMalloc(&sw.col, ne * sizeof(int32_t)));
+    EFE_HIP(hipMalloc(&sw.src, ne * sizeof(int32_t)));
+    EFE_HIP(hipMemcpy(sw.rows, rows.data(), rows.size() * sizeof(int2), hipMemcpyHostToDevice));
+    EFE_HIP(hipMemcpy(sw.more, more.data(), more.size() * sizeof(int2), hipMemcpyHostToDevice));
+    for (const SweepColor& sc : sw.color) {
+        if (sc.slices == 0) continue;
+        const int grid = grid_of(sc.slices * 64), c1 = g->cstart[1];
+        const auto fill = sc.G == 8 ? sweep_fill_kernel<8> : sc.G == 16 ? sweep_fill_kernel<16> : sweep_fill_kernel<32>;
+        fill<<<grid, BS, 0, g->ks>>>(sc, upper, c1, sw.more, sw.rows, g->fptr, g->fcol, g->dslot, g->perm, sw.col, sw.src);
+    }
+    EFE_HIP(hipGetLastError());
+    return EFE_OK;
+}
 
 int build_ilu(efe_ctx* c, GmresWork* g) {
     IluPattern ip;
@@ -638,11 +864,9 @@ int build_ilu(efe_ctx* c, GmresWork* g) {
     }
     g->ncolors = ip.ncolors;
     g->cstart.assign(ip.color_start.begin(), ip.color_start.end());
-    g->clow.assign(g->ncolors, 0);
     g->cup.assign(g->ncolors, 0);
     for (int col = 0; col < g->ncolors; ++col)
         for (int i = g->cstart[col]; i < g->cstart[col + 1]; ++i) {
-            g->clow[col] = std::max(g->clow[col], dslot[i]);
             g->cup[col] = std::max(g->cup[col], fptr[i + 1] - fptr[i] - dslot[i] - 1);
         }
     g->nbF = fptr[N];
@@ -656,8 +880,16 @@ int build_ilu(efe_ctx* c, GmresWork* g) {
     EFE_HIP(hipMemcpy(g->fidx, fidx.data(), fidx.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     EFE_HIP(hipMemcpy(g->dslot, dslot.data(), dslot.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     EFE_HIP(hipMemcpy(g->perm, ip.perm.data(), (size_t)N * sizeof(int32_t), hipMemcpyHostToDevice));
+    for (int up = 0; up < 2; ++up)
+        if (int rc = build_sweep(g, up, fptr, dslot, ip.perm)) return rc;
     g->ilu_ready = true;
     return EFE_OK;
+}
+
+template <typename T>
+T* sweep_values(const GmresWork::Sweep& sw) {
+    if constexpr (sizeof(T) == 8) return sw.v64;
+    else return sw.v32;
 }
 
 template <typename T>
@@ -694,6 +926,13 @@ int ilu_factor(efe_ctx* c, GmresWork* g, const T* K, T*& F, T*& Dinv, int pi, hi
                                                                              Dinv);
         }
     }
+    for (GmresWork::Sweep& sw : g->sweep) {
+        if (!sweep_values<T>(sw))
+            EFE_HIP(hipMalloc(sizeof(T) == 8 ? (void**)&sw.v64 : (void**)&sw.v32,
+                              std::max<size_t>(1, (size_t)sw.steps * 64 * 9) * sizeof(T)));
+        if (sw.steps)
+            sweep_pack_kernel<T><<<(unsigned)((sw.steps * 64 + BS - 1) / BS), BS, 0, st>>>(sw.steps, sw.src, F, sweep_values<T>(sw));
+    }
     EFE_HIP(hipGetLastError());
     g->factored_version[pi] = c->Kversion;
     return EFE_OK;
@@ -705,37 +944,20 @@ void apply_precond(efe_ctx* c, GmresWork* g, int precond, const T* F, const T* D
                    hipStream_t st) {
     const int N = c->N;
     if (precond == EFE_PRECOND_ILU0) {
-        T* t = (T*)g->t;
-        permute_in_kernel<T><<<grid_of(N), BS, 0, st>>>(N, g->perm, v, t);
-        const bool h8 = c->NN == 8;
         const int last = g->ncolors - 1;
-        // the last color's backward sweep rides on its forward sweep when its rows have no
-        // blocks after them; a color whose rows have no blocks before them (the first) has no
-        // forward sweep
-        const bool fuseLast = last >= 0 && g->cup[last] == 0;
-        for (int col = 0; col < g->ncolors; ++col) {
-            const int r0 = g->cstart[col], r1 = g->cstart[col + 1];
-            const bool fuse = fuseLast && col == last;
-            if (r1 <= r0 || (g->clow[col] == 0 && !fuse)) continue;
-            const T* D = fuse ? Dinv : nullptr;
-            if (h8)
-                ilu_lower_kernel<T, 8, 4><<<grid_of((r1 - r0) * 8), BS, 0, st>>>(r0, r1, g->fptr, g->fcol, g->dslot, F, t,
-                                                                              D);
-            else
-                ilu_lower_kernel<T, 16, 4><<<grid_of((r1 - r0) * 16), BS, 0, st>>>(r0, r1, g->fptr, g->fcol, g->dslot, F,
-                                                                                t, D);
-        }
-        for (int col = g->ncolors - 1; col >= 0; --col) {
-            const int r0 = g->cstart[col], r1 = g->cstart[col + 1];
-            if (r1 <= r0 || (fuseLast && col == last)) continue;
-            if (h8)
-                ilu_upper_kernel<T, 8, 4><<<grid_of((r1 - r0) * 8), BS, 0, st>>>(r0, r1, g->fptr, g->fcol, g->dslot, F,
-                                                                              Dinv, t);
-            else
-                ilu_upper_kernel<T, 16, 4><<<grid_of((r1 - r0) * 16), BS, 0, st>>>(r0, r1, g->fptr, g->fcol, g->dslot,
-                                                                                F, Dinv, t);
-        }
-        permute_out_kernel<T><<<grid_of(N), BS, 0, st>>>(N, g->perm, t, z);
+        // color 0 has no forward sweep (nothing comes before it: its forward values are v's); the
+        // last color's backward sweep rides on its forward sweep when its rows have no blocks after them
+        const bool fuseLast = last > 0 && g->cup[last] == 0;
+        auto launch = [&](int up, int col, const T* D) {
+            const GmresWork::Sweep& sw = g->sweep[up];
+            const SweepColor& sc = sw.color[col];
+            if (sc.slices == 0) return;
+            const auto kernel = sc.G == 8 ? sweep_kernel<T, 8> : sc.G == 16 ? sweep_kernel<T, 16> : sweep_kernel<T, 32>;
+            kernel<<<round8g(sc.slices), 64, 0, st>>>(sc, sw.more, sw.rows, sw.col, sweep_values<T>(sw), D, v,
+                                                      up && col > 0 ? z : v, z);
+        };
+        for (int col = 1; col < g->ncolors; ++col) launch(0, col, fuseLast && col == last ? Dinv : nullptr);
+        for (int col = fuseLast ? last - 1 : last; col >= 0; --col) launch(1, col, Dinv);
     } else {
         bjacobi_kernel<T><<<grid_of(N), BS, 0, st>>>(N, Minv, v, z);
     }
@@ -753,14 +975,13 @@ void gmres_step_launch(efe_ctx* c, GmresWork* g, int precond, const T* F, const 
     T* z = (T*)g->z;
     apply_precond<T>(c, g, precond, F, Dinv, Minv, V + (int64_t)j * D, z, st);
     gm_spmv_kernel<T><<<gs, BS, 0, st>>>(N, c->slice_off, c->scol, c->slotNode, K, z, w, nullptr);
-    for (int pass = 0; pass < 2; ++pass) {
-        mdot_kernel<T><<<dim3(g->nwg, j + 1), BS, 0, st>>>(D, V, w, g->part, g->nwg);
-        mdot_reduce_kernel<<<j + 1, BS, 0, st>>>(g->part, g->nwg, g->hdev + pass * (m + 2), 0);
-        combine_kernel<T><<<gd, BS, 0, st>>>(D, j + 1, V, g->hdev + pass * (m + 2), w, 0);
-    }
-    mdot_kernel<T><<<dim3(g->nwg, 1), BS, 0, st>>>(D, w, w, g->part, g->nwg);
-    mdot_reduce_kernel<<<1, BS, 0, st>>>(g->part, g->nwg, g->hdev + 2 * (m + 2), 0);
-    scale_kernel<T><<<gd, BS, 0, st>>>(D, w, g->hdev + 2 * (m + 2), V + (int64_t)(j + 1) * D);
+    const int nv = j + 1, nwg = dot_wgs(nv), gc = std::min(gd, kCombineWG);
+    const dim3 gdot(nwg, (nv + kDotVecs - 1) / kDotVecs);
+    orth_dot_kernel<T><<<gdot, BS, 0, st>>>(D, nv, V, w, g->part);
+    orth_combine_kernel<T, false><<<gc, BS, 0, st>>>(D, nv, nwg, V, w, g->part, g->hdev, nullptr);
+    orth_dot_kernel<T><<<gdot, BS, 0, st>>>(D, nv, V, w, g->part);
+    orth_combine_kernel<T, true><<<gc, BS, 0, st>>>(D, nv, nwg, V, w, g->part, g->hdev + (m + 2), g->pnorm);
+    orth_scale_kernel<T><<<gd, BS, 0, st>>>(D, gc, w, g->pnorm, g->hdev + 2 * (m + 2), V + (int64_t)nv * D);
 }
 
 // Step j as one replayed hipGraph (captured on first use for these buffers); with
@@ -833,8 +1054,8 @@ int gmres_solve(efe_ctx* c, GmresWork* g, const double* b, double* xout, const e
     // ||b||
     zero_kernel<T><<<gd, BS, 0, st>>>(D, x);
     gm_spmv_kernel<T><<<gs, BS, 0, st>>>(N, c->slice_off, c->scol, c->slotNode, K, x, w, b);
-    mdot_kernel<T><<<dim3(g->nwg, 1), BS, 0, st>>>(D, w, w, g->part, g->nwg);
-    mdot_reduce_kernel<<<1, BS, 0, st>>>(g->part, g->nwg, g->hdev + 2 * (m + 2), 0);
+    norm_kernel<T><<<g->nwg, BS, 0, st>>>(D, w, g->part, g->nwg);
+    norm_reduce_kernel<<<1, BS, 0, st>>>(g->part, g->nwg, g->hdev + 2 * (m + 2));
     EFE_HIP(hipMemcpyAsync(hh, g->hdev + 2 * (m + 2), sizeof(double), hipMemcpyDeviceToHost, st));
     EFE_HIP(hipStreamSynchronize(st));
     const double bnorm = sqrt(hh[0]);
@@ -895,14 +1116,14 @@ int gmres_solve(efe_ctx* c, GmresWork* g, const double* b, double* xout, const e
             y[i] = s / H[(size_t)i * (m + 1) + i];
         }
         EFE_HIP(hipMemcpyAsync(g->hdev, y.data(), (jend + 1) * sizeof(double), hipMemcpyHostToDevice, st));
-        combine_kernel<T><<<gd, BS, 0, st>>>(D, jend + 1, V, g->hdev, w, 1);
+        combine_kernel<T><<<gd, BS, 0, st>>>(D, jend + 1, V, g->hdev, w);
         apply_precond<T>(c, g, o->precond, F, Dinv, Minv, w, z, st);
         axpy_kernel<T><<<gd, BS, 0, st>>>(D, z, x);
         if (done || it >= maxit) break;
         // restart: w = b - K x
         gm_spmv_kernel<T><<<gs, BS, 0, st>>>(N, c->slice_off, c->scol, c->slotNode, K, x, w, b);
-        mdot_kernel<T><<<dim3(g->nwg, 1), BS, 0, st>>>(D, w, w, g->part, g->nwg);
-        mdot_reduce_kernel<<<1, BS, 0, st>>>(g->part, g->nwg, g->hdev + 2 * (m + 2), 0);
+        norm_kernel<T><<<g->nwg, BS, 0, st>>>(D, w, g->part, g->nwg);
+        norm_reduce_kernel<<<1, BS, 0, st>>>(g->part, g->nwg, g->hdev + 2 * (m + 2));
         EFE_HIP(hipMemcpyAsync(hh, g->hdev + 2 * (m + 2), sizeof(double), hipMemcpyDeviceToHost, st));
         EFE_HIP(hipStreamSynchronize(st));
         beta = sqrt(hh[0]);
@@ -952,7 +1173,7 @@ int ensure_gmres(efe_ctx* c, int m, int prec) {
             return EFE_ERR_ARG;
         }
         drop_step_graphs(g);
-        hipFree(g->V); hipFree(g->w); hipFree(g->z); hipFree(g->x); hipFree(g->t);
+        hipFree(g->V); hipFree(g->w); hipFree(g->z); hipFree(g->x);
         hipFree(g->part); hipFree(g->hdev);
         const size_t es = prec == EFE_FP32 ? sizeof(float) : sizeof(double);
         const size_t D = (size_t)c->D;
@@ -960,8 +1181,8 @@ int ensure_gmres(efe_ctx* c, int m, int prec) {
         EFE_HIP(hipMalloc(&g->w, D * es));
         EFE_HIP(hipMalloc(&g->z, D * es));
         EFE_HIP(hipMalloc(&g->x, D * es));
-        EFE_HIP(hipMalloc(&g->t, D * es));
-        EFE_HIP(hipMalloc(&g->part, (size_t)(m + 1) * g->nwg * sizeof(double)));
+        EFE_HIP(hipMalloc(&g->part, ((size_t)(m + 1) * g->nwg + kCombineWG) * sizeof(double)));
+        g->pnorm = g->part + (size_t)(m + 1) * g->nwg;
         EFE_HIP(hipMalloc(&g->hdev, 3 * (size_t)(m + 2) * sizeof(double)));
         g->m = m;
         g->vprec = prec;
@@ -983,9 +1204,14 @@ void efe_gmres_free(efe_ctx* c) {
     GmresWork* g = c->gw;
     if (!g) return;
     void* bufs[] = {g->fptr, g->fcol, g->fidx, g->dslot, g->perm, g->F64, g->Dinv64, g->F32, g->Dinv32,
-                    g->V, g->w, g->z, g->x, g->t, g->part, g->hdev};
+                    g->V, g->w, g->z, g->x, g->part, g->hdev};
     for (void* p : bufs)
         if (p) hipFree(p);
+    for (GmresWork::Sweep& sw : g->sweep) {
+        void* sb[] = {sw.rows, sw.more, sw.col, sw.src, sw.v64, sw.v32};
+        for (void* p : sb)
+            if (p) hipFree(p);
+    }
     drop_step_graphs(g);
     if (g->hhost) hipHostFree(g->hhost);
     if (g->ks) hipStreamDestroy(g->ks);
