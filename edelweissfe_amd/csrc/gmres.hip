@@ -539,36 +539,56 @@ __global__ void bjacobi_kernel(int N, const T* __restrict__ Minv, const T* __res
     z[3 * n + 2] = M[6] * a + M[7] * b + M[8] * c;
 }
 
-// y = K x (sliced ELL), optionally y = b - K x
+// y = K x (sliced ELL), optionally y = b - K x.  A workgroup has one slice, its wavefronts each a range
+// of the rows' blocks: with a lane for a whole row of up to 81 blocks the chain of their loads set the
+// time wherever the slices are fewer than some thousands.  hexa20R GMRES iteration at 1 / 2 / 4 / 8
+// wavefronts: 8 x 8 x 8 FP64 200 / 179 / 167 / 165 us, 24 x 22 x 20 FP64 (the product 58 us) 292 / 276 /
+// 270 / 269, 40 x 36 x 32 FP64 615 / 617 / 595 / 587, FP32 394 / 394 / 388 / 384.
+constexpr int kSpmvWaves = 8;
 template <typename T>
-__global__ __launch_bounds__(BS) void gm_spmv_kernel(int N, const int32_t* __restrict__ slice_off,
-                                                     const int32_t* __restrict__ scol,
-                                                     const int32_t* __restrict__ slotNode, const T* __restrict__ K,
-                                                     const T* __restrict__ x, T* __restrict__ y,
-                                                     const double* __restrict__ b) {
-    const int ps = xcd_block_g() * BS + threadIdx.x;  // row slot
-    if (ps >= N) return;
-    const int n = slotNode[ps];
-    const int s = ps / kSlice, l = ps - (ps / kSlice) * kSlice;
+__global__ __launch_bounds__(64 * kSpmvWaves) void gm_spmv_kernel(int N, const int32_t* __restrict__ slice_off,
+                                                         const int32_t* __restrict__ scol,
+                                                         const int32_t* __restrict__ slotNode, const T* __restrict__ K,
+                                                         const T* __restrict__ x, T* __restrict__ y,
+                                                         const double* __restrict__ b) {
+    constexpr int W = kSpmvWaves;
+    __shared__ T sh[W - 1][3][64];
+    const int s = xcd_block_g(), l = threadIdx.x & 63;
+    const int part = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const int ps = s * kSlice + l;  // row slot
+    if (s * kSlice >= N) return;
     const int o0 = slice_off[s], deg = (slice_off[s + 1] - o0) / kSlice;
+    const int n = ps < N ? slotNode[ps] : -1;
     const int32_t* cp = scol + o0 + l;
     const T* kp = K + (int64_t)o0 * 9 + l;
     T y0 = 0, y1 = 0, y2 = 0;
-    // unrolled so that the loads of several blocks are in flight together; measured on the 48^3
-    // hexa20 operator: FP64 455 / 438 / 491 / 452 us at 1 / 2 / 3 / 4 blocks, FP32 243 / 214 /
-    // 209 / 210 us
     constexpr int kUnroll = sizeof(T) == 8 ? 2 : 3;
+    const int k1 = (part + 1) * deg / W;
+    if (n >= 0)
 #pragma unroll kUnroll
-    for (int k = 0; k < deg; ++k) {
-        const int m = __builtin_nontemporal_load(cp + k * kSlice);
-        const T x0 = x[3 * m], x1 = x[3 * m + 1], x2 = x[3 * m + 2];
-        const T* v = kp + (int64_t)k * 9 * kSlice;
-        T a[9];
+        for (int k = part * deg / W; k < k1; ++k) {
+            const int m = __builtin_nontemporal_load(cp + k * kSlice);
+            const T x0 = x[3 * m], x1 = x[3 * m + 1], x2 = x[3 * m + 2];
+            const T* v = kp + (int64_t)k * 9 * kSlice;
+            T a[9];
 #pragma unroll
-        for (int i = 0; i < 9; ++i) a[i] = __builtin_nontemporal_load(v + i * kSlice);
-        y0 += a[0] * x0 + a[1] * x1 + a[2] * x2;
-        y1 += a[3] * x0 + a[4] * x1 + a[5] * x2;
-        y2 += a[6] * x0 + a[7] * x1 + a[8] * x2;
+            for (int i = 0; i < 9; ++i) a[i] = __builtin_nontemporal_load(v + i * kSlice);
+            y0 += a[0] * x0 + a[1] * x1 + a[2] * x2;
+            y1 += a[3] * x0 + a[4] * x1 + a[5] * x2;
+            y2 += a[6] * x0 + a[7] * x1 + a[8] * x2;
+        }
+    if (part > 0) {
+        sh[part - 1][0][l] = y0;
+        sh[part - 1][1][l] = y1;
+        sh[part - 1][2][l] = y2;
+    }
+    __syncthreads();
+    if (part > 0 || n < 0) return;
+#pragma unroll
+    for (int w = 0; w < W - 1; ++w) {
+        y0 += sh[w][0][l];
+        y1 += sh[w][1][l];
+        y2 += sh[w][2][l];
     }
     if (b) {
         y[3 * n] = (T)b[3 * n] - y0;
@@ -969,12 +989,12 @@ template <typename T>
 void gmres_step_launch(efe_ctx* c, GmresWork* g, int precond, const T* F, const T* Dinv, const T* Minv, const T* K,
                        int j, hipStream_t st) {
     const int D = c->D, N = c->N, m = g->m;
-    const int gd = grid_of(D), gs = round8g(grid_of(N));
+    const int gd = grid_of(D), gs = round8g((N + kSlice - 1) / kSlice);
     T* V = (T*)g->V;
     T* w = (T*)g->w;
     T* z = (T*)g->z;
     apply_precond<T>(c, g, precond, F, Dinv, Minv, V + (int64_t)j * D, z, st);
-    gm_spmv_kernel<T><<<gs, BS, 0, st>>>(N, c->slice_off, c->scol, c->slotNode, K, z, w, nullptr);
+    gm_spmv_kernel<T><<<gs, 64 * kSpmvWaves, 0, st>>>(N, c->slice_off, c->scol, c->slotNode, K, z, w, nullptr);
     const int nv = j + 1, nwg = dot_wgs(nv), gc = std::min(gd, kCombineWG);
     const dim3 gdot(nwg, (nv + kDotVecs - 1) / kDotVecs);
     orth_dot_kernel<T><<<gdot, BS, 0, st>>>(D, nv, V, w, g->part);
@@ -1049,11 +1069,11 @@ int gmres_solve(efe_ctx* c, GmresWork* g, const double* b, double* xout, const e
     T* z = (T*)g->z;
     T* x = (T*)g->x;
     const int gd = grid_of(D);
-    const int gs = round8g(grid_of(N));
+    const int gs = round8g((N + kSlice - 1) / kSlice);
     double* hh = g->hhost;
     // ||b||
     zero_kernel<T><<<gd, BS, 0, st>>>(D, x);
-    gm_spmv_kernel<T><<<gs, BS, 0, st>>>(N, c->slice_off, c->scol, c->slotNode, K, x, w, b);
+    gm_spmv_kernel<T><<<gs, 64 * kSpmvWaves, 0, st>>>(N, c->slice_off, c->scol, c->slotNode, K, x, w, b);
     norm_kernel<T><<<g->nwg, BS, 0, st>>>(D, w, g->part, g->nwg);
     norm_reduce_kernel<<<1, BS, 0, st>>>(g->part, g->nwg, g->hdev + 2 * (m + 2));
     EFE_HIP(hipMemcpyAsync(hh, g->hdev + 2 * (m + 2), sizeof(double), hipMemcpyDeviceToHost, st));
@@ -1121,7 +1141,7 @@ int gmres_solve(efe_ctx* c, GmresWork* g, const double* b, double* xout, const e
         axpy_kernel<T><<<gd, BS, 0, st>>>(D, z, x);
         if (done || it >= maxit) break;
         // restart: w = b - K x
-        gm_spmv_kernel<T><<<gs, BS, 0, st>>>(N, c->slice_off, c->scol, c->slotNode, K, x, w, b);
+        gm_spmv_kernel<T><<<gs, 64 * kSpmvWaves, 0, st>>>(N, c->slice_off, c->scol, c->slotNode, K, x, w, b);
         norm_kernel<T><<<g->nwg, BS, 0, st>>>(D, w, g->part, g->nwg);
         norm_reduce_kernel<<<1, BS, 0, st>>>(g->part, g->nwg, g->hdev + 2 * (m + 2));
         EFE_HIP(hipMemcpyAsync(hh, g->hdev + 2 * (m + 2), sizeof(double), hipMemcpyDeviceToHost, st));
