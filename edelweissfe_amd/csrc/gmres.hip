@@ -11,7 +11,8 @@
 //
 // GMRES: right preconditioning (the Arnoldi residual is the true residual of K x = b),
 // classical Gram-Schmidt with one re-orthogonalisation (all projections of a step in one
-// pass over the basis), Givens rotations on the host with one readback per step.
+// pass over the basis), Givens rotations on the host, which the device writes each step's
+// projections to and runs one step ahead of.
 #include <algorithm>
 #include <array>
 #include <cstdlib>
@@ -60,8 +61,9 @@ struct GmresWork {
     void* x = nullptr;
     int vprec = -1;
     double *part = nullptr, *pnorm = nullptr;  // [(m+1)][nwg]; behind it the partial norms
-    double* hdev = nullptr;  // [3][m+2]: h1, h2, norm
-    double* hhost = nullptr; // pinned
+    double* hdev = nullptr;  // [m+2]: ||w||^2 of a start, coefficients of the solution
+    double* hhost = nullptr; // pinned, [2][3][m+2]: h1, h2, ||w||^2 of the even and the odd steps
+    hipEvent_t step[2] = {nullptr, nullptr};  // their ends
     hipStream_t ks = nullptr;
     hipEvent_t evA = nullptr, evB = nullptr;
     hipEvent_t t0 = nullptr, t1 = nullptr, t2 = nullptr;  // timing: solve start, factor done, end
@@ -983,8 +985,10 @@ void apply_precond(efe_ctx* c, GmresWork* g, int precond, const T* F, const T* D
     }
 }
 
+inline double* step_results(const GmresWork* g, int j) { return g->hhost + (j & 1) * 3 * (g->m + 2); }
+
 // Arnoldi step j: w = K M^{-1} V_j, two classical Gram-Schmidt passes against V_0..V_j
-// (projections into hdev[0..], hdev[m+2..]), ||w||^2 into hdev[2(m+2)], V_{j+1} = w / ||w||.
+// (projections into h[0..], h[m+2..], h = step_results), ||w||^2 into h[2(m+2)], V_{j+1} = w / ||w||.
 template <typename T>
 void gmres_step_launch(efe_ctx* c, GmresWork* g, int precond, const T* F, const T* Dinv, const T* Minv, const T* K,
                        int j, hipStream_t st) {
@@ -996,12 +1000,13 @@ void gmres_step_launch(efe_ctx* c, GmresWork* g, int precond, const T* F, const 
     apply_precond<T>(c, g, precond, F, Dinv, Minv, V + (int64_t)j * D, z, st);
     gm_spmv_kernel<T><<<gs, 64 * kSpmvWaves, 0, st>>>(N, c->slice_off, c->scol, c->slotNode, K, z, w, nullptr);
     const int nv = j + 1, nwg = dot_wgs(nv), gc = std::min(gd, kCombineWG);
+    double* h = step_results(g, j);
     const dim3 gdot(nwg, (nv + kDotVecs - 1) / kDotVecs);
     orth_dot_kernel<T><<<gdot, BS, 0, st>>>(D, nv, V, w, g->part);
-    orth_combine_kernel<T, false><<<gc, BS, 0, st>>>(D, nv, nwg, V, w, g->part, g->hdev, nullptr);
+    orth_combine_kernel<T, false><<<gc, BS, 0, st>>>(D, nv, nwg, V, w, g->part, h, nullptr);
     orth_dot_kernel<T><<<gdot, BS, 0, st>>>(D, nv, V, w, g->part);
-    orth_combine_kernel<T, true><<<gc, BS, 0, st>>>(D, nv, nwg, V, w, g->part, g->hdev + (m + 2), g->pnorm);
-    orth_scale_kernel<T><<<gd, BS, 0, st>>>(D, gc, w, g->pnorm, g->hdev + 2 * (m + 2), V + (int64_t)nv * D);
+    orth_combine_kernel<T, true><<<gc, BS, 0, st>>>(D, nv, nwg, V, w, g->part, h + (m + 2), g->pnorm);
+    orth_scale_kernel<T><<<gd, BS, 0, st>>>(D, gc, w, g->pnorm, h + 2 * (m + 2), V + (int64_t)nv * D);
 }
 
 // Step j as one replayed hipGraph (captured on first use for these buffers); with
@@ -1075,8 +1080,8 @@ int gmres_solve(efe_ctx* c, GmresWork* g, const double* b, double* xout, const e
     zero_kernel<T><<<gd, BS, 0, st>>>(D, x);
     gm_spmv_kernel<T><<<gs, 64 * kSpmvWaves, 0, st>>>(N, c->slice_off, c->scol, c->slotNode, K, x, w, b);
     norm_kernel<T><<<g->nwg, BS, 0, st>>>(D, w, g->part, g->nwg);
-    norm_reduce_kernel<<<1, BS, 0, st>>>(g->part, g->nwg, g->hdev + 2 * (m + 2));
-    EFE_HIP(hipMemcpyAsync(hh, g->hdev + 2 * (m + 2), sizeof(double), hipMemcpyDeviceToHost, st));
+    norm_reduce_kernel<<<1, BS, 0, st>>>(g->part, g->nwg, g->hdev);
+    EFE_HIP(hipMemcpyAsync(hh, g->hdev, sizeof(double), hipMemcpyDeviceToHost, st));
     EFE_HIP(hipStreamSynchronize(st));
     const double bnorm = sqrt(hh[0]);
     info->rhs_norm = bnorm;
@@ -1091,18 +1096,23 @@ int gmres_solve(efe_ctx* c, GmresWork* g, const double* b, double* xout, const e
     bool done = !(bnorm > tol), bad = !(bnorm == bnorm);
     while (!done && !bad) {
         // r = b - K x is in w; V_0 = r / beta
-        scale_kernel<T><<<gd, BS, 0, st>>>(D, w, g->hdev + 2 * (m + 2), V);
+        scale_kernel<T><<<gd, BS, 0, st>>>(D, w, g->hdev, V);
         std::fill(gv.begin(), gv.end(), 0.0);
         gv[0] = beta;
-        int jend = -1;
+        int jend = -1, sent = 0;
         for (int j = 0; j < m; ++j) {
-            if (int rc = run_step<T>(c, g, o->precond, F, Dinv, Minv, K, j, st)) return rc;
-            EFE_HIP(hipMemcpyAsync(hh, g->hdev, 3 * (m + 2) * sizeof(double), hipMemcpyDeviceToHost, st));
-            EFE_HIP(hipStreamSynchronize(st));
+            // step j + 1 goes out before the host has seen step j, so that the device does not wait
+            // for it: the last step of a solve is followed by one whose results nothing reads
+            for (; sent <= j + 1 && sent < m && it + sent - j < maxit; ++sent) {
+                if (int rc = run_step<T>(c, g, o->precond, F, Dinv, Minv, K, sent, st)) return rc;
+                EFE_HIP(hipEventRecord(g->step[sent & 1], st));
+            }
+            EFE_HIP(hipEventSynchronize(g->step[j & 1]));
             ++it;
+            const double* h = step_results(g, j);
             double* col = &H[(size_t)j * (m + 1)];
-            for (int i = 0; i <= j; ++i) col[i] = hh[i] + hh[(m + 2) + i];
-            col[j + 1] = sqrt(hh[2 * (m + 2)]);
+            for (int i = 0; i <= j; ++i) col[i] = h[i] + h[(m + 2) + i];
+            col[j + 1] = sqrt(h[2 * (m + 2)]);
             for (int i = 0; i < j; ++i) {
                 const double a = cs[i] * col[i] + sn[i] * col[i + 1];
                 col[i + 1] = -sn[i] * col[i] + cs[i] * col[i + 1];
@@ -1143,8 +1153,8 @@ int gmres_solve(efe_ctx* c, GmresWork* g, const double* b, double* xout, const e
         // restart: w = b - K x
         gm_spmv_kernel<T><<<gs, 64 * kSpmvWaves, 0, st>>>(N, c->slice_off, c->scol, c->slotNode, K, x, w, b);
         norm_kernel<T><<<g->nwg, BS, 0, st>>>(D, w, g->part, g->nwg);
-        norm_reduce_kernel<<<1, BS, 0, st>>>(g->part, g->nwg, g->hdev + 2 * (m + 2));
-        EFE_HIP(hipMemcpyAsync(hh, g->hdev + 2 * (m + 2), sizeof(double), hipMemcpyDeviceToHost, st));
+        norm_reduce_kernel<<<1, BS, 0, st>>>(g->part, g->nwg, g->hdev);
+        EFE_HIP(hipMemcpyAsync(hh, g->hdev, sizeof(double), hipMemcpyDeviceToHost, st));
         EFE_HIP(hipStreamSynchronize(st));
         beta = sqrt(hh[0]);
         info->residual = beta;
@@ -1181,11 +1191,12 @@ int ensure_gmres(efe_ctx* c, int m, int prec) {
         EFE_HIP(hipStreamCreateWithFlags(&g->ks, hipStreamNonBlocking));
         EFE_HIP(hipEventCreateWithFlags(&g->evA, hipEventDisableTiming));
         EFE_HIP(hipEventCreateWithFlags(&g->evB, hipEventDisableTiming));
+        for (hipEvent_t& e : g->step) EFE_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         EFE_HIP(hipEventCreate(&g->t0));
         EFE_HIP(hipEventCreate(&g->t1));
         EFE_HIP(hipEventCreate(&g->t2));
         g->nwg = 512;
-        EFE_HIP(hipHostMalloc(&g->hhost, 3 * 258 * sizeof(double), hipHostMallocDefault));
+        EFE_HIP(hipHostMalloc(&g->hhost, 2 * 3 * 258 * sizeof(double), hipHostMallocDefault));
     }
     if (g->m != m || g->vprec != prec) {
         if (m > 256) {
@@ -1203,7 +1214,7 @@ int ensure_gmres(efe_ctx* c, int m, int prec) {
         EFE_HIP(hipMalloc(&g->x, D * es));
         EFE_HIP(hipMalloc(&g->part, ((size_t)(m + 1) * g->nwg + kCombineWG) * sizeof(double)));
         g->pnorm = g->part + (size_t)(m + 1) * g->nwg;
-        EFE_HIP(hipMalloc(&g->hdev, 3 * (size_t)(m + 2) * sizeof(double)));
+        EFE_HIP(hipMalloc(&g->hdev, (size_t)(m + 2) * sizeof(double)));
         g->m = m;
         g->vprec = prec;
     }
@@ -1237,7 +1248,7 @@ void efe_gmres_free(efe_ctx* c) {
     if (g->ks) hipStreamDestroy(g->ks);
     if (g->evA) hipEventDestroy(g->evA);
     if (g->evB) hipEventDestroy(g->evB);
-    for (hipEvent_t e : {g->t0, g->t1, g->t2})
+    for (hipEvent_t e : {g->t0, g->t1, g->t2, g->step[0], g->step[1]})
         if (e) hipEventDestroy(e);
     delete g;
     c->gw = nullptr;
