@@ -7,7 +7,7 @@
 // 8 x 8 x 4 sets found here.  The elements are split recursively across the longest side
 // (measured in mean element sizes), at a gap between layers of elements where there is one, at
 // the position that needs the fewest bricks, else nearest the middle; a set is a brick once it
-// has at most kBrick elements and kBrickNodes staged nodes, whatever the mesh.
+// has at most EB elements and NB staged nodes, whatever the mesh.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -21,7 +21,7 @@ namespace {
 struct Splitter {
     const std::vector<float>& cen;  // [3][E] element centroids in mean element sizes
     std::vector<int32_t>& order;    // element indices, rearranged in place
-    int E;
+    int E, EB, NB;
 
     // Splits [lo, hi) of the order and returns the position of the cut.
     int cut(int lo, int hi, std::vector<int32_t>& bins, std::vector<int32_t>& tmp) const {
@@ -54,7 +54,7 @@ struct Splitter {
             const int l = bins[b];
             if (4 * (int64_t)l < n || 4 * (int64_t)l > 3 * (int64_t)n) continue;
             const bool gap = bins[b + 1] == l;  // an empty bin: between two layers
-            const int64_t bricks = (l + kBrick - 1) / kBrick + (n - l + kBrick - 1) / kBrick;
+            const int64_t bricks = (l + EB - 1) / EB + (n - l + EB - 1) / EB;
             const int64_t cost = ((gap ? 0 : 1) * (int64_t)(E + 1) + bricks) * (int64_t)(n + 1) + std::abs(2 * l - n);
             if (cost < bestCost) {
                 bestCost = cost;
@@ -82,12 +82,13 @@ struct Splitter {
 struct Brick {
     int lo = 0, hi = 0;
     std::vector<int32_t> nodes;   // staged nodes (a node with more than 8 incidences repeats)
-    std::vector<uint16_t> linc;   // [nodes][8] incidences a * kBrick + t, 0xffff: none
+    std::vector<uint16_t> linc;   // [nodes][8] incidences, 0xffff: none
     std::vector<uint16_t> lidx;   // [elements][8]
 };
 
-// Fills the tables of the elements order[lo, hi); false when more than kBrickNodes are staged.
-bool fill(Brick& b, const std::vector<int32_t>& order, const int32_t* conn, std::vector<int32_t>& scratch) {
+// Fills the tables of the elements order[lo, hi); false when more than NB nodes are staged.
+bool fill(Brick& b, const Splitter& sp, const int32_t* conn, std::vector<int32_t>& scratch) {
+    const std::vector<int32_t>& order = sp.order;
     const int ne = b.hi - b.lo;
     scratch.clear();
     for (int t = 0; t < ne; ++t)
@@ -101,7 +102,7 @@ bool fill(Brick& b, const std::vector<int32_t>& order, const int32_t* conn, std:
         for (size_t k = i; k < j; k += 8) b.nodes.push_back(sorted[i]);
         i = j;
     }
-    if ((int)b.nodes.size() > kBrickNodes) return false;
+    if ((int)b.nodes.size() > sp.NB) return false;
     b.linc.assign(b.nodes.size() * 8, 0xffff);
     b.lidx.resize((size_t)ne * 8);
     std::vector<uint8_t> fillc(b.nodes.size(), 0);
@@ -111,7 +112,7 @@ bool fill(Brick& b, const std::vector<int32_t>& order, const int32_t* conn, std:
             int l = (int)(std::lower_bound(b.nodes.begin(), b.nodes.end(), nd) - b.nodes.begin());
             while (fillc[l] == 8) ++l;
             b.lidx[(size_t)t * 8 + a] = (uint16_t)l;
-            b.linc[(size_t)l * 8 + fillc[l]++] = (uint16_t)(a * kBrick + t);
+            b.linc[(size_t)l * 8 + fillc[l]++] = (uint16_t)(sp.EB == kBrick ? a * kBrick + t : 8 * t + a);
         }
     return true;
 }
@@ -128,12 +129,12 @@ std::future<void> aside(Fn fn) {
 
 void grow(const Splitter& sp, int lo, int hi, const int32_t* conn, std::vector<Brick>& out, int depth) {
     std::vector<int32_t> bins, tmp, scratch;
-    if (hi - lo <= kBrick) {
+    if (hi - lo <= sp.EB) {
         Brick b;
         b.lo = lo;
         b.hi = hi;
         std::sort(sp.order.begin() + lo, sp.order.begin() + hi);
-        if (fill(b, sp.order, conn, scratch)) {
+        if (fill(b, sp, conn, scratch)) {
             out.push_back(std::move(b));
             return;
         }
@@ -155,42 +156,56 @@ void grow(const Splitter& sp, int lo, int hi, const int32_t* conn, std::vector<B
 
 void efe_build_bricks(BrickPattern& bp, int N, int E, const int32_t* conn, const double* coords,
                       const int32_t* specOfNode) {
-    // centroids in mean element sizes
+    // centroids in the mean element sizes of their specimen, from its lowest coordinates: the bricks of a
+    // specimen are the same whatever else is in the context
+    // (numbers from 0 up; any other is taken as 0 here)
+    auto spec = [&](int n) { return specOfNode && specOfNode[n] > 0 && specOfNode[n] < N ? specOfNode[n] : 0; };
+    int nspec = 1;
+    for (int n = 0; n < N; ++n) nspec = std::max(nspec, spec(n) + 1);
     std::vector<float> cen((size_t)3 * E);
-    double lo3[3], size[3] = {0, 0, 0};
-    for (int k = 0; k < 3; ++k) lo3[k] = coords[k];
-    for (int n = 1; n < N; ++n)
-        for (int k = 0; k < 3; ++k) lo3[k] = std::min(lo3[k], coords[(size_t)3 * n + k]);
-    for (int e = 0; e < E; ++e)
+    std::vector<double> lo3((size_t)3 * nspec, INFINITY), size((size_t)3 * nspec, 0.0);
+    std::vector<int> count(nspec, 0);
+    for (int n = 0; n < N; ++n)
         for (int k = 0; k < 3; ++k) {
-            double mn = coords[(size_t)3 * conn[(size_t)8 * e] + k], mx = mn, s = 0.0;
+            double& lo = lo3[3 * (size_t)spec(n) + k];
+            lo = std::min(lo, coords[(size_t)3 * n + k]);
+        }
+    for (int e = 0; e < E; ++e) {
+        const int s = spec(conn[(size_t)8 * e]);
+        ++count[s];
+        for (int k = 0; k < 3; ++k) {
+            double mn = coords[(size_t)3 * conn[(size_t)8 * e] + k], mx = mn, sum = 0.0;
             for (int a = 0; a < 8; ++a) {
                 const double v = coords[(size_t)3 * conn[(size_t)8 * e + a] + k];
                 mn = std::min(mn, v);
                 mx = std::max(mx, v);
-                s += v;
+                sum += v;
             }
-            size[k] += mx - mn;
-            cen[(size_t)k * E + e] = (float)(s * 0.125 - lo3[k]);
+            size[(size_t)3 * s + k] += mx - mn;
+            cen[(size_t)k * E + e] = (float)(sum * 0.125 - lo3[(size_t)3 * s + k]);
         }
-    for (int k = 0; k < 3; ++k) {
-        const double h = size[k] / E;
-        if (h > 0.0 && std::isfinite(h))
-            for (int e = 0; e < E; ++e) cen[(size_t)k * E + e] = (float)(cen[(size_t)k * E + e] / h);
+    }
+    for (int e = 0; e < E; ++e) {
+        const int s = spec(conn[(size_t)8 * e]);
+        for (int k = 0; k < 3; ++k) {
+            const double h = size[(size_t)3 * s + k] / count[s];
+            if (h > 0.0 && std::isfinite(h)) cen[(size_t)k * E + e] = (float)(cen[(size_t)k * E + e] / h);
+        }
     }
     std::vector<int32_t> order(E);
     for (int e = 0; e < E; ++e) order[e] = e;
     std::vector<int> seg;  // a brick holds elements of one specimen
     if (specOfNode) {
-        auto spec = [&](int e) { return specOfNode[conn[(size_t)8 * e]]; };
-        std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) { return spec(a) < spec(b); });
+        auto of = [&](int e) { return specOfNode[conn[(size_t)8 * e]]; };
+        std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) { return of(a) < of(b); });
         for (int i = 0; i < E; ++i)
-            if (i == 0 || spec(order[i]) != spec(order[i - 1])) seg.push_back(i);
+            if (i == 0 || of(order[i]) != of(order[i - 1])) seg.push_back(i);
     } else {
         seg.push_back(0);
     }
     seg.push_back(E);
-    Splitter sp{cen, order, E};
+    const int EB = bp.EB, NB = bp.NB = EB == kBrick ? kBrickNodes : 8 * EB;
+    Splitter sp{cen, order, E, EB, NB};
     std::vector<Brick> bricks;
     if (seg.size() == 2) {
         grow(sp, 0, E, conn, bricks, 3);
@@ -209,17 +224,17 @@ void efe_build_bricks(BrickPattern& bp, int N, int E, const int32_t* conn, const
     const int G = bp.G = (int)bricks.size();
     // tables at a fixed pitch per brick, so that a workgroup finds its own without reading offsets
     bp.pos.resize(E);
-    bp.lidx.assign((size_t)G * kBrick * 8, 0xffff);
-    bp.lnode.assign((size_t)G * kBrickNodes, -1);
-    bp.lpos.assign((size_t)G * kBrickNodes, 0);
-    bp.linc.assign((size_t)G * kBrickNodes * 8, 0xffff);
+    bp.lidx.assign((size_t)G * EB * 8, 0xffff);
+    bp.lnode.assign((size_t)G * NB, -1);
+    bp.lpos.assign((size_t)G * NB, 0);
+    bp.linc.assign((size_t)G * NB * 8, 0xffff);
     bp.pptr.assign(N + 1, 0);
     for (int g = 0; g < G; ++g) {
         const Brick& b = bricks[g];
-        std::copy(b.nodes.begin(), b.nodes.end(), bp.lnode.begin() + (size_t)g * kBrickNodes);
-        std::copy(b.linc.begin(), b.linc.end(), bp.linc.begin() + (size_t)g * kBrickNodes * 8);
-        std::copy(b.lidx.begin(), b.lidx.end(), bp.lidx.begin() + (size_t)g * kBrick * 8);
-        for (int i = b.lo; i < b.hi; ++i) bp.pos[order[i]] = g * kBrick + (i - b.lo);
+        std::copy(b.nodes.begin(), b.nodes.end(), bp.lnode.begin() + (size_t)g * NB);
+        std::copy(b.linc.begin(), b.linc.end(), bp.linc.begin() + (size_t)g * NB * 8);
+        std::copy(b.lidx.begin(), b.lidx.end(), bp.lidx.begin() + (size_t)g * EB * 8);
+        for (int i = b.lo; i < b.hi; ++i) bp.pos[order[i]] = g * EB + (i - b.lo);
         for (int32_t nd : b.nodes) ++bp.pptr[nd + 1];
         if (specOfNode) bp.spec.push_back(specOfNode[b.nodes[0]]);
     }

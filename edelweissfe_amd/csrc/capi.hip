@@ -248,6 +248,7 @@ int efe_ctx_create(const efe_mesh_desc* d, efe_ctx** out) {
         }
     // the bricks of the matrix-free product, beside the pattern
     BrickPattern bp;
+    bp.EB = !d->specimen_of_node && c->E <= kSplitElements ? kBrickSplit : kBrick;
     std::future<void> bricks;
     if (c->eltype == EFE_C3D8) {
         auto build = [&bp, N = c->N, E = c->E, conn = d->conn, xyz = d->coords, spec = d->specimen_of_node] {

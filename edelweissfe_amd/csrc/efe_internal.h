@@ -45,6 +45,39 @@ __device__ __forceinline__ void add_block(const KT* src, KT (&acc)[9]) {
     for (int v = 0; v < 9; ++v) acc[v] += src[v];
 }
 
+// value of the lane whose number differs in bit H (1, 2 or 4) of the lane number
+template <int H>
+__device__ __forceinline__ double lane_xor8(double v) {
+    int lo = __double2loint(v), hi = __double2hiint(v);
+    if constexpr (H == 1) {  // quad_perm [1, 0, 3, 2]
+        lo = __builtin_amdgcn_update_dpp(0, lo, 0xB1, 0xF, 0xF, true);
+        hi = __builtin_amdgcn_update_dpp(0, hi, 0xB1, 0xF, 0xF, true);
+    } else if constexpr (H == 2) {  // quad_perm [2, 3, 0, 1]
+        lo = __builtin_amdgcn_update_dpp(0, lo, 0x4E, 0xF, 0xF, true);
+        hi = __builtin_amdgcn_update_dpp(0, hi, 0x4E, 0xF, 0xF, true);
+    } else {  // row_half_mirror (xor 7), then quad_perm [3, 2, 1, 0] (xor 3)
+        lo = __builtin_amdgcn_update_dpp(0, lo, 0x141, 0xF, 0xF, true);
+        hi = __builtin_amdgcn_update_dpp(0, hi, 0x141, 0xF, 0xF, true);
+        lo = __builtin_amdgcn_update_dpp(0, lo, 0x1B, 0xF, 0xF, true);
+        hi = __builtin_amdgcn_update_dpp(0, hi, 0x1B, 0xF, 0xF, true);
+    }
+    return __hiloint2double(hi, lo);
+}
+
+template <int H>
+__device__ __forceinline__ float lane_xor8(float v) {
+    int b = __float_as_int(v);
+    if constexpr (H == 1) {
+        b = __builtin_amdgcn_update_dpp(0, b, 0xB1, 0xF, 0xF, true);
+    } else if constexpr (H == 2) {
+        b = __builtin_amdgcn_update_dpp(0, b, 0x4E, 0xF, 0xF, true);
+    } else {
+        b = __builtin_amdgcn_update_dpp(0, b, 0x141, 0xF, 0xF, true);
+        b = __builtin_amdgcn_update_dpp(0, b, 0x1B, 0xF, 0xF, true);
+    }
+    return __int_as_float(b);
+}
+
 struct HostPattern {
     int N = 0, E = 0, NN = 0;
     std::vector<int32_t> bptr, bcol;      // node adjacency (block CSR), columns ascending
@@ -62,24 +95,41 @@ struct HostPattern {
     int64_t padded_blocks = 0;
 };
 
-// Bricks of the hexa8 matrix-free operator: at most kBrick elements and kBrickNodes staged nodes.
+// Bricks of the hexa8 matrix-free operator: at most kBrick elements and kBrickNodes staged nodes, or
+// (split bricks) kBrickSplit elements, whose 8 nodes each are the most that can be staged.
 constexpr int kBrick = 256;
 constexpr int kBrickNodes = 512;
+constexpr int kBrickSplit = 32;
+// Meshes of up to this many elements take split bricks (batches never: a specimen has the same bricks,
+// and so the same bits, alone and with others): fewer whole ones leave CUs idle, or at one
+// workgroup each; beyond it the repeated set-up costs more.  PCG iteration, whole / split bricks: FP64
+// 8^3 17.6 / 14.0 us, 20^3 19.9 / 16.2, 28^3 (21952) 21.4 / 20.8, 32^3 22.2 / 22.8, 40^3 30.0 / 38.3;
+// FP32 8^3 17.1 / 13.0, 20^3 18.7 / 14.6, 28^3 19.9 / 17.7, 32^3 20.3 / 18.4, 40^3 23.0 / 29.5.
+constexpr int kSplitElements = 24576;
+
+// place of QP q of the element at pos (BrickPattern) among the tangents' rows of kBrick lanes
+__host__ __device__ inline int64_t brick_slot(int32_t pos, int q, int EB) {
+    if (EB == kBrick) return (int64_t)(pos / kBrick * 8 + q) * kBrick + pos % kBrick;
+    return (int64_t)pos * 8 + q;
+}
 
 struct BrickPattern {
+    int EB = kBrick, NB = kBrickNodes;  // elements and staged entries a brick has room for
     int G = 0;
     int64_t L = 0;                // partials: (brick, node) pairs
-    std::vector<int32_t> pos;     // [E] element -> brick * kBrick + its place (ascending in a brick)
-    std::vector<uint16_t> lidx;   // [G * kBrick][8] staged entries of the element there, 0xffff: none
-    std::vector<int32_t> lnode;   // [G * kBrickNodes] node of each staged entry, -1: none (a node with
+    std::vector<int32_t> pos;     // [E] element -> brick * EB + its place (ascending in a brick)
+    std::vector<uint16_t> lidx;   // [G * EB][8] staged entries of the element there, 0xffff: none
+    std::vector<int32_t> lnode;   // [G * NB] node of each staged entry, -1: none (a node with
                                   // more than 8 incidences in a brick has several entries)
-    std::vector<int32_t> lpos;    // [G * kBrickNodes] its slot among the node's partials
-    std::vector<uint16_t> linc;   // [G * kBrickNodes][8] incidences a * kBrick + t, element order, 0xffff: none
+    std::vector<int32_t> lpos;    // [G * NB] its slot among the node's partials
+    std::vector<uint16_t> linc;   // [G * NB][8] incidences a * kBrick + t (split: 8 t + a), element order,
+                                  // 0xffff: none
     std::vector<int32_t> pptr;    // [N+1] partials of each node, in brick order
     std::vector<int32_t> spec;    // [G] specimen of each brick (specimens given)
 };
 
-// conn [E][8], coords [N][3], specOfNode [N] or null (a brick then holds one specimen's elements)
+// conn [E][8], coords [N][3], specOfNode [N] or null (given: a brick holds one specimen's elements);
+// bp.EB set
 void efe_build_bricks(BrickPattern& bp, int N, int E, const int32_t* conn, const double* coords,
                       const int32_t* specOfNode);
 
@@ -140,19 +190,20 @@ struct efe_ctx {
     double* shapeNe = nullptr;   // [Q][NN] at the evaluation points (QP coordinates)
     // matrix-free FP32 operator of hexa20: [Q][NC][E] compact tangent, [E*NN][3] node-sorted force
     // slots, dnxi32 = FP32 dNdxi then dJdxi ([2][Q][NN][3]).  hexa8 (bricks): mfC / mfC64
-    // [brick][Q][NC][kBrick] compact tangents of the last FP32 matrix-free / FP64 tangent pass
+    // compact tangents [row][NC][kBrick] (brick_slot) of the last FP32 matrix-free / FP64 tangent pass
     float *mfC = nullptr, *mfF = nullptr, *dnxi32 = nullptr;
     double* mfC64 = nullptr;
     // hexa8 bricks (bricks.cpp): BrickPattern's tables on the device, the staged nodes'
     // coordinates, and the partial forces [L][3] in the precision of the product
     bool mfb = false;
     int mfbG = 0;                // bricks
+    int mfbE = kBrick;         // BrickPattern's EB
     int64_t mfbL = 0;            // partials
     void* mfbTables = nullptr;   // one allocation: the tables below
     int32_t *mfbPos = nullptr, *mfbLnode = nullptr, *mfbLpos = nullptr, *mfbPptr = nullptr, *mfbSpec = nullptr;
     uint16_t *mfbLinc = nullptr, *mfbLidx = nullptr;
-    double* mfbX = nullptr;      // [3][G * kBrickNodes]
-    float *mfbEl = nullptr, *mfbF = nullptr;       // [2][G * kBrick] bulk modulus and 2 G; [L][3]
+    double* mfbX = nullptr;      // [3][G * NB]
+    float *mfbEl = nullptr, *mfbF = nullptr;       // [2][G * EB] bulk modulus and 2 G; [L][3]
     double *mfbEl64 = nullptr, *mfbF64 = nullptr;
     int dirVersion = 0;          // incremented by every efe_set_dirichlet
     // per specimen, the dirVersion of the last FP64 pass over it, whose tangents mfC64 holds (-1: none),

@@ -40,18 +40,18 @@ struct MatState {
 // The compact tangent of QP q of element e for the matrix-free product, from cc = [A, B, cnn, cn1,
 // c1n, n]: ncw = 8 [A, B, cnn, n], 7 (A left out), 10 [A, B, cnn, cn1, c1n, n] (cn1 = c1n = 0 but
 // DP) or 0 values, the coefficients times f = w detJ; n is deviatoric (n_33 = -n_11 - n_22): its
-// five other components are stored.  Element e lies at its place mfPos in the bricks (hexa8), or in
-// element order.  (Constant indices into cc only: a variable one would put it into scratch memory.)
+// five other components are stored.  Element e lies at its place mfPos in the bricks of mfEB elements
+// (hexa8), or in element order.  (Constant indices into cc only: a variable one would put it into scratch memory.)
 template <typename CT>
-__device__ __forceinline__ void store_compact(CT* __restrict__ mfC, const int32_t* __restrict__ mfPos, int E, int Q,
-                                              int e, int q, int ncw, double f, const double (&cc)[11]) {
+__device__ __forceinline__ void store_compact(CT* __restrict__ mfC, const int32_t* __restrict__ mfPos, int mfEB, int E,
+                                              int Q, int e, int q, int ncw, double f, const double (&cc)[11]) {
     if (!ncw) return;
     CT* dc;
     int64_t stride = E;
     if (mfPos) {
-        const int pos = mfPos[e];
+        const int64_t slot = brick_slot(mfPos[e], q, mfEB);
         stride = kBrick;
-        dc = mfC + ((int64_t)(pos / kBrick) * Q + q) * ncw * kBrick + pos % kBrick;
+        dc = mfC + slot / kBrick * ncw * kBrick + slot % kBrick;
     } else {
         dc = mfC + (int64_t)q * ncw * E + e;
     }
@@ -193,7 +193,7 @@ __global__ __launch_bounds__(64) void element_kernel(int E, int N, const double*
             *status = 1;
             if (specStatus) specStatus[specOfElem[e]] = 1;  // which specimen asked (batched contexts)
         }
-        if (mfC && formK) store_compact(mfC, (const int32_t*)nullptr, E, Q, e, q, ncw, det * qpw[q], cc);
+        if (mfC && formK) store_compact(mfC, (const int32_t*)nullptr, 0, E, Q, e, q, ncw, det * qpw[q], cc);
 #pragma unroll
         for (int c = 0; c < 6; ++c) {
             sTmp[c * EQ + sidx] = s[c];
@@ -365,25 +365,6 @@ __global__ __launch_bounds__(64) void element_kernel(int E, int N, const double*
 // The QP evaluated at (eta_q, xi_q, zeta_q) of the table lies in the octant of node q, so a
 // lane's sign pattern serves it as node and as QP.
 
-// value of the lane whose number differs in bit H (1, 2 or 4) of the lane number
-template <int H>
-__device__ __forceinline__ double lane_xor8(double v) {
-    int lo = __double2loint(v), hi = __double2hiint(v);
-    if constexpr (H == 1) {  // quad_perm [1, 0, 3, 2]
-        lo = __builtin_amdgcn_update_dpp(0, lo, 0xB1, 0xF, 0xF, true);
-        hi = __builtin_amdgcn_update_dpp(0, hi, 0xB1, 0xF, 0xF, true);
-    } else if constexpr (H == 2) {  // quad_perm [2, 3, 0, 1]
-        lo = __builtin_amdgcn_update_dpp(0, lo, 0x4E, 0xF, 0xF, true);
-        hi = __builtin_amdgcn_update_dpp(0, hi, 0x4E, 0xF, 0xF, true);
-    } else {  // row_half_mirror (xor 7), then quad_perm [3, 2, 1, 0] (xor 3)
-        lo = __builtin_amdgcn_update_dpp(0, lo, 0x141, 0xF, 0xF, true);
-        hi = __builtin_amdgcn_update_dpp(0, hi, 0x141, 0xF, 0xF, true);
-        lo = __builtin_amdgcn_update_dpp(0, lo, 0x1B, 0xF, 0xF, true);
-        hi = __builtin_amdgcn_update_dpp(0, hi, 0x1B, 0xF, 0xF, true);
-    }
-    return __hiloint2double(hi, lo);
-}
-
 // value of lane 0 of the 8 lanes of an element
 __device__ __forceinline__ double lane_first8(double v, bool upper) {
     int lo = __double2loint(v), hi = __double2hiint(v);
@@ -423,7 +404,7 @@ __global__ __launch_bounds__(64) void hex8_kernel(
     const double* __restrict__ sRef, double* __restrict__ sTmp, KT* __restrict__ Kscr, double* __restrict__ Pscr,
     int* __restrict__ status, KT* __restrict__ mfC, const int32_t* __restrict__ mfPos, int* __restrict__ specStatus,
     const int32_t* __restrict__ specOfElem, const int32_t* __restrict__ cpos, const int* __restrict__ specActive,
-    const int32_t* __restrict__ elist, int ecount, int ncw) {
+    const int32_t* __restrict__ elist, int ecount, int ncw, int mfEB) {
     using L = Hex8Lds<MAT, KT, MF, TAN>;
     constexpr int NP = (MAT == EFE_LINEAR_ELASTIC) ? 2 : 6;
     constexpr bool HAS_K = MatState<MAT>::n != 0;
@@ -528,7 +509,7 @@ __global__ __launch_bounds__(64) void hex8_kernel(
             sTmp[(6 + c) * EQ + sidx] = eps[c] + de[c];
         }
         if (HAS_K) sTmp[12 * EQ + sidx] = ms;
-        if (TAN && mfC) store_compact(mfC, mfPos, E, 8, e, j, ncw, det, cc);
+        if (TAN && mfC) store_compact(mfC, mfPos, mfEB, E, 8, e, j, ncw, det, cc);
     }
     // reference gradients of an octant pair: t*(b)[c] = (1 +- g s)(1 +- g s) / 8 of the two other axes
     double tx[2][2], ty[2][2], tz[2][2];
@@ -1241,7 +1222,7 @@ int launch_hex8(efe_ctx* c, const double* dU) {
     const int* act = c->useActive ? c->specActive : nullptr;
 #define HEX8_ARGS(T, C)                                                                                            \
     c->E, c->N, c->coords, c->conn, c->props, propStride, dU, c->stateRef, c->stateTmp, (T*)c->Kscr, c->Pscr,         \
-        c->status, C, c->mfbPos, c->specStatus, c->specOfElem, c->cpos, act, c->curList, c->curCount, c->mfNC
+        c->status, C, c->mfbPos, c->specStatus, c->specOfElem, c->cpos, act, c->curList, c->curCount, c->mfNC, c->mfbE
     if (!c->formK)
         hex8_kernel<MAT, double, false, false><<<grid, 64, 0, c->stream>>>(HEX8_ARGS(double, (double*)nullptr));
     else if (c->mfPass)

@@ -26,7 +26,8 @@
 // half of it) for the tangents (NC = 7), ~1.6 staged nodes of 48 + 2 x 24 (12) bytes, 16 of local
 // indices: 614 in FP64, against 2135 of the assembled blocks at 64^3 (27 x 72 + 27 x 4 per node).
 // Measured at 64^3 in FP64: 100 us per assembled product (5.6 TB/s), 43 us per brick product with
-// the tangents from HBM, ~36 us with them in the Infinity Cache; PCG iteration 123.7 -> 62.7 us.
+// the tangents from HBM, ~36 us with them in the Infinity Cache; PCG iteration 123.7 -> 59.0 us.  Meshes of up to
+// kSplitElements elements have bricks of 32, with 8 lanes per element.
 #include <algorithm>
 #include <cstring>
 #include <type_traits>
@@ -279,10 +280,85 @@ __device__ __forceinline__ void walsh3_t(T (&w)[8]) {
             }
 }
 
-// The element's forces in the monomial basis (fa, x 8) from those of p (cp) and of the coordinates
-// (cx), summed over its QPs, whose tangents start at Cg.  HOT: plain loads, which leave the tangents
-// in the Infinity Cache for the next product; else non-temporal ones.  The loop is not unrolled:
-// unrolled, it hoists the tangent loads of all QPs and needs half as many registers again.
+// One QP at (x, y, z): adds its share of the element's forces in the monomial basis (fa, x 8), from
+// the coefficients of p (cp) and of the coordinates (cx) and its NC values cf.
+template <int NC, typename T>
+__device__ __forceinline__ void brick_qp(const T (&cf)[NC ? NC : 1], T bulk, T shear2, T x, T y, T z,
+                                         const T (&cp)[3][8], const T (&cx)[3][8], T (&fa)[3][8]) {
+    const T xy = x * y, yz = y * z, xz = x * z;
+    // natural gradients: d/dx = c1 + c3 y + c5 z + c7 yz, d/dy = c2 + c3 x + c6 z + c7 xz,
+    // d/dz = c4 + c5 x + c6 y + c7 xy   (index = canonical monomial bits)
+    T H[9], J[9];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        H[i * 3 + 0] = cp[i][1] + cp[i][3] * y + cp[i][5] * z + cp[i][7] * yz;
+        H[i * 3 + 1] = cp[i][2] + cp[i][3] * x + cp[i][6] * z + cp[i][7] * xz;
+        H[i * 3 + 2] = cp[i][4] + cp[i][5] * x + cp[i][6] * y + cp[i][7] * xy;
+        J[0 * 3 + i] = cx[i][1] + cx[i][3] * y + cx[i][5] * z + cx[i][7] * yz;
+        J[1 * 3 + i] = cx[i][2] + cx[i][3] * x + cx[i][6] * z + cx[i][7] * xz;
+        J[2 * 3 + i] = cx[i][4] + cx[i][5] * x + cx[i][6] * y + cx[i][7] * xy;
+    }
+    const T det = J[0] * (J[4] * J[8] - J[5] * J[7]) - J[1] * (J[3] * J[8] - J[5] * J[6]) +
+                  J[2] * (J[3] * J[7] - J[4] * J[6]);
+    const T id = (T)1 / det;
+    const T iJ[9] = {(J[4] * J[8] - J[5] * J[7]) * id, (J[2] * J[7] - J[1] * J[8]) * id,
+                     (J[1] * J[5] - J[2] * J[4]) * id, (J[5] * J[6] - J[3] * J[8]) * id,
+                     (J[0] * J[8] - J[2] * J[6]) * id, (J[2] * J[3] - J[0] * J[5]) * id,
+                     (J[3] * J[7] - J[4] * J[6]) * id, (J[1] * J[6] - J[0] * J[7]) * id,
+                     (J[0] * J[4] - J[1] * J[3]) * id};
+    T gr[9];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+            gr[i * 3 + j] = H[i * 3] * iJ[j * 3] + H[i * 3 + 1] * iJ[j * 3 + 1] + H[i * 3 + 2] * iJ[j * 3 + 2];
+    const T ep[6] = {gr[0], gr[4], gr[8], gr[1] + gr[3], gr[2] + gr[6], gr[5] + gr[7]};
+    // the Gauss weights of hexa8 are 1: w detJ = det
+    const T A = NC == 10 ? cf[0] : bulk * det;
+    const T B = NC == 10 ? cf[1] : (NC == 7 ? cf[0] : shear2 * det);
+    const T tr = ep[0] + ep[1] + ep[2], t3 = tr * (T)(1.0 / 3.0);
+    T s1 = A * tr, sg[6];
+    if constexpr (NC != 0) {
+        const T* nc = cf + (NC == 10 ? 5 : 2);
+        const T n[6] = {nc[0], nc[1], -(nc[0] + nc[1]), nc[2], nc[3], nc[4]};  // n deviatoric
+        const T ne_ = n[0] * ep[0] + n[1] * ep[1] + n[2] * ep[2] + n[3] * ep[3] + n[4] * ep[4] + n[5] * ep[5];
+        T sn = (NC == 10 ? cf[2] : cf[1]) * ne_;
+        if constexpr (NC == 10) {
+            sn += cf[3] * tr;
+            s1 += cf[4] * ne_;
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i) sg[i] = s1 + B * (ep[i] - t3) + sn * n[i];
+#pragma unroll
+        for (int i = 3; i < 6; ++i) sg[i] = (T)0.5 * B * ep[i] + sn * n[i];
+    } else {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) sg[i] = s1 + B * (ep[i] - t3);
+#pragma unroll
+        for (int i = 3; i < 6; ++i) sg[i] = (T)0.5 * B * ep[i];
+    }
+    const T S[9] = {sg[0], sg[3], sg[4], sg[3], sg[1], sg[5], sg[4], sg[5], sg[2]};
+    // f_a,i += sum_k M_ik dN_a/dxi_k with M_ik = sum_j sig_ij iJ_jk, in monomials:
+    // fa[1] += M0, fa[2] += M1, fa[4] += M2, fa[3] += M0 y + M1 x, fa[5] += M0 z + M2 x,
+    // fa[6] += M1 z + M2 y, fa[7] += M0 yz + M1 xz + M2 xy   (M_k = column k, x 1/8)
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const T m0 = S[i * 3] * iJ[0] + S[i * 3 + 1] * iJ[3] + S[i * 3 + 2] * iJ[6];
+        const T m1 = S[i * 3] * iJ[1] + S[i * 3 + 1] * iJ[4] + S[i * 3 + 2] * iJ[7];
+        const T m2 = S[i * 3] * iJ[2] + S[i * 3 + 1] * iJ[5] + S[i * 3 + 2] * iJ[8];
+        fa[i][1] += m0;
+        fa[i][2] += m1;
+        fa[i][4] += m2;
+        fa[i][3] += m0 * y + m1 * x;
+        fa[i][5] += m0 * z + m2 * x;
+        fa[i][6] += m1 * z + m2 * y;
+        fa[i][7] += m0 * yz + m1 * xz + m2 * xy;
+    }
+}
+
+// The sum over the element's QPs, whose tangents start at Cg.  HOT: plain loads, which leave the
+// tangents in the Infinity Cache for the next product; else non-temporal ones.  The loop is not
+// unrolled: unrolled, it hoists the tangent loads of all QPs and needs half as many registers again.
 template <int NC, typename T, bool HOT>
 __device__ __forceinline__ void brick_qps(const T* __restrict__ Cg, T bulk, T shear2, const T (&cp)[3][8],
                                           const T (&cx)[3][8], T (&fa)[3][8]) {
@@ -292,8 +368,6 @@ __device__ __forceinline__ void brick_qps(const T* __restrict__ Cg, T bulk, T sh
         // evaluation point (eta_q, xi_q, zeta_q) of the QP table xi = (-,-,-,-,+,+,+,+),
         // eta = (-,-,+,+,-,-,+,+), zeta = (-,+,+,-,-,+,+,-) (times 1/sqrt 3)
         const int r = q & 3;
-        const T x = (r < 2 ? -gq : gq), y = (q < 4 ? -gq : gq), z = ((r == 1 || r == 2) ? gq : -gq);
-        const T xy = x * y, yz = y * z, xz = x * z;
         T cf[NC ? NC : 1];
 #pragma unroll
         for (int k = 0; k < NC; ++k) {
@@ -301,74 +375,8 @@ __device__ __forceinline__ void brick_qps(const T* __restrict__ Cg, T bulk, T sh
             if constexpr (HOT) cf[k] = *src;
             else cf[k] = __builtin_nontemporal_load(src);
         }
-        // natural gradients: d/dx = c1 + c3 y + c5 z + c7 yz, d/dy = c2 + c3 x + c6 z + c7 xz,
-        // d/dz = c4 + c5 x + c6 y + c7 xy   (index = canonical monomial bits)
-        T H[9], J[9];
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            H[i * 3 + 0] = cp[i][1] + cp[i][3] * y + cp[i][5] * z + cp[i][7] * yz;
-            H[i * 3 + 1] = cp[i][2] + cp[i][3] * x + cp[i][6] * z + cp[i][7] * xz;
-            H[i * 3 + 2] = cp[i][4] + cp[i][5] * x + cp[i][6] * y + cp[i][7] * xy;
-            J[0 * 3 + i] = cx[i][1] + cx[i][3] * y + cx[i][5] * z + cx[i][7] * yz;
-            J[1 * 3 + i] = cx[i][2] + cx[i][3] * x + cx[i][6] * z + cx[i][7] * xz;
-            J[2 * 3 + i] = cx[i][4] + cx[i][5] * x + cx[i][6] * y + cx[i][7] * xy;
-        }
-        const T det = J[0] * (J[4] * J[8] - J[5] * J[7]) - J[1] * (J[3] * J[8] - J[5] * J[6]) +
-                      J[2] * (J[3] * J[7] - J[4] * J[6]);
-        const T id = (T)1 / det;
-        const T iJ[9] = {(J[4] * J[8] - J[5] * J[7]) * id, (J[2] * J[7] - J[1] * J[8]) * id,
-                         (J[1] * J[5] - J[2] * J[4]) * id, (J[5] * J[6] - J[3] * J[8]) * id,
-                         (J[0] * J[8] - J[2] * J[6]) * id, (J[2] * J[3] - J[0] * J[5]) * id,
-                         (J[3] * J[7] - J[4] * J[6]) * id, (J[1] * J[6] - J[0] * J[7]) * id,
-                         (J[0] * J[4] - J[1] * J[3]) * id};
-        T gr[9];
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-#pragma unroll
-            for (int j = 0; j < 3; ++j)
-                gr[i * 3 + j] = H[i * 3] * iJ[j * 3] + H[i * 3 + 1] * iJ[j * 3 + 1] + H[i * 3 + 2] * iJ[j * 3 + 2];
-        const T ep[6] = {gr[0], gr[4], gr[8], gr[1] + gr[3], gr[2] + gr[6], gr[5] + gr[7]};
-        // the Gauss weights of hexa8 are 1: w detJ = det
-        const T A = NC == 10 ? cf[0] : bulk * det;
-        const T B = NC == 10 ? cf[1] : (NC == 7 ? cf[0] : shear2 * det);
-        const T tr = ep[0] + ep[1] + ep[2], t3 = tr * (T)(1.0 / 3.0);
-        T s1 = A * tr, sg[6];
-        if constexpr (NC != 0) {
-            const T* nc = cf + (NC == 10 ? 5 : 2);
-            const T n[6] = {nc[0], nc[1], -(nc[0] + nc[1]), nc[2], nc[3], nc[4]};  // n deviatoric
-            const T ne_ = n[0] * ep[0] + n[1] * ep[1] + n[2] * ep[2] + n[3] * ep[3] + n[4] * ep[4] + n[5] * ep[5];
-            T sn = (NC == 10 ? cf[2] : cf[1]) * ne_;
-            if constexpr (NC == 10) {
-                sn += cf[3] * tr;
-                s1 += cf[4] * ne_;
-            }
-#pragma unroll
-            for (int i = 0; i < 3; ++i) sg[i] = s1 + B * (ep[i] - t3) + sn * n[i];
-#pragma unroll
-            for (int i = 3; i < 6; ++i) sg[i] = (T)0.5 * B * ep[i] + sn * n[i];
-        } else {
-#pragma unroll
-            for (int i = 0; i < 3; ++i) sg[i] = s1 + B * (ep[i] - t3);
-#pragma unroll
-            for (int i = 3; i < 6; ++i) sg[i] = (T)0.5 * B * ep[i];
-        }
-        const T S[9] = {sg[0], sg[3], sg[4], sg[3], sg[1], sg[5], sg[4], sg[5], sg[2]};
-        // f_a,i += sum_k M_ik dN_a/dxi_k with M_ik = sum_j sig_ij iJ_jk, in monomials:
-        // fa[1] += M0, fa[2] += M1, fa[4] += M2, fa[3] += M0 y + M1 x, fa[5] += M0 z + M2 x,
-        // fa[6] += M1 z + M2 y, fa[7] += M0 yz + M1 xz + M2 xy   (M_k = column k, x 1/8)
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            const T m0 = S[i * 3] * iJ[0] + S[i * 3 + 1] * iJ[3] + S[i * 3 + 2] * iJ[6];
-            const T m1 = S[i * 3] * iJ[1] + S[i * 3 + 1] * iJ[4] + S[i * 3 + 2] * iJ[7];
-            const T m2 = S[i * 3] * iJ[2] + S[i * 3 + 1] * iJ[5] + S[i * 3 + 2] * iJ[8];
-            fa[i][1] += m0;
-            fa[i][2] += m1;
-            fa[i][4] += m2;
-            fa[i][3] += m0 * y + m1 * x;
-            fa[i][5] += m0 * z + m2 * x;
-            fa[i][6] += m1 * z + m2 * y;
-            fa[i][7] += m0 * yz + m1 * xz + m2 * xy;
-        }
+        brick_qp<NC, T>(cf, bulk, shear2, (r < 2 ? -gq : gq), (q < 4 ? -gq : gq), ((r == 1 || r == 2) ? gq : -gq), cp,
+                        cx, fa);
     }
 }
 
@@ -376,11 +384,12 @@ __device__ __forceinline__ void brick_qps(const T* __restrict__ Cg, T bulk, T sh
 struct BrickTables {
     const int32_t *lnode, *lpos, *spec;
     const uint16_t *linc, *lidx;
-    const double* X;  // [3][G * kBrickNodes] coordinates of the staged nodes
+    const double* X;  // [3][G * NB] coordinates of the staged nodes
     int G, hot;
 };
 
-// Hexa8 product by bricks: workgroup g takes the up to kBrick elements of brick g, one lane each.
+// Hexa8 product by bricks: workgroup g takes the up to kBrick / P elements of brick g, P = 1 or 8
+// lanes each.
 // The brick's distinct nodes (p with Dirichlet DOFs masked, and the coordinates, which lie in
 // staging order) go to LDS once, after two dependent loads (the node, then its values: the tables
 // have a fixed pitch, and the flags are waited for beside them); each lane forms its element's forces in the monomial basis and
@@ -392,37 +401,50 @@ struct BrickTables {
 // at hand; 10 with Drucker-Prager (A, B, c_nn, c_n1, c_1n and n as stored); 0 when every
 // element is linear elastic (B = 2 G w detJ likewise).  T is the precision of the arithmetic,
 // the tangents and the partials.
-template <int NC, typename T, typename TP>
+//
+// P = 8 (split bricks): a lane has one QP; its forces on the 8 nodes are summed over the element's
+// lanes by halving exchanges, which leave each lane one node's.  This repeats the element's set-up in
+// 8 lanes, but takes the tangents in one round of loads and needs 32 elements per CU, not 256: the
+// product of a small mesh is a chain of latencies (320 elements: 9.3 us on two whole bricks; PCG
+// iteration 17.4 -> 14 us).
+template <int NC, typename T, typename TP, int P>
 __global__ __launch_bounds__(kBrick) void brick_apply_kernel(
     BrickTables bt, const T* __restrict__ el, const T* __restrict__ C, const TP* __restrict__ p,
     const uint8_t* __restrict__ dirflag, int mask, const int* __restrict__ flags, T* __restrict__ Fpart,
     const int* __restrict__ active, double* __restrict__ part) {
-    // LDS, reused: first the staged nodes (x 3 doubles, p 3 T), then the element forces (24 T a lane)
-    constexpr int kStage = 3 * kBrickNodes * (int)(sizeof(double) + sizeof(T));
-    constexpr int kForce = 24 * kBrick * (int)sizeof(T);
+    constexpr int EB = kBrick / P, NB = P == 1 ? kBrickNodes : 8 * EB;
+    // LDS, reused: first the staged nodes (x 3 doubles, p 3 T), then the element forces (24 T each)
+    constexpr int kStage = 3 * NB * (int)(sizeof(double) + sizeof(T));
+    constexpr int kForce = 24 * EB * (int)sizeof(T);
     __shared__ __align__(16) char lds[kStage > kForce ? kStage : kForce];
     __shared__ double red[kBrick / 64];
     double* sx = (double*)lds;
-    T* sp = (T*)(lds + 3 * kBrickNodes * sizeof(double));
+    T* sp = (T*)(lds + 3 * NB * sizeof(double));
     T* sf = (T*)lds;
     const int g = xcd_block_mf();
     if (g >= bt.G) {  // the grid is rounded up to a multiple of 8
         if (part && threadIdx.x == 0) part[g] = 0.0;
         return;
     }
-    constexpr int NS = kBrickNodes / kBrick;  // staged nodes per lane
+    constexpr int NS = NB / kBrick;  // staged nodes per lane
     const int t = threadIdx.x;
-    const int64_t l0 = (int64_t)g * kBrickNodes + t;
+    const int64_t l0 = (int64_t)g * NB + t;
     int nd[NS];
 #pragma unroll
     for (int k = 0; k < NS; ++k) nd[k] = bt.lnode[l0 + k * kBrick];
     // the element's 8 staged entries in one 16-byte load; 0xffff: no element for this lane
-    const uint4 li4 = *reinterpret_cast<const uint4*>(bt.lidx + ((int64_t)g * kBrick + t) * 8);
-    const T bulk = NC != 10 ? el[g * kBrick + t] : (T)0;
-    const T shear2 = NC == 0 ? el[(int64_t)bt.G * kBrick + g * kBrick + t] : (T)0;
+    const int el0 = g * EB + t / P;  // the lane's element
+    const uint4 li4 = *reinterpret_cast<const uint4*>(bt.lidx + (int64_t)el0 * 8);
+    const T bulk = NC != 10 ? el[el0] : (T)0;
+    const T shear2 = NC == 0 ? el[(int64_t)bt.G * EB + el0] : (T)0;
     if (flags && flags[0]) return;
     // batched solves: a brick of a frozen specimen leaves its partials alone (nobody reads them)
     if (active && !active[bt.spec[g]]) return;
+    const T* Cg = C + (int64_t)g * (8 / P * NC * kBrick) + t;
+    T cf[NC ? NC : 1];  // P = 8: the lane's tangent
+    if constexpr (P == 8)
+#pragma unroll
+        for (int k = 0; k < NC; ++k) cf[k] = Cg[k * kBrick];
 #pragma unroll
     for (int k = 0; k < NS; ++k)
         if (nd[k] >= 0) {
@@ -431,12 +453,11 @@ __global__ __launch_bounds__(kBrick) void brick_apply_kernel(
             for (int c = 0; c < 3; ++c) {
                 T v = (T)p[3 * (int64_t)nd[k] + c];
                 if (mask && dirflag[3 * (int64_t)nd[k] + c]) v = (T)0;
-                sp[c * kBrickNodes + i] = v;
-                sx[c * kBrickNodes + i] = bt.X[(int64_t)c * bt.G * kBrickNodes + l0 + k * kBrick];
+                sp[c * NB + i] = v;
+                sx[c * NB + i] = bt.X[(int64_t)c * bt.G * NB + l0 + k * kBrick];
             }
         }
     const bool live = (li4.x & 0xffffu) != 0xffffu;
-    const T* Cg = C + (int64_t)g * (8 * NC * kBrick) + t;
     __syncthreads();
     T cp[3][8], cx[3][8];
     if (live) {
@@ -452,8 +473,8 @@ __global__ __launch_bounds__(kBrick) void brick_apply_kernel(
             const int l = loc[kHex8Canon[k]];
 #pragma unroll
             for (int i = 0; i < 3; ++i) {
-                cp[i][k] = sp[i * kBrickNodes + l];
-                const double xc = sx[i * kBrickNodes + l];
+                cp[i][k] = sp[i * NB + l];
+                const double xc = sx[i * NB + l];
                 if (k == 0) x0[i] = xc;
                 cx[i][k] = (T)(xc - x0[i]);
             }
@@ -488,8 +509,16 @@ __global__ __launch_bounds__(kBrick) void brick_apply_kernel(
         for (int i = 0; i < 3; ++i)
 #pragma unroll
             for (int k = 0; k < 8; ++k) fa[i][k] = (T)0;
-        if (g < bt.hot) brick_qps<NC, T, true>(Cg, bulk, shear2, cp, cx, fa);
-        else brick_qps<NC, T, false>(Cg, bulk, shear2, cp, cx, fa);
+        if constexpr (P == 8) {
+            const T gq = (T)0.57735026918962576451;
+            const int q = t & 7, r = q & 3;  // as in brick_qps
+            brick_qp<NC, T>(cf, bulk, shear2, (r < 2 ? -gq : gq), (q < 4 ? -gq : gq), ((r == 1 || r == 2) ? gq : -gq),
+                            cp, cx, fa);
+        } else if (g < bt.hot) {
+            brick_qps<NC, T, true>(Cg, bulk, shear2, cp, cx, fa);
+        } else {
+            brick_qps<NC, T, false>(Cg, bulk, shear2, cp, cx, fa);
+        }
         if (part)
 #pragma unroll
             for (int i = 0; i < 3; ++i)
@@ -498,12 +527,28 @@ __global__ __launch_bounds__(kBrick) void brick_apply_kernel(
         load_lists();
 #pragma unroll
         for (int i = 0; i < 3; ++i) walsh3_t(fa[i]);
-        // forces [i][a][t]: consecutive lanes in consecutive banks
+        if constexpr (P == 8) {
+            // lanes with the bit of the halved index set keep the upper half
+            const bool b4 = t & 4, b2 = t & 2, b1 = t & 1;
+            const int slot = t - (t & 7) + kHex8Canon[t & 7];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int a = kHex8Canon[k];
+            for (int i = 0; i < 3; ++i) {
+                T u[4], v[2];
 #pragma unroll
-            for (int i = 0; i < 3; ++i) sf[(i * 8 + a) * kBrick + t] = (T)0.125 * fa[i][k];
+                for (int k = 0; k < 4; ++k)
+                    u[k] = (b4 ? fa[i][k + 4] : fa[i][k]) + lane_xor8<4>(b4 ? fa[i][k] : fa[i][k + 4]);
+#pragma unroll
+                for (int k = 0; k < 2; ++k) v[k] = (b2 ? u[k + 2] : u[k]) + lane_xor8<2>(b2 ? u[k] : u[k + 2]);
+                sf[i * 8 * EB + slot] = (T)0.125 * ((b1 ? v[1] : v[0]) + lane_xor8<1>(b1 ? v[0] : v[1]));
+            }
+        } else {
+            // forces [i][a][t]: consecutive lanes in consecutive banks
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const int a = kHex8Canon[k];
+#pragma unroll
+                for (int i = 0; i < 3; ++i) sf[(i * 8 + a) * kBrick + t] = (T)0.125 * fa[i][k];
+            }
         }
     } else {
         load_lists();
@@ -520,8 +565,8 @@ __global__ __launch_bounds__(kBrick) void brick_apply_kernel(
             const uint32_t s = (w[j >> 1] >> (16 * (j & 1))) & 0xffffu;
             if (s != 0xffffu) {
                 f0 += sf[s];
-                f1 += sf[8 * kBrick + s];
-                f2 += sf[16 * kBrick + s];
+                f1 += sf[8 * EB + s];
+                f2 += sf[16 * EB + s];
             }
         }
         T* dst = Fpart + (int64_t)lp[k] * 3;
@@ -702,13 +747,19 @@ void launch_bricks(efe_ctx* c, hipStream_t st, const TP* p, int mask, const int*
         C = c->mfC;
         F = c->mfbF;
     }
-#define BRICK_ARGS bt, el, C, p, c->dirflag, mask, flags, F, active, part
+#define BRICK_ARGS <<<grid, kBrick, 0, st>>>(bt, el, C, p, c->dirflag, mask, flags, F, active, part)
+    const bool split = c->mfbE != kBrick;
     if (c->mfNC == 10) {
-        if constexpr (sizeof(T) == 4) brick_apply_kernel<10, T, TP><<<grid, kBrick, 0, st>>>(BRICK_ARGS);
+        if constexpr (sizeof(T) == 4) {
+            if (split) brick_apply_kernel<10, T, TP, 8> BRICK_ARGS;
+            else brick_apply_kernel<10, T, TP, 1> BRICK_ARGS;
+        }
     } else if (c->mfNC == 7) {
-        brick_apply_kernel<7, T, TP><<<grid, kBrick, 0, st>>>(BRICK_ARGS);
+        if (split) brick_apply_kernel<7, T, TP, 8> BRICK_ARGS;
+        else brick_apply_kernel<7, T, TP, 1> BRICK_ARGS;
     } else {
-        brick_apply_kernel<0, T, TP><<<grid, kBrick, 0, st>>>(BRICK_ARGS);
+        if (split) brick_apply_kernel<0, T, TP, 8> BRICK_ARGS;
+        else brick_apply_kernel<0, T, TP, 1> BRICK_ARGS;
     }
 #undef BRICK_ARGS
 }
@@ -766,7 +817,7 @@ int build_moduli(efe_ctx* c, T** dst) {
     std::vector<int32_t> pos(E);
     EFE_HIP(hipMemcpy(pr.data(), c->props, pr.size() * sizeof(double), hipMemcpyDeviceToHost));
     EFE_HIP(hipMemcpy(pos.data(), c->mfbPos, (size_t)E * sizeof(int32_t), hipMemcpyDeviceToHost));
-    const size_t n = (size_t)c->mfbG * kBrick;
+    const size_t n = (size_t)c->mfbG * c->mfbE;
     std::vector<T> v(2 * n, (T)0);
     for (int e = 0; e < E; ++e) {
         const double y = c->props_per_element ? pr[e] : pr[0], nu = c->props_per_element ? pr[(size_t)E + e] : pr[1];
@@ -808,13 +859,14 @@ int efe_mf_upload_bricks(efe_ctx* c, const BrickPattern& bp, const double* coord
     EFE_HIP(hipMemcpy(c->mfbTables, host.data(), total, hipMemcpyHostToDevice));
     c->mfbL = bp.L;
     c->mfbG = bp.G;
+    c->mfbE = bp.EB;
     c->mfb = true;
     return EFE_OK;
 }
 
 int efe_mf_alloc_bricks(efe_ctx* c, bool fp64) {
     EFE_HIP(hipStreamSynchronize(c->stream));  // the uploads below use the default stream
-    const size_t nc = (size_t)c->mfbG * kBrick * 8 * (c->mfNC ? c->mfNC : 1);
+    const size_t nc = (size_t)c->mfbG * c->mfbE * 8 * (c->mfNC ? c->mfNC : 1);
     if (fp64) {
         if (c->mfC64) return EFE_OK;
         if (int rc = build_moduli(c, &c->mfbEl64)) return rc;

@@ -152,3 +152,35 @@ def test_batched_bricks_solve_every_specimen_as_alone(sizes, precision):
         if precision == "fp64":
             assert rel_err(xa[sl], x1.cpu().numpy()) < tol
     batch.close()
+
+
+@pytest.mark.parametrize("n", [(24, 32, 32), (25, 32, 32)])  # the most elements of split bricks, and more
+@pytest.mark.parametrize("material", ["vonmises", "linearelastic"])
+def test_split_and_whole_bricks_step_as_the_assembled_operator(n, material):
+    """Three PCG iterations from x = 0 (six products' worth of round-off, far from convergence) on the
+    bricks and on the assembled operator of the same pass: 1e-12 relative in FP64; in FP32 the
+    tangents' and products' rounding, 1e-4."""
+    from edelweissfe_amd import _lib
+    from edelweissfe_amd.device import DeviceSystem
+
+    props = J2 if material == "vonmises" else LE
+    pm = device_model(n, (1.0, 1.0, 1.0), "C3D8", material, props, jitter=0.1, seed=3)
+    sysm = DeviceSystem(pm.coordinates, pm.connectivity, "C3D8", material, np.array(props))
+    dirs = np.r_[pm.dofsOfNodeSet("gen_bottom"), pm.dofsOfNodeSet("gen_top", [1])]
+    sysm.set_dirichlet(dirs)
+    rng = np.random.default_rng(7)
+    dU = torch.as_tensor(rng.uniform(-1, 1, sysm.n_dof) * 2e-3 / max(n), device="cuda")
+    b = torch.as_tensor(rng.standard_normal(sysm.n_dof), device="cuda")
+    P, F = sysm.zeros(), sysm.zeros()
+    x32, xb, xa = sysm.zeros(), sysm.zeros(), sysm.zeros()
+    sysm.compute_elements(dU, P, F, precision=_lib.EFE_FP32_MATFREE)
+    sysm.linsolve(b, x32, precision=_lib.EFE_FP32_MATFREE, rtol=0.0, max_iter=3)
+    sysm.compute_elements(dU, P, F)
+    sysm.linsolve(b, xb, rtol=0.0, max_iter=3)
+    sysm.set_dirichlet(dirs)  # leaves the assembled operator as the only one of its set
+    sysm.linsolve(b, xa, rtol=0.0, max_iter=3)
+    sysm.close()
+    xa = xa.cpu().numpy()
+    assert np.linalg.norm(xa) > 0
+    assert rel_err(xb.cpu().numpy(), xa) < 1e-12
+    assert rel_err(x32.cpu().numpy(), xa) < 1e-4
