@@ -25,15 +25,21 @@ namespace {
 constexpr int kBS = 256;            // threads per workgroup
 constexpr int kLanesPerRow = 16;    // SpMV lanes per row
 constexpr int kMaxWG = kCsrPartials;  // partials per dot product (vector kernels stride)
+constexpr int kMaxSpmvWG = 2048;      // workgroups of the CG product, all of whose partials every update adds up
+
+__device__ __forceinline__ double wave_sum(double v) {
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m);
+    return v;
+}
 
 __device__ __forceinline__ double wg_sum(double v, double* sh) {
-    sh[threadIdx.x] = v;
+    v = wave_sum(v);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x / 64] = v;
     __syncthreads();
-    for (int s = kBS / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) sh[threadIdx.x] += sh[threadIdx.x + s];
-        __syncthreads();
-    }
-    const double r = sh[0];
+    double r = sh[0];
+#pragma unroll
+    for (int w = 1; w < kBS / 64; ++w) r += sh[w];
     __syncthreads();
     return r;
 }
@@ -95,19 +101,168 @@ __global__ __launch_bounds__(kBS) void csr_spmv_kernel(int n, const int32_t* __r
 // part[wg] = sum over the workgroup's rows of u.w (grid-stride, fixed assignment)
 __global__ __launch_bounds__(kBS) void csr_dot_kernel(int n, const double* __restrict__ u,
                                                       const double* __restrict__ w, double* __restrict__ part) {
-    __shared__ double sh[kBS];
+    __shared__ double sh[kBS / 64];
     double s = 0.0;
     for (int i = blockIdx.x * kBS + threadIdx.x; i < n; i += gridDim.x * kBS) s += u[i] * w[i];
     s = wg_sum(s, sh);
     if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
-// CG scalars, sc: [0] r.z, [1] alpha, [2] r.r, [3] tol^2, [4] done flag (as double), [5] iterations
-// z = Dinv r; partials of r.z (slot 0) and r.r (slot 1)
-__global__ __launch_bounds__(kBS) void cg_precond_kernel(int n, const double* __restrict__ dinv,
-                                                         const double* __restrict__ r, double* __restrict__ z,
-                                                         double* __restrict__ part) {
-    __shared__ double sh[kBS];
+// CG, three kernels per iteration.  Scalars sc: [0] and [6] r.z of the even and the odd iterations (a
+// kernel that stores the next one still reads the last), [2] r.r, [3] tol^2, [4] done flag (as
+// double), [5] iterations.
+//
+// An iteration of a mid-sized system is a chain of launches: product, dot, update, preconditioner,
+// direction and scalars as kernels of their own took 25 us at 26775 rows and 2 M entries, the product
+// (8.8) waiting for its indices, the fixed flags and the entries of x in turn.  The product now
+// loads kStep entries of a lane together and forms p.q; z = Dinv r is formed where it is needed, not
+// stored; p and r are 0 on prescribed rows, so their columns need no flag.
+// 25.4 -> 16.2 us an iteration there.  kStep 4 / 6: 8.75 / 8.6 ms for the whole call of 448
+// iterations (49.9 / 48.8 ms at 40^3 elements); at most 1024 / 2048 workgroups of the product 8.6 / 8.6
+// (52.1 / 48.8).
+
+// q = A p on free rows, 0 on prescribed ones; part[wg] = partial of p.q
+__global__ __launch_bounds__(kBS) void cg_spmv_kernel(int n, const int32_t* __restrict__ ip,
+                                                      const int32_t* __restrict__ ix, const double* __restrict__ v,
+                                                      const uint8_t* __restrict__ fixed, const double* __restrict__ p,
+                                                      double* __restrict__ q, double* __restrict__ part,
+                                                      const double* __restrict__ sc) {
+    constexpr int kStep = 6, R = kBS / kLanesPerRow;
+    __shared__ double sh[kBS / 64];
+    const int l = threadIdx.x & (kLanesPerRow - 1);
+    double dot = 0.0;
+    if (sc[4] != 0.0) return;
+    for (int row = blockIdx.x * R + threadIdx.x / kLanesPerRow; row < n; row += gridDim.x * R) {
+        const int a = ip[row], e = fixed[row] ? a : ip[row + 1];
+        const double pr = p[row];
+        double acc = 0.0;
+        for (int k = a + l; k < e; k += kStep * kLanesPerRow) {
+            int c[kStep];
+            double av[kStep], xv[kStep];
+#pragma unroll
+            for (int u = 0; u < kStep; ++u) {
+                const int ku = k + u * kLanesPerRow;
+                const bool in = ku < e;
+                c[u] = in ? ix[ku] : -1;
+                av[u] = in ? v[ku] : 0.0;
+            }
+#pragma unroll
+            for (int u = 0; u < kStep; ++u) xv[u] = c[u] >= 0 ? p[c[u]] : 0.0;
+#pragma unroll
+            for (int u = 0; u < kStep; ++u)
+                if (c[u] >= 0) acc += av[u] * xv[u];
+        }
+#pragma unroll
+        for (int o = kLanesPerRow / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, kLanesPerRow);
+        if (l == 0) {
+            q[row] = acc;
+            dot += pr * acc;
+        }
+    }
+    dot = wg_sum(dot, sh);
+    if (threadIdx.x == 0) part[blockIdx.x] = dot;
+}
+
+// first: p = Dinv r; else x += alpha p, r -= alpha q with alpha = r.z / (p.q).  Partials of the new r.z
+// (slot 0) and r.r (slot 1).
+__global__ __launch_bounds__(kBS) void cg_update_kernel(int n, const double* __restrict__ dinv,
+                                                        double* __restrict__ x, double* __restrict__ r,
+                                                        double* __restrict__ p, const double* __restrict__ q,
+                                                        const double* __restrict__ pq, int npq,
+                                                        double* __restrict__ part, const double* __restrict__ sc,
+                                                        int rz, int first) {
+    __shared__ double sh[kBS / 64];
+    int i = blockIdx.x * kBS + threadIdx.x;
+    double d = 0, ri = 0, pi = 0, qi = 0, xi = 0;
+    auto load = [&] {
+        d = dinv[i];
+        ri = r[i];
+        if (!first) {
+            pi = p[i];
+            qi = q[i];
+            xi = x[i];
+        }
+    };
+    if (i < n) load();  // beside the sum of the partials
+    double alpha = 0.0;
+    if (!first) {
+        if (sc[4] != 0.0) return;
+        alpha = sc[rz] / sum_partials(pq, npq, sh);
+    }
+    double rzn = 0.0, rr = 0.0;
+    while (i < n) {
+        if (first) {
+            p[i] = d * ri;
+        } else {
+            x[i] = xi + alpha * pi;
+            ri -= alpha * qi;
+            r[i] = ri;
+        }
+        rzn += ri * (d * ri);
+        rr += ri * ri;
+        i += gridDim.x * kBS;
+        if (i < n) load();
+    }
+    rzn = wg_sum(rzn, sh);
+    rr = wg_sum(rr, sh);
+    if (threadIdx.x == 0) {
+        part[blockIdx.x] = rzn;
+        part[kMaxWG + blockIdx.x] = rr;
+    }
+}
+
+// the stop test, then p = Dinv r + beta p with beta = r.z new / old.  The first workgroup stores the
+// scalars; one that sees its done flag early skips a direction that nothing reads.
+__global__ __launch_bounds__(kBS) void cg_direction_kernel(int n, const double* __restrict__ dinv,
+                                                           const double* __restrict__ r, double* __restrict__ p,
+                                                           const double* __restrict__ part, int nwg,
+                                                           double* __restrict__ sc, int rz) {
+    __shared__ double sh[kBS / 64];
+    int i = blockIdx.x * kBS + threadIdx.x;
+    double zi = 0, pi = 0;
+    if (i < n) {
+        zi = dinv[i] * r[i];
+        pi = p[i];
+    }
+    if (sc[4] != 0.0) return;
+    const double rzn = sum_partials(part, nwg, sh);
+    const double rr = sum_partials(part + kMaxWG, nwg, sh);
+    const bool done = !(rr > sc[3]);  // converged (or NaN)
+    const double beta = rzn / sc[rz];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        sc[6 - rz] = rzn;
+        sc[2] = rr;
+        sc[5] += 1.0;
+        if (done) sc[4] = 1.0;
+    }
+    if (done) return;
+    while (i < n) {
+        p[i] = zi + beta * pi;
+        i += gridDim.x * kBS;
+        if (i < n) {
+            zi = dinv[i] * r[i];
+            pi = p[i];
+        }
+    }
+}
+
+// one workgroup: the scalars of the start
+__global__ void cg_scalars_kernel(const double* __restrict__ part, int nwg, double* __restrict__ sc) {
+    __shared__ double sh[kBS / 64];
+    const double rz = sum_partials(part, nwg, sh);
+    const double rr = sum_partials(part + kMaxWG, nwg, sh);
+    if (threadIdx.x == 0) {
+        sc[0] = rz;
+        sc[2] = rr;
+        if (!(rr > sc[3])) sc[4] = 1.0;  // converged (or NaN)
+    }
+}
+
+// partials of r.z with z = Dinv r (slot 0) and r.r (slot 1); z
+__global__ __launch_bounds__(kBS) void precond_kernel(int n, const double* __restrict__ dinv,
+                                                      const double* __restrict__ r, double* __restrict__ z,
+                                                      double* __restrict__ part) {
+    __shared__ double sh[kBS / 64];
     double rz = 0.0, rr = 0.0;
     for (int i = blockIdx.x * kBS + threadIdx.x; i < n; i += gridDim.x * kBS) {
         const double zi = dinv[i] * r[i];
@@ -120,48 +275,6 @@ __global__ __launch_bounds__(kBS) void cg_precond_kernel(int n, const double* __
     if (threadIdx.x == 0) {
         part[blockIdx.x] = rz;
         part[kMaxWG + blockIdx.x] = rr;
-    }
-}
-
-// p = z + beta p with beta = rz_new / rz_old (rz_old in sc[0]); first: p = z
-__global__ __launch_bounds__(kBS) void cg_direction_kernel(int n, const double* __restrict__ z, double* __restrict__ p,
-                                                           const double* __restrict__ part, int nwg,
-                                                           const double* __restrict__ sc, int first) {
-    __shared__ double sh[kBS];
-    if (sc[4] != 0.0) return;
-    const double rz = sum_partials(part, nwg, sh);
-    const double beta = first ? 0.0 : rz / sc[0];
-    // first: p = z, whatever the workspace held before
-    for (int i = blockIdx.x * kBS + threadIdx.x; i < n; i += gridDim.x * kBS) p[i] = first ? z[i] : z[i] + beta * p[i];
-}
-
-// one workgroup: rz_old <- rz (after the direction), rr and the stop test; count: the call
-// ends an iteration (sc[5] counts the iterations run)
-__global__ void cg_scalars_kernel(const double* __restrict__ part, int nwg, double* __restrict__ sc, int count) {
-    __shared__ double sh[kBS];
-    if (sc[4] != 0.0) return;
-    const double rz = sum_partials(part, nwg, sh);
-    const double rr = sum_partials(part + kMaxWG, nwg, sh);
-    if (threadIdx.x == 0) {
-        sc[0] = rz;
-        sc[2] = rr;
-        if (count) sc[5] += 1.0;
-        if (!(rr > sc[3])) sc[4] = 1.0;  // converged (or NaN)
-    }
-}
-
-// x += alpha p, r -= alpha q with alpha = rz / (p.q)
-__global__ __launch_bounds__(kBS) void cg_update_kernel(int n, double* __restrict__ x, double* __restrict__ r,
-                                                        const double* __restrict__ p, const double* __restrict__ q,
-                                                        const double* __restrict__ part, int nwg,
-                                                        const double* __restrict__ sc) {
-    __shared__ double sh[kBS];
-    if (sc[4] != 0.0) return;
-    const double pq = sum_partials(part, nwg, sh);
-    const double alpha = sc[0] / pq;
-    for (int i = blockIdx.x * kBS + threadIdx.x; i < n; i += gridDim.x * kBS) {
-        x[i] += alpha * p[i];
-        r[i] -= alpha * q[i];
     }
 }
 
@@ -197,7 +310,7 @@ __global__ __launch_bounds__(kBS) void bicg_alpha_kernel(int n, double* __restri
                                                          const double* __restrict__ v,
                                                          const double* __restrict__ part, int nwg,
                                                          double* __restrict__ sc) {
-    __shared__ double sh[kBS];
+    __shared__ double sh[kBS / 64];
     if (sc[4] != 0.0) return;
     const double rv = sum_partials(part, nwg, sh);
     const double alpha = sc[0] / rv;
@@ -211,7 +324,7 @@ __global__ __launch_bounds__(kBS) void bicg_alpha_kernel(int n, double* __restri
 // partials of t.s (slot 0) and t.t (slot 1), s in r
 __global__ __launch_bounds__(kBS) void bicg_ts_kernel(int n, const double* __restrict__ t, const double* __restrict__ s,
                                                       double* __restrict__ part, const double* __restrict__ sc) {
-    __shared__ double sh[kBS];
+    __shared__ double sh[kBS / 64];
     if (sc[4] != 0.0) return;
     double ts = 0.0, tt = 0.0;
     for (int i = blockIdx.x * kBS + threadIdx.x; i < n; i += gridDim.x * kBS) {
@@ -233,7 +346,7 @@ __global__ __launch_bounds__(kBS) void bicg_omega_kernel(int n, double* __restri
                                                          const double* __restrict__ r0,
                                                          const double* __restrict__ part_in, int nwg,
                                                          double* __restrict__ part_out, double* __restrict__ sc) {
-    __shared__ double sh[kBS];
+    __shared__ double sh[kBS / 64];
     if (sc[4] != 0.0) return;
     const double ts = sum_partials(part_in, nwg, sh);
     const double tt = sum_partials(part_in + kMaxWG, nwg, sh);
@@ -257,7 +370,7 @@ __global__ __launch_bounds__(kBS) void bicg_omega_kernel(int n, double* __restri
 
 // one workgroup: rho_new, r.r, stop test, beta into sc[7] = rho_new, sc[1] beta-ready
 __global__ void bicg_scalars_kernel(const double* __restrict__ part, int nwg, double* __restrict__ sc) {
-    __shared__ double sh[kBS];
+    __shared__ double sh[kBS / 64];
     if (sc[4] != 0.0) return;
     const double rho = sum_partials(part, nwg, sh);
     const double rr = sum_partials(part + kMaxWG, nwg, sh);
@@ -303,7 +416,7 @@ __global__ void jacobi_kernel(int n, const double* __restrict__ dinv, const doub
 
 // first rho = r0.r and rr, stop test
 __global__ void bicg_init_scalars_kernel(const double* __restrict__ part, int nwg, double* __restrict__ sc) {
-    __shared__ double sh[kBS];
+    __shared__ double sh[kBS / 64];
     const double rho = sum_partials(part, nwg, sh);
     const double rr = sum_partials(part + kMaxWG, nwg, sh);
     if (threadIdx.x == 0) {
@@ -373,7 +486,7 @@ namespace {
 // part[i][wg] = partial of V_i . w over the workgroup's rows, i < cnt (grid-stride)
 __global__ __launch_bounds__(kBS) void csr_multidot_kernel(int n, const double* __restrict__ V, int cnt,
                                                            const double* __restrict__ w, double* __restrict__ part) {
-    __shared__ double sh[kBS];
+    __shared__ double sh[kBS / 64];
     for (int i = 0; i < cnt; ++i) {
         const double* vi = V + (size_t)i * n;
         double s = 0.0;
@@ -615,18 +728,17 @@ int efe_csr_solve_ws(int32_t n, const int32_t* ip, const int32_t* ix, const doub
         set_scalars_kernel<<<1, 64, 0, st>>>(sc, tol * tol);
         int it = 0;
         if (cg) {
-            double *z = vecs + 2 * (size_t)n, *p = vecs + 3 * (size_t)n, *q = vecs + 4 * (size_t)n;
-            cg_precond_kernel<<<nwg, kBS, 0, st>>>(n, dinv, r, z, part);
-            cg_direction_kernel<<<nwg, kBS, 0, st>>>(n, z, p, part, nwg, sc, 1);
-            cg_scalars_kernel<<<1, kBS, 0, st>>>(part, nwg, sc, 0);
+            // p.q's partials lie where z would (n doubles, a workgroup has kBS / kLanesPerRow rows)
+            double *pq = vecs + 2 * (size_t)n, *p = vecs + 3 * (size_t)n, *q = vecs + 4 * (size_t)n;
+            const int gq = gs < kMaxSpmvWG ? gs : kMaxSpmvWG;
+            cg_update_kernel<<<nwg, kBS, 0, st>>>(n, dinv, x, r, p, q, pq, gq, part, sc, 0, 1);
+            cg_scalars_kernel<<<1, kBS, 0, st>>>(part, nwg, sc);
+            int rz = 0;
             while (true) {
-                for (int j = 0; j < check; ++j) {
-                    csr_spmv_kernel<<<gs, kBS, 0, st>>>(n, ip, ix, v, fixed, p, q, nullptr);
-                    csr_dot_kernel<<<nwg, kBS, 0, st>>>(n, p, q, part);
-                    cg_update_kernel<<<nwg, kBS, 0, st>>>(n, x, r, p, q, part, nwg, sc);
-                    cg_precond_kernel<<<nwg, kBS, 0, st>>>(n, dinv, r, z, part);
-                    cg_direction_kernel<<<nwg, kBS, 0, st>>>(n, z, p, part, nwg, sc, 0);
-                    cg_scalars_kernel<<<1, kBS, 0, st>>>(part, nwg, sc, 1);
+                for (int j = 0; j < check; ++j, rz = 6 - rz) {
+                    cg_spmv_kernel<<<gq, kBS, 0, st>>>(n, ip, ix, v, fixed, p, q, pq, sc);
+                    cg_update_kernel<<<nwg, kBS, 0, st>>>(n, dinv, x, r, p, q, pq, gq, part, sc, rz, 0);
+                    cg_direction_kernel<<<nwg, kBS, 0, st>>>(n, dinv, r, p, part, nwg, sc, rz);
                 }
                 EFE_HIP(hipGetLastError());
                 EFE_HIP(hipMemcpyAsync(hs, sc, 16 * sizeof(double), hipMemcpyDeviceToHost, st));
@@ -644,7 +756,7 @@ int efe_csr_solve_ws(int32_t n, const int32_t* ip, const int32_t* ix, const doub
             double *vv = vecs + 5 * (size_t)n, *sh = vecs + 6 * (size_t)n, *t = vecs + 7 * (size_t)n;
             double* part2 = part + 2 * kMaxWG;  // the omega kernel reads part while it writes these
             copy_kernel<<<gd, kBS, 0, st>>>(n, r, r0);
-            cg_precond_kernel<<<nwg, kBS, 0, st>>>(n, dinv, r, ph, part);  // slot 0 unused, slot 1 = r.r
+            precond_kernel<<<nwg, kBS, 0, st>>>(n, dinv, r, ph, part);  // slot 0 unused, slot 1 = r.r
             csr_dot_kernel<<<nwg, kBS, 0, st>>>(n, r0, r, part);
             bicg_init_scalars_kernel<<<1, kBS, 0, st>>>(part, nwg, sc);
             bicg_p_kernel<<<nwg, kBS, 0, st>>>(n, r, p, vv, sc, 1);
