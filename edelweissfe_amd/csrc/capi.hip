@@ -162,8 +162,8 @@ int efe_prepare_elements(efe_ctx* c, int precision) {
     }
     if (precision == EFE_FP32_MATFREE)
         if (int rc = efe_mf_alloc(c)) return rc;
-    // the FP64 CG on hexa8 with a symmetric tangent runs on the bricks (krylov.hip)
-    if (precision == EFE_FP64 && c->eltype == EFE_C3D8 && c->mfNC != 10)
+    // the FP64 CG on hexa8 with a symmetric tangent runs on the bricks (krylov.hip), but for small meshes
+    if (precision == EFE_FP64 && c->eltype == EFE_C3D8 && c->mfNC != 10 && c->mfbE == kBrick)
         if (int rc = efe_mf_alloc_bricks(c, true)) return rc;
     return EFE_OK;
 }

@@ -95,16 +95,70 @@ struct HostPattern {
     int64_t padded_blocks = 0;
 };
 
+// The convergence quantities over a range: max |R| with its first index, max |ddU|, sum |F|, any NaN.
+struct NormSums {
+    double mr = -1.0, ir = 1e300, md = 0.0, sf = 0.0, nan = 0.0;
+    __device__ __forceinline__ void add(double i, double r, double d, double f) {
+        r = fabs(r);
+        d = fabs(d);
+        if (!(r == r) || !(d == d)) nan = 1.0;
+        if (r > mr) {
+            mr = r;
+            ir = i;
+        }
+        md = d > md ? d : md;
+        sf += fabs(f);
+    }
+    __device__ __forceinline__ void merge(const NormSums& o) {
+        if (o.mr > mr || (o.mr == mr && o.ir < ir)) {
+            mr = o.mr;
+            ir = o.ir;
+        }
+        md = fmax(md, o.md);
+        sf += o.sf;
+        nan = fmax(nan, o.nan);
+    }
+    // over a workgroup of NW wavefronts, in a fixed order; valid in every thread.  sh: [NW][5]
+    template <int NW>
+    __device__ __forceinline__ void reduce(double* sh) {
+#pragma unroll
+        for (int m = 32; m >= 1; m >>= 1) {
+            NormSums o;
+            o.mr = __shfl_xor(mr, m);
+            o.ir = __shfl_xor(ir, m);
+            o.md = __shfl_xor(md, m);
+            o.sf = __shfl_xor(sf, m);
+            o.nan = __shfl_xor(nan, m);
+            merge(o);
+        }
+        const int w = threadIdx.x / 64;
+        if ((threadIdx.x & 63) == 0) {
+            double* d = sh + w * 5;
+            d[0] = mr, d[1] = ir, d[2] = md, d[3] = sf, d[4] = nan;
+        }
+        __syncthreads();
+        *this = NormSums();
+        for (int k = 0; k < NW; ++k) {
+            NormSums o;
+            const double* d = sh + k * 5;
+            o.mr = d[0], o.ir = d[1], o.md = d[2], o.sf = d[3], o.nan = d[4];
+            merge(o);
+        }
+    }
+};
+
 // Bricks of the hexa8 matrix-free operator: at most kBrick elements and kBrickNodes staged nodes, or
 // (split bricks) kBrickSplit elements, whose 8 nodes each are the most that can be staged.
 constexpr int kBrick = 256;
 constexpr int kBrickNodes = 512;
 constexpr int kBrickSplit = 32;
-// Meshes of up to this many elements take split bricks (batches never: a specimen has the same bricks,
-// and so the same bits, alone and with others): fewer whole ones leave CUs idle, or at one
-// workgroup each; beyond it the repeated set-up costs more.  PCG iteration, whole / split bricks: FP64
-// 8^3 17.6 / 14.0 us, 20^3 19.9 / 16.2, 28^3 (21952) 21.4 / 20.8, 32^3 22.2 / 22.8, 40^3 30.0 / 38.3;
-// FP32 8^3 17.1 / 13.0, 20^3 18.7 / 14.6, 28^3 19.9 / 17.7, 32^3 20.3 / 18.4, 40^3 23.0 / 29.5.
+// Meshes of up to this many elements take split bricks in FP32 and the assembled operator, which their
+// FP64 passes form anyway, in FP64 (batches always whole bricks: a specimen has the same bricks, and so
+// the same bits, alone and with others).  Fewer whole bricks leave CUs idle, or at one workgroup each;
+// beyond it the repeated set-up, and the assembled operator's bytes, cost more.  PCG iteration, FP32 whole
+// / split bricks: 8^3 17.1 / 13.0 us, 20^3 18.7 / 14.6, 28^3 (21952) 19.9 / 17.7, 32^3 20.3 / 18.4, 40^3
+// 23.0 / 29.5; FP64 whole / split / assembled: 8^3 17.6 / 13.6 / 11.7, 20^3 19.9 / 16.1 / 13.5, 28^3 21.4 /
+// 20.9 / 19.1, 32^3 22.2 / 22.3 / 25.3, 40^3 30.0 / 38.3 / 39.5.
 constexpr int kSplitElements = 24576;
 
 // place of QP q of the element at pos (BrickPattern) among the tangents' rows of kBrick lanes

@@ -41,6 +41,7 @@ struct KrylovWork {
     // thread, nwgv workgroups; [0] FP64, [1] FP32
     int krvp[2] = {1, 1}, nwgvp[2] = {0, 0};
     int krv = 1, nwgv = 0;
+    int krs = 1, nwgs = 0;
     int ps = 0;  // row stride of the partials array (the largest workgroup count)
     // FP64 and FP32 vector sets
     double *x64 = nullptr, *r64 = nullptr, *z64 = nullptr, *p64 = nullptr, *q64 = nullptr;
@@ -127,8 +128,8 @@ __device__ __forceinline__ void reduce_partials_n(const double* __restrict__ par
 // reduce_partials_n with a count per array; each array's sum is formed in the same order as
 // reduce_partials_n would form it.
 template <int BS, int K>
-__device__ __forceinline__ void reduce_partials_nv(const double* __restrict__ part, const int (&offs)[K],
-                                                   const int (&ns)[K], double (&out)[K], double* sh) {
+__device__ __forceinline__ void reduce_partials_nv(const double* __restrict__ part, const int* offs,
+                                                   const int* ns, double (&out)[K], double* sh) {
     int nmax = 0;
 #pragma unroll
     for (int k = 0; k < K; ++k) {
@@ -151,48 +152,74 @@ __device__ __forceinline__ double reduce_partials(const double* __restrict__ par
     return out[0];
 }
 
-template <typename T, int BS>
-__global__ __launch_bounds__(BS) void spmv_kernel(int N, const int32_t* __restrict__ slice_off,
-                                                  const int32_t* __restrict__ scol,
-                                                  const int32_t* __restrict__ slotNode, const T* __restrict__ K,
-                                                  const T* __restrict__ x, T* __restrict__ y,
-                                                  double* __restrict__ part, const int* __restrict__ flags,
-                                                  int kr) {
-    __shared__ double sh[BS];
+// y = K x, a workgroup per ks slices, its wavefronts each a range of a slice's blocks (as in the GMRES
+// product, gmres.hip); with part, the workgroup's partial of x . y.  One product, a lane per row ->
+// 8 wavefronts per slice: hexa8 FP64 20^3 13.6 -> 5.4 us, 48^3 40.2 -> 38.9, 64^3 102 -> 94 (5.9 TB/s),
+// hexa20 FP64 6^3 35.7 -> 10.3, 16^3 50.6 -> 26.2; 4 wavefronts the same within 5 %, 2 up to 30 % slower.
+// At most 2048 workgroups, whose partials every update adds up: FP32 CG 64^3 63.9 us at 2048, 67.7 at
+// 1024, 80^3 121 at 2048, 119 at 4096.
+constexpr int kSpmvWaves = 8;
+
+template <typename T>
+__global__ __launch_bounds__(64 * kSpmvWaves) void spmv_kernel(int N, const int32_t* __restrict__ slice_off,
+                                                               const int32_t* __restrict__ scol,
+                                                               const int32_t* __restrict__ slotNode,
+                                                               const T* __restrict__ K, const T* __restrict__ x,
+                                                               T* __restrict__ y, double* __restrict__ part,
+                                                               const int* __restrict__ flags, int ks) {
+    constexpr int W = kSpmvWaves;
+    __shared__ T sh[W - 1][3][64];
     if (flags && flags[0]) return;
-    const int blk = xcd_block();
+    const int blk = xcd_block(), l = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     double dot = 0.0;
-    for (int it = 0; it < kr; ++it) {
-        const int ps = (blk * kr + it) * BS + threadIdx.x;  // row slot
-        if (ps >= N) break;
-        const int n = slotNode[ps];
-        const int s = ps / kSlice, l = ps - (ps / kSlice) * kSlice;
+    for (int it = 0; it < ks; ++it) {
+        const int s = blk * ks + it;
+        if (s * kSlice >= N) break;
+        const int ps = s * kSlice + l;  // row slot
         const int o0 = slice_off[s], deg = (slice_off[s + 1] - o0) / kSlice;
+        const int n = ps < N ? slotNode[ps] : -1;
         const int32_t* cp = scol + o0 + l;
         const T* kp = K + (int64_t)o0 * 9 + l;
         T y0 = 0, y1 = 0, y2 = 0;
+        const int k1 = (wave + 1) * deg / W;
         // matrix values and indices are streamed once per product: non-temporal loads
         // keep them from displacing the gathered x in L2
+        if (n >= 0)
 #pragma unroll 3
-        for (int k = 0; k < deg; ++k) {
-            const int m = __builtin_nontemporal_load(cp + k * kSlice);
-            const T x0 = x[3 * m], x1 = x[3 * m + 1], x2 = x[3 * m + 2];
-            const T* v = kp + (int64_t)k * 9 * kSlice;
-            T a[9];
+            for (int k = wave * deg / W; k < k1; ++k) {
+                const int m = __builtin_nontemporal_load(cp + k * kSlice);
+                const T x0 = x[3 * m], x1 = x[3 * m + 1], x2 = x[3 * m + 2];
+                const T* v = kp + (int64_t)k * 9 * kSlice;
+                T a[9];
 #pragma unroll
-            for (int i = 0; i < 9; ++i) a[i] = __builtin_nontemporal_load(v + i * kSlice);
-            y0 += a[0] * x0 + a[1] * x1 + a[2] * x2;
-            y1 += a[3] * x0 + a[4] * x1 + a[5] * x2;
-            y2 += a[6] * x0 + a[7] * x1 + a[8] * x2;
+                for (int i = 0; i < 9; ++i) a[i] = __builtin_nontemporal_load(v + i * kSlice);
+                y0 += a[0] * x0 + a[1] * x1 + a[2] * x2;
+                y1 += a[3] * x0 + a[4] * x1 + a[5] * x2;
+                y2 += a[6] * x0 + a[7] * x1 + a[8] * x2;
+            }
+        if (it > 0) __syncthreads();  // the first wavefront has read the last slice's sums
+        if (wave > 0) {
+            sh[wave - 1][0][l] = y0;
+            sh[wave - 1][1][l] = y1;
+            sh[wave - 1][2][l] = y2;
+        }
+        __syncthreads();
+        if (wave > 0 || n < 0) continue;
+#pragma unroll
+        for (int w = 0; w < W - 1; ++w) {
+            y0 += sh[w][0][l];
+            y1 += sh[w][1][l];
+            y2 += sh[w][2][l];
         }
         y[3 * n] = y0;
         y[3 * n + 1] = y1;
         y[3 * n + 2] = y2;
         if (part) dot += (double)x[3 * n] * y0 + (double)x[3 * n + 1] * y1 + (double)x[3 * n + 2] * y2;
     }
-    if (part) {
-        double s = block_sum<BS>(dot, sh);
-        if (threadIdx.x == 0) part[blk] = s;
+    if (part && wave == 0) {
+        dot = wave_sum(dot);
+        if (threadIdx.x == 0) part[blk] = dot;
     }
 }
 
@@ -248,117 +275,51 @@ __global__ __launch_bounds__(BS) void pcg_init_kernel(int N, const double* __res
     }
 }
 
-template <typename T, int BS>
-__global__ __launch_bounds__(BS) void pcg_update_kernel(int N, const T* __restrict__ Minv, T* __restrict__ x,
-                                                        T* __restrict__ r, T* __restrict__ z,
-                                                        const T* __restrict__ p, const T* __restrict__ q,
-                                                        double* __restrict__ part, int ps, int nop, int nvec,
-                                                        int par, const int* __restrict__ flags, int kr) {
-    __shared__ double sh[BS];
-    if (flags[0]) return;
-    // p.q: nop partials of the operator's grid; r.z: nvec partials of this grid
-    const int offs[2] = {0, (1 + par) * ps};
-    const int ns[2] = {nop, nvec};
-    double sc[2];
-    reduce_partials_nv<BS, 2>(part, offs, ns, sc, sh);
-    const double pq = sc[0], rz = sc[1];
-    const T alpha = (T)(rz / pq);
-    const int blk = xcd_block();
-    double rzn = 0, rr = 0;
-    for (int it = 0; it < kr; ++it) {
-        const int n = (blk * kr + it) * BS + threadIdx.x;
-        if (n >= N) break;
-        T rv[3];
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            x[3 * n + i] += alpha * p[3 * n + i];
-            rv[i] = r[3 * n + i] - alpha * q[3 * n + i];
-            r[3 * n + i] = rv[i];
-            rr += (double)rv[i] * rv[i];
-        }
-        const T* M = Minv + (int64_t)n * 9;
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            T zi = M[3 * i] * rv[0] + M[3 * i + 1] * rv[1] + M[3 * i + 2] * rv[2];
-            z[3 * n + i] = zi;
-            rzn += (double)rv[i] * zi;
-        }
-    }
-    double sums[2] = {rzn, rr};
-    block_sums<BS, 2>(sums, sh);
-    const double s1 = sums[0], s2 = sums[1];
-    if (threadIdx.x == 0) {
-        part[(2 - par) * ps + blk] = s1;
-        part[3 * ps + blk] = s2;
-    }
-}
-
-template <typename T, int BS>
-__global__ __launch_bounds__(BS) void pcg_direction_kernel(int N, const T* __restrict__ z, T* __restrict__ p,
-                                                           double* __restrict__ part, int ps, int nvec,
-                                                           int par, int jlocal, const double* __restrict__ dtol2,
-                                                           int* __restrict__ flags, int kr) {
-    __shared__ double sh[BS];
-    if (flags[0]) return;
-    const int offs[3] = {(1 + par) * ps, (2 - par) * ps, 3 * ps};
-    double sc[3];
-    reduce_partials_n<BS, 3>(part, offs, nvec, sc, sh);
-    const double rzo = sc[0], rzn = sc[1], rr = sc[2];
-    const bool bad = !(rr == rr) || !(rzn == rzn);
-    const bool done = bad || rr <= dtol2[0];
-    if (done) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            flags[2] = jlocal + 1;
-            flags[1] = bad ? 1 : 0;
-            flags[0] = 1;
-        }
-        return;
-    }
-    const T beta = (T)(rzn / rzo);
-    const int blk = xcd_block();
-    for (int it = 0; it < kr; ++it) {
-        const int n = (blk * kr + it) * BS + threadIdx.x;
-        if (n >= N) break;
-#pragma unroll
-        for (int i = 0; i < 3; ++i) p[3 * n + i] = z[3 * n + i] + beta * p[3 * n + i];
-    }
-}
-
-// What B on the bricks reads of row n, loaded before the scalars are reduced.
-template <typename T>
-struct BrickRow {
+// What the update reads of row n, loaded before the scalars are reduced.  BRICK: q is the sum of the
+// node's brick partials (gptr, gF), p on its Dirichlet DOFs; else it is stored (gF).
+template <typename T, bool BRICK>
+struct UpdateRow {
     T r[3], M[9], q[3];
     __device__ __forceinline__ void load(int n, const T* __restrict__ rv, const T* __restrict__ Minv,
                                          const T* __restrict__ p, const int32_t* __restrict__ gptr,
                                          const T* __restrict__ gF, const uint8_t* __restrict__ dirflag) {
-        const int g0 = gptr[n], g1 = gptr[n + 1];
+        int g0 = 0, g1 = 0;
+        if constexpr (BRICK) {
+            g0 = gptr[n];
+            g1 = gptr[n + 1];
+        }
 #pragma unroll
         for (int i = 0; i < 3; ++i) r[i] = rv[3 * (int64_t)n + i];
 #pragma unroll
         for (int i = 0; i < 9; ++i) M[i] = Minv[(int64_t)n * 9 + i];
-        bool d[3];
+        if constexpr (BRICK) {
+            bool d[3];
 #pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            d[i] = dirflag[3 * (int64_t)n + i];
-            q[i] = (T)0;
+            for (int i = 0; i < 3; ++i) {
+                d[i] = dirflag[3 * (int64_t)n + i];
+                q[i] = (T)0;
+            }
+            for (int c = g0; c < g1; ++c)
+#pragma unroll
+                for (int i = 0; i < 3; ++i) q[i] += gF[3 * (int64_t)c + i];
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+                if (d[i]) q[i] = p[3 * (int64_t)n + i];
+        } else {
+#pragma unroll
+            for (int i = 0; i < 3; ++i) q[i] = gF[3 * (int64_t)n + i];
         }
-        for (int c = g0; c < g1; ++c)
-#pragma unroll
-            for (int i = 0; i < 3; ++i) q[i] += gF[3 * (int64_t)c + i];
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-            if (d[i]) q[i] = p[3 * (int64_t)n + i];
     }
 };
 
-// B for the hexa8 brick operator: p.q = the bricks' partials (nop of them) + the Dirichlet p.p
-// partials; q of node n = the sum of its brick partials (in brick order), p on its Dirichlet DOFs,
-// formed here and not stored.  x waits for C, which reads p anyway; alpha goes to *alphaOut.
-// The first row's loads run beside the scalars' reduction.  PCG iteration with x updated here and
-// the loads behind the reduction -> now (both kernels, and the fixed-pitch brick tables): FP64 20^3 20.4
-// -> 19.3, 40^3 33.0 -> 30.0, 64^3 62.7 -> 59.0 us, FP32 96^3 118.4 -> 113.3 us.
-template <typename T, int BS>
-__global__ __launch_bounds__(BS) void pcg_update_mfb_kernel(
+// B: alpha = r.z / p.q, r -= alpha q, z = Minv r and their partials; p.q = the operator's partials (nop
+// of them), on the bricks + the Dirichlet p.p partials.  x waits for C, which reads p anyway; alpha
+// goes to *alphaOut.  The first row's loads run beside the scalars' reduction.  PCG iteration on the
+// bricks with x updated here and the loads behind the reduction -> now (both kernels, and the
+// fixed-pitch brick tables): FP64 20^3 20.4 -> 19.3, 40^3 33.0 -> 30.0, 64^3 62.7 -> 59.0 us, FP32 96^3
+// 118.4 -> 113.3 us.
+template <typename T, int BS, bool BRICK>
+__global__ __launch_bounds__(BS) void pcg_update_kernel(
     int N, const T* __restrict__ Minv, T* __restrict__ r, T* __restrict__ z, const T* __restrict__ p,
     const int32_t* __restrict__ gptr, const T* __restrict__ gF, const uint8_t* __restrict__ dirflag,
     double* __restrict__ part, int ps, int nop, int nvec, int par, const int* __restrict__ done,
@@ -366,14 +327,17 @@ __global__ __launch_bounds__(BS) void pcg_update_mfb_kernel(
     __shared__ double sh[BS];
     const int blk = xcd_block();
     int n = blk * kr * BS + threadIdx.x;
-    BrickRow<T> row;
+    UpdateRow<T, BRICK> row;
     if (n < N) row.load(n, r, Minv, p, gptr, gF, dirflag);
     if (*done) return;
-    const int offs[3] = {0, 5 * ps, (1 + par) * ps};
+    constexpr int NS = BRICK ? 3 : 2;
+    const int offs[3] = {0, (1 + par) * ps, 5 * ps};
     const int ns[3] = {nop, nvec, nvec};
-    double sc[3];
-    reduce_partials_nv<BS, 3>(part, offs, ns, sc, sh);
-    const double al = sc[2] / (sc[0] + sc[1]);
+    double sc[NS];
+    reduce_partials_nv<BS, NS>(part, offs, ns, sc, sh);
+    double pq = sc[0];
+    if constexpr (BRICK) pq += sc[2];
+    const double al = sc[1] / pq;
     const T alpha = (T)al;
     if (blk == 0 && threadIdx.x == 0) *alphaOut = al;
     double rzn = 0, rr = 0;
@@ -402,11 +366,11 @@ __global__ __launch_bounds__(BS) void pcg_update_mfb_kernel(
     }
 }
 
-// C on the bricks: x += alpha p, the convergence test, p = z + beta p and the Dirichlet p.p partials.
+// C: x += alpha p, the convergence test, p = z + beta p and, on the bricks, the Dirichlet p.p partials.
 // As every workgroup has to add its alpha p in the last iteration too, the flag of the next iteration
 // (doneNext) is not the one this kernel reads (done): the two alternate.
-template <typename T, int BS>
-__global__ __launch_bounds__(BS) void pcg_direction_mfb_kernel(
+template <typename T, int BS, bool BRICK>
+__global__ __launch_bounds__(BS) void pcg_direction_kernel(
     int N, T* __restrict__ x, const T* __restrict__ z, T* __restrict__ p, double* __restrict__ part, int ps, int nvec,
     int par, int jlocal, const double* __restrict__ dtol2, const double* __restrict__ alphaIn,
     const int* __restrict__ done, int* __restrict__ doneNext, int* __restrict__ flags, int kr,
@@ -451,14 +415,16 @@ __global__ __launch_bounds__(BS) void pcg_direction_mfb_kernel(
             if (!stop) {
                 const T v = zv[i] + beta * pv[i];
                 p[3 * (int64_t)n + i] = v;
-                if (dirflag[3 * (int64_t)n + i]) pd += (double)v * v;
+                if (BRICK && dirflag[3 * (int64_t)n + i]) pd += (double)v * v;
             }
         }
         n += BS;
         if (it + 1 < kr && n < N) load();
     }
-    const double s = block_sum<BS>(pd, sh);
-    if (threadIdx.x == 0) part[5 * ps + blk] = s;
+    if constexpr (BRICK) {
+        const double s = block_sum<BS>(pd, sh);
+        if (threadIdx.x == 0) part[5 * ps + blk] = s;
+    }
 }
 
 // x_out = x (converted), with Dirichlet DOFs taken from b exactly.
@@ -475,58 +441,18 @@ template <int BS>
 __global__ __launch_bounds__(BS) void norms_stage1(int D, const double* __restrict__ R, const double* __restrict__ ddU,
                                                    const double* __restrict__ F, double* __restrict__ part,
                                                    int nwg) {
-    __shared__ double sv[BS];
-    __shared__ long long si[BS];
-    __shared__ double sh[BS];
-    double mr = -1.0, md = 0.0, sf = 0.0, nan = 0.0;
-    long long ir = 0x7fffffffffffffffLL;
-    for (int i = blockIdx.x * BS + threadIdx.x; i < D; i += BS * gridDim.x) {
-        const double a = fabs(R[i]);
-        if (!(a == a)) nan = 1.0;
-        if (a > mr) {
-            mr = a;
-            ir = i;
-        }
-        if (ddU) {
-            const double d = fabs(ddU[i]);
-            if (!(d == d)) nan = 1.0;
-            md = d > md ? d : md;
-        }
-        sf += fabs(F[i]);
-    }
-    sv[threadIdx.x] = mr;
-    si[threadIdx.x] = ir;
-    __syncthreads();
-    for (int s = BS / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) {
-            const double o = sv[threadIdx.x + s];
-            const long long oi = si[threadIdx.x + s];
-            if (o > sv[threadIdx.x] || (o == sv[threadIdx.x] && oi < si[threadIdx.x])) {
-                sv[threadIdx.x] = o;
-                si[threadIdx.x] = oi;
-            }
-        }
-        __syncthreads();
-    }
-    const double smax = sv[0];
-    const long long simax = si[0];
-    __syncthreads();
-    sh[threadIdx.x] = md;
-    __syncthreads();
-    for (int s = BS / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) sh[threadIdx.x] = fmax(sh[threadIdx.x], sh[threadIdx.x + s]);
-        __syncthreads();
-    }
-    const double dmax = sh[0];
-    __syncthreads();
-    const double fsum = block_sum<BS>(sf, sh);
-    const double nn = block_sum<BS>(nan, sh);
+    __shared__ double sh[BS / 64 * 5];
+    NormSums v;
+#pragma unroll 4
+    for (int i = blockIdx.x * BS + threadIdx.x; i < D; i += BS * gridDim.x)
+        v.add((double)i, R[i], ddU ? ddU[i] : 0.0, F[i]);
+    v.reduce<BS / 64>(sh);
     if (threadIdx.x == 0) {
-        part[0 * nwg + blockIdx.x] = smax;
-        part[1 * nwg + blockIdx.x] = (double)simax;
-        part[2 * nwg + blockIdx.x] = dmax;
-        part[3 * nwg + blockIdx.x] = fsum;
-        part[4 * nwg + blockIdx.x] = nn;
+        part[0 * nwg + blockIdx.x] = v.mr;
+        part[1 * nwg + blockIdx.x] = v.ir;
+        part[2 * nwg + blockIdx.x] = v.md;
+        part[3 * nwg + blockIdx.x] = v.sf;
+        part[4 * nwg + blockIdx.x] = v.nan;
     }
 }
 
@@ -541,125 +467,57 @@ __global__ __launch_bounds__(256) void sum_partials_kernel(const double* __restr
 // Final reduction of the per-workgroup norms by one 256-thread workgroup (fixed order).
 __global__ __launch_bounds__(256) void norms_stage2(const double* __restrict__ part, int nwg,
                                                     double* __restrict__ out) {
-    __shared__ double sv[256];
-    __shared__ double si[256];
-    __shared__ double sh[256];
-    double mr = -1.0, ir = 1e300, md = 0;
+    __shared__ double sh[4 * 5];
+    NormSums v;
+#pragma unroll 4
     for (int w = threadIdx.x; w < nwg; w += 256) {
-        const double v = part[w];
-        if (v > mr || (v == mr && part[nwg + w] < ir)) {
-            mr = v;
-            ir = part[nwg + w];
-        }
-        md = fmax(md, part[2 * nwg + w]);
+        NormSums o;
+        o.mr = part[w];
+        o.ir = part[nwg + w];
+        o.md = part[2 * nwg + w];
+        o.sf = part[3 * nwg + w];
+        o.nan = part[4 * nwg + w];
+        v.merge(o);
     }
-    sv[threadIdx.x] = mr;
-    si[threadIdx.x] = ir;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) {
-            const double o = sv[threadIdx.x + s], oi = si[threadIdx.x + s];
-            if (o > sv[threadIdx.x] || (o == sv[threadIdx.x] && oi < si[threadIdx.x])) {
-                sv[threadIdx.x] = o;
-                si[threadIdx.x] = oi;
-            }
-        }
-        __syncthreads();
-    }
-    const double rmax = sv[0], rarg = si[0];
-    __syncthreads();
-    sh[threadIdx.x] = md;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) sh[threadIdx.x] = fmax(sh[threadIdx.x], sh[threadIdx.x + s]);
-        __syncthreads();
-    }
-    const double dmax = sh[0];
-    __syncthreads();
-    const double sf = reduce_partials<256>(part + 3 * nwg, nwg, sh);
-    const double nn = reduce_partials<256>(part + 4 * nwg, nwg, sh);
+    v.reduce<4>(sh);
     if (threadIdx.x == 0) {
-        out[0] = rmax < 0 ? 0.0 : rmax;
-        out[1] = rmax < 0 ? 0.0 : rarg;
-        out[2] = dmax;
-        out[3] = sf;
-        out[4] = nn > 0 ? 1.0 : 0.0;
-    }
-}
-
-// Per-specimen norms (batched contexts): one workgroup per specimen over its DOF range.
-template <int BS>
-__global__ __launch_bounds__(BS) void norms_batched_kernel(const int64_t* __restrict__ dofoff,
-                                                           const double* __restrict__ R,
-                                                           const double* __restrict__ ddU,
-                                                           const double* __restrict__ F, double* __restrict__ out) {
-    __shared__ double sh[BS];
-    const int sp = blockIdx.x;
-    double mr = 0, md = 0, sf = 0, nan = 0;
-    for (int64_t i = dofoff[sp] + threadIdx.x; i < dofoff[sp + 1]; i += BS) {
-        const double a = fabs(R[i]);
-        if (!(a == a)) nan = 1.0;
-        mr = fmax(mr, a);
-        if (ddU) {
-            const double d = fabs(ddU[i]);
-            if (!(d == d)) nan = 1.0;
-            md = fmax(md, d);
-        }
-        sf += fabs(F[i]);
-    }
-    sh[threadIdx.x] = mr;
-    __syncthreads();
-    for (int s = BS / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) sh[threadIdx.x] = fmax(sh[threadIdx.x], sh[threadIdx.x + s]);
-        __syncthreads();
-    }
-    const double rmax = sh[0];
-    __syncthreads();
-    sh[threadIdx.x] = md;
-    __syncthreads();
-    for (int s = BS / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) sh[threadIdx.x] = fmax(sh[threadIdx.x], sh[threadIdx.x + s]);
-        __syncthreads();
-    }
-    const double dmax = sh[0];
-    __syncthreads();
-    const double fs = block_sum<BS>(sf, sh);
-    const double nn = block_sum<BS>(nan, sh);
-    if (threadIdx.x == 0) {
-        out[sp * 4 + 0] = rmax;
-        out[sp * 4 + 1] = dmax;
-        out[sp * 4 + 2] = fs;
-        out[sp * 4 + 3] = nn > 0 ? 1.0 : 0.0;
+        out[0] = v.mr < 0 ? 0.0 : v.mr;
+        out[1] = v.mr < 0 ? 0.0 : v.ir;
+        out[2] = v.md;
+        out[3] = v.sf;
+        out[4] = v.nan;
     }
 }
 
 template <typename T, int BS>
 void launch_iter(efe_ctx* c, KrylovWork* w, hipStream_t st, T* x, T* r, T* z, T* p, T* q, const T* K,
                  const T* Minv, bool bricks, int par, int j) {
-    const int grid = w->nwg;
-    const int kr = w->kr;
     const int gv = w->nwgv, krv = w->krv;
+    const int *done = w->flags + (par ? 3 : 0);
+    int* doneNext = w->flags + (par ? 0 : 3);
     if (bricks) {  // hexa8 bricks: the product's partials gathered by the update
         const T* gF;
         if constexpr (sizeof(T) == 8) gF = c->mfbF64;
         else gF = c->mfbF;
-        const int *done = w->flags + (par ? 3 : 0);
         efe_mf_launch_apply_partials(c, st, p, w->part, done);
-        pcg_update_mfb_kernel<T, BS><<<gv, BS, 0, st>>>(c->N, Minv, r, z, p, c->mfbPptr, gF, c->dirflag, w->part, w->ps,
-                                                        round8(c->mfbG), gv, par, done, w->dscal + 2, krv);
-        pcg_direction_mfb_kernel<T, BS><<<gv, BS, 0, st>>>(c->N, x, z, p, w->part, w->ps, gv, par, j, w->dscal,
-                                                           w->dscal + 2, done, w->flags + (par ? 0 : 3), w->flags,
-                                                           krv, c->dirflag);
+        pcg_update_kernel<T, BS, true><<<gv, BS, 0, st>>>(c->N, Minv, r, z, p, c->mfbPptr, gF, c->dirflag, w->part,
+                                                          w->ps, round8(c->mfbG), gv, par, done, w->dscal + 2, krv);
+        pcg_direction_kernel<T, BS, true><<<gv, BS, 0, st>>>(c->N, x, z, p, w->part, w->ps, gv, par, j, w->dscal,
+                                                             w->dscal + 2, done, doneNext, w->flags, krv, c->dirflag);
         return;
     }
-    if (K)
-        spmv_kernel<T, BS><<<grid, BS, 0, st>>>(c->N, c->slice_off, c->scol, c->slotNode, K, p, q, w->part, w->flags,
-                                                kr);
-    else  // matrix-free FP32 operator
-        efe_mf_launch_operator(c, st, (const float*)p, (float*)q, w->part, w->flags, grid, BS, kr);
-    pcg_update_kernel<T, BS><<<gv, BS, 0, st>>>(c->N, Minv, x, r, z, p, q, w->part, w->ps, grid, gv, par, w->flags,
-                                                krv);
-    pcg_direction_kernel<T, BS><<<gv, BS, 0, st>>>(c->N, z, p, w->part, w->ps, gv, par, j, w->dscal, w->flags, krv);
+    int nop = w->nwg;
+    if (K) {
+        nop = w->nwgs;
+        spmv_kernel<T><<<nop, 64 * kSpmvWaves, 0, st>>>(c->N, c->slice_off, c->scol, c->slotNode, K, p, q, w->part, done,
+                                                        w->krs);
+    } else {  // matrix-free FP32 operator of hexa20
+        efe_mf_launch_operator(c, st, (const float*)p, (float*)q, w->part, done, nop, BS, w->kr);
+    }
+    pcg_update_kernel<T, BS, false><<<gv, BS, 0, st>>>(c->N, Minv, r, z, p, nullptr, q, nullptr, w->part, w->ps, nop, gv,
+                                                       par, done, w->dscal + 2, krv);
+    pcg_direction_kernel<T, BS, false><<<gv, BS, 0, st>>>(c->N, x, z, p, w->part, w->ps, gv, par, j, w->dscal,
+                                                          w->dscal + 2, done, doneNext, w->flags, krv, nullptr);
 }
 
 template <typename T>
@@ -752,7 +610,10 @@ int ensure_work(efe_ctx* c) {
         w->nwgvp[i] = round8((c->N + block * w->krvp[i] - 1) / (block * w->krvp[i]));
         w->ps = std::max(w->ps, std::max(w->nwgp[i], w->nwgvp[i]));
     }
-    w->ps = std::max(w->ps, need);
+    const int slices = (c->N + kSlice - 1) / kSlice, scap = 2048;
+    w->krs = (slices + scap - 1) / scap;
+    w->nwgs = round8((slices + w->krs - 1) / w->krs);
+    w->ps = std::max(std::max(w->ps, w->nwgs), need);
     w->kr = w->krp[0];
     w->nwg = w->nwgp[0];
     w->krv = w->krvp[0];
@@ -882,9 +743,9 @@ int efe_krylov_solve(efe_ctx* c, const double* b, double* x, const efe_solve_opt
     if (o->precision == EFE_FP32)
         return pcg_solve<float>(c, b, x, o, info, w->x32, w->r32, w->z32, w->p32, w->q32, c->K32, c->Minv32, false, 1);
     // hexa8 with a symmetric tangent: the FP64 brick product moves 614 bytes per element where the
-    // assembled one moves 2135.  PCG iteration at 8^3 / 20^3 / 40^3 / 64^3: 19.8 / 22.9 / 46.9 /
-    // 123.7 us assembled, 18.9 / 20.7 / 31.2 / 62.7 us on the bricks.  The assembled operator serves
-    // the other elements and materials, and a Dirichlet set changed since the pass.
+    // assembled one moves 2135.  PCG iteration at 32^3 / 40^3 / 64^3: 25.3 / 39.5 / 118 us assembled,
+    // 22.2 / 30.0 / 59.0 us on the bricks.  The assembled operator serves smaller meshes
+    // (kSplitElements), the other elements and materials, and a Dirichlet set changed since the pass.
     if (efe_mf_bricks64(c))
         return pcg_solve<double>(c, b, x, o, info, w->x64, w->r64, w->z64, w->p64, w->q64, nullptr, c->Minv64, true, 3);
     return pcg_solve<double>(c, b, x, o, info, w->x64, w->r64, w->z64, w->p64, w->q64, c->K64, c->Minv64, false, 0);
@@ -895,7 +756,7 @@ int efe_launch_spmv64(efe_ctx* c, const double* x, double* y) {
         efe_set_error("efe_spmv needs an FP64 operator");
         return EFE_ERR_STATE;
     }
-    spmv_kernel<double, 256><<<round8((c->N + 255) / 256), 256, 0, c->stream>>>(
+    spmv_kernel<double><<<round8((c->N + kSlice - 1) / kSlice), 64 * kSpmvWaves, 0, c->stream>>>(
         c->N, c->slice_off, c->scol, c->slotNode, c->K64, x, y, nullptr, nullptr, 1);
     EFE_HIP(hipGetLastError());
     return EFE_OK;

@@ -25,9 +25,10 @@
 // runs on them instead of the assembled operator.  Bytes per element and product: 64 NC / 8 (FP32
 // half of it) for the tangents (NC = 7), ~1.6 staged nodes of 48 + 2 x 24 (12) bytes, 16 of local
 // indices: 614 in FP64, against 2135 of the assembled blocks at 64^3 (27 x 72 + 27 x 4 per node).
-// Measured at 64^3 in FP64: 100 us per assembled product (5.6 TB/s), 43 us per brick product with
-// the tangents from HBM, ~36 us with them in the Infinity Cache; PCG iteration 123.7 -> 59.0 us.  Meshes of up to
-// kSplitElements elements have bricks of 32, with 8 lanes per element.
+// Measured at 64^3 in FP64: 94 us per assembled product (5.9 TB/s), 43 us per brick product with
+// the tangents from HBM, ~34 us with them in the Infinity Cache; PCG iteration 123.7 -> 59.0 us.
+// Meshes of up to kSplitElements elements have, in FP32, bricks of 32 with 8 lanes per element and, in
+// FP64, the assembled operator.
 #include <algorithm>
 #include <cstring>
 #include <type_traits>
@@ -405,8 +406,7 @@ struct BrickTables {
 // P = 8 (split bricks): a lane has one QP; its forces on the 8 nodes are summed over the element's
 // lanes by halving exchanges, which leave each lane one node's.  This repeats the element's set-up in
 // 8 lanes, but takes the tangents in one round of loads and needs 32 elements per CU, not 256: the
-// product of a small mesh is a chain of latencies (320 elements: 9.3 us on two whole bricks; PCG
-// iteration 17.4 -> 14 us).
+// product of a small mesh is a chain of latencies (320 elements: 9.3 us on two whole bricks).
 template <int NC, typename T, typename TP, int P>
 __global__ __launch_bounds__(kBrick) void brick_apply_kernel(
     BrickTables bt, const T* __restrict__ el, const T* __restrict__ C, const TP* __restrict__ p,
@@ -748,19 +748,20 @@ void launch_bricks(efe_ctx* c, hipStream_t st, const TP* p, int mask, const int*
         F = c->mfbF;
     }
 #define BRICK_ARGS <<<grid, kBrick, 0, st>>>(bt, el, C, p, c->dirflag, mask, flags, F, active, part)
-    const bool split = c->mfbE != kBrick;
-    if (c->mfNC == 10) {
-        if constexpr (sizeof(T) == 4) {
-            if (split) brick_apply_kernel<10, T, TP, 8> BRICK_ARGS;
-            else brick_apply_kernel<10, T, TP, 1> BRICK_ARGS;
+    if constexpr (sizeof(T) == 4) {
+        if (c->mfbE != kBrick) {
+            if (c->mfNC == 10) brick_apply_kernel<10, T, TP, 8> BRICK_ARGS;
+            else if (c->mfNC == 7) brick_apply_kernel<7, T, TP, 8> BRICK_ARGS;
+            else brick_apply_kernel<0, T, TP, 8> BRICK_ARGS;
+            return;
         }
-    } else if (c->mfNC == 7) {
-        if (split) brick_apply_kernel<7, T, TP, 8> BRICK_ARGS;
-        else brick_apply_kernel<7, T, TP, 1> BRICK_ARGS;
-    } else {
-        if (split) brick_apply_kernel<0, T, TP, 8> BRICK_ARGS;
-        else brick_apply_kernel<0, T, TP, 1> BRICK_ARGS;
+        if (c->mfNC == 10) {
+            brick_apply_kernel<10, T, TP, 1> BRICK_ARGS;
+            return;
+        }
     }
+    if (c->mfNC == 7) brick_apply_kernel<7, T, TP, 1> BRICK_ARGS;
+    else brick_apply_kernel<0, T, TP, 1> BRICK_ARGS;
 #undef BRICK_ARGS
 }
 

@@ -16,6 +16,10 @@ J2 = [210000.0, 0.3, 250.0, 1000.0, 0.0, 0.0]
 LE = [180000.0, 0.25]
 
 
+# a context of one specimen takes the bricks at any size (without specimens, small meshes do not)
+_ALONE = lambda pm: dict(specimen_of_node=np.zeros(pm.coordinates.shape[0], dtype=np.int32), n_specimens=1)
+
+
 def _sections(E):
     names = np.where(np.arange(E) % 3 == 0, "linearelastic", "vonmises").tolist()
     rows = np.tile(J2, (E, 1))
@@ -48,7 +52,7 @@ def test_fp64_bricks_solve_the_assembled_system(n, material, perm):
         props = np.tile(J2, (E, 1))
         props[:, 0] *= np.exp(0.1 * rng.standard_normal(E))
         props[:, 2] *= np.exp(0.1 * rng.standard_normal(E))
-    sysm = DeviceSystem(pm.coordinates, np.ascontiguousarray(conn), "C3D8", name, props)
+    sysm = DeviceSystem(pm.coordinates, np.ascontiguousarray(conn), "C3D8", name, props, **_ALONE(pm))
     dirs = np.r_[pm.dofsOfNodeSet("gen_bottom"), pm.dofsOfNodeSet("gen_top", [1])]
     sysm.set_dirichlet(dirs)
     dU = torch.as_tensor(rng.uniform(-1, 1, sysm.n_dof) * 2e-3 / max(n), device="cuda")
@@ -75,7 +79,7 @@ def test_fp64_bricks_follow_a_changed_dirichlet_set():
     pm = device_model((5, 4, 6), (1.0, 1.0, 1.0), "C3D8", "vonmises", J2, jitter=0.1, seed=3)
     from edelweissfe_amd.device import DeviceSystem
 
-    sysm = DeviceSystem(pm.coordinates, pm.connectivity, "C3D8", "vonmises", J2)
+    sysm = DeviceSystem(pm.coordinates, pm.connectivity, "C3D8", "vonmises", J2, **_ALONE(pm))
     rng = np.random.default_rng(6)
     b = torch.as_tensor(rng.standard_normal(sysm.n_dof), device="cuda")
     P, F, x, y = (sysm.zeros() for _ in range(4))
@@ -154,22 +158,32 @@ def test_batched_bricks_solve_every_specimen_as_alone(sizes, precision):
     batch.close()
 
 
-@pytest.mark.parametrize("n", [(24, 32, 32), (25, 32, 32)])  # the most elements of split bricks, and more
-@pytest.mark.parametrize("material", ["vonmises", "linearelastic"])
+@pytest.mark.parametrize("n,material", [
+    ((1, 1, 1), "vonmises"),
+    ((33, 1, 1), "linearelastic"),   # one more than a split brick in a row
+    ((9, 7, 5), "vonmises"),
+    ((9, 7, 5), "druckerprager"),
+    ((24, 32, 32), "vonmises"),      # the most elements of split bricks, and more
+    ((24, 32, 32), "linearelastic"),
+    ((25, 32, 32), "vonmises"),
+    ((25, 32, 32), "linearelastic"),
+])
 def test_split_and_whole_bricks_step_as_the_assembled_operator(n, material):
     """Three PCG iterations from x = 0 (six products' worth of round-off, far from convergence) on the
-    bricks and on the assembled operator of the same pass: 1e-12 relative in FP64; in FP32 the
-    tangents' and products' rounding, 1e-4."""
+    FP32 bricks (split ones, then whole ones), on what the FP64 CG takes after a pass (the assembled
+    operator, then bricks) and on the assembled operator: 1e-12 relative in FP64; in FP32 the tangents'
+    and products' rounding, 1e-4.  (Drucker-Prager at an elastic state, whose tangent is symmetric.)"""
     from edelweissfe_amd import _lib
     from edelweissfe_amd.device import DeviceSystem
 
-    props = J2 if material == "vonmises" else LE
+    props = {"vonmises": J2, "linearelastic": LE, "druckerprager": [30000.0, 0.2, 30.0, 10.0, 10.0, 0.0]}[material]
     pm = device_model(n, (1.0, 1.0, 1.0), "C3D8", material, props, jitter=0.1, seed=3)
     sysm = DeviceSystem(pm.coordinates, pm.connectivity, "C3D8", material, np.array(props))
     dirs = np.r_[pm.dofsOfNodeSet("gen_bottom"), pm.dofsOfNodeSet("gen_top", [1])]
     sysm.set_dirichlet(dirs)
     rng = np.random.default_rng(7)
-    dU = torch.as_tensor(rng.uniform(-1, 1, sysm.n_dof) * 2e-3 / max(n), device="cuda")
+    scale = 1e-6 if material == "druckerprager" else 2e-3
+    dU = torch.as_tensor(rng.uniform(-1, 1, sysm.n_dof) * scale / max(n), device="cuda")
     b = torch.as_tensor(rng.standard_normal(sysm.n_dof), device="cuda")
     P, F = sysm.zeros(), sysm.zeros()
     x32, xb, xa = sysm.zeros(), sysm.zeros(), sysm.zeros()
