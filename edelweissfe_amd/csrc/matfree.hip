@@ -803,29 +803,28 @@ void launch_gather_op(efe_ctx* c, hipStream_t st, const float* p, float* q, doub
 }  // namespace
 
 namespace {
+// bulk modulus and 2 G of the elements, brick by brick (n places)
 template <typename T>
-int up(T** dst, const std::vector<T>& v) {
-    EFE_HIP(hipMalloc((void**)dst, (v.size() ? v.size() : 1) * sizeof(T)));
-    if (!v.empty()) EFE_HIP(hipMemcpy((void*)*dst, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
-    return EFE_OK;
+__global__ void brick_moduli_kernel(int E, const double* __restrict__ props, int propStride,
+                                    const int32_t* __restrict__ pos, int64_t n, T* __restrict__ el) {
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= E) return;
+    const double y = propStride ? props[e] : props[0], nu = propStride ? props[propStride + e] : props[1];
+    el[pos[e]] = (T)(y / (3.0 * (1.0 - 2.0 * nu)));
+    el[n + pos[e]] = (T)(y / (1.0 + nu));
 }
 
-// bulk modulus and 2 G of the elements, brick by brick
+// the tangents, the moduli and the partials of one precision, in one allocation (at *C)
 template <typename T>
-int build_moduli(efe_ctx* c, T** dst) {
-    const int E = c->E;
-    std::vector<double> pr(c->props_per_element ? (size_t)2 * E : 2);
-    std::vector<int32_t> pos(E);
-    EFE_HIP(hipMemcpy(pr.data(), c->props, pr.size() * sizeof(double), hipMemcpyDeviceToHost));
-    EFE_HIP(hipMemcpy(pos.data(), c->mfbPos, (size_t)E * sizeof(int32_t), hipMemcpyDeviceToHost));
-    const size_t n = (size_t)c->mfbG * c->mfbE;
-    std::vector<T> v(2 * n, (T)0);
-    for (int e = 0; e < E; ++e) {
-        const double y = c->props_per_element ? pr[e] : pr[0], nu = c->props_per_element ? pr[(size_t)E + e] : pr[1];
-        v[pos[e]] = (T)(y / (3.0 * (1.0 - 2.0 * nu)));
-        v[n + pos[e]] = (T)(y / (1.0 + nu));
-    }
-    return up(dst, v);
+int alloc_bricks(efe_ctx* c, T** C, T** el, T** F) {
+    const size_t n = (size_t)c->mfbG * c->mfbE, nc = n * 8 * (c->mfNC ? c->mfNC : 1);
+    EFE_HIP(hipMalloc((void**)C, (nc + 2 * n + (size_t)c->mfbL * 3) * sizeof(T)));
+    *el = *C + nc;
+    *F = *el + 2 * n;
+    brick_moduli_kernel<T><<<(c->E + 255) / 256, 256, 0, c->stream>>>(c->E, c->props, c->props_per_element ? c->E : 0,
+                                                                      c->mfbPos, (int64_t)n, *el);
+    EFE_HIP(hipGetLastError());
+    return EFE_OK;
 }
 }  // namespace
 
@@ -866,20 +865,8 @@ int efe_mf_upload_bricks(efe_ctx* c, const BrickPattern& bp, const double* coord
 }
 
 int efe_mf_alloc_bricks(efe_ctx* c, bool fp64) {
-    EFE_HIP(hipStreamSynchronize(c->stream));  // the uploads below use the default stream
-    const size_t nc = (size_t)c->mfbG * c->mfbE * 8 * (c->mfNC ? c->mfNC : 1);
-    if (fp64) {
-        if (c->mfC64) return EFE_OK;
-        if (int rc = build_moduli(c, &c->mfbEl64)) return rc;
-        EFE_HIP(hipMalloc(&c->mfbF64, (size_t)c->mfbL * 3 * sizeof(double)));
-        EFE_HIP(hipMalloc(&c->mfC64, nc * sizeof(double)));
-    } else {
-        if (c->mfC) return EFE_OK;
-        if (int rc = build_moduli(c, &c->mfbEl)) return rc;
-        EFE_HIP(hipMalloc(&c->mfbF, (size_t)c->mfbL * 3 * sizeof(float)));
-        EFE_HIP(hipMalloc(&c->mfC, nc * sizeof(float)));
-    }
-    return EFE_OK;
+    if (fp64) return c->mfC64 ? EFE_OK : alloc_bricks(c, &c->mfC64, &c->mfbEl64, &c->mfbF64);
+    return c->mfC ? EFE_OK : alloc_bricks(c, &c->mfC, &c->mfbEl, &c->mfbF);
 }
 
 bool efe_mf_bricks64(const efe_ctx* c, const uint8_t* which) {
@@ -993,7 +980,8 @@ void efe_mf_launch_operator_batched(efe_ctx* c, hipStream_t st, const float* p, 
 }
 
 void efe_mf_free(efe_ctx* c) {
-    void* b[] = {c->mfC, c->mfF, c->dnxi32, c->mfC64, c->mfbTables, c->mfbEl, c->mfbF, c->mfbEl64, c->mfbF64};
+    // mfC and mfC64 hold the bricks' moduli and partials too
+    void* b[] = {c->mfC, c->mfF, c->dnxi32, c->mfC64, c->mfbTables};
     for (void* q : b)
         if (q) hipFree(q);
     c->mfC = c->mfF = c->dnxi32 = nullptr;
