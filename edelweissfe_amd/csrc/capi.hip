@@ -246,11 +246,15 @@ int efe_ctx_create(const efe_mesh_desc* d, efe_ctx** out) {
             delete c;
             return EFE_ERR_ARG;
         }
-    // the bricks of the matrix-free product, beside the pattern
+    // the bricks of the matrix-free product, beside the pattern; a small mesh's, which its FP64 passes
+    // do without, at the first matrix-free pass (efe_mf_alloc)
     BrickPattern bp;
-    bp.EB = !d->specimen_of_node && c->E <= kSplitElements ? kBrickSplit : kBrick;
     std::future<void> bricks;
-    if (c->eltype == EFE_C3D8) {
+    if (c->eltype == EFE_C3D8 && !d->specimen_of_node && c->E <= kSplitElements) {
+        c->mfbE = kBrickSplit;
+        c->brickConn.assign(d->conn, d->conn + (size_t)8 * c->E);
+        c->brickXyz.assign(d->coords, d->coords + (size_t)3 * c->N);
+    } else if (c->eltype == EFE_C3D8) {
         auto build = [&bp, N = c->N, E = c->E, conn = d->conn, xyz = d->coords, spec = d->specimen_of_node] {
             efe_build_bricks(bp, N, E, conn, xyz, spec);
         };
@@ -391,7 +395,7 @@ int efe_ctx_create(const efe_mesh_desc* d, efe_ctx** out) {
     if ((rc = dalloc((void**)&c->red, (size_t)c->redn * sizeof(double)))) return fail(rc);
     for (auto& ev : c->ev) EFE_HIP(hipEventCreate(&ev));
     EFE_HIP(hipStreamSynchronize(st));
-    if (c->eltype == EFE_C3D8) {
+    if (bricks.valid()) {
         bricks.get();
         if ((rc = efe_mf_upload_bricks(c, bp, d->coords))) return fail(rc);
     }

@@ -251,7 +251,9 @@ struct efe_ctx {
     // coordinates, and the partial forces [L][3] in the precision of the product
     bool mfb = false;
     int mfbG = 0;                // bricks
-    int mfbE = kBrick;         // BrickPattern's EB
+    int mfbE = kBrick;           // BrickPattern's EB
+    std::vector<int32_t> brickConn;  // the mesh until a small one's bricks are built
+    std::vector<double> brickXyz;
     int64_t mfbL = 0;            // partials
     void* mfbTables = nullptr;   // one allocation: the tables below
     int32_t *mfbPos = nullptr, *mfbLnode = nullptr, *mfbLpos = nullptr, *mfbPptr = nullptr, *mfbSpec = nullptr;

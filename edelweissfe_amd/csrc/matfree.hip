@@ -886,7 +886,17 @@ int efe_mf_alloc(efe_ctx* c) {
     const int NC = c->mfNC;
     if (c->mfC) return EFE_OK;
     if (!c->Minv32) EFE_HIP(hipMalloc(&c->Minv32, (size_t)c->N * 9 * sizeof(float)));
-    if (c->eltype == EFE_C3D8) return efe_mf_alloc_bricks(c, false);
+    if (c->eltype == EFE_C3D8) {
+        if (!c->mfb) {
+            BrickPattern bp;
+            bp.EB = c->mfbE;
+            efe_build_bricks(bp, c->N, c->E, c->brickConn.data(), c->brickXyz.data(), nullptr);
+            if (int rc = efe_mf_upload_bricks(c, bp, c->brickXyz.data())) return rc;
+            std::vector<int32_t>().swap(c->brickConn);
+            std::vector<double>().swap(c->brickXyz);
+        }
+        return efe_mf_alloc_bricks(c, false);
+    }
     const size_t EQ = (size_t)c->E * c->Q;
     const int64_t L = (int64_t)c->E * c->NN;
     EFE_HIP(hipMalloc(&c->mfC, EQ * NC * sizeof(float)));
