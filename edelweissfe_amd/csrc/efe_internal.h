@@ -333,7 +333,7 @@ struct efe_ctx {
 
     // launch configuration
     int epw = 0;       // elements per workgroup of the element kernel (0 = default)
-    int kblock = 256;  // threads per workgroup of Krylov kernels
+    int kblock = 0;  // threads per workgroup of the PCG's vector kernels, 0: by size
 
     // phase timing: the last call of each phase, and totals over the context's life
     hipEvent_t ev[8] = {};

@@ -553,6 +553,10 @@ void launch_init_bs(efe_ctx* c, KrylovWork* w, hipStream_t st, const double* b, 
 
 int ensure_work(efe_ctx* c) {
     int block = c->kblock;
+    // Unless set: small meshes' rows over as many CUs as they give wavefronts.  PCG iteration at 64 / 128
+    // / 256 / 512: 525 nodes 10.9 / 11.4 / 11.6 / 12.7 us, 3375 11.8 / 12.0 / 12.4 / 13.5, 9261 14.2 / 13.2 / 13.4 /
+    // 14.2, 274625 76.7 / 63.4 / 59.3 / 63.4.
+    if (block <= 0) block = c->N <= 4096 ? 64 : 256;
     if (block != 64 && block != 128 && block != 256 && block != 512) block = 256;
     KrylovWork* w = c->kw;
     // the brick operator writes one p.Kp partial per brick into the partials array
