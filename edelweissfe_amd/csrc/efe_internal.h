@@ -157,8 +157,8 @@ constexpr int kBrickSplit = 32;
 // the same bits, alone and with others).  Fewer whole bricks leave CUs idle, or at one workgroup each;
 // beyond it the repeated set-up, and the assembled operator's bytes, cost more.  PCG iteration, FP32 whole
 // / split bricks: 8^3 17.1 / 13.0 us, 20^3 18.7 / 14.6, 28^3 (21952) 19.9 / 17.7, 32^3 20.3 / 18.4, 40^3
-// 23.0 / 29.5; FP64 whole / split / assembled: 8^3 17.6 / 13.6 / 11.7, 20^3 19.9 / 16.1 / 13.5, 28^3 21.4 /
-// 20.9 / 19.1, 32^3 22.2 / 22.3 / 25.3, 40^3 30.0 / 38.3 / 39.5.
+// 23.0 / 29.5; FP64 whole / split / assembled: 8^3 17.6 / 13.6 / 9.5, 20^3 19.9 / 16.1 / 10.3, 28^3 21.4 /
+// 20.9 / 18.1, 32^3 22.2 / 22.3 / 22.4, 40^3 30.0 / 38.3 / 39.5.
 constexpr int kSplitElements = 24576;
 
 // place of QP q of the element at pos (BrickPattern) among the tangents' rows of kBrick lanes

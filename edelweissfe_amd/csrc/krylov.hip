@@ -42,6 +42,7 @@ struct KrylovWork {
     int krvp[2] = {1, 1}, nwgvp[2] = {0, 0};
     int krv = 1, nwgv = 0;
     int krs = 1, nwgs = 0;
+    double* pb = nullptr;  // second direction vector of the folded iteration
     int ps = 0;  // row stride of the partials array (the largest workgroup count)
     // FP64 and FP32 vector sets
     double *x64 = nullptr, *r64 = nullptr, *z64 = nullptr, *p64 = nullptr, *q64 = nullptr;
@@ -223,6 +224,109 @@ __global__ __launch_bounds__(64 * kSpmvWaves) void spmv_kernel(int N, const int3
     }
 }
 
+// The iteration of a small assembled system in two launches: the direction (stop test, p = z + beta p)
+// in the product that follows it.  Every gather forms its entry of p, the row's owner stores it, and the
+// two p alternate, as neighbours still gather the old one.  The first blocks of a row are loaded beside
+// the scalars' reduction.  What an update ends with is tested by the next launch of this kernel.  PCG
+// iteration in three launches -> two: hexa8 FP64 525 nodes 11.1 -> 9.4 us, 3375 11.7 -> 9.7, 9261 13.3 ->
+// 10.3, 24389 19.0 -> 18.1, 35937 22.4 -> 22.4; FP32 9261 11.1 -> 8.7; hexa20R FP64 2673 19.8 -> 16.0, 26353
+// 36.2 -> 29.1.  (On 64^3 the same fold cost more than the launch: a second gathered vector.)
+template <typename T>
+__global__ __launch_bounds__(64 * kSpmvWaves) void pcg_fold_kernel(
+    int N, const int32_t* __restrict__ slice_off, const int32_t* __restrict__ scol,
+    const int32_t* __restrict__ slotNode, const T* __restrict__ K, const T* __restrict__ z, const T* __restrict__ p,
+    T* __restrict__ pNew, T* __restrict__ q, double* __restrict__ part, int ps, int nvec, int par, int jlocal,
+    const double* __restrict__ dtol2, int* __restrict__ flags) {
+    constexpr int W = kSpmvWaves, U = 4;
+    __shared__ T sh[W - 1][3][64];
+    __shared__ double sd[3 * W];
+    const int s = xcd_block(), l = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const bool slice = s * kSlice < N;
+    const int ps_ = s * kSlice + l;  // row slot
+    const int n = slice && ps_ < N ? slotNode[ps_] : -1;
+    int o0 = 0, k0 = 0, k1 = 0;
+    if (slice) {
+        o0 = slice_off[s];
+        const int deg = (slice_off[s + 1] - o0) / kSlice;
+        k0 = wave * deg / W;
+        k1 = (wave + 1) * deg / W;
+    }
+    const int32_t* cp = scol + o0 + l;
+    const T* kp = K + (int64_t)o0 * 9 + l;
+    T a[U][9], zv[U][3], pv[U][3];
+    auto load = [&](int k) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (k + u < k1) {  // uniform over the wavefront
+                const int m = cp[(k + u) * kSlice];
+#pragma unroll
+                for (int i = 0; i < 9; ++i) a[u][i] = kp[(int64_t)((k + u) * 9 + i) * kSlice];
+#pragma unroll
+                for (int i = 0; i < 3; ++i) {
+                    zv[u][i] = z[3 * m + i];
+                    pv[u][i] = p[3 * m + i];
+                }
+            }
+    };
+    if (n >= 0) load(k0);
+    if (flags[0]) return;
+    const int offs[3] = {(1 + par) * ps, (2 - par) * ps, 3 * ps};
+    double sc[3];
+    reduce_partials_n<64 * W, 3>(part, offs, nvec, sc, sd);
+    const double rz = sc[0], rzo = sc[1], rr = sc[2];
+    const bool bad = !(rr == rr) || !(rz == rz);
+    if (bad || rr <= dtol2[0]) {  // the last iteration's result
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            flags[2] = jlocal;
+            flags[1] = bad ? 1 : 0;
+            flags[0] = 1;
+        }
+        return;
+    }
+    const T beta = (T)(rz / rzo);
+    T y0 = 0, y1 = 0, y2 = 0;
+    if (n >= 0)
+        for (int k = k0; k < k1; k += U) {
+            if (k > k0) load(k);
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (k + u < k1) {
+                    const T x0 = zv[u][0] + beta * pv[u][0], x1 = zv[u][1] + beta * pv[u][1],
+                            x2 = zv[u][2] + beta * pv[u][2];
+                    y0 += a[u][0] * x0 + a[u][1] * x1 + a[u][2] * x2;
+                    y1 += a[u][3] * x0 + a[u][4] * x1 + a[u][5] * x2;
+                    y2 += a[u][6] * x0 + a[u][7] * x1 + a[u][8] * x2;
+                }
+        }
+    if (wave > 0) {
+        sh[wave - 1][0][l] = y0;
+        sh[wave - 1][1][l] = y1;
+        sh[wave - 1][2][l] = y2;
+    }
+    __syncthreads();
+    if (wave > 0) return;
+    double dot = 0.0;
+    if (n >= 0) {
+#pragma unroll
+        for (int w = 0; w < W - 1; ++w) {
+            y0 += sh[w][0][l];
+            y1 += sh[w][1][l];
+            y2 += sh[w][2][l];
+        }
+        const T y[3] = {y0, y1, y2};
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const T v = z[3 * n + i] + beta * p[3 * n + i];
+            pNew[3 * n + i] = v;
+            q[3 * n + i] = y[i];
+            dot += (double)v * y[i];
+        }
+    }
+    dot = wave_sum(dot);
+    if (threadIdx.x == 0) part[s] = dot;
+}
+
 // x = 0, r = b (b_dir = b on Dirichlet DOFs is part of the system), z = Minv r, p = z,
 // partials r.z -> part[1], b.b -> part[4].
 template <typename T, int BS, bool DP2 = false>
@@ -266,6 +370,9 @@ __global__ __launch_bounds__(BS) void pcg_init_kernel(int N, const double* __res
         part[1 * ps + blk] = s1;
         part[4 * ps + blk] = s2;
         if constexpr (DP2) part[5 * ps + blk] = sums[NS - 1];
+        // the folded iteration's beta = r.z / (r.z before) and stop test: 0 and no before the first
+        part[2 * ps + blk] = INFINITY;
+        part[3 * ps + blk] = INFINITY;
         if (blk == 0) {
             flags[0] = 0;
             flags[1] = 0;
@@ -318,12 +425,14 @@ struct UpdateRow {
 // bricks with x updated here and the loads behind the reduction -> now (both kernels, and the
 // fixed-pitch brick tables): FP64 20^3 20.4 -> 19.3, 40^3 33.0 -> 30.0, 64^3 62.7 -> 59.0 us, FP32 96^3
 // 118.4 -> 113.3 us.
-template <typename T, int BS, bool BRICK>
+// FOLD: x is updated here, after pcg_fold_kernel.
+template <typename T, int BS, bool BRICK, bool FOLD = false>
 __global__ __launch_bounds__(BS) void pcg_update_kernel(
     int N, const T* __restrict__ Minv, T* __restrict__ r, T* __restrict__ z, const T* __restrict__ p,
     const int32_t* __restrict__ gptr, const T* __restrict__ gF, const uint8_t* __restrict__ dirflag,
     double* __restrict__ part, int ps, int nop, int nvec, int par, const int* __restrict__ done,
-    double* __restrict__ alphaOut, int kr) {
+    double* __restrict__ alphaOut, int kr,
+    T* __restrict__ x = nullptr) {
     __shared__ double sh[BS];
     const int blk = xcd_block();
     int n = blk * kr * BS + threadIdx.x;
@@ -355,6 +464,9 @@ __global__ __launch_bounds__(BS) void pcg_update_kernel(
             z[3 * (int64_t)n + i] = zi;
             rzn += (double)rv[i] * zi;
         }
+        if constexpr (FOLD)
+#pragma unroll
+            for (int i = 0; i < 3; ++i) x[3 * (int64_t)n + i] += alpha * p[3 * (int64_t)n + i];
         n += BS;
         if (it + 1 < kr && n < N) row.load(n, r, Minv, p, gptr, gF, dirflag);
     }
@@ -489,6 +601,10 @@ __global__ __launch_bounds__(256) void norms_stage2(const double* __restrict__ p
     }
 }
 
+// Assembled systems of up to this many nodes take the folded iteration (at 35937 it is no faster).
+constexpr int kFoldNodes = 28000;
+inline bool fold_iteration(const efe_ctx* c) { return c->N <= kFoldNodes; }
+
 template <typename T, int BS>
 void launch_iter(efe_ctx* c, KrylovWork* w, hipStream_t st, T* x, T* r, T* z, T* p, T* q, const T* K,
                  const T* Minv, bool bricks, int par, int j) {
@@ -507,6 +623,16 @@ void launch_iter(efe_ctx* c, KrylovWork* w, hipStream_t st, T* x, T* r, T* z, T*
         return;
     }
     int nop = w->nwg;
+    if (K && fold_iteration(c)) {
+        nop = w->nwgs;
+        T *pa = p, *pb = (T*)w->pb;
+        T *pOld = par ? pb : pa, *pNew = par ? pa : pb;
+        pcg_fold_kernel<T><<<nop, 64 * kSpmvWaves, 0, st>>>(c->N, c->slice_off, c->scol, c->slotNode, K, z, pOld, pNew, q,
+                                                            w->part, w->ps, gv, par, j, w->dscal, w->flags);
+        pcg_update_kernel<T, BS, false, true><<<gv, BS, 0, st>>>(c->N, Minv, r, z, pNew, nullptr, q, nullptr, w->part,
+                                                                 w->ps, nop, gv, par, w->flags, w->dscal + 2, krv, x);
+        return;
+    }
     if (K) {
         nop = w->nwgs;
         spmv_kernel<T><<<nop, 64 * kSpmvWaves, 0, st>>>(c->N, c->slice_off, c->scol, c->slotNode, K, p, q, w->part, done,
@@ -580,6 +706,7 @@ int ensure_work(efe_ctx* c) {
         EFE_HIP(hipMalloc(&w->q32, D * sizeof(float)));
         EFE_HIP(hipMalloc(&w->flags, 4 * sizeof(int)));
         EFE_HIP(hipMalloc(&w->dscal, 4 * sizeof(double)));
+        if (fold_iteration(c)) EFE_HIP(hipMalloc(&w->pb, D * sizeof(double)));
         EFE_HIP(hipHostMalloc(&w->hflags, 4 * sizeof(int), hipHostMallocDefault));
         EFE_HIP(hipHostMalloc(&w->hpart, 8 * sizeof(double), hipHostMallocDefault));
         EFE_HIP(hipStreamCreateWithFlags(&w->ks, hipStreamNonBlocking));
@@ -709,6 +836,8 @@ int pcg_solve(efe_ctx* c, const double* b, double* xout, const efe_solve_opts* o
     EFE_HIP(hipMemcpyAsync(w->hpart, w->dscal + 1, sizeof(double), hipMemcpyDeviceToHost, st));
     EFE_HIP(hipStreamSynchronize(st));
     info->residual = sqrt(w->hpart[0]);
+    // a folded iteration's result is tested by the next one
+    if (info->status == EFE_NOT_CONVERGED && w->hpart[0] <= tol2) info->status = EFE_OK;
     info->iterations = it;
     float ms = 0;
     hipEventElapsedTime(&ms, w->t0, w->t1);
@@ -786,7 +915,7 @@ void efe_krylov_free(efe_ctx* c) {
         if (w->graph[i]) hipGraphExecDestroy(w->graph[i]);
     hipFree(w->x64); hipFree(w->r64); hipFree(w->z64); hipFree(w->p64); hipFree(w->q64);
     hipFree(w->x32); hipFree(w->r32); hipFree(w->z32); hipFree(w->p32); hipFree(w->q32);
-    hipFree(w->part); hipFree(w->flags); hipFree(w->dscal);
+    hipFree(w->part); hipFree(w->flags); hipFree(w->dscal); hipFree(w->pb);
     hipHostFree(w->hflags); hipHostFree(w->hpart);
     if (w->ks) hipStreamDestroy(w->ks);
     if (w->evA) hipEventDestroy(w->evA);
