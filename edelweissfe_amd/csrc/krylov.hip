@@ -1,8 +1,8 @@
 // Krylov solvers for the assembled tangent on gfx950.
 //
 // Operator layout: sliced ELL of 3x3 blocks, slice height 64 (one wavefront).
-// Thread (slice s, lane l) owns row slot p = 64 s + l, the row of node slotNode[p] (rows
-// sorted by length inside windows of nodes); block slot k of that row
+// Lane l of a slice s's workgroup has row slot p = 64 s + l, the row of node slotNode[p] (rows
+// sorted by length inside windows of nodes), whose blocks its wavefronts share; block slot k of that row
 // stores its 9 values at Kval[slice_off[s]*9 + (9k+v)*64 + l], so every value
 // load of a wavefront is one contiguous 512 B (FP64) / 256 B (FP32) segment and
 // the block column index (1 int per 9 values) is shared by the three rows of a
@@ -12,8 +12,9 @@
 // (nonlinearimplicitstatic.py:727-751) on symmetric tangents.  One iteration is
 // three kernels:
 //   A: q = K p, per-workgroup partials of p.q
-//   B: alpha = rz/pq; x += alpha p; r -= alpha q; z = Minv r; partials of r.z, r.r
-//   C: beta = rz_new/rz; p = z + beta p; convergence test
+//   B: alpha = rz/pq; r -= alpha q; z = Minv r; partials of r.z, r.r
+//   C: x += alpha p; beta = rz_new/rz; convergence test; p = z + beta p
+// (small assembled systems two: C's test and p in the next A, x in B).
 // Global scalars are never stored by one workgroup for the others: every
 // workgroup re-reduces the (few thousand) partials of the previous kernel in the
 // same fixed order, so all workgroups hold bitwise identical scalars and the
@@ -25,7 +26,7 @@
 // With the hexa8 brick operator (matrix-free FP32, and FP64), A is the brick product alone, its
 // partials the bricks' shares of p.Kp (Dirichlet DOFs masked), and B gathers each node's
 // brick partials itself (q is never stored): p.q = the bricks' sum + the sum of p^2 over the
-// Dirichlet DOFs, whose partials C (and the init) form with p; x is updated in C.
+// Dirichlet DOFs, whose partials C (and the init) form with p.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -876,7 +877,7 @@ int efe_krylov_solve(efe_ctx* c, const double* b, double* x, const efe_solve_opt
     if (o->precision == EFE_FP32)
         return pcg_solve<float>(c, b, x, o, info, w->x32, w->r32, w->z32, w->p32, w->q32, c->K32, c->Minv32, false, 1);
     // hexa8 with a symmetric tangent: the FP64 brick product moves 614 bytes per element where the
-    // assembled one moves 2135.  PCG iteration at 32^3 / 40^3 / 64^3: 25.3 / 39.5 / 118 us assembled,
+    // assembled one moves 2135.  PCG iteration at 32^3 / 40^3 / 64^3: 22.4 / 39.5 / 118 us assembled,
     // 22.2 / 30.0 / 59.0 us on the bricks.  The assembled operator serves smaller meshes
     // (kSplitElements), the other elements and materials, and a Dirichlet set changed since the pass.
     if (efe_mf_bricks64(c))
