@@ -2,11 +2,11 @@
 //
 // hex8_kernel (hexa8) is described at its definition; element_kernel (hexa20) follows the same
 // three phases, one 64-lane wavefront owning EPW elements.
-//   phase 1, one lane per (element, QP): Jacobian from the gathered node
-//            coordinates and the shape-function derivatives at the reference's
-//            evaluation point, dN/dx, strain increment from the gathered dU,
-//            FP64 material update of the reference state into the temporary
-//            state, and (w detJ) C and (w detJ) sigma staged in LDS;
+//   phase 1: the nodes' coordinates and increments to LDS, one lane per (element, node); one
+//            lane per (element, QP): Jacobian from the coordinates and the shape-function
+//            derivatives at the reference's evaluation point; dN/dx over all lanes; one lane
+//            per (element, QP): strain increment, FP64 material update of the reference state
+//            into the temporary state, and (w detJ) C and (w detJ) sigma staged in LDS;
 //   phase 2, one lane per (element, node a, node b), b >= a for symmetric
 //            tangents: the 3x3 block
 //            K_ab = sum_q B_a^T (w detJ C_q) B_b in KT precision (and K_ba = K_ab^T), written to the
@@ -79,6 +79,13 @@ __device__ __forceinline__ void store_compact(CT* __restrict__ mfC, const int32_
 // matrix-free operator, and phase 2 forms
 // only the diagonal blocks K_aa (for block Jacobi), stored element-major [e][a][9] at the
 // start of the element scratch.
+// Phase 1 is bound by the latency of its loads, phase 2 by FP64 VALU issue and the block stores.
+// With a gather of every node by every QP lane, and the gradients on the 16 (hexa20R: 2 x 8) or 27
+// QP lanes alone, a residual pass of 17x15x13 hexa20 J2 took 47 us against 37 us now, of 24x22x20
+// hexa20R DP 56 against 43 us, the matrix-free pass of the latter mesh (J2) 51 against 40 us; the
+// FP64 tangent passes 147 -> 139 us and 263 -> 255 us.  Coordinates, inverse Jacobians and
+// increments lie where the gradients and the weighted stresses follow: in LDS of their own (3 KB
+// more) the hexa20R tangent pass got slower (32^3 DP: 705 -> 770 us; as it is, 698 us).
 template <int NN, int Q, int MAT, typename KT, int EPW, bool MF>
 __global__ __launch_bounds__(64) void element_kernel(int E, int N, const double* __restrict__ coords,
                                                      const int32_t* __restrict__ conn,
@@ -101,9 +108,17 @@ __global__ __launch_bounds__(64) void element_kernel(int E, int N, const double*
     // the tangent of every QP in compact form, w detJ [A - B/3, B/2, c_nn, (c_n1, c_1n)] then n:
     // C = A 1(x)1 + B Idev + c_nn n(x)n (+ c_n1 n(x)1 + c_1n 1(x)n for Drucker-Prager)
     constexpr int NCC = (MAT == EFE_DRUCKER_PRAGER) ? 11 : 9;
+    // g_s holds the node coordinates until the gradients are formed; w_s in turn the inverse
+    // Jacobians, the nodes' increments, and the weighted stresses with the tangents
     __shared__ double g_s[EPW][Q * NN * 3];
-    __shared__ KT fC_s[EPW][Q * NCC];
-    __shared__ double fs_s[EPW][Q][6];
+    constexpr int kW = EPW * Q * 6 + (EPW * Q * NCC * (int)sizeof(KT) + 7) / 8;
+    static_assert(EPW * Q * 9 <= kW && EPW * NN * 3 <= kW, "inverse Jacobians and increments fit");
+    static_assert(EPW * Q <= 64 && EPW * NN <= 64, "a lane per (element, QP) and per (element, node)");
+    __shared__ double w_s[kW];
+    double(*iJ_s)[Q][9] = reinterpret_cast<double(*)[Q][9]>(w_s);
+    double(*u_s)[NN][3] = reinterpret_cast<double(*)[NN][3]>(w_s);
+    double(*fs_s)[Q][6] = reinterpret_cast<double(*)[Q][6]>(w_s);
+    KT(*fC_s)[Q * NCC] = reinterpret_cast<KT(*)[Q * NCC]>(w_s + EPW * Q * 6);
     // assembled passes: blocks staged for word-by-word stores, and their positions (and those
     // of their transposes, -1: none)
     constexpr int kStage = 32;
@@ -124,29 +139,38 @@ __global__ __launch_bounds__(64) void element_kernel(int E, int N, const double*
         return (specActive && !specActive[specOfElem[e]]) ? -1 : e;
     };
 
-    for (int t = lane; t < EPW * Q; t += 64) {
-        const int el = t / Q, q = t - (t / Q) * Q;
-        const int e = elem(el);
-        if (e < 0) continue;
-        const double* dn = dNdxi + (size_t)q * NN * 3;
+    // Every node of an element is read once, not once per QP.
+    const int nel = lane / NN, na = lane - (lane / NN) * NN;
+    const bool hasNode = lane < EPW * NN && elem(nel) >= 0;
+    double un[3] = {0, 0, 0};
+    if (hasNode) {
+        const int nd = conn[(int64_t)na * E + elem(nel)];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            g_s[nel][na * 3 + c] = coords[(int64_t)c * N + nd];
+            un[c] = dU[3 * (int64_t)nd + c];
+        }
+    }
+    __syncthreads();
+    const int qel = lane / Q, q = lane - (lane / Q) * Q;
+    const int e = lane < EPW * Q ? elem(qel) : -1;
+    double det = 0.0;
+    if (e >= 0) {
         const double* dj = dJdxi + (size_t)q * NN * 3;
         double J[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll 4
         for (int a = 0; a < NN; ++a) {
-            const int nd = conn[(int64_t)a * E + e];
-            const double x = coords[nd], y = coords[N + nd], z = coords[2 * N + nd];
 #pragma unroll
             for (int r = 0; r < 3; ++r) {
                 const double d = dj[a * 3 + r];
-                J[r * 3 + 0] += d * x;
-                J[r * 3 + 1] += d * y;
-                J[r * 3 + 2] += d * z;
+#pragma unroll
+                for (int c = 0; c < 3; ++c) J[r * 3 + c] += d * g_s[qel][a * 3 + c];
             }
         }
-        const double det = J[0] * (J[4] * J[8] - J[5] * J[7]) - J[1] * (J[3] * J[8] - J[5] * J[6]) +
-                           J[2] * (J[3] * J[7] - J[4] * J[6]);
+        det = J[0] * (J[4] * J[8] - J[5] * J[7]) - J[1] * (J[3] * J[8] - J[5] * J[6]) +
+              J[2] * (J[3] * J[7] - J[4] * J[6]);
         const double id = 1.0 / det;
-        double iJ[9];
+        double* iJ = iJ_s[qel][q];
         iJ[0] = (J[4] * J[8] - J[5] * J[7]) * id;
         iJ[1] = (J[2] * J[7] - J[1] * J[8]) * id;
         iJ[2] = (J[1] * J[5] - J[2] * J[4]) * id;
@@ -156,25 +180,33 @@ __global__ __launch_bounds__(64) void element_kernel(int E, int N, const double*
         iJ[6] = (J[3] * J[7] - J[4] * J[6]) * id;
         iJ[7] = (J[1] * J[6] - J[0] * J[7]) * id;
         iJ[8] = (J[0] * J[4] - J[1] * J[3]) * id;
-        double gr[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};  // gr[i*3+j] = d u_i / d x_j
+    }
+    __syncthreads();
+    for (int t = lane; t < EPW * Q * NN; t += 64) {  // the gradients over all lanes
+        const int el = t / (Q * NN), r = t - el * Q * NN;
+        if (elem(el) < 0) continue;
+        const double d0 = dNdxi[r * 3 + 0], d1 = dNdxi[r * 3 + 1], d2 = dNdxi[r * 3 + 2];
+        const double* iJ = iJ_s[el][r / NN];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) g_s[el][r * 3 + c] = iJ[c * 3 + 0] * d0 + iJ[c * 3 + 1] * d1 + iJ[c * 3 + 2] * d2;
+    }
+    __syncthreads();
+    if (hasNode) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) u_s[nel][na][c] = un[c];
+    }
+    __syncthreads();
+    double gr[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};  // gr[i*3+j] = d u_i / d x_j
+    if (e >= 0) {
 #pragma unroll 4
-        for (int a = 0; a < NN; ++a) {
-            const double d0 = dn[a * 3 + 0], d1 = dn[a * 3 + 1], d2 = dn[a * 3 + 2];
-            double g[3];
+        for (int a = 0; a < NN; ++a)
 #pragma unroll
-            for (int c = 0; c < 3; ++c) g[c] = iJ[c * 3 + 0] * d0 + iJ[c * 3 + 1] * d1 + iJ[c * 3 + 2] * d2;
-            g_s[el][(q * NN + a) * 3 + 0] = g[0];
-            g_s[el][(q * NN + a) * 3 + 1] = g[1];
-            g_s[el][(q * NN + a) * 3 + 2] = g[2];
-            const int nd = conn[(int64_t)a * E + e];
-            const double u0 = dU[3 * nd], u1 = dU[3 * nd + 1], u2 = dU[3 * nd + 2];
+            for (int i = 0; i < 3; ++i)
 #pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                gr[0 + j] += u0 * g[j];
-                gr[3 + j] += u1 * g[j];
-                gr[6 + j] += u2 * g[j];
-            }
-        }
+                for (int j = 0; j < 3; ++j) gr[i * 3 + j] += u_s[qel][a][i] * g_s[qel][(q * NN + a) * 3 + j];
+    }
+    __syncthreads();
+    if (e >= 0) {
         double de[6] = {gr[0], gr[4], gr[8], gr[1] + gr[3], gr[2] + gr[6], gr[5] + gr[7]};
         const int64_t sidx = (int64_t)e * Q + q;
         double s[6], ms = 0.0;
@@ -203,15 +235,15 @@ __global__ __launch_bounds__(64) void element_kernel(int E, int N, const double*
         (void)NS;
         const double f = det * qpw[q];
         if (formK) {
-            fC_s[el][q * NCC + 0] = (KT)(f * (cc[0] - cc[1] * (1.0 / 3.0)));
-            fC_s[el][q * NCC + 1] = (KT)(f * (0.5 * cc[1]));
+            fC_s[qel][q * NCC + 0] = (KT)(f * (cc[0] - cc[1] * (1.0 / 3.0)));
+            fC_s[qel][q * NCC + 1] = (KT)(f * (0.5 * cc[1]));
 #pragma unroll
-            for (int k = 2; k < NCC - 6; ++k) fC_s[el][q * NCC + k] = (KT)(f * cc[k]);
+            for (int k = 2; k < NCC - 6; ++k) fC_s[qel][q * NCC + k] = (KT)(f * cc[k]);
 #pragma unroll
-            for (int k = 0; k < 6; ++k) fC_s[el][q * NCC + NCC - 6 + k] = (KT)cc[5 + k];
+            for (int k = 0; k < 6; ++k) fC_s[qel][q * NCC + NCC - 6 + k] = (KT)cc[5 + k];
         }
 #pragma unroll
-        for (int k = 0; k < 6; ++k) fs_s[el][q][k] = f * s[k];
+        for (int k = 0; k < 6; ++k) fs_s[qel][q][k] = f * s[k];
     }
     __syncthreads();
 
