@@ -1,7 +1,7 @@
 // Element, material and assembly kernels for gfx950.
 //
 // hex8_kernel (hexa8) is described at its definition; element_kernel (hexa20) follows the same
-// three phases, one 64-lane wavefront owning EPW elements.
+// three phases, one or two 64-lane wavefronts owning EPW elements.
 //   phase 1: the nodes' coordinates and increments to LDS, one lane per (element, node); one
 //            lane per (element, QP): Jacobian from the coordinates and the shape-function
 //            derivatives at the reference's evaluation point; dN/dx over all lanes; one lane
@@ -86,8 +86,10 @@ __device__ __forceinline__ void store_compact(CT* __restrict__ mfC, const int32_
 // FP64 tangent passes 147 -> 139 us and 263 -> 255 us.  Coordinates, inverse Jacobians and
 // increments lie where the gradients and the weighted stresses follow: in LDS of their own (3 KB
 // more) the hexa20R tangent pass got slower (32^3 DP: 705 -> 770 us; as it is, 698 us).
-template <int NN, int Q, int MAT, typename KT, int EPW, bool MF>
-__global__ __launch_bounds__(64) void element_kernel(int E, int N, const double* __restrict__ coords,
+// W wavefronts per workgroup: the tasks of every phase over all of them, each with its own stage
+// for the block stores.
+template <int NN, int Q, int MAT, typename KT, int EPW, bool MF, int W>
+__global__ __launch_bounds__(64 * W) void element_kernel(int E, int N, const double* __restrict__ coords,
                                                      const int32_t* __restrict__ conn,
                                                      const double* __restrict__ props, int propStride,
                                                      const double* __restrict__ dNdxi,
@@ -122,9 +124,11 @@ __global__ __launch_bounds__(64) void element_kernel(int E, int N, const double*
     // assembled passes: blocks staged for word-by-word stores, and their positions (and those
     // of their transposes, -1: none)
     constexpr int kStage = 32;
-    __shared__ KT stg_s[MF ? 1 : kStage][9];
-    __shared__ int spos_s[MF ? 1 : 2 * kStage];
-    const int lane = threadIdx.x;
+    __shared__ KT stg_w[MF ? 1 : W][MF ? 1 : kStage][9];
+    __shared__ int spos_w[MF ? 1 : W][MF ? 1 : 2 * kStage];
+    const int tid = threadIdx.x, lane = tid & 63, wave = W > 1 ? tid >> 6 : 0;
+    KT(*stg_s)[9] = stg_w[MF ? 0 : wave];
+    int* spos_s = spos_w[MF ? 0 : wave];
     const int64_t EQ = (int64_t)E * Q;
     // Grid-stride over the element list: a grid smaller than the list (a persistent launch)
     // takes EPW elements per workgroup and round.
@@ -140,8 +144,8 @@ __global__ __launch_bounds__(64) void element_kernel(int E, int N, const double*
     };
 
     // Every node of an element is read once, not once per QP.
-    const int nel = lane / NN, na = lane - (lane / NN) * NN;
-    const bool hasNode = lane < EPW * NN && elem(nel) >= 0;
+    const int nel = tid / NN, na = tid - (tid / NN) * NN;
+    const bool hasNode = tid < EPW * NN && elem(nel) >= 0;
     double un[3] = {0, 0, 0};
     if (hasNode) {
         const int nd = conn[(int64_t)na * E + elem(nel)];
@@ -152,8 +156,8 @@ __global__ __launch_bounds__(64) void element_kernel(int E, int N, const double*
         }
     }
     __syncthreads();
-    const int qel = lane / Q, q = lane - (lane / Q) * Q;
-    const int e = lane < EPW * Q ? elem(qel) : -1;
+    const int qel = tid / Q, q = tid - (tid / Q) * Q;
+    const int e = tid < EPW * Q ? elem(qel) : -1;
     double det = 0.0;
     if (e >= 0) {
         const double* dj = dJdxi + (size_t)q * NN * 3;
@@ -182,7 +186,7 @@ __global__ __launch_bounds__(64) void element_kernel(int E, int N, const double*
         iJ[8] = (J[0] * J[4] - J[1] * J[3]) * id;
     }
     __syncthreads();
-    for (int t = lane; t < EPW * Q * NN; t += 64) {  // the gradients over all lanes
+    for (int t = tid; t < EPW * Q * NN; t += 64 * W) {  // the gradients over all lanes
         const int el = t / (Q * NN), r = t - el * Q * NN;
         if (elem(el) < 0) continue;
         const double d0 = dNdxi[r * 3 + 0], d1 = dNdxi[r * 3 + 1], d2 = dNdxi[r * 3 + 2];
@@ -257,7 +261,7 @@ __global__ __launch_bounds__(64) void element_kernel(int E, int N, const double*
     // the wavefront then stores consecutive words, about seven 72-byte blocks per store
     // instruction instead of one scattered block per lane (48^3 hexa20R DP: 2.34 -> 2.27 ms).
     const int ntask = formK ? EPW * NB : 0;
-    for (int t0 = 0; t0 < ntask; t0 += 64) {
+    for (int t0 = 64 * wave; t0 < ntask; t0 += 64 * W) {
         const int t = t0 + lane;
         const int el = t / NB, r0 = t - (t / NB) * NB;
         int a = 0, b = 0;
@@ -348,7 +352,7 @@ __global__ __launch_bounds__(64) void element_kernel(int E, int N, const double*
         }
     }
 
-    for (int t = lane; t < EPW * NN; t += 64) {
+    for (int t = tid; t < EPW * NN; t += 64 * W) {
         const int el = t / NN, a = t - (t / NN) * NN;
         const int e = elem(el);
         if (e < 0) continue;
@@ -1214,16 +1218,24 @@ void launch_elem_t(efe_ctx* c, const double* dU) {
     if (cap > 0 && grid > cap) grid = cap;  // persistent: the workgroups loop over the list
     const int propStride = c->props_per_element ? c->E : 0;
     const int* act = c->useActive ? c->specActive : nullptr;
+    auto launch = [&](auto kern, int threads, auto* K, float* mfC) {
+        kern<<<grid, threads, 0, c->stream>>>(c->E, c->N, c->coords, c->conn, c->props, propStride, c->dNdxi, c->dJdxi,
+                                              c->qpw, dU, c->stateRef, c->stateTmp, K, c->Pscr, c->status, mfC,
+                                              c->specStatus, c->specOfElem, c->cpos, act, c->formK, c->curList,
+                                              c->curCount, c->mfNC);
+    };
+    // Two wavefronts per workgroup where 27 QPs' blocks are formed: the LDS of 27 QPs leaves eight
+    // workgroups per CU, too few wavefronts to hide the LDS reads of the blocks (17x15x13 hexa20 J2:
+    // 139 -> 122 us in FP64, 118 -> 107 us in FP32; 27 elements: 49 -> 31 us; 32^3: 1074 -> 1026 us).
+    // With 8 QPs a second wavefront only took registers and stage space (32^3 hexa20R DP: 698 ->
+    // 722 us), and passes without blocks leave it idle (residual of 17x15x13: 37 -> 42 us).
+    constexpr int W = Q > 8 ? 2 : 1;
     if (c->mfPass)
-        element_kernel<NN, Q, MAT, float, EPW, true><<<grid, 64, 0, c->stream>>>(
-            c->E, c->N, c->coords, c->conn, c->props, propStride, c->dNdxi, c->dJdxi, c->qpw, dU, c->stateRef, c->stateTmp,
-            (float*)c->Kscr, c->Pscr, c->status, c->mfC, c->specStatus, c->specOfElem, c->cpos, act, c->formK,
-            c->curList, c->curCount, c->mfNC);
+        launch(element_kernel<NN, Q, MAT, float, EPW, true, 1>, 64, (float*)c->Kscr, c->mfC);
+    else if (c->formK)
+        launch(element_kernel<NN, Q, MAT, KT, EPW, false, W>, 64 * W, (KT*)c->Kscr, (float*)nullptr);
     else
-        element_kernel<NN, Q, MAT, KT, EPW, false><<<grid, 64, 0, c->stream>>>(
-            c->E, c->N, c->coords, c->conn, c->props, propStride, c->dNdxi, c->dJdxi, c->qpw, dU, c->stateRef, c->stateTmp,
-            (KT*)c->Kscr, c->Pscr, c->status, nullptr, c->specStatus, c->specOfElem, c->cpos, act, c->formK,
-            c->curList, c->curCount, c->mfNC);
+        launch(element_kernel<NN, Q, MAT, KT, EPW, false, 1>, 64, (KT*)c->Kscr, (float*)nullptr);
 }
 
 template <int NN, int Q, int MAT, typename KT>
