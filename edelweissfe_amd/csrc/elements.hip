@@ -1,7 +1,7 @@
 // Element, material and assembly kernels for gfx950.
 //
 // hex8_kernel (hexa8) is described at its definition; element_kernel (hexa20) follows the same
-// three phases, one or two 64-lane wavefronts owning EPW elements.
+// three phases, one, two or four 64-lane wavefronts owning EPW elements.
 //   phase 1: the nodes' coordinates and increments to LDS, one lane per (element, node); one
 //            lane per (element, QP): Jacobian from the coordinates and the shape-function
 //            derivatives at the reference's evaluation point; dN/dx over all lanes; one lane
@@ -1229,9 +1229,15 @@ void launch_elem_t(efe_ctx* c, const double* dU) {
     // 139 -> 122 us in FP64, 118 -> 107 us in FP32; 27 elements: 49 -> 31 us; 32^3: 1074 -> 1026 us).
     // With 8 QPs a second wavefront only took registers and stage space (32^3 hexa20R DP: 698 ->
     // 722 us), and passes without blocks leave it idle (residual of 17x15x13: 37 -> 42 us).
+    // Up to three workgroups per CU the chip has wavefronts to spare, and four share an element's
+    // blocks: 8^3 hexa20 J2 45 -> 33 us, 9^3 (729 workgroups) 46 -> 38 us, but 10^3 (1000) 47 -> 52;
+    // hexa20R DP 9^3 67 -> 36 us, 11^3 (666) 68 -> 41, 12^3 (864) 70 -> 59, 16^3 (2048) 100 -> 105.
+    constexpr int kSmallGrid = 3 * 256;
     constexpr int W = Q > 8 ? 2 : 1;
     if (c->mfPass)
         launch(element_kernel<NN, Q, MAT, float, EPW, true, 1>, 64, (float*)c->Kscr, c->mfC);
+    else if (c->formK && grid <= kSmallGrid)
+        launch(element_kernel<NN, Q, MAT, KT, EPW, false, 4>, 256, (KT*)c->Kscr, (float*)nullptr);
     else if (c->formK)
         launch(element_kernel<NN, Q, MAT, KT, EPW, false, W>, 64 * W, (KT*)c->Kscr, (float*)nullptr);
     else
