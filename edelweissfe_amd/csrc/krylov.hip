@@ -49,7 +49,7 @@ struct KrylovWork {
     double *x64 = nullptr, *r64 = nullptr, *z64 = nullptr, *p64 = nullptr, *q64 = nullptr;
     float *x32 = nullptr, *r32 = nullptr, *z32 = nullptr, *p32 = nullptr, *q32 = nullptr;
     double* part = nullptr;  // [6][ps]: pq, rz0, rz1, rr, bb, p.p over the Dirichlet DOFs
-    int* flags = nullptr;    // device: [done, nan, iters_local, done of odd iterations (bricks)]
+    int* flags = nullptr;    // device: [done, nan, iters_local, done of odd iterations]
     double* dscal = nullptr; // device: [tol2, scratch sum, alpha (bricks)]
     int* hflags = nullptr;   // pinned host copy
     double* hpart = nullptr; // pinned host scalars
@@ -228,7 +228,9 @@ __global__ __launch_bounds__(64 * kSpmvWaves) void spmv_kernel(int N, const int3
 // The iteration of a small assembled system in two launches: the direction (stop test, p = z + beta p)
 // in the product that follows it.  Every gather forms its entry of p, the row's owner stores it, and the
 // two p alternate, as neighbours still gather the old one.  The first blocks of a row are loaded beside
-// the scalars' reduction.  What an update ends with is tested by the next launch of this kernel.  PCG
+// the scalars' reduction.  What an update ends with is tested by the next launch of this kernel, which
+// stores the flag of the update and of the launch after it (doneNext) and reads its own (done): the two
+// alternate, so that the wavefronts of a workgroup agree on it.  PCG
 // iteration in three launches -> two: hexa8 FP64 525 nodes 11.1 -> 9.4 us, 3375 11.7 -> 9.7, 9261 13.3 ->
 // 10.3, 24389 19.0 -> 18.1, 35937 22.4 -> 22.4; FP32 9261 11.1 -> 8.7; hexa20R FP64 2673 19.8 -> 16.0, 26353
 // 36.2 -> 29.1.  (On 64^3 the same fold cost more than the launch: a second gathered vector.)
@@ -237,7 +239,8 @@ __global__ __launch_bounds__(64 * kSpmvWaves) void pcg_fold_kernel(
     int N, const int32_t* __restrict__ slice_off, const int32_t* __restrict__ scol,
     const int32_t* __restrict__ slotNode, const T* __restrict__ K, const T* __restrict__ z, const T* __restrict__ p,
     T* __restrict__ pNew, T* __restrict__ q, double* __restrict__ part, int ps, int nvec, int par, int jlocal,
-    const double* __restrict__ dtol2, int* __restrict__ flags) {
+    const double* __restrict__ dtol2, const int* __restrict__ done, int* __restrict__ doneNext,
+    int* __restrict__ flags) {
     constexpr int W = kSpmvWaves, U = 4;
     __shared__ T sh[W - 1][3][64];
     __shared__ double sd[3 * W];
@@ -271,20 +274,25 @@ __global__ __launch_bounds__(64 * kSpmvWaves) void pcg_fold_kernel(
             }
     };
     if (n >= 0) load(k0);
-    if (flags[0]) return;
+    const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+    if (*done) {
+        if (first) *doneNext = 1;
+        return;
+    }
     const int offs[3] = {(1 + par) * ps, (2 - par) * ps, 3 * ps};
     double sc[3];
     reduce_partials_n<64 * W, 3>(part, offs, nvec, sc, sd);
     const double rz = sc[0], rzo = sc[1], rr = sc[2];
     const bool bad = !(rr == rr) || !(rz == rz);
-    if (bad || rr <= dtol2[0]) {  // the last iteration's result
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
+    const bool stop = bad || rr <= dtol2[0];  // the last iteration's result
+    if (first) {
+        if (stop) {
             flags[2] = jlocal;
             flags[1] = bad ? 1 : 0;
-            flags[0] = 1;
         }
-        return;
+        *doneNext = stop ? 1 : 0;
     }
+    if (stop) return;
     const T beta = (T)(rz / rzo);
     T y0 = 0, y1 = 0, y2 = 0;
     if (n >= 0)
@@ -629,9 +637,10 @@ void launch_iter(efe_ctx* c, KrylovWork* w, hipStream_t st, T* x, T* r, T* z, T*
         T *pa = p, *pb = (T*)w->pb;
         T *pOld = par ? pb : pa, *pNew = par ? pa : pb;
         pcg_fold_kernel<T><<<nop, 64 * kSpmvWaves, 0, st>>>(c->N, c->slice_off, c->scol, c->slotNode, K, z, pOld, pNew, q,
-                                                            w->part, w->ps, gv, par, j, w->dscal, w->flags);
+                                                            w->part, w->ps, gv, par, j, w->dscal, done, doneNext,
+                                                            w->flags);
         pcg_update_kernel<T, BS, false, true><<<gv, BS, 0, st>>>(c->N, Minv, r, z, pNew, nullptr, q, nullptr, w->part,
-                                                                 w->ps, nop, gv, par, w->flags, w->dscal + 2, krv, x);
+                                                                 w->ps, nop, gv, par, doneNext, w->dscal + 2, krv, x);
         return;
     }
     if (K) {
