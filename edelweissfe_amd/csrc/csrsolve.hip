@@ -108,9 +108,9 @@ __global__ __launch_bounds__(kBS) void csr_dot_kernel(int n, const double* __res
     if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
-// CG, three kernels per iteration.  Scalars sc: [0] and [6] r.z of the even and the odd iterations (a
-// kernel that stores the next one still reads the last), [2] r.r, [3] tol^2, [4] done flag (as
-// double), [5] iterations.
+// CG, three kernels per iteration.  Scalars sc: [0] and [6] r.z, [4] and [7] done flags (as doubles) of
+// the even and the odd iterations (a kernel that stores the next one still reads the last), [2] r.r,
+// [3] tol^2, [5] iterations.
 //
 // An iteration of a mid-sized system is a chain of launches: product, dot, update, preconditioner,
 // direction and scalars as kernels of their own took 25 us at 26775 rows and 2 M entries, the product
@@ -126,12 +126,12 @@ __global__ __launch_bounds__(kBS) void cg_spmv_kernel(int n, const int32_t* __re
                                                       const int32_t* __restrict__ ix, const double* __restrict__ v,
                                                       const uint8_t* __restrict__ fixed, const double* __restrict__ p,
                                                       double* __restrict__ q, double* __restrict__ part,
-                                                      const double* __restrict__ sc) {
+                                                      const double* __restrict__ done) {
     constexpr int kStep = 6, R = kBS / kLanesPerRow;
     __shared__ double sh[kBS / 64];
     const int l = threadIdx.x & (kLanesPerRow - 1);
     double dot = 0.0;
-    if (sc[4] != 0.0) return;
+    if (*done != 0.0) return;
     for (int row = blockIdx.x * R + threadIdx.x / kLanesPerRow; row < n; row += gridDim.x * R) {
         const int a = ip[row], e = fixed[row] ? a : ip[row + 1];
         const double pr = p[row];
@@ -170,7 +170,7 @@ __global__ __launch_bounds__(kBS) void cg_update_kernel(int n, const double* __r
                                                         double* __restrict__ p, const double* __restrict__ q,
                                                         const double* __restrict__ pq, int npq,
                                                         double* __restrict__ part, const double* __restrict__ sc,
-                                                        int rz, int first) {
+                                                        int rz, int done, int first) {
     __shared__ double sh[kBS / 64];
     int i = blockIdx.x * kBS + threadIdx.x;
     double d = 0, ri = 0, pi = 0, qi = 0, xi = 0;
@@ -186,7 +186,7 @@ __global__ __launch_bounds__(kBS) void cg_update_kernel(int n, const double* __r
     if (i < n) load();  // beside the sum of the partials
     double alpha = 0.0;
     if (!first) {
-        if (sc[4] != 0.0) return;
+        if (sc[done] != 0.0) return;
         alpha = sc[rz] / sum_partials(pq, npq, sh);
     }
     double rzn = 0.0, rr = 0.0;
@@ -212,11 +212,11 @@ __global__ __launch_bounds__(kBS) void cg_update_kernel(int n, const double* __r
 }
 
 // the stop test, then p = Dinv r + beta p with beta = r.z new / old.  The first workgroup stores the
-// scalars; one that sees its done flag early skips a direction that nothing reads.
+// scalars, the done flag among them, where no workgroup of this launch reads them.
 __global__ __launch_bounds__(kBS) void cg_direction_kernel(int n, const double* __restrict__ dinv,
                                                            const double* __restrict__ r, double* __restrict__ p,
                                                            const double* __restrict__ part, int nwg,
-                                                           double* __restrict__ sc, int rz) {
+                                                           double* __restrict__ sc, int rz, int done) {
     __shared__ double sh[kBS / 64];
     int i = blockIdx.x * kBS + threadIdx.x;
     double zi = 0, pi = 0;
@@ -224,18 +224,22 @@ __global__ __launch_bounds__(kBS) void cg_direction_kernel(int n, const double* 
         zi = dinv[i] * r[i];
         pi = p[i];
     }
-    if (sc[4] != 0.0) return;
+    const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+    if (sc[done] != 0.0) {
+        if (first) sc[11 - done] = 1.0;
+        return;
+    }
     const double rzn = sum_partials(part, nwg, sh);
     const double rr = sum_partials(part + kMaxWG, nwg, sh);
-    const bool done = !(rr > sc[3]);  // converged (or NaN)
+    const bool stop = !(rr > sc[3]);  // converged (or NaN)
     const double beta = rzn / sc[rz];
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (first) {
         sc[6 - rz] = rzn;
         sc[2] = rr;
         sc[5] += 1.0;
-        if (done) sc[4] = 1.0;
+        sc[11 - done] = stop ? 1.0 : 0.0;
     }
-    if (done) return;
+    if (stop) return;
     while (i < n) {
         p[i] = zi + beta * pi;
         i += gridDim.x * kBS;
@@ -731,20 +735,20 @@ int efe_csr_solve_ws(int32_t n, const int32_t* ip, const int32_t* ix, const doub
             // p.q's partials lie where z would (n doubles, a workgroup has kBS / kLanesPerRow rows)
             double *pq = vecs + 2 * (size_t)n, *p = vecs + 3 * (size_t)n, *q = vecs + 4 * (size_t)n;
             const int gq = gs < kMaxSpmvWG ? gs : kMaxSpmvWG;
-            cg_update_kernel<<<nwg, kBS, 0, st>>>(n, dinv, x, r, p, q, pq, gq, part, sc, 0, 1);
+            cg_update_kernel<<<nwg, kBS, 0, st>>>(n, dinv, x, r, p, q, pq, gq, part, sc, 0, 4, 1);
             cg_scalars_kernel<<<1, kBS, 0, st>>>(part, nwg, sc);
-            int rz = 0;
+            int rz = 0, done = 4;  // the places of the next iteration's r.z and done flag
             while (true) {
-                for (int j = 0; j < check; ++j, rz = 6 - rz) {
-                    cg_spmv_kernel<<<gq, kBS, 0, st>>>(n, ip, ix, v, fixed, p, q, pq, sc);
-                    cg_update_kernel<<<nwg, kBS, 0, st>>>(n, dinv, x, r, p, q, pq, gq, part, sc, rz, 0);
-                    cg_direction_kernel<<<nwg, kBS, 0, st>>>(n, dinv, r, p, part, nwg, sc, rz);
+                for (int j = 0; j < check; ++j, rz = 6 - rz, done = 11 - done) {
+                    cg_spmv_kernel<<<gq, kBS, 0, st>>>(n, ip, ix, v, fixed, p, q, pq, sc + done);
+                    cg_update_kernel<<<nwg, kBS, 0, st>>>(n, dinv, x, r, p, q, pq, gq, part, sc, rz, done, 0);
+                    cg_direction_kernel<<<nwg, kBS, 0, st>>>(n, dinv, r, p, part, nwg, sc, rz, done);
                 }
                 EFE_HIP(hipGetLastError());
                 EFE_HIP(hipMemcpyAsync(hs, sc, 16 * sizeof(double), hipMemcpyDeviceToHost, st));
                 EFE_HIP(hipStreamSynchronize(st));
                 it = (int)hs[5];
-                if (hs[4] != 0.0) break;
+                if (hs[done] != 0.0) break;
                 if (it >= maxit) {
                     info->status = EFE_NOT_CONVERGED;
                     break;

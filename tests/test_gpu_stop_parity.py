@@ -39,3 +39,38 @@ def test_folded_pcg_stops_at_the_same_iteration_in_any_batch(el_type, n, precisi
             seen.add(info.iterations % 4)
     sysm.close()
     assert len(seen) >= 3
+
+
+@pytest.mark.parametrize("n", [1, 300, 20000])
+def test_csr_cg_stops_at_the_same_iteration_in_any_batch(n):
+    import ctypes
+
+    import scipy.sparse as sp
+
+    from edelweissfe_amd import _lib
+
+    rng = np.random.default_rng(n)
+    i, j = rng.integers(0, n, 6 * n), rng.integers(0, n, 6 * n)
+    A = sp.coo_matrix((rng.uniform(-1, 1, i.size), (i, j)), shape=(n, n)).tocsr()
+    A = A + A.T
+    A = A - sp.diags(A.diagonal())
+    A = sp.csr_matrix(A + sp.diags(1.05 * np.asarray(abs(A).sum(axis=1)).ravel() + 0.01))
+    A.sort_indices()
+    ip, ix = A.indptr.astype(np.int32), A.indices.astype(np.int32)
+    b = rng.standard_normal(n)
+    seen = set()
+    for rtol in (5e-1, 2e-1, 1e-1, 3e-2, 1e-2, 1e-3, 1e-5, 1e-10):
+        want = None
+        for check_every in (1, 2, 3, 5, 32):
+            x = np.empty(n)
+            o = _lib.SolveOpts(solver=_lib.EFE_SOLVER_CG, max_iter=2000, check_every=check_every, rtol=rtol)
+            info = _lib.SolveInfo()
+            _lib.check(_lib.load().efe_csr_linsolve(n, ip.ctypes.data, ix.ctypes.data, A.data.ctypes.data,
+                                                    b.ctypes.data, x.ctypes.data, ctypes.byref(o),
+                                                    ctypes.byref(info)), "efe_csr_linsolve")
+            assert info.status == 0
+            got = (info.iterations, info.residual, x.tobytes())
+            want = want or got
+            assert got == want
+            seen.add(info.iterations % 2)
+    assert n == 1 or len(seen) == 2
