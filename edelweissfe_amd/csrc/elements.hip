@@ -844,7 +844,9 @@ __global__ __launch_bounds__(256) void assemble_kernel(
 // with nine coalesced 512-byte loads (FP64), stages it in LDS and each lane takes its own block
 // from there, loading the next run meanwhile.  A block is summed by one lane in the order of
 // assemble_kernel, so K and Minv are bitwise the same for every W; P and F are summed by the last
-// wavefront, the correction from the W parts in order.
+// wavefront, the correction from the W parts in order.  The one block of a node outside every element
+// has no contributions (every other block of the pattern has): its K stays zero and its Minv is the
+// identity.
 template <typename KT, int W>
 __global__ __launch_bounds__(64 * W) void assemble_runs_kernel(
     int N, const int32_t* __restrict__ bptr, const int32_t* __restrict__ bcol, const int32_t* __restrict__ coff,
@@ -885,6 +887,7 @@ __global__ __launch_bounds__(64 * W) void assemble_runs_kernel(
         c0 = coff[b] - first;
         c1 = coff[b1] - first;
         if (b < b1) cend = coff[b + 1] - first;
+        haveDiag = b < b1 && c0 == c1;  // a block without contributions: dg as it is
     }
     KT acc[9];
 #pragma unroll
