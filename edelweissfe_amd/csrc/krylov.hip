@@ -50,7 +50,7 @@ struct KrylovWork {
     float *x32 = nullptr, *r32 = nullptr, *z32 = nullptr, *p32 = nullptr, *q32 = nullptr;
     double* part = nullptr;  // [6][ps]: pq, rz0, rz1, rr, bb, p.p over the Dirichlet DOFs
     int* flags = nullptr;    // device: [done, nan, iters_local, done of odd iterations]
-    double* dscal = nullptr; // device: [tol2, scratch sum, alpha (bricks)]
+    double* dscal = nullptr; // device: [tol2, scratch sum, alpha, scratch sum]
     int* hflags = nullptr;   // pinned host copy
     double* hpart = nullptr; // pinned host scalars
     hipStream_t ks = nullptr;
@@ -844,10 +844,19 @@ int pcg_solve(efe_ctx* c, const double* b, double* xout, const efe_solve_opts* o
     // final residual of the recursion
     sum_partials_kernel<<<1, 256, 0, st>>>(w->part + 3 * w->ps, w->nwgv, w->dscal + 1);
     EFE_HIP(hipMemcpyAsync(w->hpart, w->dscal + 1, sizeof(double), hipMemcpyDeviceToHost, st));
+    // a folded iteration's result is tested by the next one: that of the last iteration allowed here, by its
+    // r.r and r.z (the r.z of odd iterations, as a batch ends with one)
+    const bool untested = info->status == EFE_NOT_CONVERGED && K && fold_iteration(c);
+    if (untested) {
+        sum_partials_kernel<<<1, 256, 0, st>>>(w->part + w->ps, w->nwgv, w->dscal + 3);
+        EFE_HIP(hipMemcpyAsync(w->hpart + 1, w->dscal + 3, sizeof(double), hipMemcpyDeviceToHost, st));
+    }
     EFE_HIP(hipStreamSynchronize(st));
     info->residual = sqrt(w->hpart[0]);
-    // a folded iteration's result is tested by the next one
-    if (info->status == EFE_NOT_CONVERGED && w->hpart[0] <= tol2) info->status = EFE_OK;
+    if (untested) {
+        if (!(w->hpart[0] == w->hpart[0]) || !(w->hpart[1] == w->hpart[1])) info->status = EFE_NAN;
+        else if (w->hpart[0] <= tol2) info->status = EFE_OK;
+    }
     info->iterations = it;
     float ms = 0;
     hipEventElapsedTime(&ms, w->t0, w->t1);

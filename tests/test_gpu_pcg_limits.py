@@ -1,0 +1,48 @@
+"""What a PCG solve of a small assembled system (whose iterations test the result of the one before)
+says at its limits: NaN of the very last allowed iteration.
+
+With rtol = 0 and a right-hand side near the smallest FP32 numbers the residual underflows until p.q is
+0: alpha is infinite, the residual NaN.  Which iteration that is depends on the scale of b; with as many
+iterations allowed, in batches of two, the NaN is the last one's."""
+
+import numpy as np
+import pytest
+
+from helpers import device_model
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+DP = [30000.0, 0.2, 30.0, 10.0, 10.0, 0.0]  # elastic here: symmetric, and not taken by the bricks
+
+
+def _system(n, el_type, precision):
+    from edelweissfe_amd.device import DeviceSystem
+
+    pm = device_model(n, (1.0, 1.0, 1.0), el_type, "druckerprager", DP, jitter=0.1, seed=3)
+    sysm = DeviceSystem(pm.coordinates, pm.connectivity, el_type, "druckerprager", np.array(DP))
+    sysm.set_dirichlet(pm.dofsOfNodeSet("gen_bottom"))
+    sysm.compute_elements(sysm.zeros(), sysm.zeros(), sysm.zeros(), precision=precision)
+    return sysm
+
+
+@pytest.mark.parametrize("el_type,n", [("C3D8", (3, 2, 2)), ("C3D20R", (2, 1, 1))])
+def test_nan_of_the_last_allowed_iteration(el_type, n):
+    from edelweissfe_amd import _lib
+
+    sysm = _system(n, el_type, _lib.EFE_FP32)
+    b0 = np.random.default_rng(4).standard_normal(sysm.n_dof)
+    found = 0
+    for e in np.arange(-42.0, -30.0, 0.25):
+        b = torch.as_tensor(b0 * 10.0 ** e, device="cuda")
+        kw = dict(precision=_lib.EFE_FP32, rtol=0.0, check_every=2)
+        info = sysm.linsolve(b, sysm.zeros(), max_iter=2000, **kw)
+        if info.status != _lib.EFE_NAN or info.iterations % 2:
+            continue
+        found += 1
+        last = sysm.linsolve(b, sysm.zeros(), max_iter=info.iterations, **kw)
+        assert last.status == _lib.EFE_NAN and last.iterations == info.iterations
+        if info.iterations > 2:  # not yet
+            assert sysm.linsolve(b, sysm.zeros(), max_iter=info.iterations - 2, **kw).status == _lib.EFE_NOT_CONVERGED
+    sysm.close()
+    assert found
