@@ -284,7 +284,8 @@ __global__ __launch_bounds__(64 * kSpmvWaves) void pcg_fold_kernel(
     reduce_partials_n<64 * W, 3>(part, offs, nvec, sc, sd);
     const double rz = sc[0], rzo = sc[1], rr = sc[2];
     const bool bad = !(rr == rr) || !(rz == rz);
-    const bool stop = bad || rr <= dtol2[0];  // the last iteration's result
+    // the last iteration's result; there is none before the first, whose r.z before is infinite
+    const bool stop = bad || (rr <= dtol2[0] && rzo < INFINITY);
     if (first) {
         if (stop) {
             flags[2] = jlocal;

@@ -1,5 +1,5 @@
 """What a PCG solve of a small assembled system (whose iterations test the result of the one before)
-says at its limits: NaN of the very last allowed iteration.
+says at its limits: NaN of the very last allowed iteration, tolerances whose square overflows.
 
 With rtol = 0 and a right-hand side near the smallest FP32 numbers the residual underflows until p.q is
 0: alpha is infinite, the residual NaN.  Which iteration that is depends on the scale of b; with as many
@@ -46,3 +46,22 @@ def test_nan_of_the_last_allowed_iteration(el_type, n):
             assert sysm.linsolve(b, sysm.zeros(), max_iter=info.iterations - 2, **kw).status == _lib.EFE_NOT_CONVERGED
     sysm.close()
     assert found
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("atol", [1e200, np.inf])
+def test_a_tolerance_whose_square_overflows_stops_after_one_iteration(atol, precision):
+    """Every tolerance above ||b|| ends the solve after its first iteration, also one whose square is
+    not a number that FP64 holds: the same launches as with one that is, so the same bits."""
+    from edelweissfe_amd import _lib
+
+    prec = _lib.EFE_FP64 if precision == "fp64" else _lib.EFE_FP32
+    sysm = _system((3, 2, 2), "C3D8", prec)
+    b = torch.as_tensor(np.random.default_rng(4).standard_normal(sysm.n_dof), device="cuda")
+    x, y = sysm.zeros(), sysm.zeros()
+    want = sysm.linsolve(b, x, precision=prec, rtol=0.0, atol=1e6)
+    got = sysm.linsolve(b, y, precision=prec, rtol=0.0, atol=atol)
+    sysm.close()
+    assert want.status == 0 and want.iterations == 1 and float(x.abs().max()) > 0
+    assert got.status == 0 and got.iterations == 1 and got.residual == want.residual
+    assert torch.equal(x, y)
