@@ -676,6 +676,7 @@ __global__ __launch_bounds__(256) void mf_diag_kernel(
     double dg[9];
 #pragma unroll
     for (int v = 0; v < 9; ++v) dg[v] = acc[v];
+    if (nptr[n] == nptr[n + 1]) dg[0] = dg[4] = dg[8] = 1.0;  // a node outside every element, as in the assembly
     if (ndir) {
         const bool fr[3] = {(bool)dirflag[3 * n], (bool)dirflag[3 * n + 1], (bool)dirflag[3 * n + 2]};
 #pragma unroll

@@ -88,3 +88,19 @@ def test_an_unattached_node_takes_no_part(form, precision, el_type, n, where):
     assert np.isfinite(got).all()
     assert (got[at] == 0.0).all()
     assert rel_err(np.delete(got, at, axis=0).ravel(), want) < tol
+
+
+@pytest.mark.parametrize("form", ["cg", "batched"])
+@pytest.mark.parametrize("el_type,n", [("C3D8", (4, 3, 3)), ("C3D20R", (3, 2, 2))])
+@pytest.mark.parametrize("where", ["first", "inside", "last"])
+def test_an_unattached_node_takes_no_part_matrix_free(form, el_type, n, where):
+    from edelweissfe_amd import _lib
+
+    N = len(_mesh(n, el_type, None)[0])
+    at = {"first": 0, "inside": N // 2, "last": N}[where]
+    args = (_lib.EFE_FP32_MATFREE, _lib.EFE_SOLVER_CG, form == "batched")
+    want = _solve(n, el_type, None, *args)
+    got = _solve(n, el_type, at, *args).reshape(-1, 3)
+    assert np.isfinite(got).all()
+    assert (got[at] == 0.0).all()
+    assert rel_err(np.delete(got, at, axis=0).ravel(), want) < 1e-4
