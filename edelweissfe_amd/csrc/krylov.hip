@@ -35,7 +35,8 @@
 
 struct KrylovWork {
     int D = 0, N = 0, nwg = 0, block = 0;
-    // rows per thread: a workgroup owns kr * block consecutive rows; [0] FP64, [1] FP32
+    int gblock = 0;  // threads per workgroup of the hexa20 matrix-free product's gather
+    // rows per thread: a workgroup owns kr * gblock consecutive rows; [0] FP64, [1] FP32
     int krp[2] = {1, 1}, nwgp[2] = {0, 0};
     int kr = 1;  // of the precision being solved
     // the vector kernels (init, update, direction) on their own, smaller grid: krv rows per
@@ -649,7 +650,7 @@ void launch_iter(efe_ctx* c, KrylovWork* w, hipStream_t st, T* x, T* r, T* z, T*
         spmv_kernel<T><<<nop, 64 * kSpmvWaves, 0, st>>>(c->N, c->slice_off, c->scol, c->slotNode, K, p, q, w->part, done,
                                                         w->krs);
     } else {  // matrix-free FP32 operator of hexa20
-        efe_mf_launch_operator(c, st, (const float*)p, (float*)q, w->part, done, nop, BS, w->kr);
+        efe_mf_launch_operator(c, st, (const float*)p, (float*)q, w->part, done, nop, w->gblock, w->kr);
     }
     pcg_update_kernel<T, BS, false><<<gv, BS, 0, st>>>(c->N, Minv, r, z, p, nullptr, q, nullptr, w->part, w->ps, nop, gv,
                                                        par, done, w->dscal + 2, krv);
@@ -695,10 +696,14 @@ int ensure_work(efe_ctx* c) {
     // 14.2, 274625 76.7 / 63.4 / 59.3 / 63.4.
     if (block <= 0) block = c->N <= 4096 ? 64 : 256;
     if (block != 64 && block != 128 && block != 256 && block != 512) block = 256;
+    // Unless set, the gather of the hexa20 matrix-free product keeps 256 at every size: at 64 a lane stages
+    // four times as many force slots, and the LDS that holds them serves one wavefront.  PCG iteration at 64
+    // / 256: C3D20 81 nodes 66.2 / 60.5 us, 2673 68.6 / 63.7; C3D20R 81 35.2 / 29.8, 2673 41.0 / 36.2.
+    const int gblock = c->kblock > 0 ? block : 256;
     KrylovWork* w = c->kw;
     // the brick operator writes one p.Kp partial per brick into the partials array
     const int need = c->mfb ? round8(c->mfbG) : 0;
-    if (w && w->block == block && w->ps >= need) return EFE_OK;
+    if (w && w->block == block && w->gblock == gblock && w->ps >= need) return EFE_OK;
     if (!w) {
         w = new KrylovWork();
         c->kw = w;
@@ -732,6 +737,7 @@ int ensure_work(efe_ctx* c) {
     }
     if (w->part) hipFree(w->part);
     w->block = block;
+    w->gblock = gblock;
     // bounded workgroup counts: every workgroup re-reduces all partials in a fixed order,
     // so their number must stay bounded at any mesh size.  Measured on MI355X: FP64 is
     // fastest with at most ~2048 workgroups (fewer starve its SpMV of waves), the FP32
@@ -746,8 +752,8 @@ int ensure_work(efe_ctx* c) {
     const int vcap = 512;
     w->ps = 0;
     for (int i = 0; i < 2; ++i) {
-        w->krp[i] = (groups + cap[i] - 1) / cap[i];
-        w->nwgp[i] = round8((c->N + block * w->krp[i] - 1) / (block * w->krp[i]));
+        w->krp[i] = ((c->N + gblock - 1) / gblock + cap[i] - 1) / cap[i];
+        w->nwgp[i] = round8((c->N + gblock * w->krp[i] - 1) / (gblock * w->krp[i]));
         w->krvp[i] = (groups + vcap - 1) / vcap;
         w->nwgvp[i] = round8((c->N + block * w->krvp[i] - 1) / (block * w->krvp[i]));
         w->ps = std::max(w->ps, std::max(w->nwgp[i], w->nwgvp[i]));
