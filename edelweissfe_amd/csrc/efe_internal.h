@@ -247,6 +247,7 @@ struct efe_ctx {
     // compact tangents [row][NC][kBrick] (brick_slot) of the last FP32 matrix-free / FP64 tangent pass
     float *mfC = nullptr, *mfF = nullptr, *dnxi32 = nullptr;
     double* mfC64 = nullptr;
+    bool noBricks64 = false;     // there was no memory for mfC64: the FP64 CG stays on the assembled operator
     // hexa8 bricks (bricks.cpp): BrickPattern's tables on the device, the staged nodes'
     // coordinates, and the partial forces [L][3] in the precision of the product
     bool mfb = false;

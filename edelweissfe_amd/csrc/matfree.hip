@@ -815,11 +815,18 @@ __global__ void brick_moduli_kernel(int E, const double* __restrict__ props, int
     el[n + pos[e]] = (T)(y / (1.0 + nu));
 }
 
-// the tangents, the moduli and the partials of one precision, in one allocation (at *C)
+// the tangents, the moduli and the partials of one precision, in one allocation (at *C); with
+// `optional`, *C stays null when there is no memory for them
 template <typename T>
-int alloc_bricks(efe_ctx* c, T** C, T** el, T** F) {
+int alloc_bricks(efe_ctx* c, T** C, T** el, T** F, bool optional) {
     const size_t n = (size_t)c->mfbG * c->mfbE, nc = n * 8 * (c->mfNC ? c->mfNC : 1);
-    EFE_HIP(hipMalloc((void**)C, (nc + 2 * n + (size_t)c->mfbL * 3) * sizeof(T)));
+    const hipError_t e = hipMalloc((void**)C, (nc + 2 * n + (size_t)c->mfbL * 3) * sizeof(T));
+    if (e != hipSuccess) *C = nullptr;
+    if (optional && e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();  // the next launch's check is not to find it
+        return EFE_OK;
+    }
+    EFE_HIP(e);
     *el = *C + nc;
     *F = *el + 2 * n;
     brick_moduli_kernel<T><<<(c->E + 255) / 256, 256, 0, c->stream>>>(c->E, c->props, c->props_per_element ? c->E : 0,
@@ -866,8 +873,11 @@ int efe_mf_upload_bricks(efe_ctx* c, const BrickPattern& bp, const double* coord
 }
 
 int efe_mf_alloc_bricks(efe_ctx* c, bool fp64) {
-    if (fp64) return c->mfC64 ? EFE_OK : alloc_bricks(c, &c->mfC64, &c->mfbEl64, &c->mfbF64);
-    return c->mfC ? EFE_OK : alloc_bricks(c, &c->mfC, &c->mfbEl, &c->mfbF);
+    if (!fp64) return c->mfC ? EFE_OK : alloc_bricks(c, &c->mfC, &c->mfbEl, &c->mfbF, false);
+    if (c->mfC64 || c->noBricks64) return EFE_OK;
+    const int rc = alloc_bricks(c, &c->mfC64, &c->mfbEl64, &c->mfbF64, true);
+    c->noBricks64 = !c->mfC64;  // asked for once: the passes and captured rounds keep one operator
+    return rc;
 }
 
 bool efe_mf_bricks64(const efe_ctx* c, const uint8_t* which) {
