@@ -34,15 +34,11 @@
 #include "efe_internal.h"
 
 struct KrylovWork {
-    int D = 0, N = 0, nwg = 0, block = 0;
-    int gblock = 0;  // threads per workgroup of the hexa20 matrix-free product's gather
-    // rows per thread: a workgroup owns kr * gblock consecutive rows; [0] FP64, [1] FP32
-    int krp[2] = {1, 1}, nwgp[2] = {0, 0};
-    int kr = 1;  // of the precision being solved
-    // the vector kernels (init, update, direction) on their own, smaller grid: krv rows per
-    // thread, nwgv workgroups; [0] FP64, [1] FP32
-    int krvp[2] = {1, 1}, nwgvp[2] = {0, 0};
-    int krv = 1, nwgv = 0;
+    int D = 0, N = 0;
+    // grids: the vector kernels (init, update, direction) nwgv workgroups of block threads, krv rows each;
+    // the hexa20 matrix-free product's gather nwgg of gblock, krg; the assembled product nwgs of krs slices
+    int block = 0, krv = 1, nwgv = 0;
+    int gblock = 0, krg = 1, nwgg = 0;
     int krs = 1, nwgs = 0;
     double* pb = nullptr;  // second direction vector of the folded iteration
     int ps = 0;  // row stride of the partials array (the largest workgroup count)
@@ -633,7 +629,7 @@ void launch_iter(efe_ctx* c, KrylovWork* w, hipStream_t st, T* x, T* r, T* z, T*
                                                              w->dscal + 2, done, doneNext, w->flags, krv, c->dirflag);
         return;
     }
-    int nop = w->nwg;
+    int nop = w->nwgg;
     if (K && fold_iteration(c)) {
         nop = w->nwgs;
         T *pa = p, *pb = (T*)w->pb;
@@ -650,7 +646,7 @@ void launch_iter(efe_ctx* c, KrylovWork* w, hipStream_t st, T* x, T* r, T* z, T*
         spmv_kernel<T><<<nop, 64 * kSpmvWaves, 0, st>>>(c->N, c->slice_off, c->scol, c->slotNode, K, p, q, w->part, done,
                                                         w->krs);
     } else {  // matrix-free FP32 operator of hexa20
-        efe_mf_launch_operator(c, st, (const float*)p, (float*)q, w->part, done, nop, w->gblock, w->kr);
+        efe_mf_launch_operator(c, st, (const float*)p, (float*)q, w->part, done, nop, w->gblock, w->krg);
     }
     pcg_update_kernel<T, BS, false><<<gv, BS, 0, st>>>(c->N, Minv, r, z, p, nullptr, q, nullptr, w->part, w->ps, nop, gv,
                                                        par, done, w->dscal + 2, krv);
@@ -738,34 +734,22 @@ int ensure_work(efe_ctx* c) {
     if (w->part) hipFree(w->part);
     w->block = block;
     w->gblock = gblock;
-    // bounded workgroup counts: every workgroup re-reduces all partials in a fixed order,
-    // so their number must stay bounded at any mesh size.  Measured on MI355X: FP64 is
-    // fastest with at most ~2048 workgroups (fewer starve its SpMV of waves), the FP32
-    // operators with at most ~1024; uncapped, the reductions dominate at 96^3.
-    const int groups = (c->N + block - 1) / block;
-    const int cap[2] = {2048, 1024};
-    // The vector kernels (init, update, direction) stream less per row than the product and
-    // re-reduce every partial of the previous kernel in every workgroup, so they take at most
-    // 512 workgroups of several rows per thread.  Measured at 64^3 (history Krylov iteration,
-    // FP64 / mixed): the product's grid 125.6 / 48.6 us, at most 512 123.7 / 47.4, 256 123.1 /
-    // 47.4, 128 125.9 / 49.7.
-    const int vcap = 512;
-    w->ps = 0;
-    for (int i = 0; i < 2; ++i) {
-        w->krp[i] = ((c->N + gblock - 1) / gblock + cap[i] - 1) / cap[i];
-        w->nwgp[i] = round8((c->N + gblock * w->krp[i] - 1) / (gblock * w->krp[i]));
-        w->krvp[i] = (groups + vcap - 1) / vcap;
-        w->nwgvp[i] = round8((c->N + block * w->krvp[i] - 1) / (block * w->krvp[i]));
-        w->ps = std::max(w->ps, std::max(w->nwgp[i], w->nwgvp[i]));
-    }
+    // bounded workgroup counts: every workgroup re-reduces all partials in a fixed order, so their number
+    // must stay bounded at any mesh size (uncapped, the reductions dominate at 96^3).  The vector kernels
+    // stream less per row than the product and re-reduce every partial of the previous kernel in every
+    // workgroup, so they take at most 512 workgroups of several rows per thread.  Measured at 64^3 (history
+    // Krylov iteration, FP64 / mixed): the product's grid 125.6 / 48.6 us, at most 512 123.7 / 47.4, 256
+    // 123.1 / 47.4, 128 125.9 / 49.7.  The FP32 operators are fastest with at most ~1024.
+    auto grid = [&](int threads, int cap, int* rows, int* wgs) {
+        *rows = ((c->N + threads - 1) / threads + cap - 1) / cap;
+        *wgs = round8((c->N + threads * *rows - 1) / (threads * *rows));
+    };
+    grid(block, 512, &w->krv, &w->nwgv);
+    grid(gblock, 1024, &w->krg, &w->nwgg);
     const int slices = (c->N + kSlice - 1) / kSlice, scap = 2048;
     w->krs = (slices + scap - 1) / scap;
     w->nwgs = round8((slices + w->krs - 1) / w->krs);
-    w->ps = std::max(std::max(w->ps, w->nwgs), need);
-    w->kr = w->krp[0];
-    w->nwg = w->nwgp[0];
-    w->krv = w->krvp[0];
-    w->nwgv = w->nwgvp[0];
+    w->ps = std::max(std::max(w->nwgv, w->nwgg), std::max(w->nwgs, need));
     EFE_HIP(hipMalloc(&w->part, (size_t)6 * w->ps * sizeof(double)));
     return EFE_OK;
 }
@@ -775,10 +759,6 @@ int pcg_solve(efe_ctx* c, const double* b, double* xout, const efe_solve_opts* o
               T* z, T* p, T* q, const T* K, const T* Minv, bool bricks, int gi) {
     KrylovWork* w = c->kw;
     hipStream_t st = w->ks;
-    w->kr = w->krp[sizeof(T) == 4 ? 1 : 0];
-    w->nwg = w->nwgp[sizeof(T) == 4 ? 1 : 0];
-    w->krv = w->krvp[sizeof(T) == 4 ? 1 : 0];
-    w->nwgv = w->nwgvp[sizeof(T) == 4 ? 1 : 0];
     // order after the caller's stream
     EFE_HIP(hipEventRecord(w->evA, c->stream));
     EFE_HIP(hipStreamWaitEvent(st, w->evA, 0));

@@ -580,9 +580,8 @@ __global__ __launch_bounds__(kBrick) void brick_apply_kernel(
     }
 }
 
-// Batched solves: q = K p on the nodes of active specimens and the per-node p.q values
+// Batched solves (hexa20): q = K p on the nodes of active specimens and the per-node p.q values
 // that the per-specimen reductions sum; nodes of frozen specimens are left alone (p.q 0).
-template <bool DIRECT>
 __global__ __launch_bounds__(256) void mf_gather_batched_kernel(int N, const int32_t* __restrict__ nptr,
                                                                 const float* __restrict__ Fe,
                                                                 const float* __restrict__ p,
@@ -590,13 +589,12 @@ __global__ __launch_bounds__(256) void mf_gather_batched_kernel(int N, const int
                                                                 const int32_t* __restrict__ spec,
                                                                 const int* __restrict__ active, float* __restrict__ q,
                                                                 double* __restrict__ npq) {
-    __shared__ float buf[DIRECT ? 1 : kGatherLds];
+    __shared__ float buf[kGatherLds];
     const int n0 = blockIdx.x * 256, n = n0 + threadIdx.x;
     const bool valid = n < N;
     const bool act = valid && active[spec[n]];
     float yv[3];
-    if (DIRECT) gather_direct(n, nptr, Fe, act, yv);
-    else gather_slots<256>(n0, N, nptr, Fe, act, buf, yv);
+    gather_slots<256>(n0, N, nptr, Fe, act, buf, yv);
     if (!valid) return;
     if (!act) {
         npq[n] = 0.0;
@@ -766,13 +764,9 @@ void launch_bricks(efe_ctx* c, hipStream_t st, const TP* p, int mask, const int*
 #undef BRICK_ARGS
 }
 
+// the element forces of the hexa20 product
 template <typename TP>
-void launch_apply(efe_ctx* c, hipStream_t st, const TP* p, int mask, const int* flags,
-                  const int* active = nullptr, double* part = nullptr) {
-    if (c->mfb) {
-        launch_bricks<float, TP>(c, st, p, mask, flags, active, part);
-        return;
-    }
+void launch_apply(efe_ctx* c, hipStream_t st, const TP* p, int mask, const int* flags, const int* active = nullptr) {
     const int grid = round8_mf((c->E + 255) / 256);
     const bool dp = c->mfNC == 10;
     if (c->eltype == EFE_C3D20) {
@@ -784,21 +778,26 @@ void launch_apply(efe_ctx* c, hipStream_t st, const TP* p, int mask, const int* 
     }
 }
 
-// the per-node force list the gather sums: brick partials, or one slot per (element, node)
-inline const int32_t* gather_ptr(const efe_ctx* c) { return c->mfb ? c->mfbPptr : c->nptr; }
-inline const float* gather_forces(const efe_ctx* c) { return c->mfb ? c->mfbF : c->mfF; }
-
 template <int BS>
 void launch_gather_op(efe_ctx* c, hipStream_t st, const float* p, float* q, double* part, const int* flags,
                       int nwg, int kr) {
-    if (c->mfb)
-        mf_gather_kernel<BS, 0, float, float, true><<<nwg, BS, 0, st>>>(c->N, gather_ptr(c), c->nlist,
-                                                                        gather_forces(c), p, c->dirflag, q, part,
-                                                                        flags, kr);
-    else
-        mf_gather_kernel<BS, 0, float, float><<<nwg, BS, 0, st>>>(c->N, gather_ptr(c), c->nlist,
-                                                                  gather_forces(c), p, c->dirflag, q, part,
-                                                                  flags, kr);
+    mf_gather_kernel<BS, 0, float, float><<<nwg, BS, 0, st>>>(c->N, c->nptr, c->nlist, c->mfF, p, c->dirflag, q, part,
+                                                              flags, kr);
+}
+
+// y from FP64 vectors: the product (MODE 0, p masked) or the correction (MODE 1) of mf_gather_kernel
+template <int MODE>
+void launch_fp64_vectors(efe_ctx* c, const double* p, double* y) {
+    const int grid = round8_mf((c->N + 255) / 256), mask = MODE == 0;
+    if (c->mfb) {
+        launch_bricks<float, double>(c, c->stream, p, mask, nullptr, nullptr, nullptr);
+        mf_gather_kernel<256, MODE, double, double, true><<<grid, 256, 0, c->stream>>>(
+            c->N, c->mfbPptr, c->nlist, c->mfbF, p, c->dirflag, y, nullptr, nullptr, 1);
+    } else {
+        launch_apply<double>(c, c->stream, p, mask, nullptr);
+        mf_gather_kernel<256, MODE, double, double><<<grid, 256, 0, c->stream>>>(c->N, c->nptr, c->nlist, c->mfF, p,
+                                                                                 c->dirflag, y, nullptr, nullptr, 1);
+    }
 }
 
 }  // namespace
@@ -933,15 +932,7 @@ int efe_launch_mf_assembly(efe_ctx* c, double* P, double* F, const double* dir_v
                                                            c->useActive ? c->specActive : nullptr, c->specOfNode);
     EFE_HIP(hipGetLastError());
     if (dir_values) {
-        launch_apply<double>(c, c->stream, dir_values, 0, nullptr);
-        if (c->mfb)
-            mf_gather_kernel<256, 1, double, double, true><<<round8_mf(grid), 256, 0, c->stream>>>(
-                c->N, gather_ptr(c), c->nlist, gather_forces(c), dir_values, c->dirflag, dir_correction,
-                nullptr, nullptr, 1);
-        else
-            mf_gather_kernel<256, 1, double, double><<<round8_mf(grid), 256, 0, c->stream>>>(
-                c->N, gather_ptr(c), c->nlist, gather_forces(c), dir_values, c->dirflag, dir_correction,
-                nullptr, nullptr, 1);
+        launch_fp64_vectors<1>(c, dir_values, dir_correction);
         EFE_HIP(hipGetLastError());
     }
     c->Kprec = EFE_FP32_MATFREE;
@@ -949,8 +940,8 @@ int efe_launch_mf_assembly(efe_ctx* c, double* P, double* F, const double* dir_v
     return EFE_OK;
 }
 
-// q = K p (FP32, Dirichlet eliminated) with per-workgroup partials of p.q, for the PCG:
-// nwg workgroups of bs threads, the layout of the assembled SpMV's partials.
+// q = K p (FP32, Dirichlet eliminated) with per-workgroup partials of p.q, for the hexa20 PCG:
+// nwg workgroups of bs threads with kr rows per thread.
 void efe_mf_launch_operator(efe_ctx* c, hipStream_t st, const float* p, float* q, double* part, const int* flags,
                             int nwg, int bs, int kr) {
     launch_apply<float>(c, st, p, 1, flags);
@@ -977,27 +968,17 @@ void efe_mf_launch_apply_partials(efe_ctx* c, hipStream_t st, const double* p, d
 
 // y = K x for FP64 vectors with the matrix-free FP32 operator (Dirichlet eliminated).
 int efe_launch_spmv_mf(efe_ctx* c, const double* x, double* y) {
-    launch_apply<double>(c, c->stream, x, 1, nullptr);
-    if (c->mfb)
-        mf_gather_kernel<256, 0, double, double, true><<<round8_mf((c->N + 255) / 256), 256, 0, c->stream>>>(
-            c->N, gather_ptr(c), c->nlist, gather_forces(c), x, c->dirflag, y, nullptr, nullptr, 1);
-    else
-        mf_gather_kernel<256, 0, double, double><<<round8_mf((c->N + 255) / 256), 256, 0, c->stream>>>(
-            c->N, gather_ptr(c), c->nlist, gather_forces(c), x, c->dirflag, y, nullptr, nullptr, 1);
+    launch_fp64_vectors<0>(c, x, y);
     EFE_HIP(hipGetLastError());
     return EFE_OK;
 }
 
-// Batched PCG: q = K p for the active specimens, per-node p.q into npq.
+// Batched hexa20 PCG: q = K p for the active specimens, per-node p.q into npq.
 void efe_mf_launch_operator_batched(efe_ctx* c, hipStream_t st, const float* p, float* q, double* npq,
                                     const int* active) {
     launch_apply<float>(c, st, p, 1, nullptr, active);
-    if (c->mfb)
-        mf_gather_batched_kernel<true><<<(c->N + 255) / 256, 256, 0, st>>>(
-            c->N, gather_ptr(c), gather_forces(c), p, c->dirflag, c->specOfNode, active, q, npq);
-    else
-        mf_gather_batched_kernel<false><<<(c->N + 255) / 256, 256, 0, st>>>(
-            c->N, gather_ptr(c), gather_forces(c), p, c->dirflag, c->specOfNode, active, q, npq);
+    mf_gather_batched_kernel<<<(c->N + 255) / 256, 256, 0, st>>>(c->N, c->nptr, c->mfF, p, c->dirflag, c->specOfNode,
+                                                                 active, q, npq);
 }
 
 void efe_mf_free(efe_ctx* c) {
