@@ -65,3 +65,34 @@ def test_a_tolerance_whose_square_overflows_stops_after_one_iteration(atol, prec
     assert want.status == 0 and want.iterations == 1 and float(x.abs().max()) > 0
     assert got.status == 0 and got.iterations == 1 and got.residual == want.residual
     assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("el_type,n", [
+    ("C3D8", (1, 1, 1)),
+    ("C3D8", (5, 4, 3)),
+    ("C3D8", (29, 29, 30)),   # 27900 nodes: the most of the folded iteration
+    ("C3D8", (29, 30, 30)),   # 28830
+    ("C3D20R", (3, 2, 2)),
+])
+def test_every_row_of_the_fp32_solve_is_solved(el_type, n):
+    """The FP32 solve by the residual of every row under the FP64 operator.  The recurrence's own is at
+    most rtol ||b||; each iteration may add a rounding of K x to a row, 2^-24 of its |K| |x|, and so does
+    the operator's own rounding.  A row that takes no part is left with its b, of order 1."""
+    import scipy.sparse as sp
+
+    from edelweissfe_amd import _lib
+
+    sysm = _system(n, el_type, _lib.EFE_FP32)
+    b = torch.as_tensor(np.random.default_rng(2).standard_normal(sysm.n_dof), device="cuda")
+    x, y = sysm.zeros(), sysm.zeros()
+    info = sysm.linsolve(b, x, precision=_lib.EFE_FP32, rtol=1e-5)
+    assert info.status == 0
+    sysm.compute_elements(sysm.zeros(), sysm.zeros(), sysm.zeros(), precision=_lib.EFE_FP64)
+    sysm.spmv(x, y)
+    indptr, indices = sysm.csr_pattern()
+    K = sp.csr_matrix((sysm.export_csr_values().cpu().numpy(), indices, indptr))
+    sysm.close()
+    scale = (abs(K) @ abs(x.cpu().numpy())).max()
+    bound = 1e-5 * info.rhs_norm + (info.iterations + 1) * 2.0 ** -24 * scale
+    assert bound < 0.1
+    assert float((y - b).abs().max()) <= bound
