@@ -1221,8 +1221,8 @@ void launch_elem_t(efe_ctx* c, const double* dU) {
     if (cap > 0 && grid > cap) grid = cap;  // persistent: the workgroups loop over the list
     const int propStride = c->props_per_element ? c->E : 0;
     const int* act = c->useActive ? c->specActive : nullptr;
-    auto launch = [&](auto kern, int threads, auto* K, float* mfC) {
-        kern<<<grid, threads, 0, c->stream>>>(c->E, c->N, c->coords, c->conn, c->props, propStride, c->dNdxi, c->dJdxi,
+    auto launch = [&](auto kern, int threads, auto* K, float* mfC, int reserve = 0) {
+        kern<<<grid, threads, reserve, c->stream>>>(c->E, c->N, c->coords, c->conn, c->props, propStride, c->dNdxi, c->dJdxi,
                                               c->qpw, dU, c->stateRef, c->stateTmp, K, c->Pscr, c->status, mfC,
                                               c->specStatus, c->specOfElem, c->cpos, act, c->formK, c->curList,
                                               c->curCount, c->mfNC);
@@ -1237,12 +1237,21 @@ void launch_elem_t(efe_ctx* c, const double* dU) {
     // hexa20R DP 9^3 67 -> 36 us, 11^3 (666) 68 -> 41, 12^3 (864) 70 -> 59, 16^3 (2048) 100 -> 105.
     constexpr int kSmallGrid = 3 * 256;
     constexpr int W = Q > 8 ? 2 : 1;
+    // Large FP64 passes of hexa20R store 400 scattered 72-byte blocks per element from 12 workgroups per CU,
+    // more than the memory merges: 48^3 Drucker-Prager 2110 us while the gradients were formed by the QP
+    // lanes alone, 2530 with them over all lanes, which leaves the stores a larger part of each workgroup's
+    // time.  LDS that nobody uses keeps it to 11: 40^3 1289 -> 1280 us, 44^3 1715 -> 1670, 48^3 2530 -> 2157,
+    // 56^3 4322 -> 3438 (J2 48^3 2693 -> 2667, linear elastic 2713 -> 2673).  36^3 (23328 workgroups) takes
+    // 953 us either way, 32^3 683 with 12 and 701 with 11; in FP32, whose blocks are half as large, 48^3
+    // takes 1597 with 12 and 1694 with 11.
+    constexpr int kReserve = Q == 8 && EPW == 2 && sizeof(KT) == 8 ? 2400 : 0, kLargeGrid = 25000;
     if (c->mfPass)
         launch(element_kernel<NN, Q, MAT, float, EPW, true, 1>, 64, (float*)c->Kscr, c->mfC);
     else if (c->formK && grid <= kSmallGrid)
         launch(element_kernel<NN, Q, MAT, KT, EPW, false, 4>, 256, (KT*)c->Kscr, (float*)nullptr);
     else if (c->formK)
-        launch(element_kernel<NN, Q, MAT, KT, EPW, false, W>, 64 * W, (KT*)c->Kscr, (float*)nullptr);
+        launch(element_kernel<NN, Q, MAT, KT, EPW, false, W>, 64 * W, (KT*)c->Kscr, (float*)nullptr,
+               grid > kLargeGrid ? kReserve : 0);
     else
         launch(element_kernel<NN, Q, MAT, KT, EPW, false, 1>, 64, (KT*)c->Kscr, (float*)nullptr);
 }
