@@ -124,24 +124,27 @@ __device__ __forceinline__ void reduce_partials_n(const double* __restrict__ par
     block_sums<BS, K>(out, sh);
 }
 
-// reduce_partials_n with a count per array; each array's sum is formed in the same order as
-// reduce_partials_n would form it.
+// reduce_partials_n with a count per array and its first loads (start) apart from the rest; each array's
+// sum is formed in the same order as reduce_partials_n would form it.
 template <int BS, int K>
-__device__ __forceinline__ void reduce_partials_nv(const double* __restrict__ part, const int* offs,
-                                                   const int* ns, double (&out)[K], double* sh) {
-    int nmax = 0;
+struct PartialSums {
+    double out[K];
+    __device__ __forceinline__ void start(const double* __restrict__ part, const int* offs, const int* ns) {
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-        out[k] = 0.0;
-        nmax = ns[k] > nmax ? ns[k] : nmax;
+        for (int k = 0; k < K; ++k) out[k] = (int)threadIdx.x < ns[k] ? part[offs[k] + threadIdx.x] : 0.0;
     }
-    for (int i = threadIdx.x; i < nmax; i += BS) {
+    __device__ __forceinline__ void finish(const double* __restrict__ part, const int* offs, const int* ns, double* sh) {
+        int nmax = 0;
 #pragma unroll
-        for (int k = 0; k < K; ++k)
-            if (i < ns[k]) out[k] += part[offs[k] + i];
+        for (int k = 0; k < K; ++k) nmax = ns[k] > nmax ? ns[k] : nmax;
+        for (int i = threadIdx.x + BS; i < nmax; i += BS) {
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+                if (i < ns[k]) out[k] += part[offs[k] + i];
+        }
+        block_sums<BS, K>(out, sh);
     }
-    block_sums<BS, K>(out, sh);
-}
+};
 
 template <int BS>
 __device__ __forceinline__ double reduce_partials(const double* __restrict__ part, int n, double* sh) {
@@ -225,7 +228,9 @@ __global__ __launch_bounds__(64 * kSpmvWaves) void spmv_kernel(int N, const int3
 // The iteration of a small assembled system in two launches: the direction (stop test, p = z + beta p)
 // in the product that follows it.  Every gather forms its entry of p, the row's owner stores it, and the
 // two p alternate, as neighbours still gather the old one.  The first blocks of a row are loaded beside
-// the scalars' reduction.  What an update ends with is tested by the next launch of this kernel, which
+// the scalars' reduction, once the flag has come with the slice's offsets: behind the loads, the idle
+// iterations after the stop read the whole operator (a solve of 2 of 32 iterations at 28^3 FP64 494 us,
+// now 247; the iteration is no slower).  What an update ends with is tested by the next launch of this kernel, which
 // stores the flag of the update and of the launch after it (doneNext) and reads its own (done): the two
 // alternate, so that the wavefronts of a workgroup agree on it.  PCG
 // iteration in three launches -> two: hexa8 FP64 525 nodes 11.1 -> 9.4 us, 3375 11.7 -> 9.7, 9261 13.3 ->
@@ -270,12 +275,12 @@ __global__ __launch_bounds__(64 * kSpmvWaves) void pcg_fold_kernel(
                 }
             }
     };
-    if (n >= 0) load(k0);
     const bool first = blockIdx.x == 0 && threadIdx.x == 0;
     if (*done) {
         if (first) *doneNext = 1;
         return;
     }
+    if (n >= 0) load(k0);
     const int offs[3] = {(1 + par) * ps, (2 - par) * ps, 3 * ps};
     double sc[3];
     reduce_partials_n<64 * W, 3>(part, offs, nvec, sc, sd);
@@ -428,7 +433,10 @@ struct UpdateRow {
 
 // B: alpha = r.z / p.q, r -= alpha q, z = Minv r and their partials; p.q = the operator's partials (nop
 // of them), on the bricks + the Dirichlet p.p partials.  x waits for C, which reads p anyway; alpha
-// goes to *alphaOut.  The first row's loads run beside the scalars' reduction.  PCG iteration on the
+// goes to *alphaOut.  The first row's loads run beside the scalars' reduction, behind its first loads and
+// the flag, which the idle iterations after the stop end at (both kernels: a solve of 2 of 32 iterations
+// on the 90^3 FP64 bricks 862 us with the flag behind the row, now 696; the iteration 177.3 and 176.3 us,
+// FP32 64^3 39.6 and 39.5).  PCG iteration on the
 // bricks with x updated here and the loads behind the reduction -> now (both kernels, and the
 // fixed-pitch brick tables): FP64 20^3 20.4 -> 19.3, 40^3 33.0 -> 30.0, 64^3 62.7 -> 59.0 us, FP32 96^3
 // 118.4 -> 113.3 us.
@@ -444,16 +452,17 @@ __global__ __launch_bounds__(BS) void pcg_update_kernel(
     const int blk = xcd_block();
     int n = blk * kr * BS + threadIdx.x;
     UpdateRow<T, BRICK> row;
-    if (n < N) row.load(n, r, Minv, p, gptr, gF, dirflag);
-    if (*done) return;
     constexpr int NS = BRICK ? 3 : 2;
     const int offs[3] = {0, (1 + par) * ps, 5 * ps};
     const int ns[3] = {nop, nvec, nvec};
-    double sc[NS];
-    reduce_partials_nv<BS, NS>(part, offs, ns, sc, sh);
-    double pq = sc[0];
-    if constexpr (BRICK) pq += sc[2];
-    const double al = sc[1] / pq;
+    PartialSums<BS, NS> sc;
+    sc.start(part, offs, ns);
+    if (*done) return;
+    if (n < N) row.load(n, r, Minv, p, gptr, gF, dirflag);
+    sc.finish(part, offs, ns, sh);
+    double pq = sc.out[0];
+    if constexpr (BRICK) pq += sc.out[NS - 1];
+    const double al = sc.out[1] / pq;
     const T alpha = (T)al;
     if (blk == 0 && threadIdx.x == 0) *alphaOut = al;
     double rzn = 0, rr = 0;
@@ -506,16 +515,17 @@ __global__ __launch_bounds__(BS) void pcg_direction_kernel(
             pv[i] = p[3 * (int64_t)n + i];
         }
     };
-    if (n < N) load();
+    const int offs[3] = {(1 + par) * ps, (2 - par) * ps, 3 * ps}, ns[3] = {nvec, nvec, nvec};
+    PartialSums<BS, 3> sc;
+    sc.start(part, offs, ns);
     if (*done) {
         if (blk == 0 && threadIdx.x == 0) *doneNext = 1;
         return;
     }
+    if (n < N) load();
     const T alpha = (T)*alphaIn;
-    const int offs[3] = {(1 + par) * ps, (2 - par) * ps, 3 * ps};
-    double sc[3];
-    reduce_partials_n<BS, 3>(part, offs, nvec, sc, sh);
-    const double rzo = sc[0], rzn = sc[1], rr = sc[2];
+    sc.finish(part, offs, ns, sh);
+    const double rzo = sc.out[0], rzn = sc.out[1], rr = sc.out[2];
     const bool bad = !(rr == rr) || !(rzn == rzn);
     const bool stop = bad || rr <= dtol2[0];
     if (blk == 0 && threadIdx.x == 0) {
