@@ -20,8 +20,6 @@
 
 namespace {
 
-constexpr int kAbiBS = 256;
-
 // The tangent in compact form, as in the element passes (elements.hip): with C = A 1(x)1 + B Idev +
 // cnn n(x)n + cn1 n(x)1 + c1n 1(x)n, lambda = A - B/3, mu = B/2,
 //   K_ab = sum_q (lambda g_a + cn1 h_a) g_b^T + (c1n g_a + cnn h_a) h_b^T + mu (g_b g_a^T + (g_a . g_b) I),
@@ -32,28 +30,35 @@ constexpr int kAbiBS = 256;
 // elements, one wavefront per two elements and C as a matrix 63.8 us, now 41.1 (49 MB of Ke); the whole
 // call 89 -> 69 us, 13824 hexa8 J2 elements 129 -> 99, 64 hexa20R 79 -> 48.  Held to 128 VGPRs 82 / 111 /
 // 53, 512 threads 89 / 117 / 45, one hexa20R element per 128 threads 77 / 99 / 47.
-template <int NN, int Q, int MAT, int EPW>
-__global__ __launch_bounds__(kAbiBS) void element_abi_kernel(
+//
+// KE: whether the call wants Ke.  Without it a wavefront is enough for the phases that are left, and the
+// LDS of h goes.  Whole call with 256 -> 64 threads: hexa20 12^3 Drucker-Prager 56.0 -> 49.7 us, 24^3 J2
+// 187 -> 142, hexa20R 24^3 134 -> 89.  hexa8 takes 4 elements then in lists of up to 65536 (27000 elements:
+// Drucker-Prager 120.6 -> 113.1, 118.6 with 8; linear elastic 108.9 -> 110.7, 115.0 with 8) and 8 in
+// longer ones (216000 J2 elements 658 -> 625, 661 with 4).
+template <int NN, int Q, int MAT, int EPW, bool KE>
+__global__ __launch_bounds__(KE ? 256 : 64) void element_abi_kernel(
     int cnt, const int32_t* __restrict__ kmap, const int32_t* __restrict__ emap, int E, int N,
     const double* __restrict__ coords, const int32_t* __restrict__ conn, const double* __restrict__ props,
     int propStride, const double* __restrict__ dNdxi, const double* __restrict__ dJdxi,
     const double* __restrict__ qpw, const double* __restrict__ dQ, const double* __restrict__ sRef,
     double* __restrict__ sTmp, int ns, double* __restrict__ Pe, double* __restrict__ Ke, int* __restrict__ status) {
     constexpr int NP = (MAT == EFE_LINEAR_ELASTIC) ? 2 : 6;
-    constexpr int ND = 3 * NN;
+    constexpr int ND = 3 * NN, kBS = KE ? 256 : 64;
     constexpr bool LE = MAT == EFE_LINEAR_ELASTIC;
     static_assert(NN % 2 == 0, "blocks in pairs");
     __shared__ double x_s[EPW][NN][6];                         // coordinates, increment
     __shared__ double iJ_s[EPW][Q][9];
     __shared__ double g_s[EPW][Q][NN][3];
-    __shared__ double h_s[LE ? 1 : EPW][LE ? 1 : Q][LE ? 1 : NN][3];
+    constexpr bool H = KE && !LE;
+    __shared__ double h_s[H ? EPW : 1][H ? Q : 1][H ? NN : 1][3];
     __shared__ double c_s[EPW][Q][5], n_s[LE ? 1 : EPW][LE ? 1 : Q][6];  // w detJ [lambda, mu, cnn, cn1, c1n]; n
     __shared__ double fs_s[EPW][Q][6];
     const int tid = threadIdx.x;
     const int i0 = blockIdx.x * EPW;
     const int ne = cnt - i0 < EPW ? cnt - i0 : EPW;
 
-    for (int t = tid; t < ne * NN; t += kAbiBS) {
+    for (int t = tid; t < ne * NN; t += kBS) {
         const int el = t / NN, a = t - (t / NN) * NN;
         const int nd = conn[(int64_t)a * E + emap[i0 + el]];
         const double* du = dQ + (int64_t)kmap[i0 + el] * ND + 3 * a;
@@ -95,7 +100,7 @@ __global__ __launch_bounds__(kAbiBS) void element_abi_kernel(
     }
     __syncthreads();
 
-    for (int t = tid; t < ne * Q * NN; t += kAbiBS) {
+    for (int t = tid; t < ne * Q * NN; t += kBS) {
         const int el = t / (Q * NN), r = t - el * Q * NN, q = r / NN, a = r - (r / NN) * NN;
         const double* dn = dNdxi + ((size_t)q * NN + a) * 3;
         const double d0 = dn[0], d1 = dn[1], d2 = dn[2];
@@ -155,9 +160,9 @@ __global__ __launch_bounds__(kAbiBS) void element_abi_kernel(
     }
     __syncthreads();
 
-    if (Ke) {
+    if constexpr (KE) {
         if constexpr (!LE) {
-            for (int t = tid; t < ne * Q * NN; t += kAbiBS) {
+            for (int t = tid; t < ne * Q * NN; t += kBS) {
                 const int el = t / (Q * NN), r = t - el * Q * NN, q = r / NN, a = r - (r / NN) * NN;
                 const double* n = n_s[el][q];
                 const double x = g_s[el][q][a][0], y = g_s[el][q][a][1], z = g_s[el][q][a][2];
@@ -168,7 +173,7 @@ __global__ __launch_bounds__(kAbiBS) void element_abi_kernel(
             __syncthreads();
         }
         constexpr int NB2 = NN / 2;
-        for (int t = tid; t < ne * NN * NB2; t += kAbiBS) {
+        for (int t = tid; t < ne * NN * NB2; t += kBS) {
             const int el = t / (NN * NB2), r = t - el * NN * NB2, b0 = r / NN, a = r - (r / NN) * NN;
             double acc[2][9], tr[2] = {0, 0};
 #pragma unroll
@@ -221,7 +226,7 @@ __global__ __launch_bounds__(kAbiBS) void element_abi_kernel(
         }
     }
 
-    for (int t = tid; t < ne * NN; t += kAbiBS) {
+    for (int t = tid; t < ne * NN; t += kBS) {
         const int el = t / NN, a = t - (t / NN) * NN;
         double p0 = 0, p1 = 0, p2 = 0;
         for (int q = 0; q < Q; ++q) {
@@ -242,12 +247,16 @@ template <int NN, int Q, int MAT>
 void launch_abi(efe_ctx* c, int cnt, const int32_t* kmap, const int32_t* emap, const double* dQ, const double* sRef,
                 double* sTmp, double* Pe, double* Ke) {
     constexpr int EPW = (NN == 8) ? 8 : (Q == 8 ? 2 : 1);
-    static_assert(EPW * Q <= kAbiBS, "a thread per (element, QP)");
-    const int grid = (cnt + EPW - 1) / EPW;
-    if (grid == 0) return;
-    element_abi_kernel<NN, Q, MAT, EPW><<<grid, kAbiBS, 0, c->stream>>>(
-        cnt, kmap, emap, c->E, c->N, c->coords, c->conn, c->props, c->props_per_element ? c->E : 0, c->dNdxi,
-        c->dJdxi, c->qpw, dQ, sRef, sTmp, c->nstate, Pe, Ke, c->status);
+    static_assert(EPW * Q <= 64, "a thread per (element, QP)");
+    if (cnt == 0) return;
+    auto launch = [&](auto kernel, int epw, int threads) {
+        kernel<<<(cnt + epw - 1) / epw, threads, 0, c->stream>>>(
+            cnt, kmap, emap, c->E, c->N, c->coords, c->conn, c->props, c->props_per_element ? c->E : 0, c->dNdxi,
+            c->dJdxi, c->qpw, dQ, sRef, sTmp, c->nstate, Pe, Ke, c->status);
+    };
+    if (Ke) launch(element_abi_kernel<NN, Q, MAT, EPW, true>, EPW, 256);
+    else if (NN == 8 && cnt <= 65536) launch(element_abi_kernel<NN, Q, MAT, NN == 8 ? 4 : EPW, false>, 4, 64);
+    else launch(element_abi_kernel<NN, Q, MAT, EPW, false>, EPW, 64);
 }
 
 template <int NN, int Q>
