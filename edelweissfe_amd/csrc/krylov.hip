@@ -15,10 +15,11 @@
 //   B: alpha = rz/pq; r -= alpha q; z = Minv r; partials of r.z, r.r
 //   C: x += alpha p; beta = rz_new/rz; convergence test; p = z + beta p
 // (small assembled systems two: C's test and p in the next A, x in B).
-// Global scalars are never stored by one workgroup for the others: every
+// Global scalars are never stored by one workgroup for the others of its launch: every
 // workgroup re-reduces the (few thousand) partials of the previous kernel in the
 // same fixed order, so all workgroups hold bitwise identical scalars and the
-// whole solve is deterministic.  A runs on the product's grid, B and C on a smaller
+// whole solve is deterministic.  What the first workgroup stores for the next launches (alpha, the stop
+// flags, which alternate with the iteration) no kernel reads that stores it.  A runs on the product's grid, B and C on a smaller
 // grid of their own (their partials re-reduced by every workgroup cost less).  The two
 // r.z partial buffers alternate with the iteration parity, so a batch of an even number
 // of iterations is a fixed sequence of launches that is captured once into a hipGraph
