@@ -102,7 +102,7 @@ def run_history(system, template, step_for, precision, steps, warmup):
 
 
 def spmv_roofline(system, n_launch=50):
-    """Average device duration of the FP64 sliced-ELL SpMV (the dominant kernel of the FP64 PCG)
+    """Average device duration of the FP64 sliced-ELL SpMV (efe_spmv on the assembled operator)
     measured with HIP events on the stream it is launched on."""
     import torch
 
@@ -124,6 +124,20 @@ def spmv_roofline(system, n_launch=50):
     return ms, alg
 
 
+def brick_iteration_roofline(system, ms):
+    """The FP64 PCG iteration of a J2 hexa8 history (the brick product, the update and the direction:
+    three kernels) of `ms` milliseconds against the bytes its kernels read and write once each: per
+    element 7 tangent values at 8 QPs, 8 local node indices and the bulk modulus; per node the
+    coordinates and p of the product, r (read and written), z and the inverse block of the update,
+    x and p (read and written) and z of the direction, and the Dirichlet flags.  The Infinity Cache
+    serves part of them from one iteration to the next."""
+    alg = system.n_elements * (8 * 7 * 8 + 16 + 8) + system.n_nodes * (24 + 24 + 48 + 24 + 72 + 48 + 48 + 24 + 3)
+    return {"kernel": "FP64 PCG iteration on the hexa8 bricks: brick_apply_kernel<7, double, double, 1>, "
+                      "pcg_update_kernel<double, 256, true, false>, pcg_direction_kernel<double, 256, true>",
+            "bound": "hbm", "achieved": alg / (ms * 1e-3) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+            "frac": alg / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, "algorithmic_bytes": alg, "avg_iteration_ms": ms}
+
+
 def csr_model_bytes(system):
     """Bytes of the same product in scalar CSR (8 B value + 4 B column index per nonzero, the
     row pointers, x and y once): the per-unit model of a CSR SpMV, which the 3x3 block layout
@@ -134,9 +148,9 @@ def csr_model_bytes(system):
 def profile_spmv(system, n_launch=20, copy_mb=512):
     """Counter-collection mode: one FP64 element pass and assembly of the operator, then
     n_launch FP64 SpMV launches, n_launch plain device copies of copy_mb MiB (the calibration
-    kernel whose FETCH_SIZE / WRITE_SIZE per launch are known: copy_mb MiB each), then one
-    matrix-free FP32 element pass and a block-Jacobi PCG of n_launch iterations on the
-    matrix-free operator (the mixed form's inner solve)."""
+    kernel whose FETCH_SIZE / WRITE_SIZE per launch are known: copy_mb MiB each), a block-Jacobi
+    PCG of n_launch iterations on the FP64 bricks, then one matrix-free FP32 element pass and
+    such a PCG on the matrix-free operator (the mixed form's inner solve)."""
     import torch
 
     from edelweissfe_amd import _lib
@@ -152,13 +166,14 @@ def profile_spmv(system, n_launch=20, copy_mb=512):
         system.spmv(x, y)
     for _ in range(n_launch):
         b.copy_(a)
+    system.linsolve(x, y, rtol=1e-30, max_iter=n_launch, check_every=n_launch)
     system.compute_elements(dU, P, F, precision=_lib.EFE_FP32_MATFREE)
     system.linsolve(x, y, precision=_lib.EFE_FP32_MATFREE, rtol=1e-30, max_iter=n_launch, check_every=n_launch)
     torch.cuda.synchronize()
     nb = system.nnz // 9
     alg = 8 * system.nnz + 4 * nb + 16 * system.n_dof
-    log("[profile] %d spmv launches (algorithmic %d bytes each), %d copies of %d MiB, %d matrix-free PCG "
-        "iterations" % (n_launch, alg, n_launch, copy_mb, n_launch))
+    log("[profile] %d spmv launches (algorithmic %d bytes each), %d copies of %d MiB, %d FP64 and %d matrix-free "
+        "PCG iterations" % (n_launch, alg, n_launch, copy_mb, n_launch, n_launch))
 
 
 def profile_elements(system, n_pass=3, n_spmv=5):
@@ -313,7 +328,8 @@ def bench_batched(args):
         }
         log("[bench] batched mixed: %.3f s (%.2fx), U rel err %.2e" % (wall32, wall64 / wall32, max(uerr)))
     result["roofline"] = {
-        "kernel": "spmv_kernel<double> (sliced-ELL 3x3 blocks) on the block-diagonal batch operator",
+        "kernel": "spmv_kernel<double> (sliced-ELL 3x3 blocks; efe_spmv) on the block-diagonal batch operator, "
+                  "whose own CG runs on the bricks",
         "bound": "hbm",
         "achieved": spmv_alg / (spmv_ms * 1e-3) / 1e9,
         "peak": HBM_PEAK_GBS,
@@ -491,7 +507,7 @@ def bench_footing(args):
         log("[bench] footing mixed: %.3f s (%.2fx), U rel err %.2e" % (
             wall32, wall64 / wall32, result["mixed"]["error_vs_fp64"]["U_rel_inf"]))
     result["roofline"] = {
-        "kernel": "spmv_kernel<double> (sliced-ELL 3x3 blocks)",
+        "kernel": "spmv_kernel<double> (sliced-ELL 3x3 blocks; efe_spmv, laid out and split as the GMRES product)",
         "bound": "hbm",
         "achieved": spmv_alg / (spmv_ms * 1e-3) / 1e9,
         "peak": HBM_PEAK_GBS,
@@ -679,8 +695,8 @@ def main():
             wall32 / len(t32), result["mixed"]["history_speedup_vs_fp64"], err["U_rel_inf"]))
 
     traffic = load_traffic("spmv_fp64_64cube_traffic.json") if args.n == 64 else None
-    result["roofline"] = {
-        "kernel": "spmv_kernel<double> (sliced-ELL 3x3 blocks)",
+    result["assembled_product"] = {
+        "kernel": "spmv_kernel<double> (sliced-ELL 3x3 blocks; efe_spmv)",
         "bound": "hbm",
         "achieved": spmv_alg / (spmv_ms * 1e-3) / 1e9,
         "peak": HBM_PEAK_GBS,
@@ -692,6 +708,11 @@ def main():
         "csr_model_bytes": csr_model_bytes(system),
         "csr_model_achieved": csr_model_bytes(system) / (spmv_ms * 1e-3) / 1e9,
     }
+    # the CG of more than 24,576 elements runs on the bricks, else on the assembled operator
+    if system.n_elements > 24576:
+        result["roofline"] = brick_iteration_roofline(system, ph64["krylov_iteration"])
+    else:
+        result["roofline"] = result["assembled_product"]
 
     if not args.no_cpu:
         try:

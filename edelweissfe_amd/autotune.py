@@ -15,7 +15,7 @@ import torch
 
 from . import _lib
 
-EPW_CANDIDATES = {"C3D8": (1, 2, 4, 8), "C3D20": (1, 2), "C3D20R": (2,)}
+EPW_CANDIDATES = {"C3D8": (8,), "C3D20": (1, 2), "C3D20R": (2,)}  # hexa8 passes take 8 whatever is set
 KRYLOV_CANDIDATES = (64, 128, 256, 512)
 
 
